@@ -207,3 +207,64 @@ def test_training_gain_on_solver_ringdowns():
         f"trained {after:.3f}; loss {losses[0]:.3e} -> {losses[-1]:.3e}")
     assert np.isfinite(after) and after < before
     assert losses[-1] < 0.5 * losses[0]
+
+
+# Sizes at the edges of the kernels' tiles: one sample, rows that no wide
+# load fits, k ranges split and whole, channels and modes on both sides of a
+# pass (64 channels, 16 and 32 modes), tails on both sides of a chunk of 512.
+EDGES = [
+    dict(L0=8, c=(1, 1, 1), hidden=1, modes=1, batch=1, tail=1),
+    dict(L0=16, c=(3, 5, 7), hidden=9, modes=17, batch=3, tail=511),
+    dict(L0=64, c=(64, 65, 60), hidden=66, modes=16, batch=5, tail=513),
+    dict(L0=72, c=(8, 128, 64), hidden=128, modes=33, batch=70, tail=64),
+    dict(L0=256, c=(64, 128, 128), hidden=64, modes=32, batch=20, tail=1025),
+]
+
+
+@pytest.mark.parametrize("e", EDGES, ids=lambda e: f"L{e['L0']}_c{e['c'][1]}_b{e['batch']}_m{e['modes']}_t{e['tail']}")
+def test_edges_match_oracle(e):
+    """Modes, loss and gradients at the tolerances of this file.  The tails
+    and the gradient of the last bias (the sum of dL/do over the batch) are
+    also formed in float64 from the device's own modes, which takes the
+    products' bfloat16 rounding out: left are float32 roundings of damping
+    and output, 1e-7 times the decay exponent (at most about 30 where the
+    tail still counts), hence 1e-5."""
+    od = X.Dims(L0=e["L0"], c=e["c"], hidden=e["hidden"], modes=e["modes"])
+    dims = ExtrapolatorDims(L0=e["L0"], c1=e["c"][0], c2=e["c"][1], c3=e["c"][2], hidden=e["hidden"], modes=e["modes"],
+                            batch=e["batch"], tail=e["tail"])
+    rng = np.random.default_rng(7)
+    p = {k: v.astype(np.float32).astype(np.float64) for k, v in X.init_params(od, seed=7).items()}
+    x = rng.standard_normal((e["batch"], 2, e["L0"])).astype(np.float32)
+    tgt = 0.3 * rng.standard_normal((e["batch"], 2, e["tail"])).astype(np.float32)
+    ex = Extrapolator(dims, params=pack(p, dims))
+    modes, tails = ex.forward(x)
+    ref, c = X.forward(p, x.astype(np.float64), e["tail"], od, use_bf16=True)
+    assert _rel(modes, c["o"]) < 1e-2
+    loss, g = ex.gradients(x, tgt)
+    gd = unpack(g, dims)
+    # from the device's modes
+    o = modes.astype(np.float64).reshape(e["batch"], e["modes"], 6, 1)
+    n = np.arange(e["tail"])
+    s0, s1 = 1 / (1 + np.exp(-o[:, :, 0])), 1 / (1 + np.exp(-o[:, :, 1]))
+    z = np.exp((-X.A_SCALE * np.logaddexp(0, o[:, :, 0]) + 2j * np.pi * X.F_MAX * s1) * n)
+    a = [o[:, :, 2] + 1j * o[:, :, 3], o[:, :, 4] + 1j * o[:, :, 5]]
+    own = np.stack([(v * z).real.sum(1) for v in a], 1)
+    err_t, own_loss = _rel(tails, own), ((own - tgt) ** 2).mean()
+    r = 2 * (own - tgt) / own.size
+    d = [(r[:, q, None] * z).sum(-1) for q in (0, 1)]
+    w = sum((n * r[:, q, None] * a[q] * z).sum(-1) for q in (0, 1))
+    do = np.stack([-w.real * X.A_SCALE * s0[..., 0], -2 * np.pi * w.imag * X.F_MAX * (s1 * (1 - s1))[..., 0],
+                   d[0].real, -d[0].imag, d[1].real, -d[1].imag], -1)
+    err_b = _rel(gd["b5"], do.sum(0).reshape(-1))
+    say(f"[extrap] edges: tails {err_t:.2e}, loss {abs(loss - own_loss) / own_loss:.2e}, last bias {err_b:.2e}")
+    assert err_t < 1e-5 and abs(loss - own_loss) < 1e-5 * own_loss and err_b < 1e-5
+    # the oracle's tails, and with them its gradients, hold up to a phase of
+    # 2 pi n times the modes' own error: compared where that is small
+    if e["tail"] * _rel(modes, c["o"]) > 0.1:
+        return
+    ref_loss, ref_g = X.loss_and_grads(p, x.astype(np.float64), tgt.astype(np.float64), od, use_bf16=True)
+    assert abs(loss - ref_loss) <= 1e-3 * abs(ref_loss)
+    for k in X.ORDER:
+        err = _rel(gd[k], ref_g[k])
+        say(f"[extrap] edges grad {k}: rel L2 {err:.2e}")
+        assert err < 2e-2, k
