@@ -57,32 +57,44 @@ int pow2ceil(int v) {
     return p;
 }
 
-// Automatic tile choice: 256-lane work-groups, as many lanes along k as the
-// row holds (up to one wave of 64 float4 lanes), and i-chunks sized for
-// about 16384 work-groups (64 per CU on 256 CUs), at least 4 planes deep;
-// 2 planes on planes of more than 64 work-groups (384^2 and up) and on grids
-// that 4 planes would cut into fewer than 1024 work-groups.  Measured with
-// the material table, ms per step: 100^3 ci 1 / 2 / 4 = 0.0198 / 0.0197 /
-// 0.0233; 256^3 ci 2 / 3 / 4 = 0.263 / 0.264 / 0.258; 384x384x256 with
-// every extension ci 2 / 4 = 0.650 / 0.663; 512^3 ci 1 / 2 / 3 / 4 / 8 =
-// 2.040 / 1.950 / 2.002 / 1.961 / 1.985.
+// Automatic tile choice: work-groups of at most 256 lanes, bx along k times
+// by = 256 / bx rows of j, marching ci planes of i.
+//
+// bx: whole rows where a row's lanes fit (64 float4 lanes, 128 scalar ones,
+// whose short segments cost more than idle lanes do), else the row cut into
+// equal parts of at least 32 lanes that leave the fewest lanes idle.  A power
+// of two left lanes idle on most grids: us per step at 100^3 (25 lanes)
+// 32 / 25 lanes 13.9 / 11.9; 128x192x320 (80 lanes) 64 / 40 lanes 120 / 94;
+// 256x320x384 (96 lanes) 64 / 32 lanes 466 / 426, with CPML 568 / 497; scalar
+// 200x201x75 64 / 75 lanes 84.6 / 64.3.
+//
+// ci: one plane up to 12 M cells, where more work-groups and a shorter chain
+// of loads count (with CPML, ci 1 / 2 / 4: 72x60x32 20.2 / 26.8 / 39.8,
+// 100^3 29.5 / 35.7 / 51, 160x144x120 62.4 / 65.8 / 73.5, 200x180x232 136 /
+// 142 / 141); above, two planes, which reload half as many i +- 1 planes
+// (256^3 249 / 239 / 239; plain 192 / 191 / 197; 512^3 2040 / 1950 / 1961),
+// four where the row is cut into narrow blocks (256x320x384 511 / 511 / 497).
+// Scalar lanes, whose planes are cheaper than their start, take two
+// (151x133x117 with CPML, ci 1 / 2 / 3: 82.5 / 75.0 / 81.0).
 Tiles auto_tiles(const Grid& g, int vec_req) {
     Tiles t{};
     t.vec = (vec_req == 1) ? 1 : ((g.nz % 4 == 0) ? 4 : 1);
     if (vec_req == 4 && g.nz % 4 != 0) t.vec = 1;
     const int nzv = (g.nz + t.vec - 1) / t.vec;
-    t.bx = std::min(64, pow2ceil(std::max(nzv, 1)));
+    const int widest = t.vec == 4 ? 64 : 128;
+    double best = 0.0;
+    for (int n_kb = (nzv + widest - 1) / widest; n_kb <= nzv; ++n_kb) {
+        const int bx = (nzv + n_kb - 1) / n_kb;
+        if (best > 0.0 && (best >= 0.95 || bx < 32)) break;
+        const double busy = (double)nzv * (256 / bx) / (256.0 * n_kb);
+        if (busy > best) {
+            best = busy;
+            t.bx = bx;
+        }
+    }
     t.by = 256 / t.bx;
-    const int n_kb = (nzv + t.bx - 1) / t.bx;
-    const int n_jb = (g.ny + t.by - 1) / t.by;
-    const long plane_blocks = (long)n_kb * n_jb;
-    long n_ib = (16384 + plane_blocks - 1) / plane_blocks;
-    n_ib = std::max(1L, std::min(n_ib, (long)g.nx));
-    int ci = (int)((g.nx + n_ib - 1) / n_ib);
-    ci = std::max(ci, std::min(4, g.nx));
-    const long wg_at_4 = plane_blocks * ((g.nx + 3) / 4);
-    if (plane_blocks > 64 || wg_at_4 < 1024) ci = std::min(2, g.nx);
-    t.ci = ci;
+    const int ci4 = g.N <= 12000000 ? 1 : (t.bx <= 32 && nzv > 64) ? 4 : 2;
+    t.ci = std::min(g.nx, t.vec == 4 ? ci4 : 2);
     return t;
 }
 
@@ -690,6 +702,7 @@ oe_status oe_engine_set_tiles(oe_engine* e, int bx, int by, int ci, int vec) {
         t.by = 256 / bx;
     }
     if (by > 0) {
+        if (bx <= 0) t.bx = std::min(64, pow2ceil((e->g.nz + t.vec - 1) / t.vec));
         if (by * t.bx != 256) return fail(OE_ERR_CONFIG, "bx * by must equal 256");
         t.by = by;
     }

@@ -44,8 +44,8 @@ struct Grid {
 // or i-1 (E update) plane of the marched components in registers.
 struct Tiles {
     int vec;  // 4: float4 accesses (nz % 4 == 0), 1: scalar
-    int bx;   // lanes along k (power of two)
-    int by;   // rows along j; bx * by == 256
+    int bx;   // lanes along k
+    int by;   // rows along j; bx * by <= 256
     int ci;   // planes along i per work-group
 };
 

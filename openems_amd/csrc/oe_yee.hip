@@ -14,7 +14,7 @@
 //
 // Work decomposition (CDNA4, wave64): a 256-thread work-group covers bx lanes
 // along k (each lane owns V = 4 consecutive k through 16-byte accesses, or
-// V = 1) times by rows along j, and marches along i over ci planes.  The
+// V = 1) times by = 256 / bx rows along j, and marches along i over ci planes.  The
 // marched components (Ey, Ez for H; Hy, Hz for E) are carried in registers
 // from one plane to the next, so each field element is fetched from HBM once
 // per half-step; the j +- 1 and k +- 1 neighbours are re-reads that hit L1/L2.
@@ -233,14 +233,15 @@ __device__ __forceinline__ Tile decode(const YeeArgs& a) {
     const int jb = t % B.n_jb;
     const int ib = t / B.n_jb;
     const int lane = threadIdx.x;
-    const int kx = lane % a.t.bx;
     const int jy = lane / a.t.bx;
+    const int kx = lane - jy * a.t.bx;
     Tile r;
     r.k0 = (kb * a.t.bx + kx) * V;
     r.j = B.j0 + jb * a.t.by + jy;
     r.i0 = B.i0 + ib * a.t.ci;
     r.i1 = min(r.i0 + a.t.ci, B.i1);
-    r.jend = B.j1;
+    // lanes past the last whole row get an empty row range
+    r.jend = jy < a.t.by ? B.j1 : r.j;
     r.kfirst = kx == 0 || (lane & 63) == 0;
     r.klast = kx == a.t.bx - 1 || (lane & 63) == 63;
     return r;

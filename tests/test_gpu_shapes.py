@@ -31,3 +31,16 @@ def test_shape_all_switches_off(shape):
                   materials=[(4.0, 1.0, 0.0, 0.0, (0, nx, 0, max(1, ny // 2), 0, nz))],
                   excitations=[(src, 1, True, gauss_ref(20e9))], table=0, graph=0)
     assert_parity(run_pair(sc), sc.name)
+
+
+@pytest.mark.parametrize("shape", [(3, 13, 44), (3, 21, 100), (3, 7, 320), (5, 9, 384), (2, 5, 600), (4, 9, 75),
+                                   (3, 4, 131)], ids=lambda s: "x".join(map(str, s)))
+def test_row_lengths_that_are_no_power_of_two(shape):
+    """Work-groups of whole and cut rows with idle lanes past the last row,
+    plain and with CPML faces."""
+    nx, ny, nz = shape
+    src = (nx // 2, ny // 2, nz // 2)
+    for cpml in (None, dict(layers=(1, 1, 2, 2, 8, 8), mode=1)):
+        sc = Scenario(f"rows_{nx}x{ny}x{nz}", shape, 1e-3, 30, materials=[(4.0, 1.0, 0.02, 0.0, (0, nx, 1, ny, 3, nz // 2))],
+                      excitations=[(src, 2, True, gauss_ref(20e9))], probes=[src], cpml=cpml)
+        assert_parity(run_pair(sc), sc.name)
