@@ -892,6 +892,7 @@ oe_status oe_ext_mur_create(oe_engine* e, const int enabled[6], double phase_vel
         if (n[m.ny] < 2) return fail(OE_ERR_GRID, "Mur face needs at least 2 cells along its normal");
         if (is_max) { m.line = n[m.ny] - 1; m.shift = n[m.ny] - 2; }
         else { m.line = 0; m.shift = 1; }
+        x->mur_thin = x->mur_thin || n[m.ny] < 3;
         m.s0 = n[m.nyp];
         m.s1 = n[m.nypp];
         const double c = phase_velocity > 0 ? phase_velocity : C0;
@@ -909,6 +910,24 @@ oe_status oe_ext_mur_create(oe_engine* e, const int enabled[6], double phase_vel
         m.v_nypp = x->mur_mem.as<float>() + off + cnt;
         off += 2 * cnt;
     }
+    // the faces that share an edge with face f, for k_mur_post_apply
+    for (size_t f = 0; f < x->mur_faces.size(); ++f)
+        for (int w = 0; w < 2; ++w) {
+            MurDev& m = x->mur_faces[f];
+            const int c = w ? m.nypp : m.nyp, o = 3 - m.ny - c;
+            for (size_t h = 0; h < x->mur_faces.size(); ++h) {
+                const MurDev& y = x->mur_faces[h];
+                if (y.ny != o) continue;
+                MurEdge& ed = m.e[w][y.line == 0 ? 0 : 1];
+                ed.line = y.line;
+                if (h < f) continue;
+                ed.shift = y.shift;
+                ed.coeff = y.coeff;
+                ed.v = c == y.nyp ? y.v_nyp : y.v_nypp;
+                ed.v0 = c == y.nyp ? m.line : m.line * y.s1;
+                ed.vs = c == y.nyp ? y.s1 : 1;
+            }
+        }
     HIP_OK(x->mur_dev.alloc(std::max<size_t>(x->mur_faces.size(), 1) * sizeof(MurDev)));
     if (!x->mur_faces.empty())
         HIP_OK(hipMemcpyAsync(x->mur_dev.p, x->mur_faces.data(), x->mur_faces.size() * sizeof(MurDev), hipMemcpyHostToDevice, e->stream));
@@ -2071,7 +2090,7 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         for (auto* x : murs) {
             if (fold_mur) break;
             Timed tm(e, "mur_post");
-            HIP_OK(launch_mur_post(e->F, e->g, x->mur_dev.as<MurDev>(), (int)x->mur_faces.size(), e->stream));
+            HIP_OK(launch_mur_post(e->F, e->g, x->mur_dev.as<MurDev>(), (int)x->mur_faces.size(), x->mur_thin, e->stream));
         }
         if (host) OE_TRY(run_hooks(3));
         if (point_ops) {

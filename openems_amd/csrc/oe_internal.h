@@ -267,6 +267,15 @@ hipError_t launch_energy(const float* F, size_t N, double* partials, int blocks,
                          hipStream_t s);
 int energy_blocks();
 
+// A face that shares an edge with another: its line plane on the third axis,
+// and, where it comes later in the list, what the edge's value takes: its
+// shift plane, coefficient and pre values v[v0 + vs * (component's axis)].
+struct MurEdge {
+    int line = -1, shift = -1;  // -1: none
+    float coeff = 0.f;
+    int v0 = 0, vs = 0;
+    const float* v = nullptr;
+};
 // Mur ABC face (src/extensions/mur_abc.rs:59-151).
 struct MurDev {
     int ny, nyp, nypp;
@@ -275,9 +284,11 @@ struct MurDev {
     float coeff;
     float* v_nyp;
     float* v_nypp;
+    MurEdge e[2][2];  // [component nyp, nypp][face along the third axis: min, max]
 };
 hipError_t launch_mur_pre(float* F, const Grid& g, const MurDev* faces, int n, hipStream_t s);
-hipError_t launch_mur_post(float* F, const Grid& g, const MurDev* faces, int n, hipStream_t s);
+// thin: some face's axis holds only 2 cells.
+hipError_t launch_mur_post(float* F, const Grid& g, const MurDev* faces, int n, bool thin, hipStream_t s);
 
 // ADE (src/extensions/dispersive.rs).  One thread per listed cell.
 struct AdeDev {

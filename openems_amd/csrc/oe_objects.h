@@ -77,6 +77,7 @@ struct oe_extension {
     std::vector<MurDev> mur_faces;
     DevBuf mur_mem;
     DevBuf mur_dev;     // device copy of mur_faces
+    bool mur_thin = false;  // some face's axis holds only 2 cells
     // UPML
     oe::UpmlDev upml{};
     DevBuf upml_mem;
