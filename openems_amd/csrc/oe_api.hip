@@ -372,6 +372,7 @@ oe_status engine_alloc(oe_engine* e, size_t nx, size_t ny, size_t nz, int device
     if (const char* v = getenv("OE_FOLD_MUR")) e->fold_mur = atoi(v) != 0;
     if (const char* v = getenv("OE_MERGE_ADE")) e->merge_ade = atoi(v) != 0;
     if (const char* v = getenv("OE_BYTE_INDEX")) e->byte_index = atoi(v) != 0;
+    if (const char* v = getenv("OE_RIDE")) e->ride = atoi(v) != 0;
     if (const char* v = getenv("OE_SLAB_TILES")) {  // "bx,by,ci,vec" of the CPML x/y slab launches
         Tiles t{};
         if (sscanf(v, "%d,%d,%d,%d", &t.bx, &t.by, &t.ci, &t.vec) == 4 && t.bx > 0 && t.bx <= 64 &&
@@ -1196,6 +1197,7 @@ oe_status oe_ext_dft_create(oe_engine* e, const oe_dft_config* cfg, oe_extension
     x->eng = e;
     x->dft_freqs.assign(cfg->freqs, cfg->freqs + nf);
     x->dft_stride = cfg->time_stride > 1 ? cfg->time_stride : 1;
+    x->dft_terms = nt;
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t b_off = al((n + 1) * 8), b_comp = al(std::max<size_t>(nt, 1) * 4), b_cell = al(std::max<size_t>(nt, 1) * 8);
     const size_t b_w = al(std::max<size_t>(nt, 1) * 8), b_h = al(n), b_f = al(nf * 8);
@@ -1732,6 +1734,7 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         HIP_OK(hipMemcpyAsync(e->exc_table.p, px.data(), px.size() * sizeof(PointExc), hipMemcpyHostToDevice, e->stream));
 
     // Probe tables.
+    // (count0: the probe's samples so far)
     std::vector<PointProbe> pp(probes.size());
     const uint64_t reserve_steps = num_steps == UINT64_MAX ? 0 : num_steps;
     for (size_t q = 0; q < probes.size(); ++q) {
@@ -1744,6 +1747,7 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         pp[q].out = x->probe_mem.as<double>();
         pp[q].capacity = x->probe_cap;
         pp[q].count = x->probe_cnt.as<uint64_t>();
+        pp[q].count0 = cnt;
     }
     if (pp.size() * sizeof(PointProbe) > e->probe_table.bytes) HIP_OK(e->probe_table.alloc(pp.size() * sizeof(PointProbe) + 64));
     if (!pp.empty())
@@ -1759,17 +1763,28 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     const bool host = !hosts.empty();
     const bool fused = e->fused_mode && !host && !upml && murs.empty() && ades.empty() && tl.vec == 4 &&
                        fused_supported(e->g) && (e->fused_mode == 2 || e->g.nz >= 128) && (!cp || cp->zvec);
-    // Sources are added by the E kernels themselves when nothing acts between
-    // the E update and them (no ADE, Mur or UPML post-E hooks), when every
-    // source cell is one the E update writes (i, j >= 1), the list is short
-    // and the steps are not fused (the fused kernel leaves sources to the
-    // point kernel); the point kernel then only records probes.
-    bool fold_sources = !fused && !host && !px.empty() && px.size() <= (size_t)MAX_FOLD_SOURCES && murs.empty() &&
-                        ades.empty() && !upml;
-    for (size_t q = 0; q < b->n_excitations && fold_sources; ++q)
-        if (b->excitations[q].i == 0 || b->excitations[q].j == 0) fold_sources = false;
+    // Sources are added by the E kernels themselves when nothing acts on their
+    // cells between the E update and them (no UPML, no ADE cell, no line or
+    // shift plane of a Mur face), when every source cell is one the E update
+    // writes (i, j >= 1), the list is short and the steps are not fused (the
+    // fused kernel leaves sources to the point kernel).
+    bool fold_sources = !fused && !host && !px.empty() && px.size() <= (size_t)MAX_FOLD_SOURCES && !upml;
+    for (size_t q = 0; q < b->n_excitations && fold_sources; ++q) {
+        const oe_excitation& x = b->excitations[q];
+        if (x.i == 0 || x.j == 0) fold_sources = false;
+        const int pos[3] = {(int)x.i, (int)x.j, (int)x.k};
+        for (const auto* mx : murs)
+            for (const MurDev& m : mx->mur_faces)
+                if (pos[m.ny] == m.line || pos[m.ny] == m.shift) fold_sources = false;
+        for (const auto* ax : ades)
+            if (std::binary_search(ax->ade_cells.begin(), ax->ade_cells.end(), px[q].idx)) fold_sources = false;
+    }
     if (const char* v = getenv("OE_FOLD_SOURCES")) fold_sources = fold_sources && atoi(v) != 0;
-    const bool point_ops = (!px.empty() && !fold_sources) || !pp.empty();
+    // Probes, small DFTs and the ADE and Mur captures ride in the Yee launches
+    // (oe_ride.h) unless the steps are fused or host hooks stand between them.
+    // The plan's last launch carries them: the interior, or the whole grid.
+    const bool riding = !fused && !host && e->ride && (plan.back().axes & (AX_X | AX_Y)) == 0;
+    const bool point_ops = (!px.empty() && !fold_sources) || (!pp.empty() && !riding);
     FusedArgs fa{};
     std::vector<Launch> slabs;
     if (fused) {
@@ -1840,9 +1855,21 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     // so a run of steps without host work in between (no energy sample, decay
     // check or timed step) is replayed from one captured graph.  The DFTs
     // then form their sample times from the batch's first step.
-    if (e->step_dev.bytes < sizeof(uint64_t)) HIP_OK(e->step_dev.alloc(sizeof(uint64_t)));
+    if (e->step_dev.bytes < 2 * sizeof(uint64_t)) HIP_OK(e->step_dev.alloc(2 * sizeof(uint64_t)));
     uint64_t* step_dev = e->step_dev.as<uint64_t>();  // reset below, once the step scheme is known
     const uint64_t t_batch0 = e->timestep;
+    // DFTs of a few signals sampled every step ride; the others are launches,
+    // which read the step from the device when all of them sample every step.
+    std::vector<oe_extension*> ride_dfts;
+    if (riding) {
+        std::vector<oe_extension*> rest;
+        for (auto* x : dfts) {
+            const bool small = x->dft_stride == 1 && x->dft.surf.n == 0 && x->dft.n_sig <= RIDE_SIGNALS &&
+                               (long)x->dft.n_sig * x->dft.n_f <= RIDE_PAIRS && x->dft_terms <= (size_t)RIDE_PAIRS;
+            (small && ride_dfts.size() < (size_t)MAX_RIDE_DFT ? ride_dfts : rest).push_back(x);
+        }
+        dfts.swap(rest);
+    }
     bool dev_dft = true;
     std::vector<uint64_t> dft0(dfts.size());
     for (size_t q = 0; q < dfts.size(); ++q) {
@@ -1904,6 +1931,52 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     const bool step_in_h = !fused && !plan_h.empty();
     if (step_in_h) plan_h[0].a.step_inc = step_dev;
     HIP_OK(hipMemsetAsync(step_dev, step_in_h ? 0xff : 0, sizeof(uint64_t), e->stream));
+    HIP_OK(hipMemsetAsync(step_dev + 1, 0, sizeof(uint64_t), e->stream));
+
+    // The riders' table.  The captures ride where every one of them fits.
+    bool ride_ade = riding && ades.size() <= (size_t)MAX_MERGE_ADE, ride_mur = riding && !fold_mur;
+    size_t n_faces = 0;
+    for (const auto* x : murs) n_faces += x->mur_faces.size();
+    ride_mur = ride_mur && n_faces > 0 && n_faces <= (size_t)MAX_RIDE_MUR;
+    int n_ride_h = 0, n_ride_e = 0;
+    if (riding) {
+        Ride rt{};
+        rt.F = e->F;
+        rt.g = e->g;
+        rt.t0 = (double)t_batch0;
+        rt.dt = e->dt;
+        rt.step_a = step_dev;
+        rt.step_b = step_dev + 1;
+        rt.n_probe = (int)pp.size();
+        rt.probe = e->probe_table.as<PointProbe>();
+        rt.first_dft = pp.empty() ? 0 : 1;
+        for (auto* x : ride_dfts) rt.dft[rt.n_dft++] = RideDft{x->dft, x->dft_count};
+        rt.first_ade = rt.first_dft + rt.n_dft;
+        int wg = rt.first_ade;
+        for (auto* x : ades) {
+            if (!ride_ade || x->ade.mode != OE_MODE_PHYSICAL || x->ade.n == 0) continue;
+            rt.ade_first[rt.n_ade] = wg;
+            rt.ade[rt.n_ade++] = x->ade;
+            wg += (x->ade.n + 255) / 256;
+        }
+        rt.first_mur = wg;
+        for (auto* x : murs) {
+            if (!ride_mur) continue;
+            for (size_t f = 0; f < x->mur_faces.size(); ++f) {
+                rt.mur[rt.n_mur++] = RideMur{x->mur_dev.as<MurDev>() + f, wg};
+                wg += (x->mur_faces[f].s0 * x->mur_faces[f].s1 + 255) / 256;
+            }
+        }
+        rt.n_wg = wg;
+        n_ride_h = wg;
+        n_ride_e = rt.first_ade;
+        if (e->ride_table.bytes < sizeof(Ride)) HIP_OK(e->ride_table.alloc(sizeof(Ride)));
+        HIP_OK(hipMemcpy(e->ride_table.p, &rt, sizeof(Ride), hipMemcpyHostToDevice));
+        plan_h.back().a.ride = plan_e.back().a.ride = e->ride_table.as<Ride>();
+        plan_h.back().a.n_ride = n_ride_h;
+        plan_e.back().a.n_ride = n_ride_e;
+        plan_e[0].a.step_inc = step_dev + 1;
+    }
 
     // The slab launches of a half-step write other cells than the interior
     // launch and read only the other field (and their own psi), so they run
@@ -2036,11 +2109,12 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         }
         if (host) OE_TRY(run_hooks(1));
         for (auto* x : murs) {
-            if (fold_mur) break;
+            if (fold_mur || ride_mur) break;
             Timed tm(e, "mur_pre");
             HIP_OK(launch_mur_pre(e->F, e->g, x->mur_dev.as<MurDev>(), (int)x->mur_faces.size(), e->stream));
         }
-        if (merge_ade) {
+        if (ride_ade) {
+        } else if (merge_ade) {
             if (ade_pre_m.n) {
                 Timed tm(e, "ade_pre");
                 HIP_OK(launch_ade_multi(e->F, e->Cf, e->g.N, ade_pre_m, true, e->stream));
@@ -2096,7 +2170,7 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         if (point_ops) {
             Timed tm(e, "point_ops");
             HIP_OK(launch_point_ops(e->F, e->g.N, e->exc_table.as<PointExc>(), fold_sources ? 0 : (int)px.size(), st,
-                                    e->probe_table.as<PointProbe>(), (int)pp.size(), e->stream, step_dev));
+                                    e->probe_table.as<PointProbe>(), riding ? 0 : (int)pp.size(), e->stream, step_dev));
         }
         for (size_t q = 0; q < dfts.size(); ++q) {
             oe_extension* x = dfts[q];
@@ -2157,16 +2231,18 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
             e->timestep += LG;
             executed += LG;
             st += LG;
-            for (auto* x : dfts) {
-                x->dft_seen += LG;
-                x->dft_count += LG;
-            }
+            for (auto* v : {&dfts, &ride_dfts})
+                for (auto* x : *v) {
+                    x->dft_seen += LG;
+                    x->dft_count += LG;
+                }
             continue;
         }
         e->prof_step = e->profiling > 0 && (st % (uint64_t)e->profiling) == 0;
         OE_TRY(enqueue_step(st, cur));
-        if (dev_dft)
-            for (auto* x : dfts) {
+        for (auto* v : {&dfts, &ride_dfts})
+            for (auto* x : *v) {
+                if (v == &dfts && !dev_dft) break;  // counted by its launch
                 x->dft_seen += 1;
                 x->dft_count += 1;
             }
@@ -2223,6 +2299,8 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
             collect_timing(e);
         }
     }
+    // the last step's E values (nothing follows that would carry them)
+    if (executed && n_ride_e) HIP_OK(launch_ride_last(e->ride_table.as<Ride>(), n_ride_e, e->stream));
     OE_TRY(drain());
     HIP_OK(hipStreamSynchronize(e->stream));
     if (e->profiling) collect_timing(e);

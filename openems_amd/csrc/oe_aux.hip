@@ -2,7 +2,7 @@
 // fills, excitations + probes, the float64 energy reduction, Mur ABC faces
 // and the dispersive (ADE) polarisation-current updates.
 
-#include "oe_internal.h"
+#include "oe_ride.h"
 
 #include <algorithm>
 
@@ -137,26 +137,10 @@ __global__ __launch_bounds__(EN_THREADS) void k_energy_final(const double* __res
     }
 }
 
-__device__ __forceinline__ size_t mur_cell(const Grid& g, const MurDev& m, int line, int a, int b) {
-    int pos[3];
-    pos[m.ny] = line;
-    pos[m.nyp] = a;
-    pos[m.nypp] = b;
-    return ((size_t)pos[0] * g.ny + pos[1]) * g.nz + pos[2];
-}
-
-// MurAbc::pre_voltage_update (src/extensions/mur_abc.rs:213-254).
 __global__ void k_mur_pre(const float* __restrict__ F, Grid g, const MurDev* __restrict__ faces) {
     const MurDev m = faces[blockIdx.y];
     const int cnt = m.s0 * m.s1;
-    const float* A = F + (size_t)m.nyp * g.N;
-    const float* B = F + (size_t)m.nypp * g.N;
-    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < cnt; q += gridDim.x * blockDim.x) {
-        const int a = q / m.s1, b = q % m.s1;
-        const size_t pb = mur_cell(g, m, m.line, a, b), ps = mur_cell(g, m, m.shift, a, b);
-        m.v_nyp[q] = A[ps] - m.coeff * A[pb];
-        m.v_nypp[q] = B[ps] - m.coeff * B[pb];
-    }
+    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < cnt; q += gridDim.x * blockDim.x) mur_pre_cell(F, g, m, q);
 }
 
 // MurAbc::post_voltage_update (src/extensions/mur_abc.rs:257-291) and
@@ -229,12 +213,6 @@ __global__ void k_mur_apply(float* __restrict__ F, Grid g, const MurDev* __restr
         A[pb] = m.v_nyp[q];
         B[pb] = m.v_nypp[q];
     }
-}
-
-__device__ __forceinline__ void ade_pre_cell(const float* __restrict__ F, size_t N, const AdeDev& a, int c) {
-    const size_t p = a.idx[c];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) a.Eprev[(size_t)d * a.n + c] = F[(size_t)d * N + p];
 }
 
 __global__ void k_ade_pre(const float* __restrict__ F, size_t N, AdeDev a) {
@@ -411,10 +389,7 @@ __global__ __launch_bounds__(256) void k_dft(const float* __restrict__ F, size_t
         __syncthreads();  // sv / hv written; the previous chunk's phasors read
         for (int q = t; q < 2 * nf; q += blockDim.x) {
             const int hq = q / nf, f = q - hq * nf;
-            double sn, cs;
-            sincos(2.0 * M_PI * d.freqs[f0 + f] * (hq ? tH : tE), &sn, &cs);
-            ph[hq][f][0] = cs;
-            ph[hq][f][1] = -sn;
+            dft_phasor(d.freqs[f0 + f], hq ? tH : tE, ph[hq][f][0], ph[hq][f][1]);
         }
         __syncthreads();
         for (int q = t; q < nf * nm; q += blockDim.x) {
@@ -422,21 +397,7 @@ __global__ __launch_bounds__(256) void k_dft(const float* __restrict__ F, size_t
             const double s = sv[g];
             const double cr = ph[hv[g]][f][0], ci = ph[hv[g]][f][1];
             const size_t a = (size_t)(f0 + f) * d.n_sig + m0 + g;
-            if (d.prec == 0) {
-                d.acc64[2 * a] += s * cr;
-                d.acc64[2 * a + 1] += s * ci;
-            } else {
-                const float svf = (float)s;
-                float* acc = d.acc32 + 4 * a;
-                const float yr = svf * (float)cr - acc[2];
-                const float tr = acc[0] + yr;
-                acc[2] = (tr - acc[0]) - yr;
-                acc[0] = tr;
-                const float yi = svf * (float)ci - acc[3];
-                const float ti = acc[1] + yi;
-                acc[3] = (ti - acc[1]) - yi;
-                acc[1] = ti;
-            }
+            dft_add(d, a, s, cr, ci);
         }
     }
 }
@@ -475,10 +436,7 @@ __device__ void sweep_dft_body(const SweepDft& x, uint64_t st, double dt) {
         __syncthreads();
         for (int q = threadIdx.x; q < 2 * nf; q += blockDim.x) {
             const int hq = q / nf, f = q - hq * nf;
-            double sn, cs;
-            sincos(2.0 * M_PI * d.freqs[f0 + f] * (hq ? tH : tE), &sn, &cs);
-            ph[hq][f][0] = cs;
-            ph[hq][f][1] = -sn;
+            dft_phasor(d.freqs[f0 + f], hq ? tH : tE, ph[hq][f][0], ph[hq][f][1]);
         }
         __syncthreads();
         for (int q = threadIdx.x; q < nf * d.n_sig; q += blockDim.x) {
@@ -486,21 +444,7 @@ __device__ void sweep_dft_body(const SweepDft& x, uint64_t st, double dt) {
             const double s = sv[g];
             const double cr = ph[hv[g]][f][0], ci = ph[hv[g]][f][1];
             const size_t a = (size_t)(f0 + f) * d.n_sig + g;
-            if (d.prec == 0) {
-                d.acc64[2 * a] += s * cr;
-                d.acc64[2 * a + 1] += s * ci;
-            } else {
-                const float svf = (float)s;
-                float* acc = d.acc32 + 4 * a;
-                const float yr = svf * (float)cr - acc[2];
-                const float tr = acc[0] + yr;
-                acc[2] = (tr - acc[0]) - yr;
-                acc[0] = tr;
-                const float yi = svf * (float)ci - acc[3];
-                const float ti = acc[1] + yi;
-                acc[3] = (ti - acc[1]) - yi;
-                acc[1] = ti;
-            }
+            dft_add(d, a, s, cr, ci);
         }
     }
 }
@@ -531,6 +475,8 @@ __global__ __launch_bounds__(256) void k_sweep_point(const SweepExc* __restrict_
     __syncthreads();
     sweep_dft_body(dfts[dft_of[s]], st, dt);
 }
+
+__global__ __launch_bounds__(256) void k_ride_last(const Ride* __restrict__ r) { ride(*r, blockIdx.x, true); }
 
 __global__ void k_sweep_step(uint64_t* step) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *step += 1;
@@ -700,6 +646,12 @@ hipError_t launch_sweep_point(const SweepExc* e, const int* first, const int* se
                               const int* dft_of, int n_struct, const uint64_t* step, double dt, hipStream_t s) {
     if (n_struct <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_sweep_point, dim3(n_struct), dim3(256), 0, s, e, first, serial, dfts, dft_of, step, dt);
+    return hipGetLastError();
+}
+
+hipError_t launch_ride_last(const Ride* r, int n_wg, hipStream_t s) {
+    if (n_wg <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_ride_last, dim3(n_wg), dim3(256), 0, s, r);
     return hipGetLastError();
 }
 

@@ -134,10 +134,14 @@ struct YeeArgs {
     // First-order Mur on the z faces applied by the E half-step itself (see
     // e_body): on[0] the k = 0 face, on[1] the k = nz - 1 face.
     MurZ mur_z;
-    // Non-null on one H launch per step: its first lane advances the device
-    // step counter before anything of the step reads it (the counter starts
-    // a batch at -1).
+    // Non-null on the first H launch of a step: its first lane advances the
+    // device step counter before anything of the step reads it (the counter
+    // starts a batch at -1).  On the first E launch: the counter of steps
+    // begun that the next step's riders read.
     uint64_t* step_inc;
+    // Work-groups [0, n_ride) are riders (oe_ride.h), the tiles follow.
+    const struct Ride* ride;
+    int n_ride;
 };
 
 // CPML code compiled into a launch: bit 0 x faces, bit 1 y faces, bit 2 z faces.
@@ -256,6 +260,7 @@ struct PointProbe {
     double* out;    // [capacity][6]
     uint64_t capacity;
     uint64_t* count;  // device counter
+    uint64_t count0;  // its value when the batch began
 };
 // step_dev non-null: the step index is read from the device counter.
 hipError_t launch_point_ops(float* F, size_t N, const PointExc* exc, int n_exc, uint64_t step,
@@ -363,6 +368,38 @@ hipError_t launch_dft(const float* F, size_t N, const DftDev& d, uint64_t sample
 // Step from the device counter: sample = sample0 + st, times from t0 + st.
 hipError_t launch_dft_dev(const float* F, size_t N, const DftDev& d, const uint64_t* step_dev, uint64_t sample0,
                           double t0, double dt, hipStream_t s);
+
+// The riders of a batch's Yee launches (oe_ride.h), one table in device
+// memory.  Rider work-groups: [0, first_dft) probes, [first_dft, first_ade)
+// one DFT each, and in H launches [first_ade, first_mur) ADE captures,
+// [first_mur, ...) Mur pre values.
+constexpr int RIDE_SIGNALS = 64;   // a riding DFT's signals (one lane each)
+constexpr int RIDE_PAIRS = 4096;   // and (frequency, signal) pairs, and terms
+constexpr int MAX_RIDE_DFT = 8, MAX_RIDE_MUR = 12;
+struct RideDft {
+    DftDev d;
+    uint64_t sample0;  // sample index of the batch's first step
+};
+struct RideMur {
+    const MurDev* face;
+    int first;  // its first work-group
+};
+struct Ride {
+    const float* F;
+    Grid g;
+    double t0, dt;
+    const uint64_t* step_a;
+    const uint64_t* step_b;
+    int n_probe, n_dft, n_ade, n_mur;
+    int first_dft, first_ade, first_mur, n_wg;
+    int ade_first[MAX_MERGE_ADE];
+    const PointProbe* probe;
+    RideDft dft[MAX_RIDE_DFT];
+    AdeDev ade[MAX_MERGE_ADE];
+    RideMur mur[MAX_RIDE_MUR];
+};
+// The H launches' riders alone, after a batch's last step (probes and DFTs).
+hipError_t launch_ride_last(const Ride* r, int n_wg, hipStream_t s);
 
 // Sweep step pieces (oe_aux.hip).  The step index is read from *step.
 struct SweepExc {

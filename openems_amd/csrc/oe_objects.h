@@ -97,6 +97,7 @@ struct oe_extension {
     uint64_t dft_count = 0;   // accumulated samples
     uint64_t dft_seen = 0;    // steps seen (time stride)
     uint32_t dft_stride = 1;
+    size_t dft_terms = 0;     // terms of all signals
     std::vector<double> dft_freqs;
     bool is_port = false;
     // NF2FF box: faces whose phasors are consecutive DFT signals from nf_sig0[f]
@@ -144,7 +145,9 @@ struct oe_engine {
     double* energy_host = nullptr;  // pinned
     // point ops
     DevBuf exc_samples;
-    DevBuf step_dev;       // batch-relative step read by the kernels of a step
+    DevBuf step_dev;       // batch-relative step read by the kernels of a step, and steps begun
+    DevBuf ride_table;     // the riders of the running batch (oe_ride.h)
+    int ride = 1;          // probes, small DFTs and captures in the Yee launches: 1 on, 0 off
     int graph_steps = 16;  // steps per captured graph (0: no graphs)
     // CPML slab launches on a second stream beside the interior launch of
     // the same half-step (forked and joined with events; created on first

@@ -27,7 +27,7 @@
 // slab read a zeroed dummy line -- which keeps the psi latency hidden behind
 // the bulk loads instead of serialising it after them.
 
-#include "oe_internal.h"
+#include "oe_ride.h"
 
 #pragma clang fp contract(off)
 
@@ -217,9 +217,9 @@ struct Tile {
 // run on the same XCD at the same time.
 template <int V>
 __device__ __forceinline__ Tile decode(const YeeArgs& a) {
-    int bid = blockIdx.x;
+    int bid = blockIdx.x - a.n_ride;
     if (a.xcd_remap) {
-        const int per = gridDim.x >> 3;
+        const int per = (gridDim.x - a.n_ride) >> 3;
         if (bid < (per << 3)) bid = (bid & 7) * per + (bid >> 3);
     }
     int b = 0;
@@ -689,6 +689,11 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
     }
 }
 
+// The plain and z-faces kernels carry riders (the code would cost the
+// all-faces kernels registers).
+template <int AX>
+constexpr bool RIDES = (AX & (AX_X | AX_Y)) == 0;
+
 // One grid: the tile comes from the launch's box list.  With TAB the
 // work-group first copies its half's material rows into LDS (dynamic LDS of
 // 24 bytes per row).
@@ -697,6 +702,12 @@ __global__ __launch_bounds__(256) void k_update_h(YeeArgs a, CpmlArgs c) {
     extern __shared__ float2 lds_rows[];
     // the step's first launch advances the step counter (no H lane reads it)
     if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) *a.step_inc += 1;
+    if constexpr (RIDES<AX>) {
+        if ((int)blockIdx.x < a.n_ride) {
+            ride(*a.ride, blockIdx.x, true);
+            return;
+        }
+    }
     if constexpr (TAB) {
         const float2* src = reinterpret_cast<const float2*>(a.tab_h);
         for (int q = threadIdx.x; q < 3 * a.n_mat_h; q += blockDim.x) lds_rows[q] = src[q];
@@ -706,25 +717,28 @@ __global__ __launch_bounds__(256) void k_update_h(YeeArgs a, CpmlArgs c) {
                              decode<V>(a));
 }
 
+// The z-faces kernels are held to the 128 registers of 4 waves a SIMD.
 template <int V, int AX, bool PHYS, bool TAB, bool MUR = false>
-__global__ __launch_bounds__(256) void k_update_e(YeeArgs a, CpmlArgs c) {
+__global__ __launch_bounds__(256, V == 4 && AX == AX_Z ? 4 : 1) void k_update_e(YeeArgs a, CpmlArgs c) {
     extern __shared__ float2 lds_rows[];
+    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) *a.step_inc += 1;
+    if constexpr (RIDES<AX>) {
+        if ((int)blockIdx.x < a.n_ride) {
+            ride(*a.ride, blockIdx.x, false);
+            return;
+        }
+    }
     if constexpr (TAB) {
         const float2* src = reinterpret_cast<const float2*>(a.tab_e);
         for (int q = threadIdx.x; q < 3 * a.n_mat_e; q += blockDim.x) lds_rows[q] = src[q];
         __syncthreads();
     }
     const MatIndex mat_e{a.n_mat_e == 1 ? nullptr : a.mat_e, a.mat8_e};
-    if constexpr (MUR) {
-        // sources follow the Mur step, so they are never folded with it
-        e_body<V, AX, PHYS, TAB, true>(a.g, a.Fin, a.Fout, a.Cf, mat_e, lds_rows, c, decode<V>(a), nullptr, a.mur_z);
-        return;
-    }
-    if (a.n_exc) {
+    if (MUR || a.n_exc) {
         const Sources src{a.exc, a.exc_idx, a.n_exc, a.exc_step, a.exc_step_dev};
-        e_body<V, AX, PHYS, TAB>(a.g, a.Fin, a.Fout, a.Cf, mat_e, lds_rows, c, decode<V>(a), &src);
+        e_body<V, AX, PHYS, TAB, MUR>(a.g, a.Fin, a.Fout, a.Cf, mat_e, lds_rows, c, decode<V>(a), &src, a.mur_z);
     } else {
-        e_body<V, AX, PHYS, TAB>(a.g, a.Fin, a.Fout, a.Cf, mat_e, lds_rows, c, decode<V>(a));
+        e_body<V, AX, PHYS, TAB, MUR>(a.g, a.Fin, a.Fout, a.Cf, mat_e, lds_rows, c, decode<V>(a));
     }
 }
 
@@ -799,10 +813,10 @@ __global__ __launch_bounds__(256) void k_update_e_sweep(SweepArgs a) {
 template <int V, int AX, bool PHYS>
 hipError_t launch_h_t(const YeeArgs& a, const CpmlArgs& c, hipStream_t s) {
     if (a.n_mat_h > 0)
-        hipLaunchKernelGGL((k_update_h<V, AX, PHYS, true>), dim3(a.first[a.nbox]), dim3(256),
+        hipLaunchKernelGGL((k_update_h<V, AX, PHYS, true>), dim3(a.n_ride + a.first[a.nbox]), dim3(256),
                            3 * a.n_mat_h * sizeof(float2), s, a, c);
     else
-        hipLaunchKernelGGL((k_update_h<V, AX, PHYS, false>), dim3(a.first[a.nbox]), dim3(256), 0, s, a, c);
+        hipLaunchKernelGGL((k_update_h<V, AX, PHYS, false>), dim3(a.n_ride + a.first[a.nbox]), dim3(256), 0, s, a, c);
     return hipGetLastError();
 }
 
@@ -811,10 +825,10 @@ hipError_t launch_e_t(const YeeArgs& a, const CpmlArgs& c, hipStream_t s) {
     if constexpr (V == 4) {
         if (a.mur_z.on[0] || a.mur_z.on[1]) {
             if (a.n_mat_e > 0)
-                hipLaunchKernelGGL((k_update_e<V, AX, PHYS, true, true>), dim3(a.first[a.nbox]), dim3(256),
+                hipLaunchKernelGGL((k_update_e<V, AX, PHYS, true, true>), dim3(a.n_ride + a.first[a.nbox]), dim3(256),
                                    3 * a.n_mat_e * sizeof(float2), s, a, c);
             else
-                hipLaunchKernelGGL((k_update_e<V, AX, PHYS, false, true>), dim3(a.first[a.nbox]), dim3(256), 0, s, a,
+                hipLaunchKernelGGL((k_update_e<V, AX, PHYS, false, true>), dim3(a.n_ride + a.first[a.nbox]), dim3(256), 0, s, a,
                                    c);
             return hipGetLastError();
         }
@@ -822,10 +836,10 @@ hipError_t launch_e_t(const YeeArgs& a, const CpmlArgs& c, hipStream_t s) {
         if (a.mur_z.on[0] || a.mur_z.on[1]) return hipErrorInvalidValue;  // needs float4 lanes
     }
     if (a.n_mat_e > 0)
-        hipLaunchKernelGGL((k_update_e<V, AX, PHYS, true>), dim3(a.first[a.nbox]), dim3(256),
+        hipLaunchKernelGGL((k_update_e<V, AX, PHYS, true>), dim3(a.n_ride + a.first[a.nbox]), dim3(256),
                            3 * a.n_mat_e * sizeof(float2), s, a, c);
     else
-        hipLaunchKernelGGL((k_update_e<V, AX, PHYS, false>), dim3(a.first[a.nbox]), dim3(256), 0, s, a, c);
+        hipLaunchKernelGGL((k_update_e<V, AX, PHYS, false>), dim3(a.n_ride + a.first[a.nbox]), dim3(256), 0, s, a, c);
     return hipGetLastError();
 }
 
