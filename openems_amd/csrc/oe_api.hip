@@ -78,8 +78,7 @@ int pow2ceil(int v) {
 // (151x133x117 with CPML, ci 1 / 2 / 3: 82.5 / 75.0 / 81.0).
 Tiles auto_tiles(const Grid& g, int vec_req) {
     Tiles t{};
-    t.vec = (vec_req == 1) ? 1 : ((g.nz % 4 == 0) ? 4 : 1);
-    if (vec_req == 4 && g.nz % 4 != 0) t.vec = 1;
+    t.vec = vec_req == 1 || (g.nz % 4 != 0 && g.nz < 8) ? 1 : 4;
     const int nzv = (g.nz + t.vec - 1) / t.vec;
     const int widest = t.vec == 4 ? 64 : 128;
     double best = 0.0;
@@ -111,7 +110,7 @@ Box make_box(const Tiles& t, int i0, int i1, int j0, int j1) {
     return b;
 }
 
-YeeArgs launch_args(const oe_engine* e, const Tiles& t, const std::vector<Box>& boxes) {
+YeeArgs launch_args(const oe_engine* e, const Tiles& t, const CpmlArgs* cp, const std::vector<Box>& boxes) {
     YeeArgs a{};
     a.g = e->g;
     a.Fin = e->F;
@@ -130,6 +129,7 @@ YeeArgs launch_args(const oe_engine* e, const Tiles& t, const std::vector<Box>& 
         }
     }
     a.t = t;
+    a.ragged = t.vec == 4 && (e->g.nz % 4 != 0 || (cp && !cp->zvec));
     const int nzv = (e->g.nz + t.vec - 1) / t.vec;
     a.n_kb = (nzv + t.bx - 1) / t.bx;
     a.nbox = (int)boxes.size();
@@ -151,7 +151,7 @@ std::vector<Launch> plan_launches(const oe_engine* e, const Tiles& t, const Cpml
     std::vector<Launch> out;
     const Grid& g = e->g;
     if (!cp) {
-        out.push_back({launch_args(e, t, {make_box(t, 0, g.nx, 0, g.ny)}), 0});
+        out.push_back({launch_args(e, t, nullptr, {make_box(t, 0, g.nx, 0, g.ny)}), 0});
         return out;
     }
     const int m = cp->on_mask;
@@ -165,7 +165,7 @@ std::vector<Launch> plan_launches(const oe_engine* e, const Tiles& t, const Cpml
     Tiles ts = t;  // the interior's depth measured best for the slabs too (ci 1/2/4/8 at 256^3)
     if (e->slab_tiles.bx > 0) {
         ts = e->slab_tiles;
-        if (ts.vec == 4 && g.nz % 4 != 0) ts.vec = 1;
+        if (t.vec == 1) ts.vec = 1;
     }
     if (ix0 > 0) slabs.push_back(make_box(ts, 0, ix0, 0, g.ny));
     if (ix1 < g.nx) slabs.push_back(make_box(ts, ix1, g.nx, 0, g.ny));
@@ -173,9 +173,9 @@ std::vector<Launch> plan_launches(const oe_engine* e, const Tiles& t, const Cpml
         if (jy0 > 0) slabs.push_back(make_box(ts, ix0, ix1, 0, jy0));
         if (jy1 < g.ny) slabs.push_back(make_box(ts, ix0, ix1, jy1, g.ny));
     }
-    if (!slabs.empty()) out.push_back({launch_args(e, ts, slabs), AX_X | AX_Y | AX_Z});
+    if (!slabs.empty()) out.push_back({launch_args(e, ts, cp, slabs), AX_X | AX_Y | AX_Z});
     if (ix1 > ix0 && jy1 > jy0)
-        out.push_back({launch_args(e, t, {make_box(t, ix0, ix1, jy0, jy1)}), (m & 48) ? AX_Z : 0});
+        out.push_back({launch_args(e, t, cp, {make_box(t, ix0, ix1, jy0, jy1)}), (m & 48) ? AX_Z : 0});
     return out;
 }
 
@@ -357,9 +357,9 @@ oe_status engine_alloc(oe_engine* e, size_t nx, size_t ny, size_t nz, int device
     e->g.nx = (int)nx; e->g.ny = (int)ny; e->g.nz = (int)nz;
     e->g.N = nx * ny * nz;
     HIP_OK(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
-    HIP_OK(hipMalloc(&e->F, 6 * e->g.N * sizeof(float)));
-    HIP_OK(hipMemsetAsync(e->F, 0, 6 * e->g.N * sizeof(float), e->stream));
-    HIP_OK(hipMalloc(&e->Cf, 12 * e->g.N * sizeof(float)));
+    HIP_OK(hipMalloc(&e->F, 6 * e->g.N * sizeof(float) + ARRAY_PAD));
+    HIP_OK(hipMemsetAsync(e->F, 0, 6 * e->g.N * sizeof(float) + ARRAY_PAD, e->stream));
+    HIP_OK(hipMalloc(&e->Cf, 12 * e->g.N * sizeof(float) + ARRAY_PAD));
     HIP_OK(hipMalloc(&e->partials, 2 * energy_blocks() * sizeof(double)));
     e->energy_dev_cap = 4096;
     HIP_OK(hipMalloc(&e->energy_dev, 2 * e->energy_dev_cap * sizeof(double)));
@@ -398,7 +398,7 @@ void drop_material_table(oe_engine* e) {
 oe_status build_material_tables(oe_engine* e) {
     drop_material_table(e);
     const size_t N = e->g.N;
-    HIP_OK(hipMalloc(&e->mat, 2 * N * sizeof(uint16_t)));
+    HIP_OK(hipMalloc(&e->mat, 2 * N * sizeof(uint16_t) + ARRAY_PAD));
     HIP_OK(hipMalloc(&e->mtab, 2 * (size_t)MAX_MAT_ROWS * 6 * sizeof(float)));
     int n[2] = {0, 0};
     for (int h = 0; h < 2; ++h)
@@ -414,7 +414,7 @@ oe_status build_material_tables(oe_engine* e) {
     // less per launch)
     const bool narrow[2] = {e->byte_index && n[0] >= 2 && n[0] <= 256, e->byte_index && n[1] >= 2 && n[1] <= 256};
     if (narrow[0] || narrow[1]) {
-        HIP_OK(hipMalloc(&e->mat8, 2 * N));
+        HIP_OK(hipMalloc(&e->mat8, 2 * N + ARRAY_PAD));
         for (int h = 0; h < 2; ++h)
             if (narrow[h]) HIP_OK(narrow_material_index(e->mat + (size_t)h * N, e->mat8 + (size_t)h * N, N, e->stream));
     }
@@ -792,8 +792,8 @@ oe_status oe_ext_cpml_create(oe_engine* e, const oe_cpml_config* cfg, oe_extensi
         if (on0 && on1 && a0 + a1 > (size_t)n[dir])
             return fail(OE_ERR_CONFIG, "CPML faces of axis %d overlap (%zu + %zu layers > %d cells)", dir, a0, a1, n[dir]);
     }
-    std::vector<float> tab((size_t)6 * CPML_TABLES * c.Lmax, 0.0f);
-    size_t total = 0;
+    std::vector<float> tab((size_t)6 * CPML_TABLES * c.Lmax + ARRAY_PAD / sizeof(float), 0.0f);
+    size_t total = 64;  // a straddling lane reads up to 3 floats before its slab row
     size_t offs[6];
     for (int f = 0; f < 6; ++f) {
         const int dir = f / 2;
@@ -1753,7 +1753,8 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     if (!pp.empty())
         HIP_OK(hipMemcpyAsync(e->probe_table.p, pp.data(), pp.size() * sizeof(PointProbe), hipMemcpyHostToDevice, e->stream));
     Tiles tl = e->tiles;
-    if (cp && !cp->zvec && tl.vec == 4) tl = auto_tiles(e->g, 1);  // z slabs not 4-aligned: scalar lanes
+    // a float4 lane meets at most one z slab, or lanes are scalar
+    if (cp && !cp->zvec && tl.vec == 4 && (cp->on_mask & 48) == 48 && cp->g0[5] - cp->L[4] < 3) tl = auto_tiles(e->g, 1);
     const std::vector<Launch> plan = plan_launches(e, tl, cp);
     // Fused steps (one pass per step over the plan's interior box) when no
     // extension hooks in between the half-steps and the grid suits the
@@ -1883,7 +1884,8 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     // UPML, and no ADE cell on a face's line or shift plane (ADE post runs
     // between the E update and the Mur post step).
     MurZ mz{};
-    bool fold_mur = e->fold_mur && !host && murs.size() == 1 && !upml && !fused && tl.vec == 4 && e->g.nz >= 4;
+    bool fold_mur = e->fold_mur && !host && murs.size() == 1 && !upml && !fused && tl.vec == 4 && e->g.nz >= 4 &&
+                    e->g.nz % 4 == 0 && (!cp || cp->zvec);
     if (fold_mur)
         for (const MurDev& m : murs[0]->mur_faces) {
             if (m.ny != 2) {

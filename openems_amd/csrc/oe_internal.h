@@ -43,7 +43,7 @@ struct Grid {
 // rows (j) and marches along i over `ci` planes, keeping the i+1 (H update)
 // or i-1 (E update) plane of the marched components in registers.
 struct Tiles {
-    int vec;  // 4: float4 accesses (nz % 4 == 0), 1: scalar
+    int vec;  // 4: float4 accesses, 1: scalar
     int bx;   // lanes along k
     int by;   // rows along j; bx * by <= 256
     int ci;   // planes along i per work-group
@@ -53,6 +53,9 @@ struct Tiles {
 // psi layout for face f: dims (nx,ny,nz) with axis `dir` replaced by L[f],
 // z fastest.  tab holds, per face, 6 tables of Lmax floats:
 // b_e, b_h, a_e, a_h, (1/kappa_e - 1), (1/kappa_h - 1).
+// Arrays that float4 lanes of a ragged row read past (and z psi before) their
+// ends carry this many bytes of padding there.
+constexpr size_t ARRAY_PAD = 64;
 constexpr int CPML_TABLES = 6;
 enum { TAB_BE = 0, TAB_BH = 1, TAB_AE = 2, TAB_AH = 3, TAB_KE = 4, TAB_KH = 5 };
 
@@ -116,6 +119,7 @@ struct YeeArgs {
     const float* tab_e;
     int n_mat_h, n_mat_e;
     Tiles t;
+    int ragged;            // vec 4 on rows or z slabs that are no multiple of 4
     int n_kb;              // blocks along k (every box spans all k)
     int nbox;
     Box box[MAX_BOXES];

@@ -29,6 +29,8 @@
 
 #include "oe_ride.h"
 
+#include <type_traits>
+
 #pragma clang fp contract(off)
 
 namespace oe {
@@ -39,20 +41,14 @@ struct Vec {
     float v[V];
 };
 
-template <int V>
-__device__ __forceinline__ Vec<V> ldv(const float* __restrict__ p) {
-    Vec<V> r;
-    if constexpr (V == 4) {
-        const float4 t = *reinterpret_cast<const float4*>(p);
-        r.v[0] = t.x; r.v[1] = t.y; r.v[2] = t.z; r.v[3] = t.w;
-    } else {
-        r.v[0] = *p;
-    }
-    return r;
-}
-
-template <int V>
-__device__ __forceinline__ void stv(float* __restrict__ p, const Vec<V>& a);
+// RAG: the row length (or a z slab's) is no multiple of 4, so the float4 of a
+// lane starts at any float.  Global memory takes such accesses (a wave's 1 KB
+// then meets nine lines instead of eight); the last lane of a row reads past
+// its end (arrays are padded) and stores only the row's own cells.
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+template <bool RAG>
+using F4 = std::conditional_t<RAG, f4u, f4v>;
 
 // Streaming (nontemporal) accesses for data without reuse inside a launch:
 // the coefficient arrays and the component being updated (load and store).
@@ -68,40 +64,45 @@ __device__ __forceinline__ void stv(float* __restrict__ p, const Vec<V>& a);
 #ifndef OE_NT_STORE
 #define OE_NT_STORE 1
 #endif
-typedef float f4v __attribute__((ext_vector_type(4)));
 
-template <int V, bool NT>
+template <int V, bool NT, bool RAG = false>
 __device__ __forceinline__ Vec<V> ldn(const float* __restrict__ p) {
-    if constexpr (!NT) {
-        return ldv<V>(p);
-    } else {
-        Vec<V> r;
-        if constexpr (V == 4) {
-            const f4v t = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(p));
-            r.v[0] = t.x; r.v[1] = t.y; r.v[2] = t.z; r.v[3] = t.w;
-        } else {
-            r.v[0] = __builtin_nontemporal_load(p);
-        }
-        return r;
-    }
-}
-
-template <int V, bool NT>
-__device__ __forceinline__ void stn(float* __restrict__ p, const Vec<V>& a) {
-    if constexpr (!NT) {
-        stv<V>(p, a);
-    } else if constexpr (V == 4) {
-        f4v t = {a.v[0], a.v[1], a.v[2], a.v[3]};
-        __builtin_nontemporal_store(t, reinterpret_cast<f4v*>(p));
-    } else {
-        __builtin_nontemporal_store(a.v[0], p);
-    }
-}
-
-template <int V>
-__device__ __forceinline__ void stv(float* __restrict__ p, const Vec<V>& a) {
+    Vec<V> r;
     if constexpr (V == 4) {
-        *reinterpret_cast<float4*>(p) = make_float4(a.v[0], a.v[1], a.v[2], a.v[3]);
+        const F4<RAG>* q = reinterpret_cast<const F4<RAG>*>(p);
+        f4v t;
+        if constexpr (NT) t = __builtin_nontemporal_load(q);
+        else t = *q;
+        r.v[0] = t.x; r.v[1] = t.y; r.v[2] = t.z; r.v[3] = t.w;
+    } else if constexpr (NT) {
+        r.v[0] = __builtin_nontemporal_load(p);
+    } else {
+        r.v[0] = *p;
+    }
+    return r;
+}
+
+template <int V, bool RAG = false>
+__device__ __forceinline__ Vec<V> ldv(const float* __restrict__ p) {
+    return ldn<V, false, RAG>(p);
+}
+
+// Stores the lane's first n cells (all V unless RAG).
+template <int V, bool NT, bool RAG = false>
+__device__ __forceinline__ void stn(float* __restrict__ p, const Vec<V>& a, int n = V) {
+    if constexpr (V == 4) {
+        if (!RAG || n >= V) {
+            f4v t = {a.v[0], a.v[1], a.v[2], a.v[3]};
+            F4<RAG>* q = reinterpret_cast<F4<RAG>*>(p);
+            if constexpr (NT) __builtin_nontemporal_store(t, q);
+            else *q = t;
+        } else {
+#pragma unroll
+            for (int e = 0; e < V - 1; ++e)
+                if (e < n) p[e] = a.v[e];
+        }
+    } else if constexpr (NT) {
+        __builtin_nontemporal_store(a.v[0], p);
     } else {
         *p = a.v[0];
     }
@@ -121,6 +122,8 @@ __device__ __forceinline__ Vec<V> zerov() {
 // (nontemporal, one 8-byte load for V = 4); neither stands for a table of
 // one row, whose indices are all 0 and are not read.
 typedef unsigned int u2v __attribute__((ext_vector_type(2)));
+typedef unsigned int u2u __attribute__((ext_vector_type(2), aligned(2)));
+typedef unsigned int u1u __attribute__((aligned(1)));
 
 struct MatIndex {
     const uint16_t* m16;
@@ -133,15 +136,17 @@ struct MatIdx {
     unsigned a = 0, b = 0;
 };
 
-template <int V>
+template <int V, bool RAG = false>
 __device__ __forceinline__ MatIdx coef_index(const MatIndex& mi, size_t p) {
+    using U1 = std::conditional_t<RAG, u1u, unsigned>;
+    using U2 = std::conditional_t<RAG, u2u, u2v>;
     MatIdx r;
     if (mi.m8 != nullptr) {
-        if constexpr (V == 4) r.a = __builtin_nontemporal_load(reinterpret_cast<const unsigned*>(mi.m8 + p));
+        if constexpr (V == 4) r.a = __builtin_nontemporal_load(reinterpret_cast<const U1*>(mi.m8 + p));
         else r.a = mi.m8[p];
     } else if (mi.m16 != nullptr) {
         if constexpr (V == 4) {
-            const u2v t = __builtin_nontemporal_load(reinterpret_cast<const u2v*>(mi.m16 + p));
+            const u2v t = __builtin_nontemporal_load(reinterpret_cast<const U2*>(mi.m16 + p));
             r.a = t.x;
             r.b = t.y;
         } else {
@@ -151,15 +156,21 @@ __device__ __forceinline__ MatIdx coef_index(const MatIndex& mi, size_t p) {
     return r;
 }
 
-template <int V>
+// n: the lane's cells inside its row (RAG: those past it take row 0, their
+// index may be another half's).
+template <int V, bool RAG = false>
 __device__ __forceinline__ void coef_from(const MatIndex& mi, const MatIdx& x, const float2* tab, Vec<V>& a0,
-                                          Vec<V>& a1, Vec<V>& a2, Vec<V>& b0, Vec<V>& b1, Vec<V>& b2) {
+                                          Vec<V>& a1, Vec<V>& a2, Vec<V>& b0, Vec<V>& b1, Vec<V>& b2, int n = V) {
     unsigned m[V];
     if constexpr (V == 4) {
         if (mi.m8 != nullptr) {
             m[0] = x.a & 0xffu; m[1] = (x.a >> 8) & 0xffu; m[2] = (x.a >> 16) & 0xffu; m[3] = x.a >> 24;
         } else {
             m[0] = x.a & 0xffffu; m[1] = x.a >> 16; m[2] = x.b & 0xffffu; m[3] = x.b >> 16;
+        }
+        if constexpr (RAG) {
+#pragma unroll
+            for (int e = 1; e < V; ++e) m[e] = e < n ? m[e] : 0u;
         }
     } else {
         m[0] = x.a;
@@ -174,33 +185,10 @@ __device__ __forceinline__ void coef_from(const MatIndex& mi, const MatIdx& x, c
 }
 
 // The index load and the row reads at once (the H update's form).
-template <int V>
+template <int V, bool RAG = false>
 __device__ __forceinline__ void coef_rows(const MatIndex& mi, size_t p, const float2* tab, Vec<V>& a0,
-                                          Vec<V>& a1, Vec<V>& a2, Vec<V>& b0, Vec<V>& b1, Vec<V>& b2) {
-    unsigned m[V];
-    if (mi.m8 != nullptr) {
-        if constexpr (V == 4) {
-            const unsigned t = __builtin_nontemporal_load(reinterpret_cast<const unsigned*>(mi.m8 + p));
-            m[0] = t & 0xffu; m[1] = (t >> 8) & 0xffu; m[2] = (t >> 16) & 0xffu; m[3] = t >> 24;
-        } else {
-            m[0] = mi.m8[p];
-        }
-    } else if (mi.m16 == nullptr) {
-#pragma unroll
-        for (int e = 0; e < V; ++e) m[e] = 0;
-    } else if constexpr (V == 4) {
-        const u2v t = __builtin_nontemporal_load(reinterpret_cast<const u2v*>(mi.m16 + p));
-        m[0] = t.x & 0xffffu; m[1] = t.x >> 16; m[2] = t.y & 0xffffu; m[3] = t.y >> 16;
-    } else {
-        m[0] = mi.m16[p];
-    }
-#pragma unroll
-    for (int e = 0; e < V; ++e) {
-        const float2 x = tab[3 * m[e]], y = tab[3 * m[e] + 1], z = tab[3 * m[e] + 2];
-        a0.v[e] = x.x; b0.v[e] = x.y;
-        a1.v[e] = y.x; b1.v[e] = y.y;
-        a2.v[e] = z.x; b2.v[e] = z.y;
-    }
+                                          Vec<V>& a1, Vec<V>& a2, Vec<V>& b0, Vec<V>& b1, Vec<V>& b2, int n = V) {
+    coef_from<V, RAG>(mi, coef_index<V, RAG>(mi, p), tab, a0, a1, a2, b0, b1, b2, n);
 }
 
 // kfirst / klast: the lane's left / right k neighbour along the row is not
@@ -266,14 +254,15 @@ struct Psi {
     float* wn;
     Vec<V> pp, pn;   // loaded values
     Vec<V> b, a, km; // per-cell table values
+    int e0, e1;      // RAG: the lane's cells inside the slab and the row, e0 <= e < e1
 };
 
 // Loads psi of face f (2d or 2d+1, or -1 for the dummy line) and the three
 // tables; tables of x and y faces are uniform over the V cells, those of z
 // faces step with k.  Faces are chosen with selects (no dynamic indexing of
 // the argument arrays, which would spill them to scratch).
-template <int V, bool ZAXIS>
-__device__ __forceinline__ void psi_load(Psi<V>& s, const CpmlArgs& c, int d, int f, int l, size_t q,
+template <int V, bool ZAXIS, bool RAG = false>
+__device__ __forceinline__ void psi_load(Psi<V>& s, const CpmlArgs& c, int d, int f, int l, long q,
                                          float* const* pos, float* const* neg, float* const* wpos,
                                          float* const* wneg, int tb, int ta, int tk) {
     s.f = f;
@@ -288,14 +277,14 @@ __device__ __forceinline__ void psi_load(Psi<V>& s, const CpmlArgs& c, int d, in
     s.n = on ? Q + q : c.dummy;
     s.wp = on ? WP + q : nullptr;
     s.wn = on ? WQ + q : nullptr;
-    s.pp = ldv<V>(s.p);
-    s.pn = ldv<V>(s.n);
+    s.pp = ldv<V, RAG>(s.p);
+    s.pn = ldv<V, RAG>(s.n);
     const float* T = c.tab + (size_t)fs * CPML_TABLES * c.Lmax;
     const int lt = on ? l : 0;
     if constexpr (ZAXIS) {
-        s.b = ldv<V>(T + tb * c.Lmax + lt);
-        s.a = ldv<V>(T + ta * c.Lmax + lt);
-        s.km = ldv<V>(T + tk * c.Lmax + lt);
+        s.b = ldv<V, RAG>(T + tb * c.Lmax + lt);
+        s.a = ldv<V, RAG>(T + ta * c.Lmax + lt);
+        s.km = ldv<V, RAG>(T + tk * c.Lmax + lt);
     } else {
         const float b = T[tb * c.Lmax + lt], a = T[ta * c.Lmax + lt], km = T[tk * c.Lmax + lt];
 #pragma unroll
@@ -306,7 +295,7 @@ __device__ __forceinline__ void psi_load(Psi<V>& s, const CpmlArgs& c, int d, in
 // psi <- b psi + a D for the pos and neg recursions, then (physical) the
 // correction of the Q-term component c1 (+psi) and P-term component c2 (-psi):
 //   c1 += C1 (psi_pos - km D_pos),  c2 += C2 (km D_neg - psi_neg)
-template <int V, bool PHYS>
+template <int V, bool PHYS, bool RAG = false>
 __device__ __forceinline__ void psi_apply(Psi<V>& s, const float* dpos, const float* dneg, Vec<V>& c1,
                                           const Vec<V>& C1, Vec<V>& c2, const Vec<V>& C2, const bool* upd) {
 #pragma unroll
@@ -314,7 +303,7 @@ __device__ __forceinline__ void psi_apply(Psi<V>& s, const float* dpos, const fl
         s.pp.v[e] = s.b.v[e] * s.pp.v[e] + s.a.v[e] * dpos[e];
         s.pn.v[e] = s.b.v[e] * s.pn.v[e] + s.a.v[e] * dneg[e];
         if constexpr (PHYS) {
-            if (s.f >= 0 && upd[e]) {  // off-slab cells computed psi from the dummy line: no correction
+            if (s.f >= 0 && upd[e] && (!RAG || (e >= s.e0 && e < s.e1))) {  // off-slab cells computed psi from the dummy line: no correction
                 c1.v[e] = c1.v[e] + C1.v[e] * (s.pp.v[e] - s.km.v[e] * dpos[e]);
                 c2.v[e] = c2.v[e] + C2.v[e] * (s.km.v[e] * dneg[e] - s.pn.v[e]);
             }
@@ -322,18 +311,46 @@ __device__ __forceinline__ void psi_apply(Psi<V>& s, const float* dpos, const fl
     }
 }
 
-template <int V>
+template <int V, bool RAG = false>
 __device__ __forceinline__ void psi_store(const Psi<V>& s) {
-    if (s.f >= 0) {
-        stv<V>(s.wp, s.pp);
-        stv<V>(s.wn, s.pn);
+    if (s.f < 0) return;
+    if (!RAG || (s.e0 == 0 && s.e1 == V)) {
+        stn<V, false, RAG>(s.wp, s.pp);
+        stn<V, false, RAG>(s.wn, s.pn);
+    } else {
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+            if (e >= s.e0 && e < s.e1) {
+                s.wp[e] = s.pp.v[e];
+                s.wn[e] = s.pn.v[e];
+            }
     }
+}
+
+// The z face a lane's cells [k0, k0 + V) meet, or -1, and the slab index of
+// the first one.  RAG: a lane may straddle a slab's edge (l then reaches from
+// -V + 1 on; the host keeps the two slabs 3 cells apart, so no lane meets
+// both).
+template <int V, bool RAG>
+__device__ __forceinline__ int zface_of(const CpmlArgs& c, int k0, int& l) {
+    if constexpr (!RAG) return face_of(c, 2, k0, l);
+    if ((c.on_mask >> 4 & 1) && k0 < c.L[4]) { l = k0; return 4; }
+    if ((c.on_mask >> 5 & 1) && k0 + V > c.g0[5]) { l = k0 - c.g0[5]; return 5; }
+    l = 0;
+    return -1;
+}
+
+// The lane's cells inside z slab [0, Lz) and the row (n cells).
+template <int V>
+__device__ __forceinline__ void zspan(Psi<V>& s, int l, int Lz, int n) {
+    s.e0 = max(0, -l);
+    s.e1 = min(n, Lz - l);
 }
 
 // AX: CPML axes compiled in (AX_X | AX_Y | AX_Z); PHYS: apply the field
 // correction (else psi only, as the reference); TAB: coefficients from the
 // material table (mat, tab in LDS) instead of the arrays in Cf.
-template <int V, int AX, bool PHYS, bool TAB>
+template <int V, int AX, bool PHYS, bool TAB, bool RAG = false>
 __device__ __forceinline__ void h_body(const Grid& g, const float* Fin, float* Fout, const float* __restrict__ Cf,
                                        const MatIndex mat, const float2* tab,
                                        const CpmlArgs& c, const Tile& t) {
@@ -365,10 +382,11 @@ __device__ __forceinline__ void h_body(const Grid& g, const float* Fin, float* F
     int ly = 0, lz = 0;
     int fy = -1, fz = -1;
     if constexpr ((AX & AX_Y) != 0) fy = face_of(c, 1, j, ly);
-    if constexpr ((AX & AX_Z) != 0) fz = face_of(c, 2, k0, lz);
+    if constexpr ((AX & AX_Z) != 0) fz = zface_of<V, RAG>(c, k0, lz);
+    const int nv = RAG ? min(V, nz - k0) : V;  // the lane's cells
     size_t p = (size_t)t.i0 * plane + (size_t)j * nz + k0;
-    Vec<V> ey_c = ldv<V>(Ey + p);
-    Vec<V> ez_c = ldv<V>(Ez + p);
+    Vec<V> ey_c = ldv<V, RAG>(Ey + p);
+    Vec<V> ez_c = ldv<V, RAG>(Ez + p);
     bool upd[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) upd[e] = true;
@@ -377,14 +395,14 @@ __device__ __forceinline__ void h_body(const Grid& g, const float* Fin, float* F
         const bool hi = i + 1 < nx;
         Vec<V> ey_n = ey_c, ez_n = ez_c;
         if (hi) {
-            ey_n = ldv<V>(Ey + p + plane);
-            ez_n = ldv<V>(Ez + p + plane);
+            ey_n = ldv<V, RAG>(Ey + p + plane);
+            ez_n = ldv<V, RAG>(Ez + p + plane);
         }
-        const Vec<V> ex_c = ldv<V>(Ex + p);
+        const Vec<V> ex_c = ldv<V, RAG>(Ex + p);
         Vec<V> ez_j = ez_c, ex_j = ex_c;
         if (hj) {
-            ez_j = ldv<V>(Ez + p + nz);
-            ex_j = ldv<V>(Ex + p + nz);
+            ez_j = ldv<V, RAG>(Ez + p + nz);
+            ex_j = ldv<V, RAG>(Ex + p + nz);
         }
         // the k + V neighbour: the next lane's first cell, or a load where
         // that lane holds another row (or sits in another wave)
@@ -395,34 +413,39 @@ __device__ __forceinline__ void h_body(const Grid& g, const float* Fin, float* F
             ey_kl = t.klast ? Ey[p + V] : ey_sh;
             ex_kl = t.klast ? Ex[p + V] : ex_sh;
         }
-        Vec<V> hx = ldn<V, OE_NT_OWN>(Hx + p), hy = ldn<V, OE_NT_OWN>(Hy + p), hz = ldn<V, OE_NT_OWN>(Hz + p);
+        Vec<V> hx = ldn<V, OE_NT_OWN, RAG>(Hx + p), hy = ldn<V, OE_NT_OWN, RAG>(Hy + p), hz = ldn<V, OE_NT_OWN, RAG>(Hz + p);
         Vec<V> a0, a1, a2, b0, b1, b2;
         if constexpr (TAB) {
-            coef_rows<V>(mat, p, tab, a0, a1, a2, b0, b1, b2);
+            coef_rows<V, RAG>(mat, p, tab, a0, a1, a2, b0, b1, b2, nv);
         } else {
-            a0 = ldn<V, OE_NT_COEF>(da0 + p); a1 = ldn<V, OE_NT_COEF>(da1 + p); a2 = ldn<V, OE_NT_COEF>(da2 + p);
-            b0 = ldn<V, OE_NT_COEF>(db0 + p); b1 = ldn<V, OE_NT_COEF>(db1 + p); b2 = ldn<V, OE_NT_COEF>(db2 + p);
+            a0 = ldn<V, OE_NT_COEF, RAG>(da0 + p); a1 = ldn<V, OE_NT_COEF, RAG>(da1 + p); a2 = ldn<V, OE_NT_COEF, RAG>(da2 + p);
+            b0 = ldn<V, OE_NT_COEF, RAG>(db0 + p); b1 = ldn<V, OE_NT_COEF, RAG>(db1 + p); b2 = ldn<V, OE_NT_COEF, RAG>(db2 + p);
         }
 
         Psi<V> px, py, pz;
         if constexpr ((AX & AX_X) != 0) {
             int lx;
             const int fx = face_of(c, 0, i, lx);
-            psi_load<V, false>(px, c, 0, fx, lx, ((size_t)lx * ny + j) * nz + k0, c.ph_pos, c.ph_neg, c.phw_pos, c.phw_neg, TAB_BH, TAB_AH, TAB_KH);
+            px.e0 = 0;
+            px.e1 = nv;
+            psi_load<V, false, RAG>(px, c, 0, fx, lx, ((long)lx * ny + j) * nz + k0, c.ph_pos, c.ph_neg, c.phw_pos, c.phw_neg, TAB_BH, TAB_AH, TAB_KH);
         }
         if constexpr ((AX & AX_Y) != 0) {
             const int Ly = fy == 2 ? c.L[2] : (fy == 3 ? c.L[3] : 0);
-            psi_load<V, false>(py, c, 1, fy, ly, ((size_t)i * Ly + ly) * nz + k0, c.ph_pos, c.ph_neg, c.phw_pos, c.phw_neg, TAB_BH, TAB_AH, TAB_KH);
+            py.e0 = 0;
+            py.e1 = nv;
+            psi_load<V, false, RAG>(py, c, 1, fy, ly, ((long)i * Ly + ly) * nz + k0, c.ph_pos, c.ph_neg, c.phw_pos, c.phw_neg, TAB_BH, TAB_AH, TAB_KH);
         }
         if constexpr ((AX & AX_Z) != 0) {
             const int Lz = fz == 4 ? c.L[4] : (fz == 5 ? c.L[5] : 0);
-            psi_load<V, true>(pz, c, 2, fz, lz, ((size_t)i * ny + j) * Lz + lz, c.ph_pos, c.ph_neg, c.phw_pos, c.phw_neg, TAB_BH, TAB_AH, TAB_KH);
+            zspan<V>(pz, lz, Lz, nv);
+            psi_load<V, true, RAG>(pz, c, 2, fz, lz, ((long)i * ny + j) * Lz + lz, c.ph_pos, c.ph_neg, c.phw_pos, c.phw_neg, TAB_BH, TAB_AH, TAB_KH);
         }
 
         float dEz_x[V], dEy_x[V], dEx_y[V], dEz_y[V], dEy_z[V], dEx_z[V];
 #pragma unroll
         for (int e = 0; e < V; ++e) {
-            const bool hk = (e < V - 1) || hk_last;
+            const bool hk = RAG ? k0 + e + 1 < nz : (e < V - 1) || hk_last;
             const float eyk = (e < V - 1) ? ey_c.v[(e < V - 1) ? e + 1 : e] : ey_kl;
             const float exk = (e < V - 1) ? ex_c.v[(e < V - 1) ? e + 1 : e] : ex_kl;
             const float dez_dy = hj ? ez_j.v[e] - ez_c.v[e] : 0.f;
@@ -443,18 +466,18 @@ __device__ __forceinline__ void h_body(const Grid& g, const float* Fin, float* F
         }
 
         // x: psi_pos <- dEz/dx (Hy, Q-term), psi_neg <- dEy/dx (Hz, P-term)
-        if constexpr ((AX & AX_X) != 0) psi_apply<V, PHYS>(px, dEz_x, dEy_x, hy, b1, hz, b2, upd);
+        if constexpr ((AX & AX_X) != 0) psi_apply<V, PHYS, RAG>(px, dEz_x, dEy_x, hy, b1, hz, b2, upd);
         // y: psi_pos <- dEx/dy (Hz), psi_neg <- dEz/dy (Hx)
-        if constexpr ((AX & AX_Y) != 0) psi_apply<V, PHYS>(py, dEx_y, dEz_y, hz, b2, hx, b0, upd);
+        if constexpr ((AX & AX_Y) != 0) psi_apply<V, PHYS, RAG>(py, dEx_y, dEz_y, hz, b2, hx, b0, upd);
         // z: psi_pos <- dEy/dz (Hx), psi_neg <- dEx/dz (Hy)
-        if constexpr ((AX & AX_Z) != 0) psi_apply<V, PHYS>(pz, dEy_z, dEx_z, hx, b0, hy, b1, upd);
-        if constexpr ((AX & AX_X) != 0) psi_store<V>(px);
-        if constexpr ((AX & AX_Y) != 0) psi_store<V>(py);
-        if constexpr ((AX & AX_Z) != 0) psi_store<V>(pz);
+        if constexpr ((AX & AX_Z) != 0) psi_apply<V, PHYS, RAG>(pz, dEy_z, dEx_z, hx, b0, hy, b1, upd);
+        if constexpr ((AX & AX_X) != 0) psi_store<V, RAG>(px);
+        if constexpr ((AX & AX_Y) != 0) psi_store<V, RAG>(py);
+        if constexpr ((AX & AX_Z) != 0) psi_store<V, RAG>(pz);
 
-        stn<V, OE_NT_STORE>(Hxw + p, hx);
-        stn<V, OE_NT_STORE>(Hyw + p, hy);
-        stn<V, OE_NT_STORE>(Hzw + p, hz);
+        stn<V, OE_NT_STORE, RAG>(Hxw + p, hx, nv);
+        stn<V, OE_NT_STORE, RAG>(Hyw + p, hy, nv);
+        stn<V, OE_NT_STORE, RAG>(Hzw + p, hz, nv);
         ey_c = ey_n;
         ez_c = ez_n;
     }
@@ -501,12 +524,12 @@ __device__ __forceinline__ void apply_sources(const Sources& src, size_t p, Vec<
 // update skips (i = 0 or j = 0) get the same writes from their old values.
 // Valid when no other hook acts on those cells between the E update and the
 // Mur post step (the host checks it).
-template <int V, int AX, bool PHYS, bool TAB, bool MUR = false>
+template <int V, int AX, bool PHYS, bool TAB, bool MUR = false, bool RAG = false>
 __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* Fout, const float* __restrict__ Cf,
                                        const MatIndex mat, const float2* tab,
                                        const CpmlArgs& c, const Tile& t, const Sources* src = nullptr,
                                        const MurZ& mz = MurZ{}) {
-    static_assert(!MUR || V == 4, "the folded Mur needs float4 lanes");
+    static_assert(!MUR || (V == 4 && !RAG), "the folded Mur needs whole float4 lanes");
     const int ny = g.ny, nz = g.nz;
     if (t.k0 >= nz || t.j >= t.jend) return;
     const size_t N = g.N;
@@ -535,12 +558,13 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
     int ly = 0, lz = 0;
     int fy = -1, fz = -1;
     if constexpr ((AX & AX_Y) != 0) fy = face_of(c, 1, j, ly);
-    if constexpr ((AX & AX_Z) != 0) fz = face_of(c, 2, k0, lz);
+    if constexpr ((AX & AX_Z) != 0) fz = zface_of<V, RAG>(c, k0, lz);
+    const int nv = RAG ? min(V, nz - k0) : V;  // the lane's cells
     size_t p = (size_t)t.i0 * plane + (size_t)j * nz + k0;
     Vec<V> hy_p = zerov<V>(), hz_p = zerov<V>();
     if (t.i0 > 0) {
-        hy_p = ldv<V>(Hy + p - plane);
-        hz_p = ldv<V>(Hz + p - plane);
+        hy_p = ldv<V, RAG>(Hy + p - plane);
+        hz_p = ldv<V, RAG>(Hz + p - plane);
     }
     // lanes of the folded Mur faces held by this thread
     const bool mur_lo = MUR && mz.on[0] && k0 == 0;
@@ -549,7 +573,7 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
     // plane need not wait for that plane's field loads
     MatIdx mi_c;
     if constexpr (TAB) {
-        if (gj && t.i0 > 0) mi_c = coef_index<V>(mat, p);
+        if (gj && t.i0 > 0) mi_c = coef_index<V, RAG>(mat, p);
     }
 
     for (int i = t.i0; i < t.i1; ++i, p += plane) {
@@ -557,13 +581,13 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
         const bool row = gi && gj;
         MatIdx mi_n;
         if constexpr (TAB) {
-            if (gj && i + 1 < t.i1) mi_n = coef_index<V>(mat, p + plane);
+            if (gj && i + 1 < t.i1) mi_n = coef_index<V, RAG>(mat, p + plane);
         }
-        const Vec<V> hx_c = ldv<V>(Hx + p), hy_c = ldv<V>(Hy + p), hz_c = ldv<V>(Hz + p);
+        const Vec<V> hx_c = ldv<V, RAG>(Hx + p), hy_c = ldv<V, RAG>(Hy + p), hz_c = ldv<V, RAG>(Hz + p);
         Vec<V> hz_j = hz_c, hx_j = hx_c;
         if (gj) {
-            hz_j = ldv<V>(Hz + p - nz);
-            hx_j = ldv<V>(Hx + p - nz);
+            hz_j = ldv<V, RAG>(Hz + p - nz);
+            hx_j = ldv<V, RAG>(Hx + p - nz);
         }
         // the k - 1 neighbour: the previous lane's last cell, or a load where
         // that lane holds another row (or sits in another wave)
@@ -576,12 +600,12 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
         }
         Vec<V> ex, ey, ez, c0, c1, c2, s0, s1, s2;
         if (row) {
-            ex = ldn<V, OE_NT_OWN>(Ex + p); ey = ldn<V, OE_NT_OWN>(Ey + p); ez = ldn<V, OE_NT_OWN>(Ez + p);
+            ex = ldn<V, OE_NT_OWN, RAG>(Ex + p); ey = ldn<V, OE_NT_OWN, RAG>(Ey + p); ez = ldn<V, OE_NT_OWN, RAG>(Ez + p);
             if constexpr (TAB) {
-                coef_from<V>(mat, mi_c, tab, s0, s1, s2, c0, c1, c2);
+                coef_from<V, RAG>(mat, mi_c, tab, s0, s1, s2, c0, c1, c2, nv);
             } else {
-                s0 = ldn<V, OE_NT_COEF>(ca0 + p); s1 = ldn<V, OE_NT_COEF>(ca1 + p); s2 = ldn<V, OE_NT_COEF>(ca2 + p);
-                c0 = ldn<V, OE_NT_COEF>(cb0 + p); c1 = ldn<V, OE_NT_COEF>(cb1 + p); c2 = ldn<V, OE_NT_COEF>(cb2 + p);
+                s0 = ldn<V, OE_NT_COEF, RAG>(ca0 + p); s1 = ldn<V, OE_NT_COEF, RAG>(ca1 + p); s2 = ldn<V, OE_NT_COEF, RAG>(ca2 + p);
+                c0 = ldn<V, OE_NT_COEF, RAG>(cb0 + p); c1 = ldn<V, OE_NT_COEF, RAG>(cb1 + p); c2 = ldn<V, OE_NT_COEF, RAG>(cb2 + p);
             }
         }
         // Mur pre step on the old values: v = E(shift) - c E(line)
@@ -589,8 +613,8 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
         if constexpr (MUR) {
             if (mur_lo || mur_hi) {
                 if (!row) {
-                    ex = ldn<V, OE_NT_OWN>(Ex + p);
-                    ey = ldn<V, OE_NT_OWN>(Ey + p);
+                    ex = ldn<V, OE_NT_OWN, RAG>(Ex + p);
+                    ey = ldn<V, OE_NT_OWN, RAG>(Ey + p);
                 }
                 if (mur_lo) {
                     mvx[0] = ex.v[1] - mz.coeff[0] * ex.v[0];
@@ -607,15 +631,20 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
         if constexpr ((AX & AX_X) != 0) {
             int lx;
             const int fx = face_of(c, 0, i, lx);
-            psi_load<V, false>(px, c, 0, fx, lx, ((size_t)lx * ny + j) * nz + k0, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg, TAB_BE, TAB_AE, TAB_KE);
+            px.e0 = 0;
+            px.e1 = nv;
+            psi_load<V, false, RAG>(px, c, 0, fx, lx, ((long)lx * ny + j) * nz + k0, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg, TAB_BE, TAB_AE, TAB_KE);
         }
         if constexpr ((AX & AX_Y) != 0) {
             const int Ly = fy == 2 ? c.L[2] : (fy == 3 ? c.L[3] : 0);
-            psi_load<V, false>(py, c, 1, fy, ly, ((size_t)i * Ly + ly) * nz + k0, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg, TAB_BE, TAB_AE, TAB_KE);
+            py.e0 = 0;
+            py.e1 = nv;
+            psi_load<V, false, RAG>(py, c, 1, fy, ly, ((long)i * Ly + ly) * nz + k0, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg, TAB_BE, TAB_AE, TAB_KE);
         }
         if constexpr ((AX & AX_Z) != 0) {
             const int Lz = fz == 4 ? c.L[4] : (fz == 5 ? c.L[5] : 0);
-            psi_load<V, true>(pz, c, 2, fz, lz, ((size_t)i * ny + j) * Lz + lz, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg, TAB_BE, TAB_AE, TAB_KE);
+            zspan<V>(pz, lz, Lz, nv);
+            psi_load<V, true, RAG>(pz, c, 2, fz, lz, ((long)i * ny + j) * Lz + lz, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg, TAB_BE, TAB_AE, TAB_KE);
         }
 
         float dHz_y[V], dHy_z[V], dHx_z[V], dHz_x[V], dHy_x[V], dHx_y[V];
@@ -648,14 +677,14 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
         }
 
         // x: psi_pos <- dHz/dx (Ey, Q-term), psi_neg <- dHy/dx (Ez, P-term)
-        if constexpr ((AX & AX_X) != 0) psi_apply<V, PHYS>(px, dHz_x, dHy_x, ey, c1, ez, c2, upd);
+        if constexpr ((AX & AX_X) != 0) psi_apply<V, PHYS, RAG>(px, dHz_x, dHy_x, ey, c1, ez, c2, upd);
         // y: psi_pos <- dHx/dy (Ez), psi_neg <- dHz/dy (Ex)
-        if constexpr ((AX & AX_Y) != 0) psi_apply<V, PHYS>(py, dHx_y, dHz_y, ez, c2, ex, c0, upd);
+        if constexpr ((AX & AX_Y) != 0) psi_apply<V, PHYS, RAG>(py, dHx_y, dHz_y, ez, c2, ex, c0, upd);
         // z: psi_pos <- dHy/dz (Ex), psi_neg <- dHx/dz (Ey)
-        if constexpr ((AX & AX_Z) != 0) psi_apply<V, PHYS>(pz, dHy_z, dHx_z, ex, c0, ey, c1, upd);
-        if constexpr ((AX & AX_X) != 0) psi_store<V>(px);
-        if constexpr ((AX & AX_Y) != 0) psi_store<V>(py);
-        if constexpr ((AX & AX_Z) != 0) psi_store<V>(pz);
+        if constexpr ((AX & AX_Z) != 0) psi_apply<V, PHYS, RAG>(pz, dHy_z, dHx_z, ex, c0, ey, c1, upd);
+        if constexpr ((AX & AX_X) != 0) psi_store<V, RAG>(px);
+        if constexpr ((AX & AX_Y) != 0) psi_store<V, RAG>(py);
+        if constexpr ((AX & AX_Z) != 0) psi_store<V, RAG>(pz);
 
         // Mur post step and boundary write: v += c E(shift), E(line) = v
         if constexpr (MUR) {
@@ -668,20 +697,20 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
                 ey.v[V - 1] = mvy[1] + mz.coeff[1] * ey.v[V - 2];
             }
             if (!row && (mur_lo || mur_hi)) {
-                stn<V, OE_NT_STORE>(Exw + p, ex);
-                stn<V, OE_NT_STORE>(Eyw + p, ey);
+                stn<V, OE_NT_STORE, RAG>(Exw + p, ex, nv);
+                stn<V, OE_NT_STORE, RAG>(Eyw + p, ey, nv);
             }
         }
 
         if (row) {
             if (src) apply_sources<V>(*src, p, ex, ey, ez);
-            stn<V, OE_NT_STORE>(Exw + p, ex);
-            stn<V, OE_NT_STORE>(Eyw + p, ey);
-            stn<V, OE_NT_STORE>(Ezw + p, ez);
+            stn<V, OE_NT_STORE, RAG>(Exw + p, ex, nv);
+            stn<V, OE_NT_STORE, RAG>(Eyw + p, ey, nv);
+            stn<V, OE_NT_STORE, RAG>(Ezw + p, ez, nv);
         } else if (copy_all) {  // index-0 planes and rows keep their value
-            stn<V, OE_NT_STORE>(Exw + p, ldn<V, OE_NT_OWN>(Ex + p));
-            stn<V, OE_NT_STORE>(Eyw + p, ldn<V, OE_NT_OWN>(Ey + p));
-            stn<V, OE_NT_STORE>(Ezw + p, ldn<V, OE_NT_OWN>(Ez + p));
+            stn<V, OE_NT_STORE, RAG>(Exw + p, ldn<V, OE_NT_OWN, RAG>(Ex + p), nv);
+            stn<V, OE_NT_STORE, RAG>(Eyw + p, ldn<V, OE_NT_OWN, RAG>(Ey + p), nv);
+            stn<V, OE_NT_STORE, RAG>(Ezw + p, ldn<V, OE_NT_OWN, RAG>(Ez + p), nv);
         }
         hy_p = hy_c;
         hz_p = hz_c;
@@ -697,7 +726,7 @@ constexpr bool RIDES = (AX & (AX_X | AX_Y)) == 0;
 // One grid: the tile comes from the launch's box list.  With TAB the
 // work-group first copies its half's material rows into LDS (dynamic LDS of
 // 24 bytes per row).
-template <int V, int AX, bool PHYS, bool TAB>
+template <int V, int AX, bool PHYS, bool TAB, bool RAG = false>
 __global__ __launch_bounds__(256) void k_update_h(YeeArgs a, CpmlArgs c) {
     extern __shared__ float2 lds_rows[];
     // the step's first launch advances the step counter (no H lane reads it)
@@ -713,12 +742,12 @@ __global__ __launch_bounds__(256) void k_update_h(YeeArgs a, CpmlArgs c) {
         for (int q = threadIdx.x; q < 3 * a.n_mat_h; q += blockDim.x) lds_rows[q] = src[q];
         __syncthreads();
     }
-    h_body<V, AX, PHYS, TAB>(a.g, a.Fin, a.Fout, a.Cf, MatIndex{a.n_mat_h == 1 ? nullptr : a.mat_h, a.mat8_h}, lds_rows, c,
+    h_body<V, AX, PHYS, TAB, RAG>(a.g, a.Fin, a.Fout, a.Cf, MatIndex{a.n_mat_h == 1 ? nullptr : a.mat_h, a.mat8_h}, lds_rows, c,
                              decode<V>(a));
 }
 
 // The z-faces kernels are held to the 128 registers of 4 waves a SIMD.
-template <int V, int AX, bool PHYS, bool TAB, bool MUR = false>
+template <int V, int AX, bool PHYS, bool TAB, bool MUR = false, bool RAG = false>
 __global__ __launch_bounds__(256, V == 4 && AX == AX_Z ? 4 : 1) void k_update_e(YeeArgs a, CpmlArgs c) {
     extern __shared__ float2 lds_rows[];
     if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) *a.step_inc += 1;
@@ -736,9 +765,9 @@ __global__ __launch_bounds__(256, V == 4 && AX == AX_Z ? 4 : 1) void k_update_e(
     const MatIndex mat_e{a.n_mat_e == 1 ? nullptr : a.mat_e, a.mat8_e};
     if (MUR || a.n_exc) {
         const Sources src{a.exc, a.exc_idx, a.n_exc, a.exc_step, a.exc_step_dev};
-        e_body<V, AX, PHYS, TAB, MUR>(a.g, a.Fin, a.Fout, a.Cf, mat_e, lds_rows, c, decode<V>(a), &src, a.mur_z);
+        e_body<V, AX, PHYS, TAB, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat_e, lds_rows, c, decode<V>(a), &src, a.mur_z);
     } else {
-        e_body<V, AX, PHYS, TAB, MUR>(a.g, a.Fin, a.Fout, a.Cf, mat_e, lds_rows, c, decode<V>(a));
+        e_body<V, AX, PHYS, TAB, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat_e, lds_rows, c, decode<V>(a));
     }
 }
 
@@ -810,53 +839,53 @@ __global__ __launch_bounds__(256) void k_update_e_sweep(SweepArgs a) {
     e_body<V, AX, PHYS, TAB>(S.g, S.F, S.F, S.Cf, MatIndex{S.n_mat_e == 1 ? nullptr : S.mat_e, S.mat8_e}, lds_rows, S.c, t);
 }
 
-template <int V, int AX, bool PHYS>
+template <int V, int AX, bool PHYS, bool RAG>
 hipError_t launch_h_t(const YeeArgs& a, const CpmlArgs& c, hipStream_t s) {
+    const dim3 grid(a.n_ride + a.first[a.nbox]);
     if (a.n_mat_h > 0)
-        hipLaunchKernelGGL((k_update_h<V, AX, PHYS, true>), dim3(a.n_ride + a.first[a.nbox]), dim3(256),
-                           3 * a.n_mat_h * sizeof(float2), s, a, c);
+        hipLaunchKernelGGL((k_update_h<V, AX, PHYS, true, RAG>), grid, dim3(256), 3 * a.n_mat_h * sizeof(float2), s, a,
+                           c);
     else
-        hipLaunchKernelGGL((k_update_h<V, AX, PHYS, false>), dim3(a.n_ride + a.first[a.nbox]), dim3(256), 0, s, a, c);
+        hipLaunchKernelGGL((k_update_h<V, AX, PHYS, false, RAG>), grid, dim3(256), 0, s, a, c);
     return hipGetLastError();
 }
 
-template <int V, int AX, bool PHYS>
+template <int V, int AX, bool PHYS, bool RAG>
 hipError_t launch_e_t(const YeeArgs& a, const CpmlArgs& c, hipStream_t s) {
-    if constexpr (V == 4) {
-        if (a.mur_z.on[0] || a.mur_z.on[1]) {
+    const dim3 grid(a.n_ride + a.first[a.nbox]);
+    const size_t lds = 3 * (size_t)a.n_mat_e * sizeof(float2);
+    if (a.mur_z.on[0] || a.mur_z.on[1]) {
+        if constexpr (V == 4 && !RAG) {
             if (a.n_mat_e > 0)
-                hipLaunchKernelGGL((k_update_e<V, AX, PHYS, true, true>), dim3(a.n_ride + a.first[a.nbox]), dim3(256),
-                                   3 * a.n_mat_e * sizeof(float2), s, a, c);
+                hipLaunchKernelGGL((k_update_e<V, AX, PHYS, true, true>), grid, dim3(256), lds, s, a, c);
             else
-                hipLaunchKernelGGL((k_update_e<V, AX, PHYS, false, true>), dim3(a.n_ride + a.first[a.nbox]), dim3(256), 0, s, a,
-                                   c);
+                hipLaunchKernelGGL((k_update_e<V, AX, PHYS, false, true>), grid, dim3(256), 0, s, a, c);
             return hipGetLastError();
+        } else {
+            return hipErrorInvalidValue;  // needs whole float4 lanes
         }
-    } else {
-        if (a.mur_z.on[0] || a.mur_z.on[1]) return hipErrorInvalidValue;  // needs float4 lanes
     }
     if (a.n_mat_e > 0)
-        hipLaunchKernelGGL((k_update_e<V, AX, PHYS, true>), dim3(a.n_ride + a.first[a.nbox]), dim3(256),
-                           3 * a.n_mat_e * sizeof(float2), s, a, c);
+        hipLaunchKernelGGL((k_update_e<V, AX, PHYS, true, false, RAG>), grid, dim3(256), lds, s, a, c);
     else
-        hipLaunchKernelGGL((k_update_e<V, AX, PHYS, false>), dim3(a.n_ride + a.first[a.nbox]), dim3(256), 0, s, a, c);
+        hipLaunchKernelGGL((k_update_e<V, AX, PHYS, false, false, RAG>), grid, dim3(256), 0, s, a, c);
     return hipGetLastError();
 }
 
 // Instantiated variants: plain (no CPML), z faces only (interior of a CPML
 // grid) and all faces (the x/y face slabs), each in compat and physical
 // mode, each reading the material table or the coefficient arrays.
-template <bool H, int V>
+template <bool H, int V, int AX, bool PHYS, bool RAG>
+hipError_t launch_t(const YeeArgs& a, const CpmlArgs& c, hipStream_t s) {
+    return H ? launch_h_t<V, AX, PHYS, RAG>(a, c, s) : launch_e_t<V, AX, PHYS, RAG>(a, c, s);
+}
+template <bool H, int V, bool RAG>
 hipError_t dispatch(const YeeArgs& a, const CpmlArgs* c, int axes, hipStream_t s) {
-    const CpmlArgs none{};
-    if (!c || axes == 0) return H ? launch_h_t<V, 0, false>(a, none, s) : launch_e_t<V, 0, false>(a, none, s);
-    if (axes == AX_Z) {
-        if (c->physical) return H ? launch_h_t<V, AX_Z, true>(a, *c, s) : launch_e_t<V, AX_Z, true>(a, *c, s);
-        return H ? launch_h_t<V, AX_Z, false>(a, *c, s) : launch_e_t<V, AX_Z, false>(a, *c, s);
-    }
-    constexpr int ALL = AX_X | AX_Y | AX_Z;
-    if (c->physical) return H ? launch_h_t<V, ALL, true>(a, *c, s) : launch_e_t<V, ALL, true>(a, *c, s);
-    return H ? launch_h_t<V, ALL, false>(a, *c, s) : launch_e_t<V, ALL, false>(a, *c, s);
+    if (!c || axes == 0) return launch_t<H, V, 0, false, RAG>(a, CpmlArgs{}, s);
+    if (axes == AX_Z)
+        return c->physical ? launch_t<H, V, AX_Z, true, RAG>(a, *c, s) : launch_t<H, V, AX_Z, false, RAG>(a, *c, s);
+    constexpr int all = AX_X | AX_Y | AX_Z;
+    return c->physical ? launch_t<H, V, all, true, RAG>(a, *c, s) : launch_t<H, V, all, false, RAG>(a, *c, s);
 }
 
 // ------------------------------------------------------------ fused step
@@ -1399,11 +1428,13 @@ hipError_t launch_fused_t(const FusedArgs& a, const CpmlArgs& c, hipStream_t s) 
 }  // namespace
 
 hipError_t launch_update_h(const YeeArgs& a, const CpmlArgs* c, int axes, hipStream_t s) {
-    return a.t.vec == 4 ? dispatch<true, 4>(a, c, axes, s) : dispatch<true, 1>(a, c, axes, s);
+    if (a.t.vec != 4) return dispatch<true, 1, false>(a, c, axes, s);
+    return a.ragged ? dispatch<true, 4, true>(a, c, axes, s) : dispatch<true, 4, false>(a, c, axes, s);
 }
 
 hipError_t launch_update_e(const YeeArgs& a, const CpmlArgs* c, int axes, hipStream_t s) {
-    return a.t.vec == 4 ? dispatch<false, 4>(a, c, axes, s) : dispatch<false, 1>(a, c, axes, s);
+    if (a.t.vec != 4) return dispatch<false, 1, false>(a, c, axes, s);
+    return a.ragged ? dispatch<false, 4, true>(a, c, axes, s) : dispatch<false, 4, false>(a, c, axes, s);
 }
 
 bool fused_supported(const Grid& g) { return g.nz % 4 == 0 && g.nz >= 4 && g.nz <= 256; }
