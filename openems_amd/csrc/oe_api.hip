@@ -147,7 +147,7 @@ YeeArgs launch_args(const oe_engine* e, const Tiles& t, const CpmlArgs* cp, cons
 // to the all-faces kernel in one launch of up to four boxes, and the interior
 // planes and rows -- whose only slab cells are the z faces at the ends of each
 // row -- to the lighter z-faces kernel.  The boxes tile the grid exactly once.
-std::vector<Launch> plan_launches(const oe_engine* e, const Tiles& t, const CpmlArgs* cp) {
+std::vector<Launch> plan_launches(const oe_engine* e, const Tiles& t, const CpmlArgs* cp, bool mix) {
     std::vector<Launch> out;
     const Grid& g = e->g;
     if (!cp) {
@@ -173,8 +173,14 @@ std::vector<Launch> plan_launches(const oe_engine* e, const Tiles& t, const Cpml
         if (jy0 > 0) slabs.push_back(make_box(ts, ix0, ix1, 0, jy0));
         if (jy1 < g.ny) slabs.push_back(make_box(ts, ix0, ix1, jy1, g.ny));
     }
+    const bool inner = ix1 > ix0 && jy1 > jy0;
+    if (mix && inner && !slabs.empty()) {
+        slabs.push_back(make_box(t, ix0, ix1, jy0, jy1));
+        out.push_back({launch_args(e, t, cp, slabs), AX_MIX | ((m & 48) ? AX_Z : 0)});
+        return out;
+    }
     if (!slabs.empty()) out.push_back({launch_args(e, ts, cp, slabs), AX_X | AX_Y | AX_Z});
-    if (ix1 > ix0 && jy1 > jy0)
+    if (inner)
         out.push_back({launch_args(e, t, cp, {make_box(t, ix0, ix1, jy0, jy1)}), (m & 48) ? AX_Z : 0});
     return out;
 }
@@ -373,6 +379,7 @@ oe_status engine_alloc(oe_engine* e, size_t nx, size_t ny, size_t nz, int device
     if (const char* v = getenv("OE_MERGE_ADE")) e->merge_ade = atoi(v) != 0;
     if (const char* v = getenv("OE_BYTE_INDEX")) e->byte_index = atoi(v) != 0;
     if (const char* v = getenv("OE_RIDE")) e->ride = atoi(v) != 0;
+    if (const char* v = getenv("OE_MIX_CELLS")) e->mix_cells = (size_t)std::max(0L, atol(v));
     if (const char* v = getenv("OE_SLAB_TILES")) {  // "bx,by,ci,vec" of the CPML x/y slab launches
         Tiles t{};
         if (sscanf(v, "%d,%d,%d,%d", &t.bx, &t.by, &t.ci, &t.vec) == 4 && t.bx > 0 && t.bx <= 64 &&
@@ -708,6 +715,7 @@ oe_status oe_engine_set_tiles(oe_engine* e, int bx, int by, int ci, int vec) {
         t.by = by;
     }
     if (ci > 0) t.ci = std::min(ci, e->g.nx);
+    e->tiles_auto = bx <= 0 && by <= 0 && ci <= 0;
     e->tiles = t;
     return OE_OK;
 }
@@ -1755,7 +1763,6 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     Tiles tl = e->tiles;
     // a float4 lane meets at most one z slab, or lanes are scalar
     if (cp && !cp->zvec && tl.vec == 4 && (cp->on_mask & 48) == 48 && cp->g0[5] - cp->L[4] < 3) tl = auto_tiles(e->g, 1);
-    const std::vector<Launch> plan = plan_launches(e, tl, cp);
     // Fused steps (one pass per step over the plan's interior box) when no
     // extension hooks in between the half-steps and the grid suits the
     // fused kernel; the x/y CPML slabs keep their two launches around it.
@@ -1764,6 +1771,32 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     const bool host = !hosts.empty();
     const bool fused = e->fused_mode && !host && !upml && murs.empty() && ades.empty() && tl.vec == 4 &&
                        fused_supported(e->g) && (e->fused_mode == 2 || e->g.nz >= 128) && (!cp || cp->zvec);
+    // Small CPML grids with a material table take one launch per half-step:
+    // the second launch's start and tail cost more than the interior's halved
+    // occupancy up to about 4.5 M cells.  us per step, two launches / one (the
+    // best depth of each): 72x60x32 22.0 / 12.0, 100x100x48 24.6 / 17.6,
+    // 100^3 31.5 / 27.8, 160x144x128 63.3 / 55.4, 200x160x128 78.6 / 71.6,
+    // 240x200x128 101.7 / 102.4, 256^3 241 / 265.
+    const bool mix = cp && !fused && tl.vec == 4 && !e->overlap_slabs && e->slab_tiles.bx <= 0 && e->n_mat[0] > 0 &&
+                     e->n_mat[1] > 0 && e->g.N <= e->mix_cells;
+    if (mix && e->tiles_auto) {
+        // At 2 waves a SIMD the chip holds 512 of its work-groups at a time,
+        // and such grids fill it once to a few times: the depth that wastes
+        // least of the last fill (160x144x128, ci 1 .. 8: 60.9 57.7 56.7 62.5
+        // 70.3 55.4 60.3 65.7, of which 3 and 6 fill it twice and once).
+        double best = 1e300;
+        for (int ci = 1; ci <= std::min(8, e->g.nx); ++ci) {
+            Tiles t = tl;
+            t.ci = ci;
+            const YeeArgs a = plan_launches(e, t, cp, true).back().a;
+            const double cost = std::ceil(a.first[a.nbox] / 512.0) * (ci + 0.5);
+            if (cost < best) {
+                best = cost;
+                tl.ci = ci;
+            }
+        }
+    }
+    const std::vector<Launch> plan = plan_launches(e, tl, cp, mix);
     // Sources are added by the E kernels themselves when nothing acts on their
     // cells between the E update and them (no UPML, no ADE cell, no line or
     // shift plane of a Mur face), when every source cell is one the E update

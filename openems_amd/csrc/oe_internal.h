@@ -79,9 +79,9 @@ struct CpmlArgs {
     const float* dummy;  // 16 zeroed floats: load target for cells outside every slab
 };
 
-// A launch covers up to 4 boxes [i0,i1) x [j0,j1) x [0,nz); work-group ids
+// A launch covers up to 5 boxes [i0,i1) x [j0,j1) x [0,nz); work-group ids
 // are split over the boxes by prefix sums (first[b] .. first[b+1]).
-constexpr int MAX_BOXES = 4;
+constexpr int MAX_BOXES = 5;
 struct Box {
     int i0, i1, j0, j1;
     int n_jb, n_ib;  // j-blocks, i-chunks of this box
@@ -149,7 +149,9 @@ struct YeeArgs {
 };
 
 // CPML code compiled into a launch: bit 0 x faces, bit 1 y faces, bit 2 z faces.
-enum { AX_X = 1, AX_Y = 2, AX_Z = 4 };
+// AX_MIX: the x/y slabs (all faces) and, as the last box, the interior with
+// the other bits' faces in one launch.
+enum { AX_X = 1, AX_Y = 2, AX_Z = 4, AX_MIX = 8 };
 
 // Largest material table a half-step keeps in LDS (rows of 24 bytes).
 constexpr int MAX_MAT_ROWS = 1024;

@@ -133,6 +133,7 @@ struct oe_engine {
     uint8_t* mat8 = nullptr;  // [E: N][H: N] the indices as bytes, when a half has 2 to 256 rows
     uint64_t timestep = 0;
     Tiles tiles{};
+    bool tiles_auto = true;  // no shape was asked for
     Tiles slab_tiles{};  // tiles of the CPML x/y slab launches (bx = 0: the interior's)
     int xcd_remap = 1;
     double peak_persistent = 0.0;
@@ -147,6 +148,7 @@ struct oe_engine {
     DevBuf exc_samples;
     DevBuf step_dev;       // batch-relative step read by the kernels of a step, and steps begun
     DevBuf ride_table;     // the riders of the running batch (oe_ride.h)
+    size_t mix_cells = 4500000;  // most cells of a CPML grid whose slabs and interior share a launch
     int ride = 1;          // probes, small DFTs and captures in the Yee launches: 1 on, 0 off
     int graph_steps = 16;  // steps per captured graph (0: no graphs)
     // CPML slab launches on a second stream beside the interior launch of

@@ -203,12 +203,21 @@ struct Tile {
 // work-group ids to the 8 XCDs round-robin; the remap gives XCD x the
 // contiguous logical range [x*per, (x+1)*per) so that j-neighbouring tiles
 // run on the same XCD at the same time.
-template <int V>
-__device__ __forceinline__ Tile decode(const YeeArgs& a) {
+// MIX: the launch's last box is the interior, the boxes before it are slabs,
+// and each of the two kinds is spread over the XCDs by itself (their
+// work-groups do not cost the same); inner tells them apart.
+template <int V, bool MIX = false>
+__device__ __forceinline__ Tile decode(const YeeArgs& a, bool* inner = nullptr) {
     int bid = blockIdx.x - a.n_ride;
+    int seg0 = 0, seg1 = a.first[a.nbox];
+    if constexpr (MIX) {
+        *inner = bid >= a.first[a.nbox - 1];
+        if (*inner) seg0 = a.first[a.nbox - 1];
+        else seg1 = a.first[a.nbox - 1];
+    }
     if (a.xcd_remap) {
-        const int per = (gridDim.x - a.n_ride) >> 3;
-        if (bid < (per << 3)) bid = (bid & 7) * per + (bid >> 3);
+        const int per = (seg1 - seg0) >> 3, q = bid - seg0;
+        if (q < (per << 3)) bid = seg0 + (q & 7) * per + (q >> 3);
     }
     int b = 0;
 #pragma unroll
@@ -771,6 +780,51 @@ __global__ __launch_bounds__(256, V == 4 && AX == AX_Z ? 4 : 1) void k_update_e(
     }
 }
 
+// One launch for the x/y slabs (every face) and the interior (AXI: z faces or
+// none) of a CPML grid.  The slab code's registers leave 2 waves a SIMD for
+// both, so this is for grids whose launches are bound by their start and
+// their chain of loads, not by how many are in flight (plan_launches).
+template <int AXI, bool PHYS, bool RAG>
+__global__ __launch_bounds__(256) void k_update_h_mix(YeeArgs a, CpmlArgs c) {
+    constexpr int V = 4;
+    extern __shared__ float2 lds_rows[];
+    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) *a.step_inc += 1;
+    if ((int)blockIdx.x < a.n_ride) {
+        ride(*a.ride, blockIdx.x, true);
+        return;
+    }
+    const float2* src = reinterpret_cast<const float2*>(a.tab_h);
+    for (int q = threadIdx.x; q < 3 * a.n_mat_h; q += blockDim.x) lds_rows[q] = src[q];
+    __syncthreads();
+    const MatIndex mat{a.n_mat_h == 1 ? nullptr : a.mat_h, a.mat8_h};
+    bool inner;
+    const Tile t = decode<V, true>(a, &inner);
+    if (inner) h_body<V, AXI, PHYS && AXI != 0, true, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, lds_rows, c, t);
+    else h_body<V, AX_X | AX_Y | AX_Z, PHYS, true, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, lds_rows, c, t);
+}
+
+template <int AXI, bool PHYS, bool MUR, bool RAG>
+__global__ __launch_bounds__(256) void k_update_e_mix(YeeArgs a, CpmlArgs c) {
+    constexpr int V = 4;
+    extern __shared__ float2 lds_rows[];
+    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) *a.step_inc += 1;
+    if ((int)blockIdx.x < a.n_ride) {
+        ride(*a.ride, blockIdx.x, false);
+        return;
+    }
+    const float2* src = reinterpret_cast<const float2*>(a.tab_e);
+    for (int q = threadIdx.x; q < 3 * a.n_mat_e; q += blockDim.x) lds_rows[q] = src[q];
+    __syncthreads();
+    const MatIndex mat{a.n_mat_e == 1 ? nullptr : a.mat_e, a.mat8_e};
+    const Sources ex{a.exc, a.exc_idx, a.n_exc, a.exc_step, a.exc_step_dev};
+    bool inner;
+    const Tile t = decode<V, true>(a, &inner);
+    if (inner)
+        e_body<V, AXI, PHYS && AXI != 0, true, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, lds_rows, c, t, &ex, a.mur_z);
+    else
+        e_body<V, AX_X | AX_Y | AX_Z, PHYS, true, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, lds_rows, c, t, &ex, a.mur_z);
+}
+
 // Many grids in one launch (a parameter sweep): work-group -> box of some
 // structure through the launch's table; each box has its own tile shape
 // (bx * by * ns <= 256 lanes: ns i-chunks of by rows of bx lanes; surplus
@@ -879,6 +933,28 @@ template <bool H, int V, int AX, bool PHYS, bool RAG>
 hipError_t launch_t(const YeeArgs& a, const CpmlArgs& c, hipStream_t s) {
     return H ? launch_h_t<V, AX, PHYS, RAG>(a, c, s) : launch_e_t<V, AX, PHYS, RAG>(a, c, s);
 }
+template <bool H, int AXI, bool PHYS, bool RAG>
+hipError_t launch_mix_t(const YeeArgs& a, const CpmlArgs& c, hipStream_t s) {
+    const dim3 grid(a.n_ride + a.first[a.nbox]);
+    const size_t lds = 3 * (size_t)(H ? a.n_mat_h : a.n_mat_e) * sizeof(float2);
+    if constexpr (H) {
+        hipLaunchKernelGGL((k_update_h_mix<AXI, PHYS, RAG>), grid, dim3(256), lds, s, a, c);
+    } else if (a.mur_z.on[0] || a.mur_z.on[1]) {
+        if constexpr (RAG) return hipErrorInvalidValue;
+        else hipLaunchKernelGGL((k_update_e_mix<AXI, PHYS, true, false>), grid, dim3(256), lds, s, a, c);
+    } else {
+        hipLaunchKernelGGL((k_update_e_mix<AXI, PHYS, false, RAG>), grid, dim3(256), lds, s, a, c);
+    }
+    return hipGetLastError();
+}
+// One launch for slabs and interior: float4 lanes and a material table only.
+template <bool H, bool RAG>
+hipError_t dispatch_mix(const YeeArgs& a, const CpmlArgs& c, int axes, hipStream_t s) {
+    if (a.t.vec != 4 || (H ? a.n_mat_h : a.n_mat_e) <= 0 || a.nbox < 2) return hipErrorInvalidValue;
+    if (axes & AX_Z) return c.physical ? launch_mix_t<H, AX_Z, true, RAG>(a, c, s) : launch_mix_t<H, AX_Z, false, RAG>(a, c, s);
+    return c.physical ? launch_mix_t<H, 0, true, RAG>(a, c, s) : launch_mix_t<H, 0, false, RAG>(a, c, s);
+}
+
 template <bool H, int V, bool RAG>
 hipError_t dispatch(const YeeArgs& a, const CpmlArgs* c, int axes, hipStream_t s) {
     if (!c || axes == 0) return launch_t<H, V, 0, false, RAG>(a, CpmlArgs{}, s);
@@ -1427,14 +1503,19 @@ hipError_t launch_fused_t(const FusedArgs& a, const CpmlArgs& c, hipStream_t s) 
 
 }  // namespace
 
+template <bool H>
+static hipError_t launch_update(const YeeArgs& a, const CpmlArgs* c, int axes, hipStream_t s) {
+    if (axes & AX_MIX) return a.ragged ? dispatch_mix<H, true>(a, *c, axes, s) : dispatch_mix<H, false>(a, *c, axes, s);
+    if (a.t.vec != 4) return dispatch<H, 1, false>(a, c, axes, s);
+    return a.ragged ? dispatch<H, 4, true>(a, c, axes, s) : dispatch<H, 4, false>(a, c, axes, s);
+}
+
 hipError_t launch_update_h(const YeeArgs& a, const CpmlArgs* c, int axes, hipStream_t s) {
-    if (a.t.vec != 4) return dispatch<true, 1, false>(a, c, axes, s);
-    return a.ragged ? dispatch<true, 4, true>(a, c, axes, s) : dispatch<true, 4, false>(a, c, axes, s);
+    return launch_update<true>(a, c, axes, s);
 }
 
 hipError_t launch_update_e(const YeeArgs& a, const CpmlArgs* c, int axes, hipStream_t s) {
-    if (a.t.vec != 4) return dispatch<false, 1, false>(a, c, axes, s);
-    return a.ragged ? dispatch<false, 4, true>(a, c, axes, s) : dispatch<false, 4, false>(a, c, axes, s);
+    return launch_update<false>(a, c, axes, s);
 }
 
 bool fused_supported(const Grid& g) { return g.nz % 4 == 0 && g.nz >= 4 && g.nz <= 256; }

@@ -62,3 +62,19 @@ def test_riders_equal_launches_of_their_own(monkeypatch, shape, cpml, mur, batch
     for a, b in zip(got, ref):
         assert a.shape == b.shape and np.array_equal(a, b)
     assert np.abs(got[2]).max() > 0 or np.abs(got[3]).max() > 0
+
+
+@pytest.mark.parametrize("shape,cpml,mur", [((20, 18, 24), (4, 4, 4, 4, 4, 0), (0, 0, 0, 0, 0, 1)),
+                                            ((21, 19, 23), (3, 3, 3, 3, 3, 3), None), ((17, 40, 14), (0, 5, 5, 0, 0, 0), None),
+                                            ((12, 18, 16), (6, 6, 4, 4, 4, 4), None), ((40, 10, 100), (0, 0, 2, 3, 8, 8), None)],
+                         ids=["mur_z", "ragged", "no_z", "no_interior", "no_x"])
+@pytest.mark.parametrize("graph", [0, 4])
+def test_one_launch_per_half_step_equals_two(monkeypatch, shape, cpml, mur, graph):
+    """Slabs and interior in one launch against a launch each (OE_MIX_CELLS=0)."""
+    monkeypatch.setenv("OE_MIX_CELLS", "1000000")
+    got = _run(monkeypatch, 1, shape, cpml, mur, [(STEPS, None)], graph, 0)
+    monkeypatch.setenv("OE_MIX_CELLS", "0")
+    ref = _run(monkeypatch, 0, shape, cpml, mur, [(STEPS, None)], graph, 0)
+    for a, b in zip(got, ref):
+        assert a.shape == b.shape and np.array_equal(a, b)
+    assert np.abs(got[0]).max() > 0
