@@ -589,10 +589,11 @@ uint64_t oe_engine_timestep(const oe_engine* eng) { return eng ? eng->timestep :
 oe_status oe_engine_read_fields(oe_engine* e, float* const fields[6]) {
     if (!e || !fields) return fail(OE_ERR_CONFIG, "null argument");
     HIP_OK(hipSetDevice(e->device));
+    HostCopy c[6];
+    int n = 0;
     for (int d = 0; d < 6; ++d)
-        if (fields[d])
-            HIP_OK(hipMemcpyAsync(fields[d], e->F + (size_t)d * e->g.N, e->g.N * sizeof(float), hipMemcpyDeviceToHost, e->stream));
-    HIP_OK(hipStreamSynchronize(e->stream));
+        if (fields[d]) c[n++] = HostCopy{fields[d], e->F + (size_t)d * e->g.N, e->g.N * sizeof(float)};
+    HIP_OK(copy_to_host(c, n, e->stream));
     return OE_OK;
 }
 
@@ -644,8 +645,8 @@ oe_status oe_engine_read_coefficients(oe_engine* e, int which, float* out) {
     if (!e || !out) return fail(OE_ERR_CONFIG, "null argument");
     if (which < 0 || which >= 12) return fail(OE_ERR_CONFIG, "coefficient index %d out of range", which);
     HIP_OK(hipSetDevice(e->device));
-    HIP_OK(hipMemcpyAsync(out, e->Cf + (size_t)which * e->g.N, e->g.N * sizeof(float), hipMemcpyDeviceToHost, e->stream));
-    HIP_OK(hipStreamSynchronize(e->stream));
+    const HostCopy c{out, e->Cf + (size_t)which * e->g.N, e->g.N * sizeof(float)};
+    HIP_OK(copy_to_host(&c, 1, e->stream));
     return OE_OK;
 }
 

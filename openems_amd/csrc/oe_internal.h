@@ -236,6 +236,15 @@ struct SweepArgs {
 // table, rows being the largest table of the launch's half (LDS size).
 hipError_t launch_sweep(bool h, const SweepArgs& a, int n_wg, int axes, int vec, int rows, hipStream_t s);
 
+// Device arrays to pageable host memory after the work on s (oe_copy.hip);
+// returns when they are there.
+struct HostCopy {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+hipError_t copy_to_host(const HostCopy* c, int n, hipStream_t s);
+
 // Auxiliary kernels (oe_aux.hip).
 hipError_t launch_fill(float* p, size_t n, float v, hipStream_t s);
 // One region write of the coefficient block: cells [box0, box1) x [box2,

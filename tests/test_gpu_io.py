@@ -80,3 +80,23 @@ def test_vtk_dump_of_device_fields(tmp_path):
     vals = np.array([[np.float32(v) for v in l.split()] for l in lines[k:]], np.float32)
     assert vals.shape == (12, 3)
     assert np.array_equal(vals.T, E.reshape(3, -1))
+
+
+@pytest.mark.parametrize("shape", [(64, 64, 127), (64, 64, 128), (64, 64, 129), (128, 128, 44), (100, 90, 131)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_fields_read_back_through_the_ring(shape):
+    """Fields and coefficients on both sides of the staged copy's least size
+    and of its piece sizes come back as written, all six or one half."""
+    from openems_amd import HipEngine, Operator
+
+    rng = np.random.default_rng(5)
+    F = rng.standard_normal((6,) + shape).astype(np.float32)
+    op = Operator.uniform(*shape, 1e-3)
+    op.set_material(2.0, 1.5, 0.1, 0.0, (1, shape[0], 0, shape[1] - 1, 0, shape[2]))
+    eng = HipEngine(op)
+    eng.write_fields(F[:3], F[3:])
+    for _ in range(3):
+        E, H = eng.read_fields()
+        assert np.array_equal(E, F[:3]) and np.array_equal(H, F[3:])
+    c = eng.coefficients()
+    assert len(np.unique(c[0])) == 2 and np.array_equal(c[0], c[1]) and np.array_equal(c[0][0], np.ones(shape[1:], np.float32))
