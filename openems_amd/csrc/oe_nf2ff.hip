@@ -15,6 +15,14 @@
 // axis with the fewer distinct values (|cos t| on a (t, f) grid has at most
 // n_t of them).  The second contraction, the per-angle phase and the
 // projection are float64.
+//
+// Every step is one launch over all faces (up to 6 at a time), which read
+// their sizes and buffers from a table in device memory: pack, operands
+// (phase rows and split B), the contractions, the reduction, the projection.
+// The faces of a small box are a few microseconds of work each, so a launch
+// per face and step (about 35 of them, on two streams) was what a transform
+// of two pattern cuts cost: 232 us for 181 x 2 angles and 62 x 55 x 41 nodes,
+// where six launches take 77.
 
 #include "oe_internal.h"
 
@@ -46,15 +54,73 @@ constexpr int LDS_PAD = 32;  // row stride = tile + 32 words: the two half-waves
 // MFMA 32x32x2 operands: lane l supplies A[l % 32][l / 32] and
 // B[l / 32][l % 32]; accumulator register v of lane l holds
 // C[8 (v / 4) + 4 (l / 32) + (v % 4)][l % 32].
+//
+// A launch covers the faces of kind KIND_FP32 (TILE = 64) or KIND_FP32_LARGE
+// (128), each N / TILE x M / TILE work-groups from its first one on.  Rows of
+// B at and past np (the K padding) count as zeros whatever they hold.
+enum { KIND_FP32 = 0, KIND_FP32_LARGE = 1, KIND_SPLIT16 = 2 };
+
+// One face as the kernels see it.
+struct FaceDev {
+    const void* src;
+    double scale;
+    int kind, n1, n2, swap, sign;  // source layout (0 float64 pairs, 1 float32 quads), nodes, p is axis 2
+    int np, nq, K, N, nb;          // contraction sizes; work-groups of the pack
+    const double *xp, *wp, *xq, *wq;
+    float *B, *A, *G;              // operands and result of the first contraction
+    _Float16 *Bhi, *Blo;
+    float* bsc;                    // scale of the split B and its inverse
+    double* part;                  // radiated-power partials
+    float* pmax;                   // block maxima of |B|
+    int split;                     // some chunk runs on the FP16 matrix cores
+    const double* uval;
+    int uni_p, uni_q;
+    double dxp, dxq, x0;
+    const double *kapq, *kap0;     // per angle
+    const float* usgn;             // per angle: sign of kappa_p
+    const int* uidx;               // per angle: row
+    const int* order;              // angles sorted by row
+    const int2* groups;            // (first index into order, count <= REDUCE_M)
+    const int4* mgroups;           // mirror groups (row, first index into members, count, 0)
+    const double* gkq;             // per mirror group: |kappa_q| of its first member
+    const int* members;
+    double* S;                     // [n_ang][4] complex: this face's sums
+    int a1, a2;
+};
+
+// The part of a face in one chunk of rows.
+struct ChunkDev {
+    int kind;            // KIND_*
+    int u0, u1, M;       // rows u0 .. u1 (two each), padded
+    int first;           // its first work-group in the launch of its kind
+    int mirror;          // reduced by mirror groups [g0, g1), else by groups
+    int g0, g1;
+};
+constexpr int MAX_FACES = 6;
+
+// The face whose work-groups hold blockIdx.x in a launch over kind.
+__device__ __forceinline__ int face_of_block(const ChunkDev* ch, int nf, int kind) {
+    int f = -1;
+    for (int q = 0; q < nf; ++q)
+        if (ch[q].kind == kind && (int)blockIdx.x >= ch[q].first) f = q;
+    return f;
+}
+
 template <int TILE>
-__global__ __launch_bounds__(256) void k_sgemm_mfma(const float* __restrict__ A, const float* __restrict__ B,
-                                                   float* __restrict__ C, int M, int N, int K) {
+__global__ __launch_bounds__(256) void k_sgemm_mfma(const FaceDev* __restrict__ fc, const ChunkDev* __restrict__ ch,
+                                                    int nf) {
+    const int fi = face_of_block(ch, nf, TILE == 64 ? KIND_FP32 : KIND_FP32_LARGE);
+    const FaceDev& fd = fc[fi];
+    const float* __restrict__ A = fd.A;
+    const float* __restrict__ B = fd.B;
+    float* __restrict__ C = fd.G;
+    const int N = fd.N, K = fd.K, np = fd.np, tile = blockIdx.x - ch[fi].first, tn = N / TILE;
     constexpr int MB = TILE / 64;        // MFMA blocks per wave and dimension
     constexpr int LV = TILE / 64;        // float4 loads per thread and matrix per K step
     __shared__ float As[GBK][TILE + LDS_PAD];
     __shared__ __align__(16) float Bs[GBK][TILE + LDS_PAD];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int bm = blockIdx.y * TILE, bn = blockIdx.x * TILE;
+    const int bm = tile / tn * TILE, bn = tile % tn * TILE;
     const int wm = (wave >> 1) * (TILE / 2), wn = (wave & 1) * (TILE / 2);
     // A: thread loads row ar, columns ac .. ac + 4 LV - 1 of the 16-wide K slice
     const int ar = tid & (TILE - 1), ac = (tid / TILE) * 4 * LV;
@@ -77,13 +143,15 @@ __global__ __launch_bounds__(256) void k_sgemm_mfma(const float* __restrict__ A,
         rb[q] = sb[q];
     }
     for (int k0 = 0; k0 < K; k0 += GBK) {
+        const bool row = k0 + br < np;
 #pragma unroll
         for (int q = 0; q < LV; ++q) {
             As[ac + 4 * q + 0][ar] = ra[q][0];
             As[ac + 4 * q + 1][ar] = ra[q][1];
             As[ac + 4 * q + 2][ar] = ra[q][2];
             As[ac + 4 * q + 3][ar] = ra[q][3];
-            *reinterpret_cast<floatx4*>(&Bs[br][bc + 4 * q]) = rb[q];
+            const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+            *reinterpret_cast<floatx4*>(&Bs[br][bc + 4 * q]) = row ? rb[q] : zero;
         }
         __syncthreads();
         // prefetch the next K slice; the last step re-reads its own slice
@@ -144,17 +212,24 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 constexpr int HK = 32;    // K step of the split FP16 GEMM
 constexpr int HROW = 40;  // LDS row stride in halves: 32 of K plus 8 of padding
 
-__global__ __launch_bounds__(256) void k_hgemm3(const _Float16* __restrict__ Ahi, const _Float16* __restrict__ Alo,
-                                               const _Float16* __restrict__ Bhi, const _Float16* __restrict__ Blo,
-                                               float* __restrict__ C, int M, int N, int K,
-                                               const float* __restrict__ bsc) {
+__global__ __launch_bounds__(256) void k_hgemm3(const FaceDev* __restrict__ fc, const ChunkDev* __restrict__ ch,
+                                               int nf) {
     constexpr int TILE = 128, MB = 2;
+    const int fi = face_of_block(ch, nf, KIND_SPLIT16);
+    const FaceDev& fd = fc[fi];
+    const int N = fd.N, K = fd.K, tile = blockIdx.x - ch[fi].first, tn = N / TILE;
+    const _Float16* __restrict__ Ahi = reinterpret_cast<const _Float16*>(fd.A);
+    const _Float16* __restrict__ Alo = Ahi + (size_t)ch[fi].M * K;
+    const _Float16* __restrict__ Bhi = fd.Bhi;
+    const _Float16* __restrict__ Blo = fd.Blo;
+    float* __restrict__ C = fd.G;
+    const float* __restrict__ bsc = fd.bsc;
     __shared__ __align__(16) _Float16 Ah[TILE][HROW];
     __shared__ __align__(16) _Float16 Al[TILE][HROW];
     __shared__ __align__(16) _Float16 Bh[TILE][HROW];
     __shared__ __align__(16) _Float16 Bl[TILE][HROW];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int bm = blockIdx.y * TILE, bn = blockIdx.x * TILE;
+    const int bm = tile / tn * TILE, bn = tile % tn * TILE;
     const int wm = (wave >> 1) * (TILE / 2), wn = (wave & 1) * (TILE / 2);
     // every thread copies 16 halves (2 x 16 B) of one row of each of the four tiles
     const int r = tid >> 1, kq = (tid & 1) * 16;
@@ -229,19 +304,16 @@ __global__ __launch_bounds__(256) void k_hgemm3(const _Float16* __restrict__ Ahi
 
 // B [K][N] float -> Bhi, Blo [N][K] halves of B s, s = 2^(14 - e) for the
 // largest entry m = f 2^e (0.5 <= f < 1) of the pack's block maxima
-// pmax[0..npmax) (s = 1 when m is 0 or not finite), so every scaled entry is
-// below 2^14.  Entries outside the packed p < np, n < nv (padding, which may
+// pmax[0..nb) (s = 1 when m is 0 or not finite), so every scaled entry is
+// below 2^14.  Entries outside the packed p < np, n < 8 nq (padding, which may
 // hold an earlier face's values) are written as zeros.  64 x 64 tiles through
-// LDS: reads along n, writes along k.  Work-group 0 stores (s, 1 / s) to bsc.
-__global__ __launch_bounds__(256) void k_bsplit(const float* __restrict__ B, int K, int N, int np, int nv,
-                                               const float* __restrict__ pmax, int npmax,
-                                               _Float16* __restrict__ Bhi, _Float16* __restrict__ Blo,
-                                               float* __restrict__ bsc) {
+// LDS: reads along n, writes along k.  The first work-group stores (s, 1 / s).
+__device__ __forceinline__ void bsplit(const FaceDev& f) {
     __shared__ float red[256];
     __shared__ float t[64][65];
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, K = f.K, N = f.N, nv = 8 * f.nq;
     float m = 0.f;
-    for (int q = tid; q < npmax; q += 256) m = fmaxf(m, pmax[q]);
+    for (int q = tid; q < f.nb; q += 256) m = fmaxf(m, f.pmax[q]);
     red[tid] = m;
     __syncthreads();
     for (int o = 128; o > 0; o >>= 1) {
@@ -255,57 +327,78 @@ __global__ __launch_bounds__(256) void k_bsplit(const float* __restrict__ B, int
         sc = ldexpf(1.f, 14 - e);
         inv = ldexpf(1.f, e - 14);
     }
-    if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) {
-        bsc[0] = sc;
-        bsc[1] = inv;
+    if (blockIdx.x == 0 && tid == 0) {
+        f.bsc[0] = sc;
+        f.bsc[1] = inv;
     }
-    const int k0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
+    const int tn = N / 64, tiles = tn * ((K + 63) / 64);
     const int tx = tid & 63, ty = tid >> 6;
-    for (int y = ty; y < 64; y += 4) {
-        const int k = k0 + y, n = n0 + tx;
-        t[y][tx] = (k < np && n < nv) ? B[(size_t)k * N + n] * sc : 0.f;
-    }
-    __syncthreads();
-    for (int y = ty; y < 64; y += 4) {
-        const int n = n0 + y, k = k0 + tx;
-        if (n < N && k < K) {
-            const float x = t[tx][y];
-            const _Float16 h = (_Float16)x;
-            Bhi[(size_t)n * K + k] = h;
-            Blo[(size_t)n * K + k] = (_Float16)(x - (float)h);
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int k0 = tile / tn * 64, n0 = tile % tn * 64;
+        for (int y = ty; y < 64; y += 4) {
+            const int k = k0 + y, n = n0 + tx;
+            t[y][tx] = (k < f.np && n < nv) ? f.B[(size_t)k * N + n] * sc : 0.f;
         }
+        __syncthreads();
+        for (int y = ty; y < 64; y += 4) {
+            const int n = n0 + y, k = k0 + tx;
+            if (k < K) {
+                const float x = t[tx][y];
+                const _Float16 h = (_Float16)x;
+                f.Bhi[(size_t)n * K + k] = h;
+                f.Blo[(size_t)n * K + k] = (_Float16)(x - (float)h);
+            }
+        }
+        __syncthreads();
     }
 }
 
-// Phase rows of k_phase as fp16 halves (hi, lo of the float64 value).  One
-// thread per 8 consecutive columns of a row (ld is a multiple of 8); on a
-// uniform grid (uniform, xp[i] = xp[0] + i dx) the thread takes one sincos
-// and steps the other 7 columns by angle addition in float64.
-__global__ __launch_bounds__(256) void k_phase16(_Float16* __restrict__ Ahi, _Float16* __restrict__ Alo, int ld,
-                                                size_t total, int u0, int u1, int np, const double* __restrict__ uval,
-                                                const double* __restrict__ xp, double k, int uniform, double dx) {
-    const size_t groups = total / 8;
-    for (size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x; g < groups; g += (size_t)gridDim.x * blockDim.x) {
+// Rows of A in float32: row r of the chunk holds cos (even r) or sin (odd r)
+// of k uval[u] xp[i], u = u0 + r / 2, for u < u1 and i < np, zeros elsewhere.
+__device__ __forceinline__ void phase_rows(const FaceDev& f, const ChunkDev& c, double k) {
+    const size_t total = (size_t)c.M * f.K;
+    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < total; t += (size_t)gridDim.x * 256) {
+        const int r = (int)(t / f.K), i = (int)(t - (size_t)r * f.K);
+        const int u = c.u0 + (r >> 1);
+        float v = 0.f;
+        if (u < c.u1 && i < f.np) {
+            double sn, cs;
+            sincos(k * f.uval[u] * f.xp[i], &sn, &cs);
+            v = (float)((r & 1) ? sn : cs);
+        }
+        f.A[t] = v;
+    }
+}
+
+// The same rows as fp16 halves (hi, then lo, of the float64 value).  One
+// thread per 8 consecutive columns of a row (K is a multiple of 8); on a
+// uniform grid (xp[i] = xp[0] + i dxp) the thread takes one sincos and steps
+// the other 7 columns by angle addition in float64.
+__device__ __forceinline__ void phase_rows16(const FaceDev& f, const ChunkDev& c, double k) {
+    const size_t total = (size_t)c.M * f.K, groups = total / 8;
+    _Float16* Ahi = reinterpret_cast<_Float16*>(f.A);
+    _Float16* Alo = Ahi + total;
+    for (size_t g = (size_t)blockIdx.x * 256 + threadIdx.x; g < groups; g += (size_t)gridDim.x * 256) {
         const size_t t0 = 8 * g;
-        const int r = (int)(t0 / ld), i0 = (int)(t0 - (size_t)r * ld);
-        const int u = u0 + (r >> 1);
+        const int r = (int)(t0 / f.K), i0 = (int)(t0 - (size_t)r * f.K);
+        const int u = c.u0 + (r >> 1);
         const bool odd = (r & 1) != 0;
         half8 h, l;
-        if (u < u1 && i0 < np) {
-            const double ku = k * uval[u];
+        if (u < c.u1 && i0 < f.np) {
+            const double ku = k * f.uval[u];
             double sn, cs, sd = 0.0, cd = 1.0;
-            sincos(ku * xp[i0], &sn, &cs);
-            if (uniform) sincos(ku * dx, &sd, &cd);
+            sincos(ku * f.xp[i0], &sn, &cs);
+            if (f.uni_p) sincos(ku * f.dxp, &sd, &cd);
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
                 double v = 0.0;
-                if (i0 + q < np) {
-                    if (!uniform && q > 0) sincos(ku * xp[i0 + q], &sn, &cs);
+                if (i0 + q < f.np) {
+                    if (!f.uni_p && q > 0) sincos(ku * f.xp[i0 + q], &sn, &cs);
                     v = odd ? sn : cs;
                 }
                 h[q] = (_Float16)v;
                 l[q] = (_Float16)(v - (double)h[q]);
-                if (uniform) {
+                if (f.uni_p) {
                     const double c2 = cs * cd - sn * sd;
                     sn = sn * cd + cs * sd;
                     cs = c2;
@@ -320,44 +413,27 @@ __global__ __launch_bounds__(256) void k_phase16(_Float16* __restrict__ Ahi, _Fl
     }
 }
 
-// The large contractions on the FP16 matrix cores when split16 (operands
-// split into fp16 halves), the others in FP32.
-bool use_split16(int M, int N, bool split16) { return split16 && (M / 128) * (N / 128) >= 512; }
-
-hipError_t launch_gemm(const float* A, const float* B, float* C, int M, int N, int K, hipStream_t s) {
-    if ((M / 128) * (N / 128) >= 512)
-        hipLaunchKernelGGL(k_sgemm_mfma<128>, dim3(N / 128, M / 128), dim3(256), 0, s, A, B, C, M, N, K);
-    else
-        hipLaunchKernelGGL(k_sgemm_mfma<64>, dim3(N / 64, M / 64), dim3(256), 0, s, A, B, C, M, N, K);
-    return hipGetLastError();
-}
-
-// Rows r of A (ld floats, total = rows * ld): u = u0 + r / 2 < u1 gives
-// cos (even r) or sin (odd r) of k uval[u] xp[i] for i < np, zero elsewhere.
-__global__ __launch_bounds__(256) void k_phase(float* __restrict__ A, int ld, size_t total, int u0, int u1, int np,
-                                               const double* __restrict__ uval, const double* __restrict__ xp,
-                                               double k) {
-    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-        const int r = (int)(t / ld), i = (int)(t - (size_t)r * ld);
-        const int u = u0 + (r >> 1);
-        float v = 0.f;
-        if (u < u1 && i < np) {
-            double sn, cs;
-            sincos(k * uval[u] * xp[i], &sn, &cs);
-            v = (float)((r & 1) ? sn : cs);
-        }
-        A[t] = v;
+// The contraction's operands of one chunk, every face in one launch: grid
+// (work-groups, face, 2), z = 0 the phase rows, z = 1 (first chunk) the split
+// of B for the faces that need it.
+__global__ __launch_bounds__(256) void k_nf2ff_operands(const FaceDev* __restrict__ fc, const ChunkDev* __restrict__ ch,
+                                                        double k) {
+    const FaceDev& f = fc[blockIdx.y];
+    const ChunkDev& c = ch[blockIdx.y];
+    if (blockIdx.z == 0) {
+        if (c.M == 0) return;
+        if (c.kind == KIND_SPLIT16) phase_rows16(f, c, k);
+        else phase_rows(f, c, k);
+    } else if (f.split) {
+        bsplit(f);
     }
 }
 
-// Zero rows [np, K) of B (the padding the contraction's K tiles cover), so
-// that whatever an earlier face or call left there -- a non-finite value
-// from a diverged run included -- cannot reach a product: A's padding
-// columns are zeros, and 0 * NaN would still be NaN.
-__global__ __launch_bounds__(256) void k_nf2ff_pad_rows(float* __restrict__ B, int ldb, int np, int K) {
-    const size_t n = (size_t)(K - np) * ldb;
-    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256)
-        B[(size_t)np * ldb + e] = 0.f;
+// The large contractions on the FP16 matrix cores when split16 (operands
+// split into fp16 halves), the others in FP32.
+int gemm_kind(int M, int N, bool split16) {
+    const bool large = (M / 128) * (N / 128) >= 512;
+    return !large ? KIND_FP32 : split16 ? KIND_SPLIT16 : KIND_FP32_LARGE;
 }
 
 // B = [Br | Bi] for one face: row ip, columns 4 iq + c and 4 nq + 4 iq + c
@@ -368,37 +444,38 @@ __global__ __launch_bounds__(256) void k_nf2ff_pad_rows(float* __restrict__ B, i
 // n = s e_axis.  The block partial of the radiated power,
 // 1/2 sum w_p w_q Re((E x H*) . n) (matlab/AnalyzeNF2FF.m:201-209), goes to
 // part[blockIdx.x].
-template <int KIND>
-__global__ __launch_bounds__(256) void k_nf2ff_pack(const void* __restrict__ src, double scale, int n1, int n2,
-                                                    int swap, int sign, const double* __restrict__ wp,
-                                                    const double* __restrict__ wq, float* __restrict__ B, int ldb,
-                                                    double* __restrict__ part, float* __restrict__ pmax) {
+__global__ __launch_bounds__(256) void k_nf2ff_pack(const FaceDev* __restrict__ fc) {
+    const FaceDev& f = fc[blockIdx.y];
+    if ((int)blockIdx.x >= f.nb) return;
     __shared__ double red[256];
     __shared__ float redm[256];
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, n1 = f.n1, n2 = f.n2;
     const int q = blockIdx.x * 256 + tid;
     double p = 0.0;
     float mx = 0.f;
     if (q < n1 * n2) {
         const int i1 = q / n2, i2 = q - i1 * n2;
-        const int ip = swap ? i2 : i1, iq = swap ? i1 : i2, nq = swap ? n1 : n2;
+        const int ip = f.swap ? i2 : i1, iq = f.swap ? i1 : i2, nq = f.nq;
         double vr[4], vi[4];
+        if (f.kind == 0) {
+            const double2* v = reinterpret_cast<const double2*>(f.src) + 4 * (size_t)q;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            if (KIND == 0) {
-                const double* v = reinterpret_cast<const double*>(src) + 8 * (size_t)q + 2 * c;
-                vr[c] = scale * v[0];
-                vi[c] = scale * v[1];
-            } else {
-                const float* v = reinterpret_cast<const float*>(src) + 16 * (size_t)q + 4 * c;
-                vr[c] = scale * (double)v[0];
-                vi[c] = scale * (double)v[1];
+            for (int c = 0; c < 4; ++c) {
+                vr[c] = f.scale * v[c].x;
+                vi[c] = f.scale * v[c].y;
+            }
+        } else {
+            const float4* v = reinterpret_cast<const float4*>(f.src) + 4 * (size_t)q;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                vr[c] = f.scale * (double)v[c].x;
+                vi[c] = f.scale * (double)v[c].y;
             }
         }
-        const double sg = sign, w = wp[ip];
+        const double sg = f.sign, w = f.wp[ip];
         const double cr[4] = {-sg * vr[3], sg * vr[2], sg * vr[1], -sg * vr[0]};
         const double ci[4] = {-sg * vi[3], sg * vi[2], sg * vi[1], -sg * vi[0]};
-        float* row = B + (size_t)ip * ldb;
+        float* row = f.B + (size_t)ip * f.N;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const float br = (float)(w * cr[c]), bi = (float)(w * ci[c]);
@@ -406,7 +483,7 @@ __global__ __launch_bounds__(256) void k_nf2ff_pack(const void* __restrict__ src
             row[4 * nq + 4 * iq + c] = bi;
             mx = fmaxf(mx, fmaxf(fabsf(br), fabsf(bi)));
         }
-        p = 0.5 * w * wq[iq] * sg * (vr[0] * vr[3] + vi[0] * vi[3] - vr[1] * vr[2] - vi[1] * vi[2]);
+        p = 0.5 * w * f.wq[iq] * sg * (vr[0] * vr[3] + vi[0] * vi[3] - vr[1] * vr[2] - vi[1] * vi[2]);
     }
     red[tid] = p;
     redm[tid] = mx;
@@ -419,40 +496,25 @@ __global__ __launch_bounds__(256) void k_nf2ff_pack(const void* __restrict__ src
         __syncthreads();
     }
     if (tid == 0) {
-        part[blockIdx.x] = red[0];
-        pmax[blockIdx.x] = redm[0];
+        f.part[blockIdx.x] = red[0];
+        f.pmax[blockIdx.x] = redm[0];
     }
 }
 
 #ifndef REDUCE_M
 #define REDUCE_M 2  // 2: 0.894 ms device per frequency; 3: 0.978; 4: 0.914 (fewer waves)
 #endif
-struct ReduceArgs {
-    const float* G;        // GEMM output of this chunk: rows 2 (u - u0) (C) and 2 (u - u0) + 1 (S)
-    int ldg;
-    const int* order;      // angles sorted by u
-    const int2* groups;    // (first index into order, count) of up to REDUCE_M angles of one row
-    int g0, g1;            // this chunk's range of groups[]
-    int u0;
-    const int* uidx;       // per angle
-    const float* usgn;     // per angle: sign of kappa_p
-    int nq;
-    const double* kapq;    // per angle
-    const double* kap0;    // per angle
-    const double* xq;
-    const double* wq;
-    int uniform;           // xq[i] = xq[0] + i dxq (phases by recurrence)
-    double dxq, x0, k;
-    int slot[4];           // NL slot of current c
-    double* NL;            // [n_ang][6] complex
-};
+// e^{j pi x}, x in half turns reduced to one turn first.
+__device__ __forceinline__ void cis_pi(double x, double* c, double* s) {
+    sincospi(x - 2.0 * rint(0.5 * x), s, c);
+}
 
 // Second contraction, one group of angles at a time: the angles of a group
 // share one G row (the same |kappa_p|), so each G load serves all of them.
 // QL lanes split the q sum (lane l takes q = l, l + QL, ...; consecutive
 // lanes read consecutive G entries); the QL partial sums of every angle are
 // added by a fixed xor butterfly (deterministic) and the group's first lane
-// adds the results, rotated by the face-position phase, into NL.  G = GC -/+
+// stores the results, rotated by the face-position phase, as the face's sums.  G = GC -/+
 // j GS is formed in float32 (one rounding of the matrix-core output, 6e-8
 // relative); the phase products are accumulated in float64 with fused
 // multiply-adds.
@@ -460,13 +522,18 @@ constexpr int QL = 16;
 constexpr int REDUCE_THREADS = 256;
 constexpr int REDUCE_GROUPS = REDUCE_THREADS / QL;
 
-__global__ __launch_bounds__(REDUCE_THREADS) void k_nf2ff_reduce(ReduceArgs r) {
+__global__ __launch_bounds__(REDUCE_THREADS) void k_nf2ff_reduce(const FaceDev* __restrict__ fc,
+                                                                 const ChunkDev* __restrict__ ch, double k) {
     constexpr int M = REDUCE_M;
+    const FaceDev& r = fc[blockIdx.y];
+    const ChunkDev& ck = ch[blockIdx.y];
+    if (ck.mirror) return;
     const int ql = threadIdx.x & (QL - 1);
-    const int gi = r.g0 + blockIdx.x * REDUCE_GROUPS + (int)(threadIdx.x / QL);
-    const bool act = gi < r.g1;
-    const int2 grp = r.groups[act ? gi : r.g0];
-    const int n = act ? grp.y : 0;
+    const int gi = ck.g0 + blockIdx.x * REDUCE_GROUPS + (int)(threadIdx.x / QL);
+    if (gi >= ck.g1) return;  // whole groups of QL lanes
+    const int2 grp = r.groups[gi];
+    const int n = grp.y, nq = r.nq;
+    const double kp = k * M_1_PI;
     int am[M];
     float sgf[M];
     double pr[M], pi[M], str[M], sti[M];
@@ -475,22 +542,22 @@ __global__ __launch_bounds__(REDUCE_THREADS) void k_nf2ff_reduce(ReduceArgs r) {
     for (int m = 0; m < M; ++m) {
         am[m] = r.order[grp.x + min(m, grp.y - 1)];
         sgf[m] = r.usgn[am[m]];
-        const double kk = r.k * r.kapq[am[m]];
+        const double kk = kp * r.kapq[am[m]];
         pr[m] = 1.0; pi[m] = 0.0; str[m] = 1.0; sti[m] = 0.0;
-        if (r.uniform && ql < r.nq) {
-            sincos(kk * r.xq[ql], &pi[m], &pr[m]);
-            sincos(kk * (QL * r.dxq), &sti[m], &str[m]);
+        if (r.uni_q && ql < nq) {
+            cis_pi(kk * r.xq[ql], &pr[m], &pi[m]);
+            cis_pi(kk * (QL * r.dxq), &str[m], &sti[m]);
         }
 #pragma unroll
         for (int c = 0; c < 4; ++c) sr[m][c] = si[m][c] = 0.0;
     }
-    const float* gc = r.G + (size_t)(2 * (r.uidx[am[0]] - r.u0)) * r.ldg;
-    const float* gs = gc + r.ldg;
+    const float* gc = r.G + (size_t)(2 * (r.uidx[am[0]] - ck.u0)) * r.N;
+    const float* gs = gc + r.N;
     auto body = [&](int iq, bool uniform) {
         const float4 cr4 = *reinterpret_cast<const float4*>(gc + 4 * iq);
-        const float4 ci4 = *reinterpret_cast<const float4*>(gc + 4 * r.nq + 4 * iq);
+        const float4 ci4 = *reinterpret_cast<const float4*>(gc + 4 * nq + 4 * iq);
         const float4 sr4 = *reinterpret_cast<const float4*>(gs + 4 * iq);
-        const float4 si4 = *reinterpret_cast<const float4*>(gs + 4 * r.nq + 4 * iq);
+        const float4 si4 = *reinterpret_cast<const float4*>(gs + 4 * nq + 4 * iq);
         const double w = r.wq[iq];
         const float gcr[4] = {cr4.x, cr4.y, cr4.z, cr4.w}, gci[4] = {ci4.x, ci4.y, ci4.z, ci4.w};
         const float gsr[4] = {sr4.x, sr4.y, sr4.z, sr4.w}, gsi[4] = {si4.x, si4.y, si4.z, si4.w};
@@ -502,7 +569,7 @@ __global__ __launch_bounds__(REDUCE_THREADS) void k_nf2ff_reduce(ReduceArgs r) {
                 pi[m] = pr[m] * sti[m] + pi[m] * str[m];
                 pr[m] = t;
             } else {
-                sincos(r.k * r.kapq[am[m]] * r.xq[iq], &sn, &cs);
+                cis_pi(kp * r.kapq[am[m]] * r.xq[iq], &cs, &sn);
             }
             const double wr = w * cs, wi = w * sn;
 #pragma unroll
@@ -514,10 +581,10 @@ __global__ __launch_bounds__(REDUCE_THREADS) void k_nf2ff_reduce(ReduceArgs r) {
             }
         }
     };
-    if (r.uniform) {
-        for (int iq = ql; iq < r.nq; iq += QL) body(iq, true);
+    if (r.uni_q) {
+        for (int iq = ql; iq < nq; iq += QL) body(iq, true);
     } else {
-        for (int iq = ql; iq < r.nq; iq += QL) body(iq, false);
+        for (int iq = ql; iq < nq; iq += QL) body(iq, false);
     }
 #pragma unroll
     for (int o = QL / 2; o > 0; o >>= 1)
@@ -534,13 +601,11 @@ __global__ __launch_bounds__(REDUCE_THREADS) void k_nf2ff_reduce(ReduceArgs r) {
         if (m >= n) break;
         const int a = am[m];
         double sn, cs;
-        sincos(r.k * r.kap0[a] * r.x0, &sn, &cs);
+        cis_pi(kp * r.kap0[a] * r.x0, &cs, &sn);
+        double2* o = reinterpret_cast<double2*>(r.S) + (size_t)a * 4;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            double* o = r.NL + ((size_t)a * 6 + r.slot[c]) * 2;
-            o[0] += cs * sr[m][c] - sn * si[m][c];
-            o[1] += cs * si[m][c] + sn * sr[m][c];
-        }
+        for (int c = 0; c < 4; ++c)
+            o[c] = make_double2(cs * sr[m][c] - sn * si[m][c], cs * si[m][c] + sn * sr[m][c]);
     }
 }
 
@@ -556,41 +621,59 @@ __global__ __launch_bounds__(REDUCE_THREADS) void k_nf2ff_reduce(ReduceArgs r) {
 // read once per group, and the float64 work per q is that of one angle for
 // the whole group.
 //
-// One wave per group: lane = 4 ql + c takes component c at q = ql, ql + MQ,
-// ... (the four lanes of one ql read 16 consecutive bytes, the wave 256), with
-// eight float64 accumulators, and issues the loads of four q steps before
-// using them (the reduction is bound by the latency of these loads).  An xor
-// butterfly over the MQ lanes of each component gives every lane its
-// component's sums; lane (ql, c) then finishes component c of member ql (a
-// group holds at most MQ members).
-struct MirrorArgs {
-    const int4* groups;   // (u, first index into members, count, 0)
-    const double* gkq;    // per group: |kappa_q| of its first member
-    const int* members;   // angles, grouped
-    int m0, m1;           // this chunk's range of groups[]
-};
-constexpr int MQ = 16;
+// 4 MQ lanes per group: lane = 4 ql + c takes component c at q = ql, ql + MQ,
+// ... (the four lanes of one ql read 16 consecutive bytes), with eight float64
+// accumulators, and issues the loads of four q steps before using them.  The
+// MQ lanes of each component are added by row rotations (MQ = 4: a group is
+// one 16-lane row), and lane (ql, c) then finishes component c of members ql,
+// ql + MQ, ...  What bounds it is instructions: for each group the start and
+// end phases (three sincos) and the sums over lanes cost as much as the steps
+// in q when a whole wave works on one group, so a wave takes four groups.
+// 65160 angles, 349x349x221 nodes: the six faces take 106 us, against 6 x 32
+// with a wave a group.
+constexpr int MIRROR_MAX = 16;  // most members of a group
+constexpr int MQ = 4;
 constexpr int MIRROR_THREADS = 256;
 constexpr int MIRROR_GROUPS = MIRROR_THREADS / (4 * MQ);
 
-// UNI: uniform q grid (phases by recurrence, r.uniform set)
+// v of the lane n further on in its row of 16.
+template <int N>
+__device__ __forceinline__ double row_ror(double v) {
+    union {
+        double d;
+        int i[2];
+    } x{v};
+    x.i[0] = __builtin_amdgcn_update_dpp(0, x.i[0], 0x120 + N, 0xf, 0xf, true);
+    x.i[1] = __builtin_amdgcn_update_dpp(0, x.i[1], 0x120 + N, 0xf, 0xf, true);
+    return x.d;
+}
+__device__ __forceinline__ void add_lanes(double& v) {
+    v += row_ror<4>(v);
+    v += row_ror<8>(v);
+#pragma unroll
+    for (int o = 16; o < 4 * MQ; o <<= 1) v += __shfl_xor(v, o);
+}
+
+// UNI: uniform q grid (phases by recurrence)
 template <bool UNI>
-__global__ __launch_bounds__(MIRROR_THREADS) void k_nf2ff_reduce_mirror(ReduceArgs r, MirrorArgs m) {
-    const int gi = m.m0 + blockIdx.x * MIRROR_GROUPS + (int)(threadIdx.x / (4 * MQ));
-    if (gi >= m.m1) return;  // whole waves: no lane of another group waits on this one
+__device__ __forceinline__ void mirror_reduce(const FaceDev& r, const ChunkDev& ck, double k) {
+    const int gi = ck.g0 + blockIdx.x * MIRROR_GROUPS + (int)(threadIdx.x / (4 * MQ));
+    const bool on = gi < ck.g1;  // every lane takes part in the rotations
     const int c = threadIdx.x & 3;
     const int ql = (threadIdx.x >> 2) & (MQ - 1);
-    const int4 grp = m.groups[gi];
-    const double kk = r.k * m.gkq[gi];
+    const int4 grp = r.mgroups[on ? gi : ck.g0];
+    const int nq = on ? r.nq : 0;
+    const double kp = k * M_1_PI, kk = kp * r.gkq[on ? gi : ck.g0];
     double pr = 1.0, pi = 0.0, str = 1.0, sti = 0.0;
-    if (UNI && ql < r.nq) {
-        sincos(kk * r.xq[ql], &pi, &pr);
-        sincos(kk * (MQ * r.dxq), &sti, &str);
+    if (UNI && ql < nq) {
+        cis_pi(kk * r.xq[ql], &pr, &pi);
+        cis_pi(kk * (MQ * r.dxq), &str, &sti);
     }
     // P1..P4 of component c, real and imaginary
     double p1r = 0.0, p1i = 0.0, p2r = 0.0, p2i = 0.0, p3r = 0.0, p3i = 0.0, p4r = 0.0, p4i = 0.0;
-    const float* gc = r.G + (size_t)(2 * (grp.x - r.u0)) * r.ldg + c;
-    const float* gs = gc + r.ldg;
+    const float* gc = r.G + (size_t)(2 * (grp.x - ck.u0)) * r.N + c;
+    const float* gs = gc + r.N;
+    const double* __restrict__ wq = r.wq;
     const int n4 = 4 * r.nq;
     auto step = [&](int q, float a, float b, float e, float f, double w) {
         double cs = pr, sn = pi;
@@ -599,7 +682,7 @@ __global__ __launch_bounds__(MIRROR_THREADS) void k_nf2ff_reduce_mirror(ReduceAr
             pi = pr * sti + pi * str;
             pr = t;
         } else {
-            sincos(kk * r.xq[q], &sn, &cs);
+            cis_pi(kk * r.xq[q], &cs, &sn);
         }
         const double wc = w * cs, ws = w * sn;
         p1r = fma(wc, (double)a, p1r);
@@ -612,7 +695,7 @@ __global__ __launch_bounds__(MIRROR_THREADS) void k_nf2ff_reduce_mirror(ReduceAr
         p4i = fma(ws, (double)f, p4i);
     };
     int iq = ql;
-    for (; iq + 3 * MQ < r.nq; iq += 4 * MQ) {
+    for (; iq + 3 * MQ < nq; iq += 4 * MQ) {
         float va[4], vb[4], ve[4], vf[4];
         double vw[4];
 #pragma unroll
@@ -622,45 +705,83 @@ __global__ __launch_bounds__(MIRROR_THREADS) void k_nf2ff_reduce_mirror(ReduceAr
             vb[u] = gc[n4 + 4 * q];
             ve[u] = gs[4 * q];
             vf[u] = gs[n4 + 4 * q];
-            vw[u] = r.wq[q];
+            vw[u] = wq[q];
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) step(iq + u * MQ, va[u], vb[u], ve[u], vf[u], vw[u]);
     }
-    for (; iq < r.nq; iq += MQ) step(iq, gc[4 * iq], gc[n4 + 4 * iq], gs[4 * iq], gs[n4 + 4 * iq], r.wq[iq]);
-#pragma unroll
-    for (int o = 4; o < 4 * MQ; o <<= 1) {
-        p1r += __shfl_xor(p1r, o);
-        p1i += __shfl_xor(p1i, o);
-        p2r += __shfl_xor(p2r, o);
-        p2i += __shfl_xor(p2i, o);
-        p3r += __shfl_xor(p3r, o);
-        p3i += __shfl_xor(p3i, o);
-        p4r += __shfl_xor(p4r, o);
-        p4i += __shfl_xor(p4i, o);
-    }
-    const int slot = c == 0 ? r.slot[0] : c == 1 ? r.slot[1] : c == 2 ? r.slot[2] : r.slot[3];
-    if (ql < grp.z) {
-        const int a = m.members[grp.y + ql];
+    for (; iq < nq; iq += MQ) step(iq, gc[4 * iq], gc[n4 + 4 * iq], gs[4 * iq], gs[n4 + 4 * iq], wq[iq]);
+    add_lanes(p1r);
+    add_lanes(p1i);
+    add_lanes(p2r);
+    add_lanes(p2i);
+    add_lanes(p3r);
+    add_lanes(p3i);
+    add_lanes(p4r);
+    add_lanes(p4i);
+    if (!on) return;
+    for (int m = ql; m < grp.z; m += MQ) {
+        const int a = r.members[grp.y + m];
         const double sg = (double)r.usgn[a];
         const double s = r.kapq[a] < 0.0 ? -1.0 : 1.0;
         const double ss = s * sg;
         double sn, cs;
-        sincos(r.k * r.kap0[a] * r.x0, &sn, &cs);
+        cis_pi(kp * r.kap0[a] * r.x0, &cs, &sn);
         // P1 + j sigma P2 + j s P3 - s sigma P4
         const double tr = p1r - sg * p2i - s * p3i - ss * p4r;
         const double ti = p1i + sg * p2r + s * p3r - ss * p4i;
-        double* o = r.NL + ((size_t)a * 6 + slot) * 2;
-        o[0] += cs * tr - sn * ti;
-        o[1] += cs * ti + sn * tr;
+        reinterpret_cast<double2*>(r.S)[(size_t)a * 4 + c] = make_double2(cs * tr - sn * ti, cs * ti + sn * tr);
     }
+}
+
+__global__ __launch_bounds__(MIRROR_THREADS) void k_nf2ff_reduce_mirror(const FaceDev* __restrict__ fc,
+                                                                        const ChunkDev* __restrict__ ch, double k) {
+    const FaceDev& r = fc[blockIdx.y];
+    const ChunkDev& ck = ch[blockIdx.y];
+    if (!ck.mirror || ck.g0 + (int)blockIdx.x * MIRROR_GROUPS >= ck.g1) return;
+    if (r.uni_q) mirror_reduce<true>(r, ck, k);
+    else mirror_reduce<false>(r, ck, k);
+}
+
+// N, L of angle a: nl (or zero) plus the faces' sums, in face order.
+__device__ __forceinline__ void gather_nl(const FaceDev* __restrict__ fc, int nf, const double* __restrict__ nl,
+                                          size_t a, double* v) {
+#pragma unroll
+    for (int c = 0; c < 12; ++c) v[c] = nl ? nl[12 * a + c] : 0.0;
+    for (int f = 0; f < nf; ++f) {
+        const double2* S = reinterpret_cast<const double2*>(fc[f].S) + 4 * a;
+        const int a1 = fc[f].a1;  // a2 = a1 + 1 cyclically
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const double2 s = S[c];
+            const int slot = (c >= 2 ? 3 : 0) + ((c & 1) ? (a1 == 2 ? 0 : a1 + 1) : a1);
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+                if (q == slot) {
+                    v[2 * q] += s.x;
+                    v[2 * q + 1] += s.y;
+                }
+        }
+    }
+}
+
+// Surfaces of more than MAX_FACES faces: the sums of one set of them.
+__global__ __launch_bounds__(256) void k_nf2ff_gather(const FaceDev* __restrict__ fc, int nf, double* nl, int first,
+                                                      size_t n_ang) {
+    const size_t a = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (a >= n_ang) return;
+    double v[12];
+    gather_nl(fc, nf, first ? nullptr : nl, a, v);
+#pragma unroll
+    for (int c = 0; c < 12; ++c) nl[12 * a + c] = v[c];
 }
 
 // E_theta = -fac (L_phi + Z0 N_theta), E_phi = fac (L_theta - Z0 N_phi) with
 // fac = jk e^{-jkr}/(4 pi r) (matlab/AnalyzeNF2FF.m:98-105) and
 // U = r^2/(2 Z0)(|E_theta|^2 + |E_phi|^2) (:112): out = [4][n_ang]
 // (E_theta re, im, E_phi re, im); the block maximum of U goes to umax[block].
-__global__ __launch_bounds__(256) void k_nf2ff_project(const double* __restrict__ NL, const double* __restrict__ NL2,
+__global__ __launch_bounds__(256) void k_nf2ff_project(const FaceDev* __restrict__ fc, int nf,
+                                                       const double* __restrict__ nl,
                                                        const double* __restrict__ theta,
                                                        const double* __restrict__ phi, int n_phi, size_t n_ang,
                                                        double fr, double fi, double r, double* __restrict__ out,
@@ -673,10 +794,8 @@ __global__ __launch_bounds__(256) void k_nf2ff_project(const double* __restrict_
         double st, ct, sp, cp;
         sincos(theta[it], &st, &ct);
         sincos(phi[ip], &sp, &cp);
-        // N, L summed over the faces (NL2: the side stream's faces, or null)
         double v[12];
-#pragma unroll
-        for (int c = 0; c < 12; ++c) v[c] = NL[12 * a + c] + (NL2 ? NL2[12 * a + c] : 0.0);
+        gather_nl(fc, nf, nl, a, v);
         const double ntr = v[0] * (ct * cp) + v[2] * (ct * sp) - v[4] * st;
         const double nti = v[1] * (ct * cp) + v[3] * (ct * sp) - v[5] * st;
         const double npr = -v[0] * sp + v[2] * cp, npi = -v[1] * sp + v[3] * cp;
@@ -775,7 +894,7 @@ struct Nf2ffCache {
     } ax[3];
     // Mirror groups of the faces normal to each axis (k_nf2ff_reduce_mirror):
     // the angles of every row u of that face's first-contraction axis,
-    // grouped by equal |kappa| along its second axis, at most MQ per group.
+    // grouped by equal |kappa| along its second axis, at most MIRROR_MAX each.
     struct Mirror {
         std::vector<int> mstart;  // U + 1 offsets into groups
         DevBuf groups;            // int4 (u, first index into members, count, 0)
@@ -786,20 +905,9 @@ struct Nf2ffCache {
     // timing events, created on first use and kept: [0] brackets the whole
     // transform, the others one GEMM launch each
     std::vector<std::unique_ptr<EventPair>> events;
-    // byte offset and length of the B region last zeroed in `work`
-    size_t bm_off[2] = {SIZE_MAX, SIZE_MAX}, bm_len[2] = {0, 0};
-    // the side stream of the x/y faces, created on first use
-    hipStream_t side = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     Nf2ffCache() = default;
     Nf2ffCache(const Nf2ffCache&) = delete;
     Nf2ffCache& operator=(const Nf2ffCache&) = delete;
-    ~Nf2ffCache() {
-        if (side) (void)hipStreamSynchronize(side);
-        if (ev_fork) (void)hipEventDestroy(ev_fork);
-        if (ev_join) (void)hipEventDestroy(ev_join);
-        if (side) (void)hipStreamDestroy(side);
-    }
 };
 
 Nf2ffCache* nf2ff_cache_new() { return new Nf2ffCache(); }
@@ -900,9 +1008,9 @@ static hipError_t plan_angles(Nf2ffCache& c, const double* theta, int nt, const 
             for (int i = b; i < e;) {
                 const double v0 = std::fabs(kq[members[i]]);
                 int j = i + 1;
-                // at most MQ members: one finishing pass per lane (the poles
+                // a bounded number of members (the poles
                 // alone would otherwise make one group of every phi)
-                while (j < e && j - i < MQ && std::fabs(kq[members[j]]) - v0 <= 1e-12) ++j;
+                while (j < e && j - i < MIRROR_MAX && std::fabs(kq[members[j]]) - v0 <= 1e-12) ++j;
                 groups.push_back(make_int4(u, i, j - i, 0));
                 gkq.push_back(v0);
                 i = j;
@@ -923,8 +1031,8 @@ static hipError_t plan_angles(Nf2ffCache& c, const double* theta, int nt, const 
     return hipSuccess;
 }
 
-// G stays within 64 Mi floats per GEMM launch; larger U is split into chunks
-// of u, each with the angles whose u falls in it.
+// G stays within 64 Mi floats per face; larger U is split into chunks of u,
+// each with the angles whose u falls in it.
 hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const double* theta, int n_theta,
                          const double* phi, int n_phi, double r, const double center[3], hipStream_t s,
                          Nf2ffCache* cache, Nf2ffOut* out) {
@@ -938,22 +1046,36 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
             return hipErrorInvalidValue;
         if (n1 * n2 > (size_t)INT32_MAX / 16) return hipErrorInvalidValue;
     }
-    NF_OK(hipStreamSynchronize(s));
     NF_OK(plan_angles(*cache, theta, n_theta, phi, n_phi, s));
     Nf2ffCache& C = *cache;
     const double k = 2.0 * M_PI * freq / C0;
     const double* d_kap = C.kap.as<double>();
+    // the large contractions on the FP16 matrix cores (operands split in two
+    // halves, k_hgemm3) unless OE_NF2FF_SPLIT16=0
+    bool split16 = true;
+    if (const char* v = getenv("OE_NF2FF_SPLIT16")) split16 = atoi(v) != 0;
+    // the second contraction by mirror groups where they hold two or more
+    // angles on average, unless OE_NF2FF_MIRROR=0
+    bool mirror = true;
+    if (const char* v = getenv("OE_NF2FF_MIRROR")) mirror = atoi(v) != 0;
 
     // per face: first-contraction axis p (fewer distinct |kappa|), sizes
     struct Plan {
-        int p, q, np, nq, K, N, swap;
+        int p, q, np, nq, K, N, swap, lane, chunk, n_chunks;
         std::vector<double> xp, xq;
     };
-    std::vector<Plan> plans;
-    size_t coord_len = 0, blocks = 0;
-    for (const auto& f : faces) {
+    const int nf = (int)faces.size();
+    std::vector<Plan> plans(nf);
+    // rows of one chunk: G within 64 Mi floats for the widest of the z faces,
+    // and of the others (of all, when there is only one kind)
+    bool kinds[2] = {false, false};
+    for (const auto& f : faces) kinds[f.axis != 2] = true;
+    size_t coord_len = 0, blocks = 0, Nmax[2] = {GBN, GBN};
+    int Umax[2] = {0, 0};
+    for (int q = 0; q < nf; ++q) {
+        const Nf2ffFace& f = faces[q];
+        Plan& pl = plans[q];
         const int a1 = (f.axis + 1) % 3, a2 = (f.axis + 2) % 3;
-        Plan pl{};
         pl.swap = C.ax[a2].U < C.ax[a1].U;
         pl.p = pl.swap ? a2 : a1;
         pl.q = pl.swap ? a1 : a2;
@@ -967,115 +1089,180 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
         for (double v : cq) pl.xq.push_back(v - center[pl.q]);
         coord_len += 2 * ((size_t)pl.np + pl.nq);
         blocks += (cp.size() * cq.size() + 255) / 256;
-        plans.push_back(std::move(pl));
+        pl.lane = kinds[0] && kinds[1] && f.axis != 2;
+        Nmax[pl.lane] = std::max(Nmax[pl.lane], (size_t)pl.N);
+        Umax[pl.lane] = std::max(Umax[pl.lane], C.ax[pl.p].U);
     }
-    // Faces run in up to two lanes: the z faces (the large contractions) on
-    // the caller's stream, the x and y faces on a side stream with buffers
-    // and an N/L accumulator of their own, so that their small,
-    // latency-bound launches overlap the large ones (OE_NF2FF_STREAMS=1: all
-    // on the caller's stream).
-    int n_streams = 2;
-    if (const char* v = getenv("OE_NF2FF_STREAMS")) n_streams = atoi(v) == 1 ? 1 : 2;
-    std::vector<int> lane_of(faces.size(), 0);
-    bool in_lane[2] = {false, false};
-    for (size_t fi = 0; fi < faces.size(); ++fi) {
-        lane_of[fi] = (n_streams == 2 && faces[fi].axis != 2) ? 1 : 0;
-        in_lane[lane_of[fi]] = true;
-    }
-    if (!in_lane[0] || !in_lane[1]) std::fill(lane_of.begin(), lane_of.end(), 0);
-    const int L = (in_lane[0] && in_lane[1]) ? 2 : 1;
-    struct LaneBuf {
-        size_t Kmax = KPAD, Nmax = GBN, rows = GBM, off = 0, bt_off = 0;
-        float *Bm = nullptr, *Am = nullptr, *G = nullptr;
-        _Float16* bt = nullptr;
-        double* nl = nullptr;
-    } lb[2];
     const size_t budget = (size_t)64 << 20;
-    for (int l = 0; l < L; ++l) {
-        int Umax = 0;
-        for (size_t fi = 0; fi < faces.size(); ++fi) {
-            if (lane_of[fi] != l) continue;
-            lb[l].Kmax = std::max(lb[l].Kmax, (size_t)plans[fi].K);
-            lb[l].Nmax = std::max(lb[l].Nmax, (size_t)plans[fi].N);
-            Umax = std::max(Umax, C.ax[plans[fi].p].U);
-        }
-        const size_t r0 = std::max<size_t>(GBM, budget / lb[l].Nmax / GBM * GBM);
-        lb[l].rows = std::min(r0, round_up(2 * (size_t)Umax, GBM));
+    size_t rows[2];
+    for (int l = 0; l < 2; ++l)
+        rows[l] = std::min(std::max<size_t>(GBM, budget / Nmax[l] / GBM * GBM), round_up(2 * (size_t)Umax[l], GBM));
+    // sets of up to MAX_FACES faces share the launches and, from one set to
+    // the next, the buffers
+    const int n_sets = (nf + MAX_FACES - 1) / MAX_FACES;
+    std::vector<int> set_chunks(n_sets, 0);
+    size_t n_table = 0;
+    for (int q = 0; q < nf; ++q) {
+        Plan& pl = plans[q];
+        pl.chunk = (int)(rows[pl.lane] / 2);
+        pl.n_chunks = (C.ax[pl.p].U + pl.chunk - 1) / pl.chunk;
+        int& m = set_chunks[q / MAX_FACES];
+        m = std::max(m, pl.n_chunks);
     }
+    for (int m : set_chunks) n_table += (size_t)m * MAX_FACES;
 
+    // device workspace: the tables (uploaded in one copy), then results,
+    // partials and per face slot the operands
     const size_t pblocks = (n_ang + 255) / 256;
-    const size_t n_dbl = 12 * n_ang * L + 4 * n_ang + pblocks + coord_len + blocks;
-    size_t off = round_up(n_dbl * sizeof(double), 256);
-    for (int l = 0; l < L; ++l) {
-        lb[l].off = off;
-        off = round_up(off + (lb[l].Kmax * lb[l].Nmax + lb[l].rows * lb[l].Kmax + lb[l].rows * lb[l].Nmax) *
-                                 sizeof(float), 256);
-        lb[l].bt_off = off;
-        off = round_up(off + lb[l].Kmax * lb[l].Nmax * sizeof(float), 256);
-    }
+    const size_t face_off = 0, chunk_off = round_up(nf * sizeof(FaceDev), 64);
+    const size_t coord_off = round_up(chunk_off + n_table * sizeof(ChunkDev), 64);
+    const size_t up_bytes = coord_off + coord_len * sizeof(double);
+    size_t off = round_up(up_bytes, 256);
+    const size_t out_off = off;  // E_theta, E_phi, block maxima of U, power partials
+    const size_t out_len = 4 * n_ang + pblocks + blocks;
+    off = round_up(off + out_len * sizeof(double), 256);
+    const size_t nl_off = off;
+    if (n_sets > 1) off = round_up(off + 12 * n_ang * sizeof(double), 256);
     const size_t pmax_off = off;
     off = round_up(off + blocks * sizeof(float), 256);
     const size_t bsc_off = off;
-    const size_t bytes = off + 2 * faces.size() * sizeof(float);
-    if (C.work.bytes < bytes) {
-        NF_OK(C.work.alloc(bytes));
-        C.bm_off[0] = C.bm_off[1] = SIZE_MAX;
+    off = round_up(off + 2 * (size_t)nf * sizeof(float), 256);
+    struct Slot {
+        size_t B = 0, A = 0, G = 0, S = 0, b = 0, a = 0, g = 0;
+    } slot[MAX_FACES];
+    for (int q = 0; q < nf; ++q) {
+        const Plan& pl = plans[q];
+        Slot& t = slot[q % MAX_FACES];
+        const size_t M = std::min(rows[pl.lane], round_up(2 * (size_t)C.ax[pl.p].U, GBM));
+        t.b = std::max(t.b, (size_t)pl.K * pl.N);
+        t.a = std::max(t.a, M * pl.K);
+        t.g = std::max(t.g, M * pl.N);
     }
-    char* wk = reinterpret_cast<char*>(C.work.p);
-    double* d_nl = C.work.as<double>();
-    double* d_ff = d_nl + 12 * n_ang * L;
-    double* d_umax = d_ff + 4 * n_ang;
-    double* d_coord = d_umax + pblocks;
-    double* d_part = d_coord + coord_len;
-    // B is zeroed only when its region moves or grows.  Its padding rows
-    // (p >= np) are cleared per face after the pack (k_nf2ff_pad_rows), and
-    // A's padding columns are exact zeros (k_phase), so they add signed zeros
-    // to every product; B's padding columns only reach G columns the
-    // reduction never reads.
-    for (int l = 0; l < L; ++l) {
-        LaneBuf& b = lb[l];
-        b.Bm = reinterpret_cast<float*>(wk + b.off);
-        b.Am = b.Bm + b.Kmax * b.Nmax;
-        b.G = b.Am + b.rows * b.Kmax;
-        // split fp16 halves of B (transposed, [N][K] each)
-        b.bt = reinterpret_cast<_Float16*>(wk + b.bt_off);
-        b.nl = d_nl + 12 * n_ang * l;
-        const size_t len = b.Kmax * b.Nmax * sizeof(float);
-        if (b.off != C.bm_off[l] || len > C.bm_len[l]) {
-            NF_OK(hipMemsetAsync(b.Bm, 0, len, s));
-            C.bm_off[l] = b.off;
-            C.bm_len[l] = len;
-        }
+    for (int q = 0; q < std::min(nf, MAX_FACES); ++q) {
+        Slot& t = slot[q];
+        t.B = off;  // B, then its split halves [N][K] each
+        off = round_up(off + 2 * t.b * sizeof(float), 256);
+        t.A = off;
+        off = round_up(off + t.a * sizeof(float), 256);
+        t.G = off;
+        off = round_up(off + t.g * sizeof(float), 256);
+        t.S = off;
+        off = round_up(off + 8 * n_ang * sizeof(double), 256);
     }
-    float* d_pmax = reinterpret_cast<float*>(wk + pmax_off);  // the pack's block maxima of |B|, per face as d_part
-    // per face the scale of B and its inverse
-    float* d_bsc = reinterpret_cast<float*>(wk + bsc_off);
-    if (L == 2 && !C.side) {
-        NF_OK(hipStreamCreateWithFlags(&C.side, hipStreamNonBlocking));
-        NF_OK(hipEventCreateWithFlags(&C.ev_fork, hipEventDisableTiming));
-        NF_OK(hipEventCreateWithFlags(&C.ev_join, hipEventDisableTiming));
+    if (C.work.bytes < off) {
+        NF_OK(hipStreamSynchronize(s));
+        NF_OK(C.work.alloc(off));
     }
-    // the large contractions on the FP16 matrix cores (operands split in two
-    // halves, k_hgemm3) unless OE_NF2FF_SPLIT16=0
-    bool split16 = true;
-    if (const char* v = getenv("OE_NF2FF_SPLIT16")) split16 = atoi(v) != 0;
-    // the second contraction by mirror groups where they hold two or more
-    // angles on average, unless OE_NF2FF_MIRROR=0
-    bool mirror = true;
-    if (const char* v = getenv("OE_NF2FF_MIRROR")) mirror = atoi(v) != 0;
+    const size_t host_bytes = std::max(up_bytes, out_len * sizeof(double));
+    if (C.host.bytes < host_bytes) NF_OK(C.host.alloc(host_bytes));
+    char* wk = C.work.as<char>();
+    double* d_out = reinterpret_cast<double*>(wk + out_off);
+    double* d_umax = d_out + 4 * n_ang;
+    double* d_nl = n_sets > 1 ? reinterpret_cast<double*>(wk + nl_off) : nullptr;
 
-    std::vector<double> coords;
-    coords.reserve(coord_len);
-    for (const auto& pl : plans) {
-        coords.insert(coords.end(), pl.xp.begin(), pl.xp.end());
-        const auto wp = trapz_weights(pl.xp);
-        coords.insert(coords.end(), wp.begin(), wp.end());
-        coords.insert(coords.end(), pl.xq.begin(), pl.xq.end());
-        const auto wq = trapz_weights(pl.xq);
-        coords.insert(coords.end(), wq.begin(), wq.end());
+    FaceDev* hf = reinterpret_cast<FaceDev*>(static_cast<char*>(C.host.p) + face_off);
+    ChunkDev* hc = reinterpret_cast<ChunkDev*>(static_cast<char*>(C.host.p) + chunk_off);
+    double* hx = reinterpret_cast<double*>(static_cast<char*>(C.host.p) + coord_off);
+    const double* dx = reinterpret_cast<const double*>(wk + coord_off);
+    double flop = 0.0, flop_split = 0.0;
+    struct Launch {  // one chunk of one set
+        int wg[3] = {0, 0, 0};  // work-groups per KIND_*
+        int operands = 0, mirror = 0, plain = 0, table = 0;
+    };
+    std::vector<std::vector<Launch>> launches(n_sets);
+    std::vector<int> pack_blocks(n_sets, 0);
+    size_t co = 0, bo = 0, tb = 0;
+    for (int set = 0; set < n_sets; ++set) {
+        launches[set].resize(set_chunks[set]);
+        for (size_t c = 0; c < launches[set].size(); ++c) launches[set][c].table = (int)(tb + c * MAX_FACES);
+        std::memset(hc + tb, 0, launches[set].size() * MAX_FACES * sizeof(ChunkDev));
+        for (int q = set * MAX_FACES; q < std::min(nf, (set + 1) * MAX_FACES); ++q) {
+            const Nf2ffFace& f = faces[q];
+            const Plan& pl = plans[q];
+            const auto& A = C.ax[pl.p];
+            const auto& M = C.mir[f.axis];
+            const Slot& t = slot[q % MAX_FACES];
+            FaceDev d{};
+            d.src = f.src;
+            d.scale = f.scale;
+            d.kind = f.src_kind;
+            d.n1 = (int)f.c1.size();
+            d.n2 = (int)f.c2.size();
+            d.swap = pl.swap;
+            d.sign = f.sign;
+            d.np = pl.np; d.nq = pl.nq; d.K = pl.K; d.N = pl.N;
+            d.nb = (d.n1 * d.n2 + 255) / 256;
+            auto put = [&](const std::vector<double>& v) {
+                std::copy(v.begin(), v.end(), hx + co);
+                const double* at = dx + co;
+                co += v.size();
+                return at;
+            };
+            d.xp = put(pl.xp);
+            d.wp = put(trapz_weights(pl.xp));
+            d.xq = put(pl.xq);
+            d.wq = put(trapz_weights(pl.xq));
+            d.B = reinterpret_cast<float*>(wk + t.B);
+            d.Bhi = reinterpret_cast<_Float16*>(d.B + t.b);
+            d.Blo = d.Bhi + (size_t)pl.N * pl.K;
+            d.A = reinterpret_cast<float*>(wk + t.A);
+            d.G = reinterpret_cast<float*>(wk + t.G);
+            d.S = reinterpret_cast<double*>(wk + t.S);
+            d.bsc = reinterpret_cast<float*>(wk + bsc_off) + 2 * q;
+            d.part = d_umax + pblocks + bo;
+            d.pmax = reinterpret_cast<float*>(wk + pmax_off) + bo;
+            bo += d.nb;
+            d.uval = A.uval.as<double>();
+            d.uni_p = uniform_spacing(pl.xp, &d.dxp);
+            d.uni_q = uniform_spacing(pl.xq, &d.dxq);
+            d.x0 = f.c0 - center[f.axis];
+            d.kapq = d_kap + (size_t)pl.q * n_ang;
+            d.kap0 = d_kap + (size_t)f.axis * n_ang;
+            d.usgn = A.usgn.as<float>();
+            d.uidx = A.uidx.as<int>();
+            d.order = A.order.as<int>();
+            d.groups = A.groups.as<int2>();
+            d.mgroups = M.groups.as<int4>();
+            d.gkq = M.gkq.as<double>();
+            d.members = M.members.as<int>();
+            d.a1 = (f.axis + 1) % 3;
+            d.a2 = (f.axis + 2) % 3;
+            pack_blocks[set] = std::max(pack_blocks[set], d.nb);
+            for (int c = 0; c < pl.n_chunks; ++c) {
+                Launch& L = launches[set][c];
+                ChunkDev& ck = hc[L.table + q % MAX_FACES];
+                ck.u0 = c * pl.chunk;
+                ck.u1 = std::min(A.U, ck.u0 + pl.chunk);
+                ck.M = (int)round_up(2 * (size_t)(ck.u1 - ck.u0), GBM);
+                ck.kind = gemm_kind(ck.M, pl.N, split16);
+                ck.first = L.wg[ck.kind];
+                const int tile = ck.kind == KIND_FP32 ? 64 : 128;
+                L.wg[ck.kind] += (pl.N / tile) * (ck.M / tile);
+                if (ck.kind == KIND_SPLIT16) d.split = 1;
+                const int nm = M.mstart[ck.u1] - M.mstart[ck.u0];
+                // two or more angles per mirror group on average
+                ck.mirror = mirror && 2 * (size_t)nm <= (size_t)(A.start[ck.u1] - A.start[ck.u0]);
+                const auto& gs = ck.mirror ? M.mstart : A.gstart;
+                ck.g0 = gs[ck.u0];
+                ck.g1 = gs[ck.u1];
+                const int ng = ck.g1 - ck.g0;
+                if (ck.mirror) L.mirror = std::max(L.mirror, (ng + MIRROR_GROUPS - 1) / MIRROR_GROUPS);
+                else L.plain = std::max(L.plain, (ng + REDUCE_GROUPS - 1) / REDUCE_GROUPS);
+                const size_t work = (size_t)ck.M * pl.K / (ck.kind == KIND_SPLIT16 ? 8 : 1);
+                L.operands = std::max(L.operands, (int)std::min<size_t>((work + 255) / 256, 2048));
+                const double fl = 2.0 * (2.0 * (ck.u1 - ck.u0)) * (8.0 * pl.nq) * pl.np;  // useful (unpadded) work
+                flop += fl;
+                if (ck.kind == KIND_SPLIT16) flop_split += fl;
+            }
+            hf[q] = d;
+        }
+        // a face past its last chunk: no kind of launch holds it
+        for (size_t c = 0; c < launches[set].size(); ++c)
+            for (int q = 0; q < MAX_FACES; ++q)
+                if (hc[tb + c * MAX_FACES + q].M == 0) hc[tb + c * MAX_FACES + q].kind = -1;
+        tb += launches[set].size() * MAX_FACES;
     }
-    NF_OK(hipMemcpyAsync(d_coord, coords.data(), coords.size() * 8, hipMemcpyHostToDevice, s));
-    NF_OK(hipMemsetAsync(d_nl, 0, 12 * n_ang * L * sizeof(double), s));
+    NF_OK(hipMemcpyAsync(wk, C.host.p, up_bytes, hipMemcpyHostToDevice, s));
 
     size_t n_ev = 0;
     auto next_events = [&](EventPair** out) -> hipError_t {
@@ -1092,165 +1279,50 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
     NF_OK(next_events(&all));
     std::vector<EventPair*> gemm_ev;
     std::vector<bool> gemm_split;  // launch ran the split FP16 kernel
-    double flop_split = 0.0;
     NF_OK(hipEventRecord(all->a, s));
-    if (L == 2) {
-        NF_OK(hipEventRecord(C.ev_fork, s));
-        NF_OK(hipStreamWaitEvent(C.side, C.ev_fork, 0));
-    }
-    double flop = 0.0;
-    // per face, its offsets into the coordinates and the pack's block sums
-    std::vector<size_t> co_of(faces.size()), bo_of(faces.size());
-    for (size_t fi = 0, co = 0, bo = 0; fi < faces.size(); ++fi) {
-        co_of[fi] = co;
-        bo_of[fi] = bo;
-        co += 2 * ((size_t)plans[fi].np + plans[fi].nq);
-        bo += (faces[fi].c1.size() * faces[fi].c2.size() + 255) / 256;
-    }
-    // the caller's stream first: its long contractions then start while
-    // the host still issues the side stream's faces
-    std::vector<size_t> order;
-    for (int l = 0; l < L; ++l)
-        for (size_t fi = 0; fi < faces.size(); ++fi)
-            if (lane_of[fi] == l) order.push_back(fi);
-    for (size_t fi : order) {
-        const Nf2ffFace& f = faces[fi];
-        // this face's lane: its stream and buffers
-        const int ln = lane_of[fi];
-        const hipStream_t fs = ln ? C.side : s;
-        float* Bm = lb[ln].Bm;
-        float* Am = lb[ln].Am;
-        float* G = lb[ln].G;
-        _Float16* d_bt = lb[ln].bt;
-        const size_t rows = lb[ln].rows;
-        const Plan& pl = plans[fi];
-        const auto& A = C.ax[pl.p];
-        const int n1 = (int)f.c1.size(), n2 = (int)f.c2.size();
-        const int a1 = (f.axis + 1) % 3, a2 = (f.axis + 2) % 3;
-        const double* xp = d_coord + co_of[fi];
-        const double* wp = xp + pl.np;
-        const double* xq = wp + pl.np;
-        const double* wq = xq + pl.nq;
-        const size_t bo = bo_of[fi];
-        const int nb = (n1 * n2 + 255) / 256;
-        if (f.src_kind == 0)
-            hipLaunchKernelGGL(k_nf2ff_pack<0>, dim3(nb), dim3(256), 0, fs, f.src, f.scale, n1, n2, pl.swap, f.sign,
-                               wp, wq, Bm, pl.N, d_part + bo, d_pmax + bo);
-        else
-            hipLaunchKernelGGL(k_nf2ff_pack<1>, dim3(nb), dim3(256), 0, fs, f.src, f.scale, n1, n2, pl.swap, f.sign,
-                               wp, wq, Bm, pl.N, d_part + bo, d_pmax + bo);
+    const FaceDev* d_faces = reinterpret_cast<const FaceDev*>(wk + face_off);
+    const ChunkDev* d_chunks = reinterpret_cast<const ChunkDev*>(wk + chunk_off);
+    for (int set = 0; set < n_sets; ++set) {
+        const FaceDev* fd = d_faces + set * MAX_FACES;
+        const int n = std::min(MAX_FACES, nf - set * MAX_FACES);
+        hipLaunchKernelGGL(k_nf2ff_pack, dim3(pack_blocks[set], n), dim3(256), 0, s, fd);
+        bool any_split = false;
+        for (int q = 0; q < n; ++q) any_split = any_split || hf[set * MAX_FACES + q].split;
+        for (size_t c = 0; c < launches[set].size(); ++c) {
+            const Launch& L = launches[set][c];
+            const ChunkDev* cd = d_chunks + L.table;
+            hipLaunchKernelGGL(k_nf2ff_operands, dim3(L.operands, n, c == 0 && any_split ? 2 : 1), dim3(256), 0, s, fd, cd,
+                               k);
+            for (int kind : {KIND_SPLIT16, KIND_FP32_LARGE, KIND_FP32}) {
+                if (!L.wg[kind]) continue;
+                EventPair* ev = nullptr;
+                NF_OK(next_events(&ev));
+                gemm_ev.push_back(ev);
+                gemm_split.push_back(kind == KIND_SPLIT16);
+                NF_OK(hipEventRecord(ev->a, s));
+                const dim3 grid(L.wg[kind]);
+                if (kind == KIND_SPLIT16) hipLaunchKernelGGL(k_hgemm3, grid, dim3(256), 0, s, fd, cd, n);
+                else if (kind == KIND_FP32) hipLaunchKernelGGL(k_sgemm_mfma<64>, grid, dim3(256), 0, s, fd, cd, n);
+                else hipLaunchKernelGGL(k_sgemm_mfma<128>, grid, dim3(256), 0, s, fd, cd, n);
+                NF_OK(hipEventRecord(ev->b, s));
+            }
+            if (L.mirror)
+                hipLaunchKernelGGL(k_nf2ff_reduce_mirror, dim3(L.mirror, n), dim3(MIRROR_THREADS), 0, s, fd, cd, k);
+            if (L.plain) hipLaunchKernelGGL(k_nf2ff_reduce, dim3(L.plain, n), dim3(REDUCE_THREADS), 0, s, fd, cd, k);
+        }
+        if (set + 1 < n_sets)
+            hipLaunchKernelGGL(k_nf2ff_gather, dim3((unsigned)pblocks), dim3(256), 0, s, fd, n, d_nl, set == 0, n_ang);
         NF_OK(hipGetLastError());
-        if (pl.K > pl.np) {
-            const size_t npad = (size_t)(pl.K - pl.np) * pl.N;
-            hipLaunchKernelGGL(k_nf2ff_pad_rows, dim3((unsigned)std::min<size_t>((npad + 255) / 256, 1024)), dim3(256),
-                               0, fs, Bm, pl.N, pl.np, pl.K);
-            NF_OK(hipGetLastError());
-        }
-        const float* face_pmax = d_pmax + bo;
-        const int uchunk = (int)(rows / 2);
-        bool face16 = false;  // some contraction of this face runs on the FP16 matrix cores
-        for (int u0 = 0; u0 < A.U; u0 += uchunk) {
-            const int mp = (int)round_up(2 * (size_t)(std::min(A.U, u0 + uchunk) - u0), GBM);
-            face16 = face16 || use_split16(mp, pl.N, split16);
-        }
-        _Float16* Bhi = d_bt;
-        _Float16* Blo = d_bt + (size_t)pl.N * pl.K;
-        float* bsc = d_bsc + 2 * fi;
-        if (face16) {
-            hipLaunchKernelGGL(k_bsplit, dim3(pl.N / 64 + (pl.N % 64 != 0), (pl.K + 63) / 64), dim3(256), 0, fs, Bm, pl.K,
-                               pl.N, pl.np, 8 * pl.nq, face_pmax, nb, Bhi, Blo, bsc);
-            NF_OK(hipGetLastError());
-        }
-        double dxq = 0.0, dxp = 0.0;
-        const bool uni = uniform_spacing(pl.xq, &dxq);
-        const bool uni_p = uniform_spacing(pl.xp, &dxp);
-        ReduceArgs ra{};
-        ra.G = G;
-        ra.ldg = pl.N;
-        ra.order = A.order.as<int>();
-        ra.groups = A.groups.as<int2>();
-        ra.uidx = A.uidx.as<int>();
-        ra.usgn = A.usgn.as<float>();
-        ra.nq = pl.nq;
-        ra.kapq = d_kap + (size_t)pl.q * n_ang;
-        ra.kap0 = d_kap + (size_t)f.axis * n_ang;
-        ra.xq = xq;
-        ra.wq = wq;
-        ra.uniform = uni ? 1 : 0;
-        ra.dxq = dxq;
-        ra.x0 = f.c0 - center[f.axis];
-        ra.k = k;
-        ra.slot[0] = a1; ra.slot[1] = a2; ra.slot[2] = 3 + a1; ra.slot[3] = 3 + a2;
-        ra.NL = lb[ln].nl;
-        for (int u0 = 0; u0 < A.U; u0 += uchunk) {
-            const int u1 = std::min(A.U, u0 + uchunk);
-            const int mp = (int)round_up(2 * (size_t)(u1 - u0), GBM);
-            const size_t total = (size_t)mp * pl.K;
-            const int pb = (int)std::min<size_t>((total + 255) / 256, 16384);
-            const bool fp16 = use_split16(mp, pl.N, split16);
-            _Float16* Ahi = reinterpret_cast<_Float16*>(Am);
-            _Float16* Alo = Ahi + total;
-            if (fp16)
-                hipLaunchKernelGGL(k_phase16, dim3(std::max(1, pb / 8)), dim3(256), 0, fs, Ahi, Alo, pl.K, total, u0, u1,
-                                   pl.np, A.uval.as<double>(), xp, k, uni_p ? 1 : 0, dxp);
-            else
-                hipLaunchKernelGGL(k_phase, dim3(pb), dim3(256), 0, fs, Am, pl.K, total, u0, u1, pl.np,
-                                   A.uval.as<double>(), xp, k);
-            NF_OK(hipGetLastError());
-            EventPair* ev = nullptr;
-            NF_OK(next_events(&ev));
-            gemm_ev.push_back(ev);
-            NF_OK(hipEventRecord(ev->a, fs));
-            if (fp16) {
-                hipLaunchKernelGGL(k_hgemm3, dim3(pl.N / 128, mp / 128), dim3(256), 0, fs, Ahi, Alo, Bhi, Blo, G, mp, pl.N,
-                                   pl.K, bsc);
-                NF_OK(hipGetLastError());
-            } else {
-                NF_OK(launch_gemm(Am, Bm, G, mp, pl.N, pl.K, fs));
-            }
-            NF_OK(hipEventRecord(gemm_ev.back()->b, fs));
-            gemm_split.push_back(fp16);
-            const double fl = 2.0 * (2.0 * (u1 - u0)) * (8.0 * pl.nq) * pl.np;  // useful (unpadded) work
-            flop += fl;
-            if (fp16) flop_split += fl;
-            ra.g0 = A.gstart[u0];
-            ra.g1 = A.gstart[u1];
-            ra.u0 = u0;
-            const auto& M = C.mir[f.axis];
-            const int nm = M.mstart[u1] - M.mstart[u0];
-            if (mirror && 2 * (size_t)nm <= (size_t)(A.start[u1] - A.start[u0])) {
-                // two or more angles per mirror group on average
-                MirrorArgs ma{M.groups.as<int4>(), M.gkq.as<double>(), M.members.as<int>(), M.mstart[u0],
-                              M.mstart[u1]};
-                const dim3 grid((nm + MIRROR_GROUPS - 1) / MIRROR_GROUPS);
-                if (ra.uniform)
-                    hipLaunchKernelGGL(k_nf2ff_reduce_mirror<true>, grid, dim3(MIRROR_THREADS), 0, fs, ra, ma);
-                else
-                    hipLaunchKernelGGL(k_nf2ff_reduce_mirror<false>, grid, dim3(MIRROR_THREADS), 0, fs, ra, ma);
-            } else {
-                const int ng = ra.g1 - ra.g0;
-                hipLaunchKernelGGL(k_nf2ff_reduce, dim3((ng + REDUCE_GROUPS - 1) / REDUCE_GROUPS),
-                                   dim3(REDUCE_THREADS), 0, fs, ra);
-            }
-            NF_OK(hipGetLastError());
-        }
-    }
-    if (L == 2) {
-        NF_OK(hipEventRecord(C.ev_join, C.side));
-        NF_OK(hipStreamWaitEvent(s, C.ev_join, 0));
     }
     typedef std::complex<double> cd;
     const cd fac = cd(0.0, k) * std::exp(cd(0.0, -k * r)) / (4.0 * M_PI * r);
-    hipLaunchKernelGGL(k_nf2ff_project, dim3((unsigned)pblocks), dim3(256), 0, s, d_nl, L == 2 ? lb[1].nl : nullptr,
-                       d_kap + 3 * n_ang,
-                       d_kap + 3 * n_ang + n_theta, n_phi, n_ang, fac.real(), fac.imag(), r, d_ff, d_umax);
+    hipLaunchKernelGGL(k_nf2ff_project, dim3((unsigned)pblocks), dim3(256), 0, s, d_faces + (n_sets - 1) * MAX_FACES,
+                       nf - (n_sets - 1) * MAX_FACES, d_nl, d_kap + 3 * n_ang, d_kap + 3 * n_ang + n_theta, n_phi, n_ang,
+                       fac.real(), fac.imag(), r, d_out, d_umax);
     NF_OK(hipGetLastError());
     NF_OK(hipEventRecord(all->b, s));
-    const size_t hb = (4 * n_ang + pblocks + blocks) * sizeof(double);
-    if (C.host.bytes < hb) NF_OK(C.host.alloc(hb));
     double* h = reinterpret_cast<double*>(C.host.p);
-    NF_OK(hipMemcpyAsync(h, d_ff, (4 * n_ang + pblocks) * sizeof(double), hipMemcpyDeviceToHost, s));
-    NF_OK(hipMemcpyAsync(h + 4 * n_ang + pblocks, d_part, blocks * sizeof(double), hipMemcpyDeviceToHost, s));
+    NF_OK(hipMemcpyAsync(h, d_out, out_len * sizeof(double), hipMemcpyDeviceToHost, s));
     NF_OK(hipStreamSynchronize(s));
     float ms = 0.f;
     NF_OK(hipEventElapsedTime(&ms, all->a, all->b));

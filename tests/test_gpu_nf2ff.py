@@ -267,6 +267,43 @@ def test_fdtd_dipole_fp32_kahan_far_field():
         assert abs(gb.prad / ga.prad - 1) < 1e-5
 
 
+@pytest.mark.parametrize("mirror", ["1", "0"])
+@pytest.mark.parametrize("steps,extra,nt,np_", [
+    ((2, 3, 4), 0, 5, 3),        # fewer nodes than lanes of a group
+    ((1, 17, 16), 1, 19, 2),     # an axis of one node; seven faces
+    ((9, 65, 33), 6, 37, 72),    # twelve faces, tiles and remainders
+    ((20, 21, 5), 7, 1, 1),      # thirteen faces, one angle
+], ids=["tiny", "seven", "twelve", "thirteen"])
+def test_faces_share_launches(monkeypatch, steps, extra, nt, np_, mirror):
+    """All faces of a surface go through common launches, six at a time: any
+    number of faces, with sizes below and beside the tiles and group widths,
+    gives the oracle's far field (PATTERN_TOL; P_rad is summed in float64),
+    and a second call repeats the first bit for bit."""
+    monkeypatch.setenv("OE_NF2FF_MIRROR", mirror)
+    rng = np.random.default_rng(sum(steps) + extra)
+    f = 8e9
+    faces = []
+    for q in range(6 + extra):
+        axis, sign = q % 3, 1 if q % 2 else -1
+        n1, n2 = steps[(axis + 1) % 3] + q // 6, steps[(axis + 2) % 3] + q // 5
+        c1, c2 = np.linspace(-0.02, 0.03, n1), np.sort(rng.uniform(-0.02, 0.02, n2))
+        E = rng.standard_normal((3, n1, n2)) + 1j * rng.standard_normal((3, n1, n2))
+        H = (rng.standard_normal((3, n1, n2)) + 1j * rng.standard_normal((3, n1, n2))) / N.Z0
+        faces.append(N.Face(axis, sign, 0.02 * sign + 0.001 * q, c1, c2, E, H))
+    th = np.linspace(0, math.pi, nt) if nt > 1 else np.array([0.7])
+    ph = np.linspace(0, 2 * math.pi, np_ + 1)[:-1]
+    Et, Ep, prad, _ = N.far_field(faces, f, th, ph)
+    g = _gpu_far_field(faces, f, th, ph)
+    err = math.sqrt((np.linalg.norm(g.e_theta - Et) ** 2 + np.linalg.norm(g.e_phi - Ep) ** 2)
+                    / (np.linalg.norm(Et) ** 2 + np.linalg.norm(Ep) ** 2))
+    scale = sum(np.abs(N.radiated_power([fc])) for fc in faces)
+    say(f"[nf2ff] {len(faces)} faces of {steps}, {nt}x{np_} angles, mirror {mirror}: rel L2 {err:.2e}")
+    assert err <= PATTERN_TOL
+    assert abs(g.prad - prad) <= 1e-12 * scale
+    again = _gpu_far_field(faces, f, th, ph)
+    assert np.array_equal(again.e_theta, g.e_theta) and np.array_equal(again.e_phi, g.e_phi)
+
+
 def test_split_fp16_contraction_against_oracle_and_fp32(monkeypatch):
     """z faces of 100 x 300 nodes and 181 x 180 irregular angles: the large
     contractions run on the FP16 matrix cores with split operands over
