@@ -134,9 +134,9 @@ def fused_index_bytes(rows):
 
 
 def launch_bytes(name, shape, layers, coef="arrays", rows=(0, 0)):
-    """Algorithmic bytes of one launch of the plan: 'grid' (no CPML), or
-    'interior' (x/y slabs excluded; z-face psi at the row ends) and 'slabs'
-    (the x/y face slabs with all faces) when a CPML is attached.  A fused
+    """Algorithmic bytes of one launch of the plan: 'grid' (the whole grid,
+    with its CPML if layers), or 'interior' (x/y slabs excluded; z-face psi at
+    the row ends) and 'slabs' (the x/y face slabs with all faces).  A fused
     launch ('fused:interior', 'fused:grid') covers both half-steps of its
     box: FUSED_CELL_BYTES per cell, 32 B per z-slab cell (H and E psi).
     rows: the material table's rows of E and H (a half of one row reads no
@@ -150,7 +150,7 @@ def launch_bytes(name, shape, layers, coef="arrays", rows=(0, 0)):
         return fb * ix * jy * nz + 32 * ix * jy * zl
     coef = half_coef(coef, rows, kind == "update_h")
     if part == "grid" or not layers:
-        return kernel_bytes(shape, 0, coef)
+        return kernel_bytes(shape, layers, coef)
     ix, jy = nx - 2 * layers, ny - 2 * layers
     interior = CELL_BYTES[coef] * ix * jy * nz + 16 * ix * jy * 2 * layers
     if part == "interior":
@@ -792,6 +792,9 @@ def yee_point(wl, mode, steps, warmup, period, tiles="", coef_opt="auto", fused=
         "bound": "hbm",
         "kernel": {"update_h:interior": "k_update_h<4,AX_Z,phys> (interior box, z-face CPML)",
                    "update_e:interior": "k_update_e<4,AX_Z,phys> (interior box, z-face CPML)",
+                   **({"update_h:grid": "k_update_h_mix<AX_Z,phys> (whole grid with its CPML)",
+                       "update_e:grid": "k_update_e_mix<AX_Z,phys> (whole grid with its CPML)"}
+                      if wl.cpml_layers else {}),
                    "fused:interior": "k_fused_rows<AX_Z,phys> (H and E of the interior box in one pass)"}.get(dom, dom),
         "achieved": round(achieved, 1),
         "peak": HBM_PEAK_GBS,

@@ -249,9 +249,9 @@ oe_status oe_engine_run_batch(oe_engine* eng, const oe_batch_desc* batch, oe_bat
 
 /* Kernel timing accumulated while profiling is on, measured with HIP events
  * on the engine's stream around every launch.  Names: "update_h:grid" and
- * "update_e:grid" (no CPML), or "update_h:interior" / "update_h:slabs" and
- * the "update_e:" pair (CPML: interior box with z-face CPML, x/y face slabs
- * with all faces), "mur_pre", "mur_post", "ade_pre", "ade_post",
+ * "update_e:grid" (one launch over the grid), or "update_h:interior" /
+ * "update_h:slabs" and the "update_e:" pair (CPML in two launches: interior
+ * box with z-face CPML, x/y face slabs with all faces), "mur_pre", "mur_post", "ade_pre", "ade_post",
  * "point_ops", "energy".  Returns the launch count and total milliseconds. */
 oe_status oe_engine_kernel_time(oe_engine* eng, const char* name, uint64_t* launches, double* total_ms);
 

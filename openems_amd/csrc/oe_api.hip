@@ -76,9 +76,13 @@ int pow2ceil(int v) {
 // four where the row is cut into narrow blocks (256x320x384 511 / 511 / 497).
 // Scalar lanes, whose planes are cheaper than their start, take two
 // (151x133x117 with CPML, ci 1 / 2 / 3: 82.5 / 75.0 / 81.0).
+// Whether a plane's byte offsets fit the float4 kernels' 32 bits (one row
+// beyond either end included).
+bool narrow_plane(const Grid& g) { return ((size_t)g.ny + 2) * g.nz < ((size_t)1 << 30); }
+
 Tiles auto_tiles(const Grid& g, int vec_req) {
     Tiles t{};
-    t.vec = vec_req == 1 || (g.nz % 4 != 0 && g.nz < 8) ? 1 : 4;
+    t.vec = vec_req == 1 || (g.nz % 4 != 0 && g.nz < 8) || !narrow_plane(g) ? 1 : 4;
     const int nzv = (g.nz + t.vec - 1) / t.vec;
     const int widest = t.vec == 4 ? 64 : 128;
     double best = 0.0;
@@ -142,8 +146,15 @@ YeeArgs launch_args(const oe_engine* e, const Tiles& t, const CpmlArgs* cp, cons
     return a;
 }
 
+// The profile's name of a launch.
+const char* launch_name(int axes, const CpmlArgs* cp, bool h) {
+    if (axes & (AX_X | AX_Y)) return h ? "update_h:slabs" : "update_e:slabs";
+    if (cp && !(axes & AX_MIX)) return h ? "update_h:interior" : "update_e:interior";
+    return h ? "update_h:grid" : "update_e:grid";
+}
+
 // Launch plan of one half-step.  Without CPML: one launch of the plain kernel
-// over the grid.  With CPML: the x and y face slabs (whole planes / rows) go
+// over the grid.  With CPML (mix false): the x and y face slabs (whole planes / rows) go
 // to the all-faces kernel in one launch of up to four boxes, and the interior
 // planes and rows -- whose only slab cells are the z faces at the ends of each
 // row -- to the lighter z-faces kernel.  The boxes tile the grid exactly once.
@@ -174,8 +185,25 @@ std::vector<Launch> plan_launches(const oe_engine* e, const Tiles& t, const Cpml
         if (jy1 < g.ny) slabs.push_back(make_box(ts, ix0, ix1, jy1, g.ny));
     }
     const bool inner = ix1 > ix0 && jy1 > jy0;
-    if (mix && inner && !slabs.empty()) {
-        slabs.push_back(make_box(t, ix0, ix1, jy0, jy1));
+    if (mix && !slabs.empty()) {
+        // One launch over whole-grid tiles, the body chosen per work-group.
+        // j-blocks of the whole grid: those that meet a y slab (the first lo
+        // and the last hi of them) run the slab code for all their rows
+        const int n = (g.ny + t.by - 1) / t.by;
+        const int lo = std::min(n, (jy0 + t.by - 1) / t.by);
+        const int hi = jy1 < g.ny ? std::min(n - lo, n - jy1 / t.by) : 0;
+        slabs.clear();
+        if (ix0 > 0) slabs.push_back(make_box(t, 0, ix0, 0, g.ny));
+        if (ix1 < g.nx) slabs.push_back(make_box(t, ix1, g.nx, 0, g.ny));
+        if (ix1 > ix0 && lo + hi > 0) {
+            Box b = make_box(t, ix0, ix1, 0, g.ny);
+            b.n_jb = lo + hi;
+            b.jb_cut = lo;
+            b.j_skip = (n - hi - lo) * t.by;
+            slabs.push_back(b);
+        }
+        slabs.push_back(make_box(t, ix0, std::max(ix0, ix1), lo * t.by, std::max(lo, n - hi) * t.by));
+        slabs.back().j1 = std::min(slabs.back().j1, g.ny);
         out.push_back({launch_args(e, t, cp, slabs), AX_MIX | ((m & 48) ? AX_Z : 0)});
         return out;
     }
@@ -1763,6 +1791,7 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         HIP_OK(hipMemcpyAsync(e->probe_table.p, pp.data(), pp.size() * sizeof(PointProbe), hipMemcpyHostToDevice, e->stream));
     Tiles tl = e->tiles;
     // a float4 lane meets at most one z slab, or lanes are scalar
+    if (tl.vec == 4 && !narrow_plane(e->g)) tl = auto_tiles(e->g, 1);
     if (cp && !cp->zvec && tl.vec == 4 && (cp->on_mask & 48) == 48 && cp->g0[5] - cp->L[4] < 3) tl = auto_tiles(e->g, 1);
     // Fused steps (one pass per step over the plan's interior box) when no
     // extension hooks in between the half-steps and the grid suits the
@@ -1772,25 +1801,27 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     const bool host = !hosts.empty();
     const bool fused = e->fused_mode && !host && !upml && murs.empty() && ades.empty() && tl.vec == 4 &&
                        fused_supported(e->g) && (e->fused_mode == 2 || e->g.nz >= 128) && (!cp || cp->zvec);
-    // Small CPML grids with a material table take one launch per half-step:
-    // the second launch's start and tail cost more than the interior's halved
-    // occupancy up to about 4.5 M cells.  us per step, two launches / one (the
-    // best depth of each): 72x60x32 22.0 / 12.0, 100x100x48 24.6 / 17.6,
-    // 100^3 31.5 / 27.8, 160x144x128 63.3 / 55.4, 200x160x128 78.6 / 71.6,
-    // 240x200x128 101.7 / 102.4, 256^3 241 / 265.
+    // CPML grids with a material table take one launch per half-step.  Two
+    // launches cost a second start and tail, and work-groups of a slab's few
+    // rows leave most of their lanes idle.  us per step, two launches / one:
+    // 72x60x32 22.0 / 11.2, 200x150x40 39 / 27.0, 144^3 61 / 52.5, 256x200x128
+    // 100.9 / 92.1, 256^3 227.8 / 218.5, 384x384x256 557 / 547, 800x500x40
+    // 287.6 / 262.7.  (Overlapped or separately tiled slab launches, scalar
+    // lanes and grids without a table keep the two.)
     const bool mix = cp && !fused && tl.vec == 4 && !e->overlap_slabs && e->slab_tiles.bx <= 0 && e->n_mat[0] > 0 &&
                      e->n_mat[1] > 0 && e->g.N <= e->mix_cells;
     if (mix && e->tiles_auto) {
-        // At 2 waves a SIMD the chip holds 512 of its work-groups at a time,
-        // and such grids fill it once to a few times: the depth that wastes
-        // least of the last fill (160x144x128, ci 1 .. 8: 60.9 57.7 56.7 62.5
-        // 70.3 55.4 60.3 65.7, of which 3 and 6 fill it twice and once).
+        // At 3 waves a SIMD the chip holds 768 of its work-groups at a time,
+        // and such grids fill it once to a few times: the depth, 1 or 2, that
+        // wastes less of the last fill (us per step at 1 / 2: 100^3 22.7 /
+        // 21.0, 200x150x40 27.6 / 27.0, 140x90x40 14.3 / 16.6; deeper ones are
+        // slower at nearly every size).
         double best = 1e300;
-        for (int ci = 1; ci <= std::min(8, e->g.nx); ++ci) {
+        for (int ci = 1; ci <= std::min(2, e->g.nx); ++ci) {
             Tiles t = tl;
             t.ci = ci;
             const YeeArgs a = plan_launches(e, t, cp, true).back().a;
-            const double cost = std::ceil(a.first[a.nbox] / 512.0) * (ci + 0.5);
+            const double cost = std::ceil(a.first[a.nbox] / 768.0) * (ci + 0.5);
             if (cost < best) {
                 best = cost;
                 tl.ci = ci;
@@ -1814,11 +1845,12 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         for (const auto* ax : ades)
             if (std::binary_search(ax->ade_cells.begin(), ax->ade_cells.end(), px[q].idx)) fold_sources = false;
     }
-    if (const char* v = getenv("OE_FOLD_SOURCES")) fold_sources = fold_sources && atoi(v) != 0;
     // Probes, small DFTs and the ADE and Mur captures ride in the Yee launches
     // (oe_ride.h) unless the steps are fused or host hooks stand between them.
     // The plan's last launch carries them: the interior, or the whole grid.
     const bool riding = !fused && !host && e->ride && (plan.back().axes & (AX_X | AX_Y)) == 0;
+    fold_sources = fold_sources && riding;  // a rider looks their values up
+    if (const char* v = getenv("OE_FOLD_SOURCES")) fold_sources = fold_sources && atoi(v) != 0;
     const bool point_ops = (!px.empty() && !fold_sources) || (!pp.empty() && !riding);
     FusedArgs fa{};
     std::vector<Launch> slabs;
@@ -1985,7 +2017,20 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         rt.step_b = step_dev + 1;
         rt.n_probe = (int)pp.size();
         rt.probe = e->probe_table.as<PointProbe>();
-        rt.first_dft = pp.empty() ? 0 : 1;
+        const size_t val_off = (sizeof(Ride) + 63) / 64 * 64;
+        const size_t ride_bytes = val_off + MAX_FOLD_SOURCES * sizeof(SourceValue);
+        if (e->ride_table.bytes < ride_bytes) HIP_OK(e->ride_table.alloc(ride_bytes));
+        if (fold_sources) {
+            rt.n_src = (int)px.size();
+            rt.src = e->exc_table.as<PointExc>();
+            rt.src_val = reinterpret_cast<SourceValue*>(e->ride_table.as<char>() + val_off);
+            for (Launch& L : plan_e) {
+                L.a.src_val = rt.src_val;
+                L.a.n_src = rt.n_src;
+                for (size_t q = 0; q < px.size(); ++q) L.a.src_idx[q] = px[q].idx;
+            }
+        }
+        rt.first_dft = pp.empty() && !fold_sources ? 0 : 1;
         for (auto* x : ride_dfts) rt.dft[rt.n_dft++] = RideDft{x->dft, x->dft_count};
         rt.first_ade = rt.first_dft + rt.n_dft;
         int wg = rt.first_ade;
@@ -2006,7 +2051,6 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         rt.n_wg = wg;
         n_ride_h = wg;
         n_ride_e = rt.first_ade;
-        if (e->ride_table.bytes < sizeof(Ride)) HIP_OK(e->ride_table.alloc(sizeof(Ride)));
         HIP_OK(hipMemcpy(e->ride_table.p, &rt, sizeof(Ride), hipMemcpyHostToDevice));
         plan_h.back().a.ride = plan_e.back().a.ride = e->ride_table.as<Ride>();
         plan_h.back().a.n_ride = n_ride_h;
@@ -2030,17 +2074,10 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         HIP_OK(hipEventCreateWithFlags(&e->ev_fork, hipEventDisableTiming));
         HIP_OK(hipEventCreateWithFlags(&e->ev_join, hipEventDisableTiming));
     }
-    auto overlapped_half = [&](bool h, uint64_t st) -> oe_status {
+    auto overlapped_half = [&](bool h) -> oe_status {
         auto one = [&](const Launch& L, hipStream_t s) -> hipError_t {
             if (h) return launch_update_h(L.a, cp, L.axes, s);
-            if (!fold_sources) return launch_update_e(L.a, cp, L.axes, s);
-            YeeArgs a = L.a;
-            a.exc = e->exc_table.as<PointExc>();
-            a.n_exc = (int)px.size();
-            for (size_t q = 0; q < px.size(); ++q) a.exc_idx[q] = px[q].idx;
-            a.exc_step = st;
-            a.exc_step_dev = step_dev;
-            return launch_update_e(a, cp, L.axes, s);
+            return launch_update_e(L.a, cp, L.axes, s);
         };
         const std::vector<Launch>& pl = h ? plan_h : plan_e;
         HIP_OK(hipEventRecord(e->ev_fork, e->stream));
@@ -2133,10 +2170,10 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         }
         if (host) OE_TRY(run_hooks(0));
         if (!fused && ovl) {
-            OE_TRY(overlapped_half(true, st));
+            OE_TRY(overlapped_half(true));
         } else if (!fused)
             for (const Launch& L : plan_h) {
-                Timed tm(e, (L.axes & (AX_X | AX_Y)) ? "update_h:slabs" : (cp ? "update_h:interior" : "update_h:grid"));
+                Timed tm(e, launch_name(L.axes, cp, true));
                 HIP_OK(launch_update_h(L.a, cp, L.axes, e->stream));
             }
         if (upml) {
@@ -2168,21 +2205,11 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         }
         if (host) OE_TRY(run_hooks(2));
         if (!fused && ovl) {
-            OE_TRY(overlapped_half(false, st));
+            OE_TRY(overlapped_half(false));
         } else if (!fused)
             for (const Launch& L : plan_e) {
-                Timed tm(e, (L.axes & (AX_X | AX_Y)) ? "update_e:slabs" : (cp ? "update_e:interior" : "update_e:grid"));
-                if (fold_sources) {
-                    YeeArgs a = L.a;
-                    a.exc = e->exc_table.as<PointExc>();
-                    a.n_exc = (int)px.size();
-                    for (size_t q = 0; q < px.size(); ++q) a.exc_idx[q] = px[q].idx;
-                    a.exc_step = st;
-                    a.exc_step_dev = step_dev;
-                    HIP_OK(launch_update_e(a, cp, L.axes, e->stream));
-                } else {
-                    HIP_OK(launch_update_e(L.a, cp, L.axes, e->stream));
-                }
+                Timed tm(e, launch_name(L.axes, cp, false));
+                HIP_OK(launch_update_e(L.a, cp, L.axes, e->stream));
             }
         if (upml) {
             Timed tm(e, "upml");

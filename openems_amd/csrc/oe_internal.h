@@ -85,10 +85,14 @@ constexpr int MAX_BOXES = 5;
 struct Box {
     int i0, i1, j0, j1;
     int n_jb, n_ib;  // j-blocks, i-chunks of this box
+    int jb_cut, j_skip;  // j-blocks from jb_cut on start j_skip rows further
 };
 
-struct PointExc;
 constexpr int MAX_FOLD_SOURCES = 8;
+struct SourceValue {
+    float v;
+    uint32_t code;  // 0 nothing this step, else 1 | soft << 1 | component << 2
+};
 
 // Mur faces folded into the E update: a z face's line and shift cells are
 // lanes of one float4 lane group, so the thread that updates them also takes
@@ -127,14 +131,13 @@ struct YeeArgs {
     int xcd_remap;         // 1: make consecutive tiles share an XCD (L2)
     // Point sources added by the E half-step after its update (when no
     // extension acts between the E update and the sources): the lane holding
-    // a source's cell adds or sets samples[exc_step], in list order.  The
-    // cell indices travel in the kernel arguments, so the per-plane test is
-    // a comparison with uniform values.
-    const PointExc* exc;
-    int n_exc;
-    uint32_t exc_idx[MAX_FOLD_SOURCES];
-    uint64_t exc_step;
-    const uint64_t* exc_step_dev;  // non-null: the step comes from the device counter
+    // a source's cell adds or sets its value, in list order.  The cell
+    // indices travel in the kernel arguments, so the per-plane test is a
+    // comparison with uniform values; the values of the step come from the
+    // riders of the H launch (oe_ride.h).
+    const struct SourceValue* src_val;
+    int n_src;
+    uint32_t src_idx[MAX_FOLD_SOURCES];
     // First-order Mur on the z faces applied by the E half-step itself (see
     // e_body): on[0] the k = 0 face, on[1] the k = nz - 1 face.
     MurZ mur_z;
@@ -408,6 +411,9 @@ struct Ride {
     int n_probe, n_dft, n_ade, n_mur;
     int first_dft, first_ade, first_mur, n_wg;
     int ade_first[MAX_MERGE_ADE];
+    int n_src;                // folded sources: values of the step to come
+    const struct PointExc* src;
+    SourceValue* src_val;
     const PointProbe* probe;
     RideDft dft[MAX_RIDE_DFT];
     AdeDev ade[MAX_MERGE_ADE];

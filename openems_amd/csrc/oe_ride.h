@@ -8,7 +8,8 @@
 //
 //   H launch of step s    E^(s) is still: E probes and E signals of step
 //                         s - 1 (after its sources and post-E hooks), the
-//                         ADE and Mur captures for step s
+//                         ADE and Mur captures for step s, the values of
+//                         the sources that the E launch of step s adds
 //   E launch of step s    H is still: H probes and H signals of step s
 //
 // After the batch's last step a launch of the H launch's part alone records
@@ -99,6 +100,12 @@ __device__ __forceinline__ void ride(const Ride& r, int wg, bool h) {
     uint64_t st;
     if (h) {
         const uint64_t b = *r.step_b;
+        if (wg == 0 && r.first_dft > 0 && tid < r.n_src) {
+            const PointExc& x = r.src[tid];
+            SourceValue v{0.f, 0};
+            if (b < x.n_samples) v = SourceValue{x.samples[b], 1u | (x.soft ? 2u : 0u) | (x.comp << 2)};
+            r.src_val[tid] = v;
+        }
         if (b == 0) return;  // the batch's first step has no step before it
         st = b - 1;
     } else {

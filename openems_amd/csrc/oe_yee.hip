@@ -116,41 +116,66 @@ __device__ __forceinline__ Vec<V> zerov() {
     return r;
 }
 
+// A cell of an array as (cells u, bytes o): u the same for every lane (whole
+// planes), o the lane's place in the plane.  For V = 4 o is 32 bits, which
+// lets a load take its base from scalar registers and its lane's part from
+// one register for all arrays; the host keeps planes of 2^30 cells and more
+// on V = 1.
+template <int V>
+using LaneOffset = std::conditional_t<V == 4, uint32_t, size_t>;
+template <class O>
+__device__ __forceinline__ const float* at(const float* base, size_t u, O o) {
+    return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base + u) + o);
+}
+template <class O>
+__device__ __forceinline__ float* at(float* base, size_t u, O o) {
+    return reinterpret_cast<float*>(reinterpret_cast<char*>(base + u) + o);
+}
+
+// Keeps the compiler from forming base + o of every array outside the plane
+// loop, a register pair each.
+template <class O>
+__device__ __forceinline__ void keep_offset(O& o) {
+    __asm__ volatile("" : "+v"(o));
+}
+
 // Material table (oe_coef.hip): V row indices of a lane at cell p and the
 // rows' (a, b) pairs of x, y, z from LDS.  The index is read from m8 (one
-// byte per cell, tables of at most 256 rows) when present, else from m16
-// (nontemporal, one 8-byte load for V = 4); neither stands for a table of
-// one row, whose indices are all 0 and are not read.
+// byte per cell, tables of at most 256 rows) when present, else from m16;
+// neither stands for a table of one row, whose indices are all 0 and are not
+// read.
 typedef unsigned int u2v __attribute__((ext_vector_type(2)));
-typedef unsigned int u2u __attribute__((ext_vector_type(2), aligned(2)));
-typedef unsigned int u1u __attribute__((aligned(1)));
+typedef unsigned int u2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef unsigned int u2b __attribute__((ext_vector_type(2), aligned(1)));
 
 struct MatIndex {
-    const uint16_t* m16;
-    const uint8_t* m8;
+    const char* base;
+    unsigned size;  // bytes per index, 0 for a table of one row
+    __device__ __forceinline__ MatIndex(const uint16_t* m16, const uint8_t* m8)
+        : base(m8 ? reinterpret_cast<const char*>(m8) : reinterpret_cast<const char*>(m16)),
+          size(m8 ? 1u : m16 ? 2u : 0u) {}
 };
 
 // A lane's V row indices at cell p, as loaded (unpacked by coef_from): the E
-// update loads them one plane ahead.
+// update loads them one plane ahead.  For V = 4 always 8 bytes, of which
+// byte-wide indices fill the first four (the arrays are padded): a load of
+// its own for each width would put a branch among the field loads.
 struct MatIdx {
     unsigned a = 0, b = 0;
 };
 
 template <int V, bool RAG = false>
-__device__ __forceinline__ MatIdx coef_index(const MatIndex& mi, size_t p) {
-    using U1 = std::conditional_t<RAG, u1u, unsigned>;
-    using U2 = std::conditional_t<RAG, u2u, u2v>;
+__device__ __forceinline__ MatIdx coef_index(const MatIndex& mi, size_t u, LaneOffset<V> o = 0) {
+    using U = std::conditional_t<RAG, u2b, u2u>;
     MatIdx r;
-    if (mi.m8 != nullptr) {
-        if constexpr (V == 4) r.a = __builtin_nontemporal_load(reinterpret_cast<const U1*>(mi.m8 + p));
-        else r.a = mi.m8[p];
-    } else if (mi.m16 != nullptr) {
+    if (mi.size != 0) {
+        const char* q = mi.base + mi.size * u + (mi.size == 1 ? o / 4 : o / 2);
         if constexpr (V == 4) {
-            const u2v t = __builtin_nontemporal_load(reinterpret_cast<const U2*>(mi.m16 + p));
+            const u2v t = __builtin_nontemporal_load(reinterpret_cast<const U*>(q));
             r.a = t.x;
             r.b = t.y;
         } else {
-            r.a = mi.m16[p];
+            r.a = mi.size == 1 ? *reinterpret_cast<const uint8_t*>(q) : *reinterpret_cast<const uint16_t*>(q);
         }
     }
     return r;
@@ -163,11 +188,12 @@ __device__ __forceinline__ void coef_from(const MatIndex& mi, const MatIdx& x, c
                                           Vec<V>& a1, Vec<V>& a2, Vec<V>& b0, Vec<V>& b1, Vec<V>& b2, int n = V) {
     unsigned m[V];
     if constexpr (V == 4) {
-        if (mi.m8 != nullptr) {
-            m[0] = x.a & 0xffu; m[1] = (x.a >> 8) & 0xffu; m[2] = (x.a >> 16) & 0xffu; m[3] = x.a >> 24;
-        } else {
-            m[0] = x.a & 0xffffu; m[1] = x.a >> 16; m[2] = x.b & 0xffffu; m[3] = x.b >> 16;
-        }
+        const bool byte = mi.size == 1;
+        const unsigned mask = byte ? 0xffu : 0xffffu;
+        m[0] = x.a & mask;
+        m[1] = (byte ? x.a >> 8 : x.a >> 16) & mask;
+        m[2] = (byte ? x.a >> 16 : x.b) & mask;
+        m[3] = (byte ? x.a >> 24 : x.b >> 16) & mask;
         if constexpr (RAG) {
 #pragma unroll
             for (int e = 1; e < V; ++e) m[e] = e < n ? m[e] : 0u;
@@ -189,6 +215,49 @@ template <int V, bool RAG = false>
 __device__ __forceinline__ void coef_rows(const MatIndex& mi, size_t p, const float2* tab, Vec<V>& a0,
                                           Vec<V>& a1, Vec<V>& a2, Vec<V>& b0, Vec<V>& b1, Vec<V>& b2, int n = V) {
     coef_from<V, RAG>(mi, coef_index<V, RAG>(mi, p), tab, a0, a1, a2, b0, b1, b2, n);
+}
+
+// Adds one to a step counter (without a read to wait for).
+__device__ __forceinline__ void advance(uint64_t* step) {
+    atomicAdd(reinterpret_cast<unsigned long long*>(step), 1ull);
+}
+
+// The work-group's copy of its half's material rows.  LATE: it is made
+// (fill) after the first plane's loads are issued, so there is one wait for
+// both; every wave then reaches fill, the lanes outside the box computing
+// cell (i, 0, 0) and storing nothing.  Else the rows are there before the
+// body begins.
+template <bool LATE>
+struct Rows {
+    static constexpr bool late = LATE;
+    float2* lds;
+    const float2* src;
+    int n;
+    const SourceValue* val = nullptr;  // folded sources' values of the step,
+    SourceValue* lds_val = nullptr;    // copied with the rows
+    int n_val = 0;
+    __device__ __forceinline__ void fill() const {
+        if ((int)threadIdx.x < n_val) lds_val[threadIdx.x] = val[threadIdx.x];
+        for (int q = threadIdx.x; q < n; q += 256) lds[q] = src[q];
+        __syncthreads();
+    }
+};
+
+// Reads one word of each 64-byte line of the kernel's arguments at once.
+// Loaded where they are used, the lines (13 of a Yee launch) arrive one
+// after the other, each a miss of its work-group's scalar cache: a step of
+// 72x60x32 with CPML took 13.4 us, 12.5 with this.
+template <int BYTES>
+__device__ __forceinline__ void touch_args() {
+    using Arg = const __attribute__((address_space(4))) unsigned*;
+    const Arg k = (Arg)__builtin_amdgcn_kernarg_segment_ptr();
+    constexpr int L = (BYTES + 63) / 64;
+    static_assert(L >= 1 && L <= 16, "arguments beyond 1 KB");
+    unsigned t[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) t[q] = k[16 * (q < L ? q : L - 1)];
+    __asm__ volatile("" ::"s"(t[0]), "s"(t[1]), "s"(t[2]), "s"(t[3]), "s"(t[4]), "s"(t[5]), "s"(t[6]), "s"(t[7]),
+                     "s"(t[8]), "s"(t[9]), "s"(t[10]), "s"(t[11]), "s"(t[12]), "s"(t[13]), "s"(t[14]), "s"(t[15]));
 }
 
 // kfirst / klast: the lane's left / right k neighbour along the row is not
@@ -234,7 +303,7 @@ __device__ __forceinline__ Tile decode(const YeeArgs& a, bool* inner = nullptr) 
     const int kx = lane - jy * a.t.bx;
     Tile r;
     r.k0 = (kb * a.t.bx + kx) * V;
-    r.j = B.j0 + jb * a.t.by + jy;
+    r.j = B.j0 + jb * a.t.by + jy + (jb >= B.jb_cut ? B.j_skip : 0);
     r.i0 = B.i0 + ib * a.t.ci;
     r.i1 = min(r.i0 + a.t.ci, B.i1);
     // lanes past the last whole row get an empty row range
@@ -271,7 +340,7 @@ struct Psi {
 // faces step with k.  Faces are chosen with selects (no dynamic indexing of
 // the argument arrays, which would spill them to scratch).
 template <int V, bool ZAXIS, bool RAG = false>
-__device__ __forceinline__ void psi_load(Psi<V>& s, const CpmlArgs& c, int d, int f, int l, long q,
+__device__ __forceinline__ void psi_load(Psi<V>& s, const CpmlArgs& c, int d, int f, int l, size_t u, LaneOffset<V> o,
                                          float* const* pos, float* const* neg, float* const* wpos,
                                          float* const* wneg, int tb, int ta, int tk) {
     s.f = f;
@@ -282,10 +351,11 @@ __device__ __forceinline__ void psi_load(Psi<V>& s, const CpmlArgs& c, int d, in
     float* Q = lo ? neg[2 * d] : neg[2 * d + 1];
     float* WP = lo ? wpos[2 * d] : wpos[2 * d + 1];
     float* WQ = lo ? wneg[2 * d] : wneg[2 * d + 1];
-    s.p = on ? P + q : c.dummy;
-    s.n = on ? Q + q : c.dummy;
-    s.wp = on ? WP + q : nullptr;
-    s.wn = on ? WQ + q : nullptr;
+    const LaneOffset<V> oo = on ? o : 0;
+    s.p = at(on ? P + u : c.dummy, 0, oo);
+    s.n = at(on ? Q + u : c.dummy, 0, oo);
+    s.wp = at(on ? WP + u : nullptr, 0, oo);
+    s.wn = at(on ? WQ + u : nullptr, 0, oo);
     s.pp = ldv<V, RAG>(s.p);
     s.pn = ldv<V, RAG>(s.n);
     const float* T = c.tab + (size_t)fs * CPML_TABLES * c.Lmax;
@@ -356,17 +426,33 @@ __device__ __forceinline__ void zspan(Psi<V>& s, int l, int Lz, int n) {
     s.e1 = min(n, Lz - l);
 }
 
+// Whether some lane of the wave meets a slab of the axis asked about.  The
+// all-faces kernels pass over an axis's psi where none does (an x slab's
+// inner rows, a y slab's inner planes); a launch of one slab's own cells
+// (AX with x or y alone) has it everywhere.
+template <int AX>
+__device__ __forceinline__ bool any_lane(bool on) {
+    return (AX & (AX_X | AX_Y)) != (AX_X | AX_Y) || __any(on);
+}
+
 // AX: CPML axes compiled in (AX_X | AX_Y | AX_Z); PHYS: apply the field
 // correction (else psi only, as the reference); TAB: coefficients from the
 // material table (mat, tab in LDS) instead of the arrays in Cf.
-template <int V, int AX, bool PHYS, bool TAB, bool RAG = false>
+template <int V, int AX, bool PHYS, bool TAB, bool RAG = false, class R>
 __device__ __forceinline__ void h_body(const Grid& g, const float* Fin, float* Fout, const float* __restrict__ Cf,
-                                       const MatIndex mat, const float2* tab,
+                                       const MatIndex mat, R& rows,
                                        const CpmlArgs& c, const Tile& t) {
     const int nx = g.nx, ny = g.ny, nz = g.nz;
-    if (t.k0 >= nz || t.j >= t.jend) return;
+    const bool live = t.k0 < nz && t.j < t.jend;
+    if constexpr (!R::late) {
+        if (!live) return;
+    } else if (!__any(live)) {
+        rows.fill();
+        return;
+    }
     const size_t N = g.N;
     const size_t plane = (size_t)ny * nz;
+    using O = LaneOffset<V>;
     const float* __restrict__ Ex = Fin;
     const float* __restrict__ Ey = Fin + N;
     const float* __restrict__ Ez = Fin + 2 * N;
@@ -385,72 +471,85 @@ __device__ __forceinline__ void h_body(const Grid& g, const float* Fin, float* F
     const float* __restrict__ db1 = Cf + 10 * N;
     const float* __restrict__ db2 = Cf + 11 * N;
 
-    const int j = t.j, k0 = t.k0;
+    const int j = live ? t.j : 0, k0 = live ? t.k0 : 0;
     const bool hj = j + 1 < ny;
     const bool hk_last = k0 + V < nz;
     int ly = 0, lz = 0;
     int fy = -1, fz = -1;
-    if constexpr ((AX & AX_Y) != 0) fy = face_of(c, 1, j, ly);
-    if constexpr ((AX & AX_Z) != 0) fz = zface_of<V, RAG>(c, k0, lz);
+    if constexpr ((AX & AX_Y) != 0) fy = live ? face_of(c, 1, j, ly) : -1;
+    const bool ony = (AX & AX_Y) != 0 && any_lane<AX>(fy >= 0);
+    if constexpr ((AX & AX_Z) != 0) fz = live ? zface_of<V, RAG>(c, k0, lz) : -1;
     const int nv = RAG ? min(V, nz - k0) : V;  // the lane's cells
-    size_t p = (size_t)t.i0 * plane + (size_t)j * nz + k0;
-    Vec<V> ey_c = ldv<V, RAG>(Ey + p);
-    Vec<V> ez_c = ldv<V, RAG>(Ez + p);
+    size_t u = (size_t)t.i0 * plane;
+    O o = ((O)j * nz + k0) * (O)sizeof(float), oj = o + (hj ? (O)nz * (O)sizeof(float) : 0);
+    Vec<V> ey_c = ldv<V, RAG>(at(Ey, u, o));
+    Vec<V> ez_c = ldv<V, RAG>(at(Ez, u, o));
     bool upd[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) upd[e] = true;
 
-    for (int i = t.i0; i < t.i1; ++i, p += plane) {
+    for (int i = t.i0; i < t.i1; ++i, u += plane) {
+        keep_offset(o);
+        keep_offset(oj);
         const bool hi = i + 1 < nx;
-        Vec<V> ey_n = ey_c, ez_n = ez_c;
-        if (hi) {
-            ey_n = ldv<V, RAG>(Ey + p + plane);
-            ez_n = ldv<V, RAG>(Ez + p + plane);
-        }
-        const Vec<V> ex_c = ldv<V, RAG>(Ex + p);
-        Vec<V> ez_j = ez_c, ex_j = ex_c;
-        if (hj) {
-            ez_j = ldv<V, RAG>(Ez + p + nz);
-            ex_j = ldv<V, RAG>(Ex + p + nz);
-        }
-        // the k + V neighbour: the next lane's first cell, or a load where
-        // that lane holds another row (or sits in another wave)
-        const float ey_sh = __shfl_down(ey_c.v[0], 1, 64);
-        const float ex_sh = __shfl_down(ex_c.v[0], 1, 64);
+        Vec<V> ey_n, ez_n, ex_c, ez_j, ex_j, hx, hy, hz, a0, a1, a2, b0, b1, b2;
         float ey_kl = 0.f, ex_kl = 0.f;
-        if (hk_last) {
-            ey_kl = t.klast ? Ey[p + V] : ey_sh;
-            ex_kl = t.klast ? Ex[p + V] : ex_sh;
-        }
-        Vec<V> hx = ldn<V, OE_NT_OWN, RAG>(Hx + p), hy = ldn<V, OE_NT_OWN, RAG>(Hy + p), hz = ldn<V, OE_NT_OWN, RAG>(Hz + p);
-        Vec<V> a0, a1, a2, b0, b1, b2;
+        MatIdx mi;
+        Psi<V> px, py, pz;
+        bool onx = false;
+        const size_t un = u + (hi ? plane : 0);
+        ey_n = ldv<V, RAG>(at(Ey, un, o));
+        ez_n = ldv<V, RAG>(at(Ez, un, o));
+        ex_c = ldv<V, RAG>(at(Ex, u, o));
+        ez_j = ldv<V, RAG>(at(Ez, u, oj));
+        ex_j = ldv<V, RAG>(at(Ex, u, oj));
+        hx = ldn<V, OE_NT_OWN, RAG>(at(Hx, u, o)), hy = ldn<V, OE_NT_OWN, RAG>(at(Hy, u, o)), hz = ldn<V, OE_NT_OWN, RAG>(at(Hz, u, o));
         if constexpr (TAB) {
-            coef_rows<V, RAG>(mat, p, tab, a0, a1, a2, b0, b1, b2, nv);
+            mi = coef_index<V, RAG>(mat, u, o);
         } else {
-            a0 = ldn<V, OE_NT_COEF, RAG>(da0 + p); a1 = ldn<V, OE_NT_COEF, RAG>(da1 + p); a2 = ldn<V, OE_NT_COEF, RAG>(da2 + p);
-            b0 = ldn<V, OE_NT_COEF, RAG>(db0 + p); b1 = ldn<V, OE_NT_COEF, RAG>(db1 + p); b2 = ldn<V, OE_NT_COEF, RAG>(db2 + p);
+            a0 = ldn<V, OE_NT_COEF, RAG>(at(da0, u, o)); a1 = ldn<V, OE_NT_COEF, RAG>(at(da1, u, o)); a2 = ldn<V, OE_NT_COEF, RAG>(at(da2, u, o));
+            b0 = ldn<V, OE_NT_COEF, RAG>(at(db0, u, o)); b1 = ldn<V, OE_NT_COEF, RAG>(at(db1, u, o)); b2 = ldn<V, OE_NT_COEF, RAG>(at(db2, u, o));
         }
 
-        Psi<V> px, py, pz;
         if constexpr ((AX & AX_X) != 0) {
             int lx;
             const int fx = face_of(c, 0, i, lx);
             px.e0 = 0;
             px.e1 = nv;
-            psi_load<V, false, RAG>(px, c, 0, fx, lx, ((long)lx * ny + j) * nz + k0, c.ph_pos, c.ph_neg, c.phw_pos, c.phw_neg, TAB_BH, TAB_AH, TAB_KH);
+            onx = any_lane<AX>(fx >= 0);
+            if (onx)
+                psi_load<V, false, RAG>(px, c, 0, fx, lx, lx * plane, o, c.ph_pos, c.ph_neg, c.ph_pos, c.ph_neg, TAB_BH, TAB_AH, TAB_KH);
+            px.f = live ? fx : -1;
         }
         if constexpr ((AX & AX_Y) != 0) {
             const int Ly = fy == 2 ? c.L[2] : (fy == 3 ? c.L[3] : 0);
+            py.f = fy;
             py.e0 = 0;
             py.e1 = nv;
-            psi_load<V, false, RAG>(py, c, 1, fy, ly, ((long)i * Ly + ly) * nz + k0, c.ph_pos, c.ph_neg, c.phw_pos, c.phw_neg, TAB_BH, TAB_AH, TAB_KH);
+            if (ony)
+                psi_load<V, false, RAG>(py, c, 1, fy, ly, ((size_t)i * Ly + ly) * nz + k0, 0, c.ph_pos, c.ph_neg, c.ph_pos, c.ph_neg, TAB_BH, TAB_AH, TAB_KH);
         }
         if constexpr ((AX & AX_Z) != 0) {
             const int Lz = fz == 4 ? c.L[4] : (fz == 5 ? c.L[5] : 0);
             zspan<V>(pz, lz, Lz, nv);
-            psi_load<V, true, RAG>(pz, c, 2, fz, lz, ((long)i * ny + j) * Lz + lz, c.ph_pos, c.ph_neg, c.phw_pos, c.phw_neg, TAB_BH, TAB_AH, TAB_KH);
+            psi_load<V, true, RAG>(pz, c, 2, fz, lz, ((size_t)i * ny + j) * Lz + lz, 0, c.ph_pos, c.ph_neg, c.phw_pos, c.phw_neg, TAB_BH, TAB_AH, TAB_KH);
         }
-
+        if (hk_last && t.klast) {
+            ey_kl = at(Ey, u, o)[V];
+            ex_kl = at(Ex, u, o)[V];
+        }
+        if constexpr (TAB && R::late) {
+            if (i == t.i0) rows.fill();
+        }
+        if constexpr (TAB) coef_from<V, RAG>(mat, mi, rows.lds, a0, a1, a2, b0, b1, b2, nv);
+        // the k + V neighbour: the next lane's first cell, or the load where
+        // that lane holds another row (or sits in another wave)
+        const float ey_sh = __shfl_down(ey_c.v[0], 1, 64);
+        const float ex_sh = __shfl_down(ex_c.v[0], 1, 64);
+        if (!t.klast) {
+            ey_kl = ey_sh;
+            ex_kl = ex_sh;
+        }
         float dEz_x[V], dEy_x[V], dEx_y[V], dEz_y[V], dEy_z[V], dEx_z[V];
 #pragma unroll
         for (int e = 0; e < V; ++e) {
@@ -475,18 +574,20 @@ __device__ __forceinline__ void h_body(const Grid& g, const float* Fin, float* F
         }
 
         // x: psi_pos <- dEz/dx (Hy, Q-term), psi_neg <- dEy/dx (Hz, P-term)
-        if constexpr ((AX & AX_X) != 0) psi_apply<V, PHYS, RAG>(px, dEz_x, dEy_x, hy, b1, hz, b2, upd);
+        if (onx) psi_apply<V, PHYS, RAG>(px, dEz_x, dEy_x, hy, b1, hz, b2, upd);
         // y: psi_pos <- dEx/dy (Hz), psi_neg <- dEz/dy (Hx)
-        if constexpr ((AX & AX_Y) != 0) psi_apply<V, PHYS, RAG>(py, dEx_y, dEz_y, hz, b2, hx, b0, upd);
+        if (ony) psi_apply<V, PHYS, RAG>(py, dEx_y, dEz_y, hz, b2, hx, b0, upd);
         // z: psi_pos <- dEy/dz (Hx), psi_neg <- dEx/dz (Hy)
         if constexpr ((AX & AX_Z) != 0) psi_apply<V, PHYS, RAG>(pz, dEy_z, dEx_z, hx, b0, hy, b1, upd);
         if constexpr ((AX & AX_X) != 0) psi_store<V, RAG>(px);
         if constexpr ((AX & AX_Y) != 0) psi_store<V, RAG>(py);
         if constexpr ((AX & AX_Z) != 0) psi_store<V, RAG>(pz);
 
-        stn<V, OE_NT_STORE, RAG>(Hxw + p, hx, nv);
-        stn<V, OE_NT_STORE, RAG>(Hyw + p, hy, nv);
-        stn<V, OE_NT_STORE, RAG>(Hzw + p, hz, nv);
+        if (live) {
+            stn<V, OE_NT_STORE, RAG>(at(Hxw, u, o), hx, nv);
+            stn<V, OE_NT_STORE, RAG>(at(Hyw, u, o), hy, nv);
+            stn<V, OE_NT_STORE, RAG>(at(Hzw, u, o), hz, nv);
+        }
         ey_c = ey_n;
         ez_c = ez_n;
     }
@@ -495,33 +596,33 @@ __device__ __forceinline__ void h_body(const Grid& g, const float* Fin, float* F
 // Point sources of the lane's V cells (BasicEngine::apply_excitations,
 // src/fdtd/basic_engine.rs:313-395): list order, soft adds, hard sets.
 struct Sources {
-    const PointExc* exc;
-    const uint32_t* idx;  // cell indices (kernel arguments)
-    int n;
-    uint64_t step;
-    const uint64_t* step_dev;  // non-null: read the step here (graph replay)
+    const YeeArgs& a;        // cell indices (kernel arguments)
+    const SourceValue* val;  // the step's values
 };
 
 template <int V>
-__device__ __forceinline__ void apply_sources(const Sources& src, size_t p, Vec<V>& ex, Vec<V>& ey, Vec<V>& ez) {
-    for (int q = 0; q < src.n; ++q) {
-        const size_t idx = src.idx[q];
-        if (idx < p || idx >= p + V) continue;
-        const PointExc* x = src.exc + q;
-        const uint64_t step = src.step_dev ? *src.step_dev : src.step;
-        if (step >= x->n_samples) continue;
-        const float v = x->samples[step];
-        const bool soft = x->soft != 0;
-        const uint32_t comp = x->comp;
+__device__ __forceinline__ void apply_sources(const Sources& src, size_t plane, size_t u, LaneOffset<V> o, Vec<V>& ex,
+                                              Vec<V>& ey, Vec<V>& ez) {
+    const LaneOffset<V> cell = o / sizeof(float);
+#pragma unroll
+    for (int q = 0; q < MAX_FOLD_SOURCES; ++q) {
+        const size_t d = (size_t)src.a.src_idx[q] - u;
+        if (q >= src.a.n_src || d >= plane) continue;  // in another plane, the same for every lane
+        const LaneOffset<V> in = (LaneOffset<V>)d;
+        if (in - cell >= (LaneOffset<V>)V) continue;
+        const SourceValue x = src.val[q];
+        if (x.code == 0) continue;
+        const bool soft = (x.code & 2u) != 0;
+        const uint32_t comp = x.code >> 2;
 #pragma unroll
         for (int m = 0; m < V; ++m) {
-            if (idx != p + m) continue;
-            const float fx = soft ? ex.v[m] + v : v;
-            const float fy = soft ? ey.v[m] + v : v;
-            const float fz = soft ? ez.v[m] + v : v;
-            ex.v[m] = comp == 0 ? fx : ex.v[m];
-            ey.v[m] = comp == 1 ? fy : ey.v[m];
-            ez.v[m] = comp == 2 ? fz : ez.v[m];
+            const bool hit = in == cell + m;
+            const float fx = soft ? ex.v[m] + x.v : x.v;
+            const float fy = soft ? ey.v[m] + x.v : x.v;
+            const float fz = soft ? ez.v[m] + x.v : x.v;
+            ex.v[m] = hit && comp == 0 ? fx : ex.v[m];
+            ey.v[m] = hit && comp == 1 ? fy : ey.v[m];
+            ez.v[m] = hit && comp == 2 ? fz : ez.v[m];
         }
     }
 }
@@ -533,16 +634,23 @@ __device__ __forceinline__ void apply_sources(const Sources& src, size_t p, Vec<
 // update skips (i = 0 or j = 0) get the same writes from their old values.
 // Valid when no other hook acts on those cells between the E update and the
 // Mur post step (the host checks it).
-template <int V, int AX, bool PHYS, bool TAB, bool MUR = false, bool RAG = false>
+template <int V, int AX, bool PHYS, bool TAB, bool MUR = false, bool RAG = false, class R>
 __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* Fout, const float* __restrict__ Cf,
-                                       const MatIndex mat, const float2* tab,
+                                       const MatIndex mat, R& rows,
                                        const CpmlArgs& c, const Tile& t, const Sources* src = nullptr,
                                        const MurZ& mz = MurZ{}) {
     static_assert(!MUR || (V == 4 && !RAG), "the folded Mur needs whole float4 lanes");
     const int ny = g.ny, nz = g.nz;
-    if (t.k0 >= nz || t.j >= t.jend) return;
+    const bool live = t.k0 < nz && t.j < t.jend;
+    if constexpr (!R::late) {
+        if (!live) return;
+    } else if (!__any(live)) {
+        rows.fill();
+        return;
+    }
     const size_t N = g.N;
     const size_t plane = (size_t)ny * nz;
+    using O = LaneOffset<V>;
     // old E from Fin, new E to Fout; the new H (already in Fout) is read
     const bool copy_all = Fin != Fout;
     const float* Ex = Fin;
@@ -561,70 +669,85 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
     const float* __restrict__ cb1 = Cf + 4 * N;
     const float* __restrict__ cb2 = Cf + 5 * N;
 
-    const int j = t.j, k0 = t.k0;
+    const int j = live ? t.j : 0, k0 = live ? t.k0 : 0;
     const bool gj = j > 0;
     const bool gk_first = k0 > 0;
     int ly = 0, lz = 0;
     int fy = -1, fz = -1;
-    if constexpr ((AX & AX_Y) != 0) fy = face_of(c, 1, j, ly);
-    if constexpr ((AX & AX_Z) != 0) fz = zface_of<V, RAG>(c, k0, lz);
+    if constexpr ((AX & AX_Y) != 0) fy = live ? face_of(c, 1, j, ly) : -1;
+    const bool ony = (AX & AX_Y) != 0 && any_lane<AX>(fy >= 0);
+    if constexpr ((AX & AX_Z) != 0) fz = live ? zface_of<V, RAG>(c, k0, lz) : -1;
     const int nv = RAG ? min(V, nz - k0) : V;  // the lane's cells
-    size_t p = (size_t)t.i0 * plane + (size_t)j * nz + k0;
-    Vec<V> hy_p = zerov<V>(), hz_p = zerov<V>();
-    if (t.i0 > 0) {
-        hy_p = ldv<V, RAG>(Hy + p - plane);
-        hz_p = ldv<V, RAG>(Hz + p - plane);
-    }
+    size_t u = (size_t)t.i0 * plane;
+    O o = ((O)j * nz + k0) * (O)sizeof(float), oj = o - (gj ? (O)nz * (O)sizeof(float) : 0);
+    const size_t up = u - (t.i0 > 0 ? plane : 0);
+    Vec<V> hy_p = ldv<V, RAG>(at(Hy, up, o)), hz_p = ldv<V, RAG>(at(Hz, up, o));
     // lanes of the folded Mur faces held by this thread
-    const bool mur_lo = MUR && mz.on[0] && k0 == 0;
-    const bool mur_hi = MUR && mz.on[1] && k0 + V == nz;
+    const bool mur_lo = MUR && live && mz.on[0] && k0 == 0;
+    const bool mur_hi = MUR && live && mz.on[1] && k0 + V == nz;
     // material-table row indices one plane ahead: the LDS row reads of a
     // plane need not wait for that plane's field loads
     MatIdx mi_c;
     if constexpr (TAB) {
-        if (gj && t.i0 > 0) mi_c = coef_index<V, RAG>(mat, p);
+        mi_c = coef_index<V, RAG>(mat, u, o);
     }
 
-    for (int i = t.i0; i < t.i1; ++i, p += plane) {
+    for (int i = t.i0; i < t.i1; ++i, u += plane) {
+        keep_offset(o);
+        keep_offset(oj);
         const bool gi = i > 0;
-        const bool row = gi && gj;
+        const bool row = live && gi && gj;
         MatIdx mi_n;
-        if constexpr (TAB) {
-            if (gj && i + 1 < t.i1) mi_n = coef_index<V, RAG>(mat, p + plane);
-        }
-        const Vec<V> hx_c = ldv<V, RAG>(Hx + p), hy_c = ldv<V, RAG>(Hy + p), hz_c = ldv<V, RAG>(Hz + p);
-        Vec<V> hz_j = hz_c, hx_j = hx_c;
-        if (gj) {
-            hz_j = ldv<V, RAG>(Hz + p - nz);
-            hx_j = ldv<V, RAG>(Hx + p - nz);
-        }
-        // the k - 1 neighbour: the previous lane's last cell, or a load where
-        // that lane holds another row (or sits in another wave)
-        const float hy_sh = __shfl_up(hy_c.v[V - 1], 1, 64);
-        const float hx_sh = __shfl_up(hx_c.v[V - 1], 1, 64);
+        Vec<V> hx_c, hy_c, hz_c, hz_j, hx_j, ex, ey, ez, c0, c1, c2, s0, s1, s2;
         float hy_kf = 0.f, hx_kf = 0.f;
-        if (gk_first) {
-            hy_kf = t.kfirst ? Hy[p - 1] : hy_sh;
-            hx_kf = t.kfirst ? Hx[p - 1] : hx_sh;
+        Psi<V> px, py, pz;
+        bool onx = false;
+        if constexpr (TAB) mi_n = coef_index<V, RAG>(mat, u + (i + 1 < t.i1 ? plane : 0), o);
+        hx_c = ldv<V, RAG>(at(Hx, u, o)), hy_c = ldv<V, RAG>(at(Hy, u, o)), hz_c = ldv<V, RAG>(at(Hz, u, o));
+        hz_j = ldv<V, RAG>(at(Hz, u, oj));
+        hx_j = ldv<V, RAG>(at(Hx, u, oj));
+        ex = ldn<V, OE_NT_OWN, RAG>(at(Ex, u, o)); ey = ldn<V, OE_NT_OWN, RAG>(at(Ey, u, o)); ez = ldn<V, OE_NT_OWN, RAG>(at(Ez, u, o));
+        if constexpr (!TAB) {
+            s0 = ldn<V, OE_NT_COEF, RAG>(at(ca0, u, o)); s1 = ldn<V, OE_NT_COEF, RAG>(at(ca1, u, o)); s2 = ldn<V, OE_NT_COEF, RAG>(at(ca2, u, o));
+            c0 = ldn<V, OE_NT_COEF, RAG>(at(cb0, u, o)); c1 = ldn<V, OE_NT_COEF, RAG>(at(cb1, u, o)); c2 = ldn<V, OE_NT_COEF, RAG>(at(cb2, u, o));
         }
-        Vec<V> ex, ey, ez, c0, c1, c2, s0, s1, s2;
-        if (row) {
-            ex = ldn<V, OE_NT_OWN, RAG>(Ex + p); ey = ldn<V, OE_NT_OWN, RAG>(Ey + p); ez = ldn<V, OE_NT_OWN, RAG>(Ez + p);
-            if constexpr (TAB) {
-                coef_from<V, RAG>(mat, mi_c, tab, s0, s1, s2, c0, c1, c2, nv);
-            } else {
-                s0 = ldn<V, OE_NT_COEF, RAG>(ca0 + p); s1 = ldn<V, OE_NT_COEF, RAG>(ca1 + p); s2 = ldn<V, OE_NT_COEF, RAG>(ca2 + p);
-                c0 = ldn<V, OE_NT_COEF, RAG>(cb0 + p); c1 = ldn<V, OE_NT_COEF, RAG>(cb1 + p); c2 = ldn<V, OE_NT_COEF, RAG>(cb2 + p);
-            }
+        if constexpr ((AX & AX_X) != 0) {
+            int lx;
+            const int fx = face_of(c, 0, i, lx);
+            px.e0 = 0;
+            px.e1 = nv;
+            onx = any_lane<AX>(fx >= 0);
+            if (onx)
+                psi_load<V, false, RAG>(px, c, 0, fx, lx, lx * plane, o, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg, TAB_BE, TAB_AE, TAB_KE);
+            px.f = live ? fx : -1;
+        }
+        if constexpr ((AX & AX_Y) != 0) {
+            const int Ly = fy == 2 ? c.L[2] : (fy == 3 ? c.L[3] : 0);
+            py.f = fy;
+            py.e0 = 0;
+            py.e1 = nv;
+            if (ony)
+                psi_load<V, false, RAG>(py, c, 1, fy, ly, ((size_t)i * Ly + ly) * nz + k0, 0, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg, TAB_BE, TAB_AE, TAB_KE);
+        }
+        if constexpr ((AX & AX_Z) != 0) {
+            const int Lz = fz == 4 ? c.L[4] : (fz == 5 ? c.L[5] : 0);
+            zspan<V>(pz, lz, Lz, nv);
+            psi_load<V, true, RAG>(pz, c, 2, fz, lz, ((size_t)i * ny + j) * Lz + lz, 0, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg, TAB_BE, TAB_AE, TAB_KE);
+        }
+        if (gk_first && t.kfirst) {
+            hy_kf = at(Hy, u, o)[-1];
+            hx_kf = at(Hx, u, o)[-1];
+        }
+        if constexpr (TAB && R::late) {
+            if (i == t.i0) rows.fill();
+        }
+        if constexpr (TAB) {
+            coef_from<V, RAG>(mat, mi_c, rows.lds, s0, s1, s2, c0, c1, c2, nv);
         }
         // Mur pre step on the old values: v = E(shift) - c E(line)
         float mvx[2] = {0.f, 0.f}, mvy[2] = {0.f, 0.f};
         if constexpr (MUR) {
             if (mur_lo || mur_hi) {
-                if (!row) {
-                    ex = ldn<V, OE_NT_OWN, RAG>(Ex + p);
-                    ey = ldn<V, OE_NT_OWN, RAG>(Ey + p);
-                }
                 if (mur_lo) {
                     mvx[0] = ex.v[1] - mz.coeff[0] * ex.v[0];
                     mvy[0] = ey.v[1] - mz.coeff[0] * ey.v[0];
@@ -636,26 +759,14 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
             }
         }
 
-        Psi<V> px, py, pz;
-        if constexpr ((AX & AX_X) != 0) {
-            int lx;
-            const int fx = face_of(c, 0, i, lx);
-            px.e0 = 0;
-            px.e1 = nv;
-            psi_load<V, false, RAG>(px, c, 0, fx, lx, ((long)lx * ny + j) * nz + k0, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg, TAB_BE, TAB_AE, TAB_KE);
+        // the k - 1 neighbour: the previous lane's last cell, or the load
+        // where that lane holds another row (or sits in another wave)
+        const float hy_sh = __shfl_up(hy_c.v[V - 1], 1, 64);
+        const float hx_sh = __shfl_up(hx_c.v[V - 1], 1, 64);
+        if (!t.kfirst) {
+            hy_kf = hy_sh;
+            hx_kf = hx_sh;
         }
-        if constexpr ((AX & AX_Y) != 0) {
-            const int Ly = fy == 2 ? c.L[2] : (fy == 3 ? c.L[3] : 0);
-            py.e0 = 0;
-            py.e1 = nv;
-            psi_load<V, false, RAG>(py, c, 1, fy, ly, ((long)i * Ly + ly) * nz + k0, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg, TAB_BE, TAB_AE, TAB_KE);
-        }
-        if constexpr ((AX & AX_Z) != 0) {
-            const int Lz = fz == 4 ? c.L[4] : (fz == 5 ? c.L[5] : 0);
-            zspan<V>(pz, lz, Lz, nv);
-            psi_load<V, true, RAG>(pz, c, 2, fz, lz, ((long)i * ny + j) * Lz + lz, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg, TAB_BE, TAB_AE, TAB_KE);
-        }
-
         float dHz_y[V], dHy_z[V], dHx_z[V], dHz_x[V], dHy_x[V], dHx_y[V];
         bool upd[V];
 #pragma unroll
@@ -686,9 +797,9 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
         }
 
         // x: psi_pos <- dHz/dx (Ey, Q-term), psi_neg <- dHy/dx (Ez, P-term)
-        if constexpr ((AX & AX_X) != 0) psi_apply<V, PHYS, RAG>(px, dHz_x, dHy_x, ey, c1, ez, c2, upd);
+        if (onx) psi_apply<V, PHYS, RAG>(px, dHz_x, dHy_x, ey, c1, ez, c2, upd);
         // y: psi_pos <- dHx/dy (Ez), psi_neg <- dHz/dy (Ex)
-        if constexpr ((AX & AX_Y) != 0) psi_apply<V, PHYS, RAG>(py, dHx_y, dHz_y, ez, c2, ex, c0, upd);
+        if (ony) psi_apply<V, PHYS, RAG>(py, dHx_y, dHz_y, ez, c2, ex, c0, upd);
         // z: psi_pos <- dHy/dz (Ex), psi_neg <- dHx/dz (Ey)
         if constexpr ((AX & AX_Z) != 0) psi_apply<V, PHYS, RAG>(pz, dHy_z, dHx_z, ex, c0, ey, c1, upd);
         if constexpr ((AX & AX_X) != 0) psi_store<V, RAG>(px);
@@ -706,20 +817,20 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
                 ey.v[V - 1] = mvy[1] + mz.coeff[1] * ey.v[V - 2];
             }
             if (!row && (mur_lo || mur_hi)) {
-                stn<V, OE_NT_STORE, RAG>(Exw + p, ex, nv);
-                stn<V, OE_NT_STORE, RAG>(Eyw + p, ey, nv);
+                stn<V, OE_NT_STORE, RAG>(at(Exw, u, o), ex, nv);
+                stn<V, OE_NT_STORE, RAG>(at(Eyw, u, o), ey, nv);
             }
         }
 
         if (row) {
-            if (src) apply_sources<V>(*src, p, ex, ey, ez);
-            stn<V, OE_NT_STORE, RAG>(Exw + p, ex, nv);
-            stn<V, OE_NT_STORE, RAG>(Eyw + p, ey, nv);
-            stn<V, OE_NT_STORE, RAG>(Ezw + p, ez, nv);
-        } else if (copy_all) {  // index-0 planes and rows keep their value
-            stn<V, OE_NT_STORE, RAG>(Exw + p, ldn<V, OE_NT_OWN, RAG>(Ex + p), nv);
-            stn<V, OE_NT_STORE, RAG>(Eyw + p, ldn<V, OE_NT_OWN, RAG>(Ey + p), nv);
-            stn<V, OE_NT_STORE, RAG>(Ezw + p, ldn<V, OE_NT_OWN, RAG>(Ez + p), nv);
+            if (src) apply_sources<V>(*src, plane, u, o, ex, ey, ez);
+            stn<V, OE_NT_STORE, RAG>(at(Exw, u, o), ex, nv);
+            stn<V, OE_NT_STORE, RAG>(at(Eyw, u, o), ey, nv);
+            stn<V, OE_NT_STORE, RAG>(at(Ezw, u, o), ez, nv);
+        } else if (copy_all && live) {  // index-0 planes and rows keep their value
+            stn<V, OE_NT_STORE, RAG>(at(Exw, u, o), ex, nv);
+            stn<V, OE_NT_STORE, RAG>(at(Eyw, u, o), ey, nv);
+            stn<V, OE_NT_STORE, RAG>(at(Ezw, u, o), ez, nv);
         }
         hy_p = hy_c;
         hz_p = hz_c;
@@ -733,96 +844,94 @@ template <int AX>
 constexpr bool RIDES = (AX & (AX_X | AX_Y)) == 0;
 
 // One grid: the tile comes from the launch's box list.  With TAB the
-// work-group first copies its half's material rows into LDS (dynamic LDS of
-// 24 bytes per row).
+// work-group copies its half's material rows into LDS (dynamic LDS of 24
+// bytes per row).
 template <int V, int AX, bool PHYS, bool TAB, bool RAG = false>
-__global__ __launch_bounds__(256) void k_update_h(YeeArgs a, CpmlArgs c) {
+__global__ __launch_bounds__(256, V == 4 && AX == 7 ? 3 : 1) void k_update_h(YeeArgs a, CpmlArgs c) {
     extern __shared__ float2 lds_rows[];
     // the step's first launch advances the step counter (no H lane reads it)
-    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) *a.step_inc += 1;
+    touch_args<sizeof(YeeArgs) + sizeof(CpmlArgs)>();
+    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(a.step_inc);
     if constexpr (RIDES<AX>) {
         if ((int)blockIdx.x < a.n_ride) {
             ride(*a.ride, blockIdx.x, true);
             return;
         }
     }
-    if constexpr (TAB) {
-        const float2* src = reinterpret_cast<const float2*>(a.tab_h);
-        for (int q = threadIdx.x; q < 3 * a.n_mat_h; q += blockDim.x) lds_rows[q] = src[q];
-        __syncthreads();
-    }
-    h_body<V, AX, PHYS, TAB, RAG>(a.g, a.Fin, a.Fout, a.Cf, MatIndex{a.n_mat_h == 1 ? nullptr : a.mat_h, a.mat8_h}, lds_rows, c,
+    Rows<TAB> rows{lds_rows, reinterpret_cast<const float2*>(a.tab_h), 3 * a.n_mat_h};
+    h_body<V, AX, PHYS, TAB, RAG>(a.g, a.Fin, a.Fout, a.Cf, MatIndex{a.n_mat_h == 1 ? nullptr : a.mat_h, a.mat8_h}, rows, c,
                              decode<V>(a));
 }
 
 // The z-faces kernels are held to the 128 registers of 4 waves a SIMD.
 template <int V, int AX, bool PHYS, bool TAB, bool MUR = false, bool RAG = false>
-__global__ __launch_bounds__(256, V == 4 && AX == AX_Z ? 4 : 1) void k_update_e(YeeArgs a, CpmlArgs c) {
+__global__ __launch_bounds__(256, V == 4 && AX == AX_Z ? 4 : V == 4 && AX == 7 ? 3 : 1) void k_update_e(YeeArgs a, CpmlArgs c) {
     extern __shared__ float2 lds_rows[];
-    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) *a.step_inc += 1;
+    touch_args<sizeof(YeeArgs) + sizeof(CpmlArgs)>();
+    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(a.step_inc);
     if constexpr (RIDES<AX>) {
         if ((int)blockIdx.x < a.n_ride) {
             ride(*a.ride, blockIdx.x, false);
             return;
         }
     }
-    if constexpr (TAB) {
-        const float2* src = reinterpret_cast<const float2*>(a.tab_e);
-        for (int q = threadIdx.x; q < 3 * a.n_mat_e; q += blockDim.x) lds_rows[q] = src[q];
-        __syncthreads();
-    }
+    __shared__ SourceValue lds_val[MAX_FOLD_SOURCES];
+    Rows<TAB> rows{lds_rows, reinterpret_cast<const float2*>(a.tab_e), 3 * a.n_mat_e, a.src_val, lds_val, a.n_src};
     const MatIndex mat_e{a.n_mat_e == 1 ? nullptr : a.mat_e, a.mat8_e};
-    if (MUR || a.n_exc) {
-        const Sources src{a.exc, a.exc_idx, a.n_exc, a.exc_step, a.exc_step_dev};
-        e_body<V, AX, PHYS, TAB, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat_e, lds_rows, c, decode<V>(a), &src, a.mur_z);
+    if (MUR || a.n_src) {
+        const Sources src{a, TAB ? lds_val : a.src_val};
+        e_body<V, AX, PHYS, TAB, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat_e, rows, c, decode<V>(a), &src, a.mur_z);
     } else {
-        e_body<V, AX, PHYS, TAB, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat_e, lds_rows, c, decode<V>(a));
+        e_body<V, AX, PHYS, TAB, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat_e, rows, c, decode<V>(a));
     }
 }
 
-// One launch for the x/y slabs (every face) and the interior (AXI: z faces or
-// none) of a CPML grid.  The slab code's registers leave 2 waves a SIMD for
-// both, so this is for grids whose launches are bound by their start and
-// their chain of loads, not by how many are in flight (plan_launches).
+// One launch over a CPML grid: work-groups that meet an x or y slab run the
+// body of all faces, the others the interior's (AXI: z faces or none).  The
+// slab body's registers are the launch's: held to 168 they leave 3 waves a
+// SIMD.  What bounds small grids is the chain from a work-group's start to
+// its stores, so the arguments, the table rows and all of a plane's loads are
+// each waited for once; large ones run at memory speed (256^3, 8 layers, 64
+// boxes' table: 109 us a launch, 121 when the slabs were a launch of their
+// own and a plane's loads came in three waits).
 template <int AXI, bool PHYS, bool RAG>
-__global__ __launch_bounds__(256) void k_update_h_mix(YeeArgs a, CpmlArgs c) {
+__global__ __launch_bounds__(256, 3) void k_update_h_mix(YeeArgs a, CpmlArgs c) {
     constexpr int V = 4;
     extern __shared__ float2 lds_rows[];
-    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) *a.step_inc += 1;
+    touch_args<sizeof(YeeArgs) + sizeof(CpmlArgs)>();
+    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(a.step_inc);
     if ((int)blockIdx.x < a.n_ride) {
         ride(*a.ride, blockIdx.x, true);
         return;
     }
-    const float2* src = reinterpret_cast<const float2*>(a.tab_h);
-    for (int q = threadIdx.x; q < 3 * a.n_mat_h; q += blockDim.x) lds_rows[q] = src[q];
-    __syncthreads();
+    Rows<true> rows{lds_rows, reinterpret_cast<const float2*>(a.tab_h), 3 * a.n_mat_h};
     const MatIndex mat{a.n_mat_h == 1 ? nullptr : a.mat_h, a.mat8_h};
     bool inner;
     const Tile t = decode<V, true>(a, &inner);
-    if (inner) h_body<V, AXI, PHYS && AXI != 0, true, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, lds_rows, c, t);
-    else h_body<V, AX_X | AX_Y | AX_Z, PHYS, true, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, lds_rows, c, t);
+    if (inner) h_body<V, AXI, PHYS && AXI != 0, true, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t);
+    else h_body<V, AX_X | AX_Y | AX_Z, PHYS, true, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t);
 }
 
 template <int AXI, bool PHYS, bool MUR, bool RAG>
-__global__ __launch_bounds__(256) void k_update_e_mix(YeeArgs a, CpmlArgs c) {
+__global__ __launch_bounds__(256, 3) void k_update_e_mix(YeeArgs a, CpmlArgs c) {
     constexpr int V = 4;
     extern __shared__ float2 lds_rows[];
-    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) *a.step_inc += 1;
+    touch_args<sizeof(YeeArgs) + sizeof(CpmlArgs)>();
+    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(a.step_inc);
     if ((int)blockIdx.x < a.n_ride) {
         ride(*a.ride, blockIdx.x, false);
         return;
     }
-    const float2* src = reinterpret_cast<const float2*>(a.tab_e);
-    for (int q = threadIdx.x; q < 3 * a.n_mat_e; q += blockDim.x) lds_rows[q] = src[q];
-    __syncthreads();
+    __shared__ SourceValue lds_val[MAX_FOLD_SOURCES];
+    Rows<true> rows{lds_rows, reinterpret_cast<const float2*>(a.tab_e), 3 * a.n_mat_e, a.src_val, lds_val, a.n_src};
     const MatIndex mat{a.n_mat_e == 1 ? nullptr : a.mat_e, a.mat8_e};
-    const Sources ex{a.exc, a.exc_idx, a.n_exc, a.exc_step, a.exc_step_dev};
+    const Sources ex{a, lds_val};
     bool inner;
     const Tile t = decode<V, true>(a, &inner);
     if (inner)
-        e_body<V, AXI, PHYS && AXI != 0, true, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, lds_rows, c, t, &ex, a.mur_z);
+        e_body<V, AXI, PHYS && AXI != 0, true, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t, &ex, a.mur_z);
     else
-        e_body<V, AX_X | AX_Y | AX_Z, PHYS, true, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, lds_rows, c, t, &ex, a.mur_z);
+        e_body<V, AX_X | AX_Y | AX_Z, PHYS, true, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t, &ex, a.mur_z);
 }
 
 // Many grids in one launch (a parameter sweep): work-group -> box of some
@@ -865,17 +974,16 @@ __device__ __forceinline__ bool decode_sweep(const SweepArgs& a, Tile& r, int& s
 template <int V, int AX, bool PHYS, bool TAB>
 __global__ __launch_bounds__(256) void k_update_h_sweep(SweepArgs a) {
     extern __shared__ float2 lds_rows[];
-    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) *a.step_inc += 1;
+    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(a.step_inc);
     Tile t;
     int sid;
     decode_sweep<V>(a, t, sid);
     const SweepStruct& S = a.st[sid];
+    Rows<false> rows{lds_rows, reinterpret_cast<const float2*>(S.tab_h), 3 * S.n_mat_h};
     if constexpr (TAB) {
-        const float2* src = reinterpret_cast<const float2*>(S.tab_h);
-        for (int q = threadIdx.x; q < 3 * S.n_mat_h; q += blockDim.x) lds_rows[q] = src[q];
-        __syncthreads();
+            rows.fill();
     }
-    h_body<V, AX, PHYS, TAB>(S.g, S.F, S.F, S.Cf, MatIndex{S.n_mat_h == 1 ? nullptr : S.mat_h, S.mat8_h}, lds_rows, S.c, t);
+    h_body<V, AX, PHYS, TAB>(S.g, S.F, S.F, S.Cf, MatIndex{S.n_mat_h == 1 ? nullptr : S.mat_h, S.mat8_h}, rows, S.c, t);
 }
 
 template <int V, int AX, bool PHYS, bool TAB>
@@ -885,12 +993,11 @@ __global__ __launch_bounds__(256) void k_update_e_sweep(SweepArgs a) {
     int sid;
     decode_sweep<V>(a, t, sid);
     const SweepStruct& S = a.st[sid];
+    Rows<false> rows{lds_rows, reinterpret_cast<const float2*>(S.tab_e), 3 * S.n_mat_e};
     if constexpr (TAB) {
-        const float2* src = reinterpret_cast<const float2*>(S.tab_e);
-        for (int q = threadIdx.x; q < 3 * S.n_mat_e; q += blockDim.x) lds_rows[q] = src[q];
-        __syncthreads();
+            rows.fill();
     }
-    e_body<V, AX, PHYS, TAB>(S.g, S.F, S.F, S.Cf, MatIndex{S.n_mat_e == 1 ? nullptr : S.mat_e, S.mat8_e}, lds_rows, S.c, t);
+    e_body<V, AX, PHYS, TAB>(S.g, S.F, S.F, S.Cf, MatIndex{S.n_mat_e == 1 ? nullptr : S.mat_e, S.mat8_e}, rows, S.c, t);
 }
 
 template <int V, int AX, bool PHYS, bool RAG>
@@ -1066,7 +1173,7 @@ __global__ __launch_bounds__((FUSED_ROWS + 1) * 64) void k_fused(FusedArgs a, Cp
             b1 = ldn<V, OE_NT_COEF>(a.Cf + 10 * N + p); b2 = ldn<V, OE_NT_COEF>(a.Cf + 11 * N + p);
         }
         if constexpr (ZC)
-            psi_load<V, true>(pz, c, 2, fz, lz, ((size_t)i * ny + j) * Lz + lz, c.ph_pos, c.ph_neg, c.phw_pos,
+            psi_load<V, true>(pz, c, 2, fz, lz, ((size_t)i * ny + j) * Lz + lz, 0, c.ph_pos, c.ph_neg, c.phw_pos,
                               c.phw_neg, TAB_BH, TAB_AH, TAB_KH);
         float dEy_z[V], dEx_z[V];
 #pragma unroll
@@ -1133,7 +1240,7 @@ __global__ __launch_bounds__((FUSED_ROWS + 1) * 64) void k_fused(FusedArgs a, Cp
                 c1 = ldn<V, OE_NT_COEF>(a.Cf + 4 * N + p); c2 = ldn<V, OE_NT_COEF>(a.Cf + 5 * N + p);
             }
             if constexpr (ZC)
-                psi_load<V, true>(pe, c, 2, fz, lz, ((size_t)i * ny + j) * Lz + lz, c.pe_pos, c.pe_neg, c.pe_pos,
+                psi_load<V, true>(pe, c, 2, fz, lz, ((size_t)i * ny + j) * Lz + lz, 0, c.pe_pos, c.pe_neg, c.pe_pos,
                                   c.pe_neg, TAB_BE, TAB_AE, TAB_KE);
         };
         if (comp) {
@@ -1313,7 +1420,7 @@ __global__ __launch_bounds__(FUSED_ROWS * 64) void k_fused_rows(FusedArgs a, Cpm
         Vec<V> a0, a1, a2, b0, b1, b2;
         h_coef(p, a0, a1, a2, b0, b1, b2);
         if constexpr (ZC)
-            psi_load<V, true>(pz, c, 2, fz, lz, ((size_t)i * ny + j) * Lz + lz, c.ph_pos, c.ph_neg, c.phw_pos,
+            psi_load<V, true>(pz, c, 2, fz, lz, ((size_t)i * ny + j) * Lz + lz, 0, c.ph_pos, c.ph_neg, c.phw_pos,
                               c.phw_neg, TAB_BH, TAB_AH, TAB_KH);
         float dEy_z[V], dEx_z[V];
 #pragma unroll
@@ -1354,7 +1461,7 @@ __global__ __launch_bounds__(FUSED_ROWS * 64) void k_fused_rows(FusedArgs a, Cpm
         h_coef(pm, a0, a1, a2, b0, b1, b2);
         Psi<V> pz;
         if constexpr (ZC)
-            psi_load<V, true>(pz, c, 2, fz, lz, ((size_t)i * ny + (j - 1)) * Lz + lz, c.ph_pos, c.ph_neg,
+            psi_load<V, true>(pz, c, 2, fz, lz, ((size_t)i * ny + (j - 1)) * Lz + lz, 0, c.ph_pos, c.ph_neg,
                               c.phw_pos, c.phw_neg, TAB_BH, TAB_AH, TAB_KH);
         float dEy_z[V];
 #pragma unroll
@@ -1443,7 +1550,7 @@ __global__ __launch_bounds__(FUSED_ROWS * 64) void k_fused_rows(FusedArgs a, Cpm
         }
         Psi<V> pe;
         if constexpr (ZC)
-            psi_load<V, true>(pe, c, 2, fz, lz, ((size_t)i * ny + j) * Lz + lz, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg,
+            psi_load<V, true>(pe, c, 2, fz, lz, ((size_t)i * ny + j) * Lz + lz, 0, c.pe_pos, c.pe_neg, c.pe_pos, c.pe_neg,
                               TAB_BE, TAB_AE, TAB_KE);
         Vec<V> ex = ex_c, ey = ey_c, ez = ez_c;
         float dHy_z[V], dHx_z[V];

@@ -78,3 +78,36 @@ def test_one_launch_per_half_step_equals_two(monkeypatch, shape, cpml, mur, grap
     for a, b in zip(got, ref):
         assert a.shape == b.shape and np.array_equal(a, b)
     assert np.abs(got[0]).max() > 0
+
+
+@pytest.mark.parametrize("shape,cpml", [((14, 70, 64), (2, 3, 3, 20, 4, 4)), ((11, 33, 64), (0, 3, 17, 0, 0, 5)),
+                                        ((9, 23, 256), (3, 0, 4, 5, 8, 0)), ((10, 31, 262), (2, 2, 0, 9, 7, 6)),
+                                        ((8, 16, 130), (2, 2, 8, 8, 5, 5))],
+                         ids=["blocks", "one_face", "rows_of_64", "ragged", "all_slab"])
+@pytest.mark.parametrize("rows", [1, 86, 300])
+def test_tiles_that_meet_a_slab(monkeypatch, shape, cpml, rows):
+    """j-blocks that lie inside, across and outside the y slabs, with tables
+    of one row, of more float2 than a work-group has lanes and of 16-bit
+    indices; hard and soft sources, four of them in one lane, that end before
+    the batch does: one launch per half-step with its riders against a launch
+    for each part, bit for bit."""
+    def run(cells, ride):
+        monkeypatch.setenv("OE_MIX_CELLS", cells)
+        monkeypatch.setenv("OE_RIDE", ride)
+        nx, ny, nz = shape
+        op = Operator.uniform(nx, ny, nz, 0.5e-3)
+        for q in range(rows - 1):
+            at = (q * 7) % nx, (q * 5) % ny, (q * 11) % nz
+            op.set_material(1.5 + 0.01 * q, 1.0, 0.001 * (q % 3), 0.0,
+                            (at[0], at[0] + 1, at[1], at[1] + 1, at[2], at[2] + 1))
+        eng = HipEngine(op)
+        cp = eng.cpml(CpmlBoundaries(layers=cpml, mode=MODE_PHYSICAL))
+        pulse = (0.3 * np.arange(1, 31)).astype(np.float32)
+        exc = [ScheduledExcitation((nx // 2, ny // 2, 8 + q), q % 3, pulse[q:25], q % 2 == 0) for q in range(4)]
+        exc += [ScheduledExcitation((nx // 2, 1 + q, nz // 2), 2, pulse[:9 + q], True) for q in range(4)]
+        eng.run_batch(EngineBatch(num_steps=30, excitations=exc, extensions=[cp]))
+        return eng.read_fields()
+
+    got, ref = run("1000000000", "1"), run("0", "0")
+    for a, b in zip(got, ref):
+        assert np.array_equal(a, b) and np.abs(b).max() > 0
