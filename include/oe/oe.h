@@ -505,7 +505,7 @@ typedef struct {
     double energy_decay_db;
     uint32_t check_interval;  /* 0: 100 */
     int use_graph;            /* replay captured graphs (else plain launches) */
-    int autotune;             /* time candidate tile depths on the zero state first */
+    int autotune;             /* time candidate tile depths over the run's first steps */
 } oe_sweep_config;
 typedef struct {
     uint64_t timesteps_executed;

@@ -57,6 +57,10 @@ int pow2ceil(int v) {
     return p;
 }
 
+// Whether a plane's byte offsets fit the float4 kernels' 32 bits (one row
+// beyond either end included).
+bool narrow_plane(const Grid& g) { return ((size_t)g.ny + 2) * g.nz < ((size_t)1 << 30); }
+
 // Automatic tile choice: work-groups of at most 256 lanes, bx along k times
 // by = 256 / bx rows of j, marching ci planes of i.
 //
@@ -76,10 +80,6 @@ int pow2ceil(int v) {
 // four where the row is cut into narrow blocks (256x320x384 511 / 511 / 497).
 // Scalar lanes, whose planes are cheaper than their start, take two
 // (151x133x117 with CPML, ci 1 / 2 / 3: 82.5 / 75.0 / 81.0).
-// Whether a plane's byte offsets fit the float4 kernels' 32 bits (one row
-// beyond either end included).
-bool narrow_plane(const Grid& g) { return ((size_t)g.ny + 2) * g.nz < ((size_t)1 << 30); }
-
 Tiles auto_tiles(const Grid& g, int vec_req) {
     Tiles t{};
     t.vec = vec_req == 1 || (g.nz % 4 != 0 && g.nz < 8) || !narrow_plane(g) ? 1 : 4;
@@ -491,7 +491,32 @@ void engine_free(oe_engine* e) {
     delete e;
 }
 
+bool close_z_slabs(const CpmlArgs* cp) {
+    return cp && !cp->zvec && (cp->on_mask & 48) == 48 && cp->g0[5] - cp->L[4] < 3;
+}
+
 }  // namespace
+
+namespace oe {
+
+bool dft_rides(const oe_extension* x) {
+    return x->dft_stride == 1 && x->dft.surf.n == 0 && x->dft.n_sig <= RIDE_SIGNALS &&
+           (long)x->dft.n_sig * x->dft.n_f <= RIDE_PAIRS && x->dft_terms <= (size_t)RIDE_PAIRS;
+}
+
+bool one_launch_plan(const oe_engine* e, const CpmlArgs* cp, int ci, YeeArgs* a, int* axes) {
+    if (e->n_mat[0] <= 0 || e->n_mat[1] <= 0) return false;
+    Tiles t = auto_tiles(e->g, 0);
+    if (t.vec != 4 || close_z_slabs(cp)) return false;
+    t.ci = std::min(ci, e->g.nx);
+    const std::vector<Launch> plan = plan_launches(e, t, cp, true);
+    if (plan.size() != 1 || (plan[0].axes & (AX_X | AX_Y)) != 0) return false;
+    *a = plan[0].a;
+    *axes = plan[0].axes;
+    return true;
+}
+
+}  // namespace oe
 
 // =================================================================== C ABI
 extern "C" {
@@ -1792,7 +1817,7 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     Tiles tl = e->tiles;
     // a float4 lane meets at most one z slab, or lanes are scalar
     if (tl.vec == 4 && !narrow_plane(e->g)) tl = auto_tiles(e->g, 1);
-    if (cp && !cp->zvec && tl.vec == 4 && (cp->on_mask & 48) == 48 && cp->g0[5] - cp->L[4] < 3) tl = auto_tiles(e->g, 1);
+    if (tl.vec == 4 && close_z_slabs(cp)) tl = auto_tiles(e->g, 1);
     // Fused steps (one pass per step over the plan's interior box) when no
     // extension hooks in between the half-steps and the grid suits the
     // fused kernel; the x/y CPML slabs keep their two launches around it.
@@ -1931,9 +1956,7 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     if (riding) {
         std::vector<oe_extension*> rest;
         for (auto* x : dfts) {
-            const bool small = x->dft_stride == 1 && x->dft.surf.n == 0 && x->dft.n_sig <= RIDE_SIGNALS &&
-                               (long)x->dft.n_sig * x->dft.n_f <= RIDE_PAIRS && x->dft_terms <= (size_t)RIDE_PAIRS;
-            (small && ride_dfts.size() < (size_t)MAX_RIDE_DFT ? ride_dfts : rest).push_back(x);
+            (dft_rides(x) && ride_dfts.size() < (size_t)MAX_RIDE_DFT ? ride_dfts : rest).push_back(x);
         }
         dfts.swap(rest);
     }

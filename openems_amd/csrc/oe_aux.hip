@@ -116,6 +116,8 @@ __global__ __launch_bounds__(EN_THREADS) void k_energy(const float* __restrict__
 __global__ __launch_bounds__(EN_THREADS) void k_energy_final(const double* __restrict__ partials, int nb,
                                                              double* __restrict__ out) {
     __shared__ double se[EN_THREADS], sh[EN_THREADS];
+    partials += 2 * (size_t)nb * blockIdx.x;  // one grid's per work-group
+    out += 2 * blockIdx.x;
     double ae = 0.0, ah = 0.0;
     for (int b = threadIdx.x; b < nb; b += EN_THREADS) {
         ae += partials[2 * b];
@@ -478,6 +480,11 @@ __global__ __launch_bounds__(256) void k_sweep_point(const SweepExc* __restrict_
 
 __global__ __launch_bounds__(256) void k_ride_last(const Ride* __restrict__ r) { ride(*r, blockIdx.x, true); }
 
+__global__ __launch_bounds__(256) void k_ride_last_many(const Ride* __restrict__ table, const int* __restrict__ ids) {
+    const Ride& r = table[ids[blockIdx.y]];
+    if ((int)blockIdx.x < r.first_ade) ride(r, blockIdx.x, true);
+}
+
 __global__ void k_sweep_step(uint64_t* step) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *step += 1;
 }
@@ -655,6 +662,12 @@ hipError_t launch_ride_last(const Ride* r, int n_wg, hipStream_t s) {
     return hipGetLastError();
 }
 
+hipError_t launch_ride_last_many(const Ride* table, const int* ids, int n, int n_wg, hipStream_t s) {
+    if (n <= 0 || n_wg <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_ride_last_many, dim3(n_wg, n), dim3(256), 0, s, table, ids);
+    return hipGetLastError();
+}
+
 hipError_t launch_sweep_step(uint64_t* step, hipStream_t s) {
     hipLaunchKernelGGL(k_sweep_step, dim3(1), dim3(64), 0, s, step);
     return hipGetLastError();
@@ -664,9 +677,7 @@ hipError_t launch_sweep_energy(const SweepStruct* st, const int* ids, int n, dou
                                hipStream_t s) {
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_sweep_energy, dim3(EN_BLOCKS, n), dim3(EN_THREADS), 0, s, st, ids, partials);
-    for (int q = 0; q < n; ++q)
-        hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(EN_THREADS), 0, s, partials + (size_t)q * 2 * EN_BLOCKS,
-                           EN_BLOCKS, out + 2 * q);
+    hipLaunchKernelGGL(k_energy_final, dim3(n), dim3(EN_THREADS), 0, s, partials, EN_BLOCKS, out);
     return hipGetLastError();
 }
 

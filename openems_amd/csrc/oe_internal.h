@@ -239,6 +239,21 @@ struct SweepArgs {
 // table, rows being the largest table of the launch's half (LDS size).
 hipError_t launch_sweep(bool h, const SweepArgs& a, int n_wg, int axes, int vec, int rows, hipStream_t s);
 
+// The other grids of a sweep (float4 lanes, a material table for both halves):
+// one launch per kind of axes (0, AX_Z, with or without AX_MIX) and ragged.
+struct SweepUnit {
+    YeeArgs a;
+    CpmlArgs c;
+    int first;  // first work-group of the grid's launch
+};
+struct UnitArgs {
+    const SweepUnit* unit;
+    const int* wg_unit;  // work-group -> unit
+    int xcd_remap;
+    uint64_t* step_inc;  // non-null on a half's first launch: lane 0 advances the counter
+};
+hipError_t launch_units(bool h, const UnitArgs& a, int n_wg, int axes, bool ragged, int rows, hipStream_t s);
+
 // Device arrays to pageable host memory after the work on s (oe_copy.hip);
 // returns when they are there.
 struct HostCopy {
@@ -268,7 +283,7 @@ struct PointExc {
     uint32_t idx;   // linear cell index
     uint32_t comp;  // 0..2 (E component)
     uint32_t soft;
-    uint32_t pad;
+    uint32_t zero_after;  // past its samples the source's value is 0 (else it does nothing)
     const float* samples;
     uint64_t n_samples;
 };
@@ -421,6 +436,8 @@ struct Ride {
 };
 // The H launches' riders alone, after a batch's last step (probes and DFTs).
 hipError_t launch_ride_last(const Ride* r, int n_wg, hipStream_t s);
+// Several structures' at once: those of table[ids[0..n)], n_wg work-groups each.
+hipError_t launch_ride_last_many(const Ride* table, const int* ids, int n, int n_wg, hipStream_t s);
 
 // Sweep step pieces (oe_aux.hip).  The step index is read from *step.
 struct SweepExc {

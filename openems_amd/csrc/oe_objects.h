@@ -180,3 +180,10 @@ struct oe_engine {
     float* host_fields = nullptr;
 };
 
+namespace oe {
+// Whether a DFT is small enough to ride (oe_ride.h).
+bool dft_rides(const oe_extension* x);
+// The single launch of a half-step with ci planes per work-group; false for
+// grids that need scalar lanes or have no material table.
+bool one_launch_plan(const oe_engine* e, const CpmlArgs* cp, int ci, YeeArgs* a, int* axes);
+}  // namespace oe

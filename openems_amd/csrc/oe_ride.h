@@ -103,7 +103,9 @@ __device__ __forceinline__ void ride(const Ride& r, int wg, bool h) {
         if (wg == 0 && r.first_dft > 0 && tid < r.n_src) {
             const PointExc& x = r.src[tid];
             SourceValue v{0.f, 0};
-            if (b < x.n_samples) v = SourceValue{x.samples[b], 1u | (x.soft ? 2u : 0u) | (x.comp << 2)};
+            const uint32_t code = 1u | (x.soft ? 2u : 0u) | (x.comp << 2);
+            if (b < x.n_samples) v = SourceValue{x.samples[b], code};
+            else if (x.zero_after) v.code = code;
             r.src_val[tid] = v;
         }
         if (b == 0) return;  // the batch's first step has no step before it

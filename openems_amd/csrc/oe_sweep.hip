@@ -3,12 +3,14 @@
 //
 // The reference runs one Simulation at a time (Simulation::run,
 // src/fdtd/simulation.rs:255-326, batching timesteps per call,
-// src/fdtd/batch.rs:17-34); it has no multi-structure launcher.  Here every
-// half-step of all active structures is one launch per kernel variant (the
-// work-groups of all structures share the grid through a box table), the
-// excitations, port DFTs and the step counter follow as one launch each, and
-// the step sequence between two termination checks is captured once as a
-// HIP graph and replayed.  Each structure stops on its own energy decay or at
+// src/fdtd/batch.rs:17-34); it has no multi-structure launcher.  Here a
+// half-step of all active structures is one launch: the work-groups of each
+// structure's own launch (its tiles, and as riders its port DFT and source
+// values) stand one after the other, found through a table.  Structures that
+// need scalar lanes or have no material table go in launches per kernel
+// variant beside it, sources and DFTs too large to ride in a point launch
+// after it.  The step sequence between two termination checks is captured
+// once as a HIP graph and replayed.  Each structure stops on its own energy decay or at
 // max_steps; stopped structures leave the tables.  Checks fall on the
 // engines' absolute timesteps and the peak is kept in the engine, so a run
 // can continue where an earlier one stopped with the same result as one run.
@@ -33,7 +35,20 @@ struct Item {
     std::vector<SweepExc> exc;              // target filled at run time
     std::vector<std::vector<float>> samples;
     std::vector<size_t> exc_off;            // element offsets of the targets
-    int vec = 4;
+    // of the running run
+    bool unit = false;       // in a UnitGroup
+    bool fold = false;       // sources added by the E launch
+    bool ride_port = false;  // port DFT carried by the launches
+};
+
+struct UnitGroup {  // one launch: the grids of one kind
+    int axes;
+    bool ragged;
+    std::vector<SweepUnit> units;
+    std::vector<int> wg_unit;
+    int rows_h = 0, rows_e = 0;  // largest material tables
+    const SweepUnit* d_unit = nullptr;  // device copies
+    const int* d_wg = nullptr;
 };
 
 struct Group {      // one launch: all boxes of one (vec, axes) kind
@@ -59,18 +74,22 @@ struct oe_sweep {
     int device = 0;
     hipStream_t stream = nullptr;
     std::vector<Item> items;
-    int ci = 8;            // planes per work-group along i
+    // planes per work-group along i: 32 microstrips of 0.2 to 1.3 M cells
+    // take 317 / 305 / 306 / 320 us a step at 1 / 2 / 4 / 8
+    int ci = 2;
     int xcd_remap = 1;
-    // largest material table of the run per half (0: some structure reads
-    // its coefficient arrays, so every structure does)
+    // largest material table per half of the structures outside the units
+    // (0: some structure reads its coefficient arrays, so every one does)
     int rows_h = 0, rows_e = 0;
     double tune_ms[4] = {0, 0, 0, 0};
     int tune_ci[4] = {1, 2, 4, 8};
     // device state of a run
-    DevBuf structs, tables, excs, exc_first, exc_serial, exc_samples, dfts, dft_of, ids, partials, energy, step;
+    DevBuf structs, tables, rides, excs, exc_first, exc_serial, exc_samples, dfts, dft_of, ids, partials, energy, step;
     double* energy_host = nullptr;
     size_t energy_host_n = 0;
     std::vector<Group> groups;
+    std::vector<UnitGroup> unit_groups;
+    std::vector<Ride> ride_host;  // per structure, of the run (n_wg 0: none)
     // per structure, the (timestep, E + H energy) of every check of the last run
     std::vector<std::vector<std::pair<uint64_t, double>>> history;
     hipGraph_t graph = nullptr;
@@ -120,7 +139,7 @@ namespace {
 // (plain kernel).
 void structure_boxes(const oe_sweep* sw, int sid, const Item& it, std::vector<Group>& groups) {
     const Grid& g = it.eng->g;
-    const int vec = it.vec;
+    const int vec = g.nz % 4 == 0 && (!it.cpml || it.cpml->cpml.zvec) ? 4 : 1;
     const int nzv = ceil_div(g.nz, vec);
     SweepBox proto{};
     proto.sid = sid;
@@ -179,39 +198,86 @@ void structure_boxes(const oe_sweep* sw, int sid, const Item& it, std::vector<Gr
 // Launch tables of the active structures, uploaded into sw->tables.
 oe_status build_tables(oe_sweep* sw, const std::vector<int>& active) {
     sw->groups.clear();
-    for (int sid : active) structure_boxes(sw, sid, sw->items[sid], sw->groups);
-    size_t nb = 0, nw = 0;
-    std::vector<size_t> box_off, wg_off;
-    for (auto& G : sw->groups) {
-        box_off.push_back(nb);
-        wg_off.push_back(nw);
-        nb += G.boxes.size();
-        nw += G.wg_box.size();
+    sw->unit_groups.clear();
+    for (int sid : active) {
+        const Item& it = sw->items[sid];
+        if (!it.unit) {
+            structure_boxes(sw, sid, it, sw->groups);
+            continue;
+        }
+        SweepUnit u{};
+        int axes = 0;
+        if (!one_launch_plan(it.eng, it.cpml ? &it.cpml->cpml : nullptr, sw->ci, &u.a, &axes))
+            return fail(OE_ERR_CONFIG, "structure %d has no single launch", sid);
+        if (it.cpml) u.c = it.cpml->cpml;
+        u.a.xcd_remap = 0;
+        const Ride& r = sw->ride_host[sid];
+        if (r.n_wg > 0) {
+            u.a.ride = sw->rides.as<Ride>() + sid;
+            u.a.n_ride = r.n_wg;
+            u.a.src_val = r.src_val;
+            u.a.n_src = r.n_src;
+            for (int q = 0; q < r.n_src; ++q) u.a.src_idx[q] = (uint32_t)(it.exc_off[q] % it.eng->g.N);
+        }
+        UnitGroup* G = nullptr;
+        for (auto& q : sw->unit_groups)
+            if (q.axes == axes && q.ragged == (u.a.ragged != 0)) G = &q;
+        if (!G) {
+            sw->unit_groups.emplace_back();
+            G = &sw->unit_groups.back();
+            G->axes = axes;
+            G->ragged = u.a.ragged != 0;
+        }
+        u.first = (int)G->wg_unit.size();
+        G->wg_unit.insert(G->wg_unit.end(), u.a.n_ride + u.a.first[u.a.nbox], (int)G->units.size());
+        G->units.push_back(u);
+        G->rows_h = std::max(G->rows_h, u.a.n_mat_h);
+        G->rows_e = std::max(G->rows_e, u.a.n_mat_e);
     }
-    const size_t bbytes = (nb * sizeof(SweepBox) + 255) & ~(size_t)255;
-    std::vector<char> host(bbytes + nw * sizeof(int));
-    for (size_t q = 0; q < sw->groups.size(); ++q) {
-        const Group& G = sw->groups[q];
-        std::memcpy(host.data() + box_off[q] * sizeof(SweepBox), G.boxes.data(), G.boxes.size() * sizeof(SweepBox));
-        std::memcpy(host.data() + bbytes + wg_off[q] * sizeof(int), G.wg_box.data(), G.wg_box.size() * sizeof(int));
+    std::vector<char> host;
+    auto put = [&](const void* p, size_t bytes) {
+        const size_t at = host.size();
+        host.resize((at + bytes + 63) / 64 * 64);
+        std::memcpy(host.data() + at, p, bytes);
+        return at;
+    };
+    std::vector<std::pair<size_t, size_t>> at;
+    for (const auto& G : sw->groups) {
+        const size_t b = put(G.boxes.data(), G.boxes.size() * sizeof(SweepBox));
+        at.push_back({b, put(G.wg_box.data(), G.wg_box.size() * sizeof(int))});
+    }
+    for (const auto& G : sw->unit_groups) {
+        const size_t b = put(G.units.data(), G.units.size() * sizeof(SweepUnit));
+        at.push_back({b, put(G.wg_unit.data(), G.wg_unit.size() * sizeof(int))});
     }
     if (sw->tables.bytes < host.size()) HIP_OK(sw->tables.alloc(host.size()));
     HIP_OK(hipMemcpyAsync(sw->tables.p, host.data(), host.size(), hipMemcpyHostToDevice, sw->stream));
     HIP_OK(hipStreamSynchronize(sw->stream));
-    for (size_t q = 0; q < sw->groups.size(); ++q) {
-        sw->groups[q].d_box = reinterpret_cast<const SweepBox*>(sw->tables.as<char>() + box_off[q] * sizeof(SweepBox));
-        sw->groups[q].d_wg = reinterpret_cast<const int*>(sw->tables.as<char>() + bbytes + wg_off[q] * sizeof(int));
+    const char* base = sw->tables.as<char>();
+    size_t q = 0;
+    for (auto& G : sw->groups) {
+        G.d_box = reinterpret_cast<const SweepBox*>(base + at[q].first);
+        G.d_wg = reinterpret_cast<const int*>(base + at[q++].second);
+    }
+    for (auto& G : sw->unit_groups) {
+        G.d_unit = reinterpret_cast<const SweepUnit*>(base + at[q].first);
+        G.d_wg = reinterpret_cast<const int*>(base + at[q++].second);
     }
     return OE_OK;
 }
 
-// step_inc (H half only): the first launch advances this step counter.  The
-// launches of one half write disjoint cells and read only the other field,
-// so with sw->overlap the slab groups (x/y CPML faces) go to side streams,
-// forked from and joined back into the sweep stream around its interior
-// launch.
-hipError_t yee_half(oe_sweep* sw, bool h, uint64_t* step_inc = nullptr) {
-    bool first = true;
+// The first launch advances the half's step counter.  The launches of one
+// half write disjoint cells and read only the other field, so with
+// sw->overlap the slab groups (x/y CPML faces) go to side streams, forked
+// from and joined back into the sweep stream around its interior launch.
+hipError_t yee_half(oe_sweep* sw, bool h) {
+    uint64_t* inc = sw->step.as<uint64_t>() + (h ? 0 : 1);
+    for (const auto& G : sw->unit_groups) {
+        const UnitArgs a{G.d_unit, G.d_wg, sw->xcd_remap, inc};
+        inc = nullptr;
+        HIP_RET(launch_units(h, a, (int)G.wg_unit.size(), G.axes, G.ragged, h ? G.rows_h : G.rows_e, sw->stream));
+    }
+    if (sw->groups.empty()) return hipSuccess;
     const bool ov = sw->overlap && sw->groups.size() > 1;
     const int n_side = sw->overlap == 2 ? 3 : 1;
     int used = 0;  // side streams forked so far
@@ -222,8 +288,8 @@ hipError_t yee_half(oe_sweep* sw, bool h, uint64_t* step_inc = nullptr) {
         a.box = G.d_box;
         a.wg_box = G.d_wg;
         a.xcd_remap = sw->xcd_remap;
-        a.step_inc = (h && first) ? step_inc : nullptr;
-        first = false;
+        a.step_inc = inc;
+        inc = nullptr;
         hipStream_t st = sw->stream;
         if (ov && (G.axes & (AX_X | AX_Y)) != 0) {
             // slab group: the next side stream (or the one side stream)
@@ -246,8 +312,7 @@ hipError_t yee_half(oe_sweep* sw, bool h, uint64_t* step_inc = nullptr) {
 
 // Point and DFT tables of the active structures.
 struct StepTables {
-    int n_struct = 0;
-    int n_dft = 0;
+    int n_struct = 0;  // structures with sources or a DFT of the point launch
 };
 
 oe_status build_step_tables(oe_sweep* sw, const std::vector<int>& active, StepTables& t) {
@@ -255,17 +320,23 @@ oe_status build_step_tables(oe_sweep* sw, const std::vector<int>& active, StepTa
     std::vector<int> first{0};
     std::vector<int> serial, dft_of;
     std::vector<SweepDft> dft;
+    int n = 0;
     for (int sid : active) {
         const Item& it = sw->items[sid];
-        for (const auto& e : it.exc) ex.push_back(e);
+        const bool own_exc = !it.fold && !it.exc.empty(), own_dft = it.port && !it.ride_port;
+        if (!own_exc && !own_dft) continue;
+        ++n;
+        if (own_exc)
+            for (const auto& e : it.exc) ex.push_back(e);
         first.push_back((int)ex.size());
         // sources on one cell apply in list order: then one thread does them all
         std::vector<const float*> cells;
-        for (const auto& e : it.exc) cells.push_back(e.target);
+        if (own_exc)
+            for (const auto& e : it.exc) cells.push_back(e.target);
         std::sort(cells.begin(), cells.end());
         serial.push_back(std::adjacent_find(cells.begin(), cells.end()) != cells.end() ? 1 : 0);
-        dft_of.push_back(it.port ? (int)dft.size() : -1);
-        if (it.port) {
+        dft_of.push_back(own_dft ? (int)dft.size() : -1);
+        if (own_dft) {
             SweepDft d{};
             d.F = it.eng->F;
             d.N = it.eng->g.N;
@@ -281,7 +352,7 @@ oe_status build_step_tables(oe_sweep* sw, const std::vector<int>& active, StepTa
     const size_t nb_struct = std::max<size_t>(active.size(), 1) * sizeof(int);
     if (sw->exc_serial.bytes < nb_struct) HIP_OK(sw->exc_serial.alloc(nb_struct));
     if (sw->dft_of.bytes < nb_struct) HIP_OK(sw->dft_of.alloc(nb_struct));
-    if (!active.empty()) {
+    if (n > 0) {
         HIP_OK(hipMemcpyAsync(sw->exc_serial.p, serial.data(), serial.size() * sizeof(int), hipMemcpyHostToDevice,
                               sw->stream));
         HIP_OK(hipMemcpyAsync(sw->dft_of.p, dft_of.data(), dft_of.size() * sizeof(int), hipMemcpyHostToDevice,
@@ -297,8 +368,7 @@ oe_status build_step_tables(oe_sweep* sw, const std::vector<int>& active, StepTa
     if (!active.empty())
         HIP_OK(hipMemcpyAsync(sw->ids.p, active.data(), active.size() * sizeof(int), hipMemcpyHostToDevice, sw->stream));
     HIP_OK(hipStreamSynchronize(sw->stream));
-    t.n_struct = (int)active.size();
-    t.n_dft = (int)dft.size();
+    t.n_struct = n;
     return OE_OK;
 }
 
@@ -306,8 +376,9 @@ oe_status build_step_tables(oe_sweep* sw, const std::vector<int>& active, StepTa
 hipError_t sweep_step(oe_sweep* sw, const StepTables& t, double dt) {
     hipError_t e;
     // the first H launch advances the step counter (from -1: step st reads st)
-    if ((e = yee_half(sw, true, sw->step.as<uint64_t>())) != hipSuccess) return e;
+    if ((e = yee_half(sw, true)) != hipSuccess) return e;
     if ((e = yee_half(sw, false)) != hipSuccess) return e;
+    if (t.n_struct == 0) return hipSuccess;
     return launch_sweep_point(sw->excs.as<SweepExc>(), sw->exc_first.as<int>(), sw->exc_serial.as<int>(),
                               sw->dfts.as<SweepDft>(), sw->dft_of.as<int>(), t.n_struct, sw->step.as<uint64_t>(), dt,
                               sw->stream);
@@ -327,6 +398,79 @@ oe_status capture(oe_sweep* sw, const StepTables& t, double dt, int steps) {
     sw->graph = g;
     HIP_OK(hipGraphInstantiate(&sw->exec, sw->graph, nullptr, nullptr, 0));
     sw->graph_steps = steps;
+    return OE_OK;
+}
+
+// The riders of the run: port DFTs and source values of the structures in
+// units.  Samples are on the device (it.exc[q].samples).
+oe_status build_rides(oe_sweep* sw, uint64_t t0, double dt) {
+    const size_t n = sw->items.size();
+    sw->ride_host.assign(n, Ride{});
+    std::vector<PointExc> src;
+    for (auto& it : sw->items) {
+        const Grid& g = it.eng->g;
+        YeeArgs a;
+        int axes;
+        it.unit = one_launch_plan(it.eng, it.cpml ? &it.cpml->cpml : nullptr, 1, &a, &axes);
+        const bool riding = it.unit && it.eng->ride;
+        it.fold = riding && !it.exc.empty() && it.exc.size() <= (size_t)MAX_FOLD_SOURCES;
+        for (size_t off : it.exc_off) {  // cells the E update writes
+            const size_t cell = off % g.N, plane = (size_t)g.ny * g.nz;
+            if (cell < plane || cell % plane < (size_t)g.nz) it.fold = false;
+        }
+        it.ride_port = riding && it.port && dft_rides(it.port);
+        if (it.fold) src.resize(src.size() + it.exc.size());
+    }
+    const size_t src_off = (n * sizeof(Ride) + 63) / 64 * 64;
+    const size_t val_off = (src_off + src.size() * sizeof(PointExc) + 63) / 64 * 64;
+    const size_t bytes = val_off + n * MAX_FOLD_SOURCES * sizeof(SourceValue);
+    if (sw->rides.bytes < bytes) HIP_OK(sw->rides.alloc(bytes));
+    size_t at = 0;
+    for (size_t s = 0; s < n; ++s) {
+        const Item& it = sw->items[s];
+        Ride& r = sw->ride_host[s];
+        r.F = it.eng->F;
+        r.g = it.eng->g;
+        r.t0 = (double)t0;
+        r.dt = dt;
+        r.step_a = sw->step.as<uint64_t>();
+        r.step_b = sw->step.as<uint64_t>() + 1;
+        if (it.fold) {
+            r.n_src = (int)it.exc.size();
+            r.src = reinterpret_cast<const PointExc*>(sw->rides.as<char>() + src_off) + at;
+            r.src_val = reinterpret_cast<SourceValue*>(sw->rides.as<char>() + val_off) + s * MAX_FOLD_SOURCES;
+            for (size_t q = 0; q < it.exc.size(); ++q) {
+                PointExc& x = src[at++];
+                x.idx = (uint32_t)(it.exc_off[q] % it.eng->g.N);
+                x.comp = (uint32_t)(it.exc_off[q] / it.eng->g.N);
+                x.soft = it.exc[q].soft;
+                x.zero_after = 1;  // as the point launch does
+                x.samples = it.exc[q].samples;
+                x.n_samples = it.exc[q].n_samples;
+            }
+        }
+        r.first_dft = it.fold ? 1 : 0;
+        if (it.ride_port) r.dft[r.n_dft++] = RideDft{it.port->dft, it.port->dft_count};
+        r.first_ade = r.first_mur = r.n_wg = r.first_dft + r.n_dft;
+    }
+    HIP_OK(hipMemcpyAsync(sw->rides.p, sw->ride_host.data(), n * sizeof(Ride), hipMemcpyHostToDevice, sw->stream));
+    if (!src.empty())
+        HIP_OK(hipMemcpyAsync(sw->rides.as<char>() + src_off, src.data(), src.size() * sizeof(PointExc),
+                              hipMemcpyHostToDevice, sw->stream));
+    HIP_OK(hipStreamSynchronize(sw->stream));
+    return OE_OK;
+}
+
+// The E signals of the last step of structures that stop.
+oe_status ride_last(oe_sweep* sw, const std::vector<int>& stopping) {
+    std::vector<int> ids;
+    for (int s : stopping)
+        if (sw->items[s].ride_port) ids.push_back(s);
+    if (ids.empty()) return OE_OK;
+    if (sw->ids.bytes < ids.size() * sizeof(int)) HIP_OK(sw->ids.alloc(ids.size() * sizeof(int)));
+    HIP_OK(hipMemcpyAsync(sw->ids.p, ids.data(), ids.size() * sizeof(int), hipMemcpyHostToDevice, sw->stream));
+    HIP_OK(launch_ride_last_many(sw->rides.as<Ride>(), sw->ids.as<int>(), (int)ids.size(), 2, sw->stream));
+    HIP_OK(hipStreamSynchronize(sw->stream));
     return OE_OK;
 }
 
@@ -369,7 +513,7 @@ oe_status oe_sweep_create(int device, oe_sweep** out) {
             HIP_OK(hipEventCreateWithFlags(&sw->ev_join[q], hipEventDisableTiming));
         }
     }
-    HIP_OK(sw->step.alloc(sizeof(uint64_t)));
+    HIP_OK(sw->step.alloc(2 * sizeof(uint64_t)));  // step under way, steps whose E half has begun
     *out = sw.release();
     return OE_OK;
 }
@@ -398,7 +542,6 @@ oe_status oe_sweep_add(oe_sweep* sw, oe_engine* e, oe_extension* cpml, oe_extens
     it.eng = e;
     it.cpml = cpml;
     it.port = port;
-    it.vec = (e->g.nz % 4 == 0 && (!cpml || cpml->cpml.zvec)) ? 4 : 1;
     for (size_t q = 0; q < n_exc; ++q) {
         const oe_excitation& x = exc[q];
         if (x.i >= (uint32_t)e->g.nx || x.j >= (uint32_t)e->g.ny || x.k >= (uint32_t)e->g.nz || x.direction > 2)
@@ -456,16 +599,6 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
         }
         for (const auto& v : it.samples) total += v.size();
     }
-    sw->rows_e = sw->rows_h = 0;
-    bool all_e = true, all_h = true;
-    for (int s = 0; s < n; ++s) {
-        all_e = all_e && st[s].n_mat_e > 0;
-        all_h = all_h && st[s].n_mat_h > 0;
-        sw->rows_e = std::max(sw->rows_e, st[s].n_mat_e);
-        sw->rows_h = std::max(sw->rows_h, st[s].n_mat_h);
-    }
-    if (!all_e) sw->rows_e = 0;
-    if (!all_h) sw->rows_h = 0;
     HIP_OK(sw->structs.alloc(n * sizeof(SweepStruct)));
     HIP_OK(hipMemcpyAsync(sw->structs.p, st.data(), n * sizeof(SweepStruct), hipMemcpyHostToDevice, sw->stream));
     HIP_OK(sw->exc_samples.alloc(std::max<size_t>(total, 1) * sizeof(float)));
@@ -480,6 +613,19 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
             off += it.samples[q].size();
         }
     HIP_OK(hipMemsetAsync(sw->step.p, 0xff, sizeof(uint64_t), sw->stream));  // -1: the first step's H launch makes it 0
+    HIP_OK(hipMemsetAsync(sw->step.as<uint64_t>() + 1, 0, sizeof(uint64_t), sw->stream));
+    OE_TRY(build_rides(sw, T0, dt));
+    sw->rows_e = sw->rows_h = 0;
+    bool all_e = true, all_h = true;
+    for (int s = 0; s < n; ++s) {
+        if (sw->items[s].unit) continue;
+        all_e = all_e && st[s].n_mat_e > 0;
+        all_h = all_h && st[s].n_mat_h > 0;
+        sw->rows_e = std::max(sw->rows_e, st[s].n_mat_e);
+        sw->rows_h = std::max(sw->rows_h, st[s].n_mat_h);
+    }
+    if (!all_e) sw->rows_e = 0;
+    if (!all_h) sw->rows_h = 0;
 
     std::vector<int> active(n);
     for (int s = 0; s < n; ++s) active[s] = s;
@@ -491,47 +637,22 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
         results[s].termination_reason = OE_TERM_STEPS_COMPLETED;
     }
 
-    // Autotune the i-depth of the work-groups on the zero state: with zero
-    // fields and no sources every update leaves the state exactly zero.
-    if (cfg->autotune) {
-        HIP_OK(sw->ids.alloc(n * sizeof(int)));
-        HIP_OK(hipMemcpyAsync(sw->ids.p, active.data(), n * sizeof(int), hipMemcpyHostToDevice, sw->stream));
-        OE_TRY(energies(sw, n));
-        bool zero = true;
-        for (int s = 0; s < n; ++s) zero = zero && sw->energy_host[2 * s] == 0.0 && sw->energy_host[2 * s + 1] == 0.0;
-        if (zero) {
-            hipEvent_t a, b;
-            HIP_OK(hipEventCreate(&a));
-            HIP_OK(hipEventCreate(&b));
-            double best = 1e300;
-            int best_ci = sw->ci;
-            for (int q = 0; q < 4; ++q) {
-                sw->ci = sw->tune_ci[q];
-                OE_TRY(build_tables(sw, active));
-                for (int w = 0; w < 2; ++w) {
-                    HIP_OK(yee_half(sw, true));
-                    HIP_OK(yee_half(sw, false));
-                }
-                HIP_OK(hipEventRecord(a, sw->stream));
-                constexpr int TUNE_STEPS = 12;  // 6 left candidates within 1% to chance
-                for (int w = 0; w < TUNE_STEPS; ++w) {
-                    HIP_OK(yee_half(sw, true));
-                    HIP_OK(yee_half(sw, false));
-                }
-                HIP_OK(hipEventRecord(b, sw->stream));
-                HIP_OK(hipEventSynchronize(b));
-                float ms = 0.f;
-                HIP_OK(hipEventElapsedTime(&ms, a, b));
-                sw->tune_ms[q] = ms / TUNE_STEPS;
-                if (ms < best) {
-                    best = ms;
-                    best_ci = sw->tune_ci[q];
-                }
-            }
-            (void)hipEventDestroy(a);
-            (void)hipEventDestroy(b);
-            sw->ci = best_ci;
+    // The i-depth of the work-groups, timed over the run's own first steps
+    // after its first check (no result depends on it): TUNE_STEPS of each
+    // candidate, one more before them.
+    struct Events {
+        hipEvent_t a = nullptr, b = nullptr;
+        ~Events() {
+            if (a) (void)hipEventDestroy(a);
+            if (b) (void)hipEventDestroy(b);
         }
+    } ev;
+    constexpr int TUNE_STEPS = 4;
+    int tune_next = cfg->autotune ? 0 : 4, tune_best = 0;
+    if (cfg->autotune) {
+        HIP_OK(hipEventCreate(&ev.a));
+        HIP_OK(hipEventCreate(&ev.b));
+        for (double& ms : sw->tune_ms) ms = 0.0;
     }
 
     OE_TRY(build_tables(sw, active));
@@ -548,7 +669,28 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
         const uint64_t ts = T0 + done;                            // timestep of the next step
         const uint64_t next_check = (ts + check - 1) / check * check;  // first check at or after it
         const uint64_t chunk = std::min<uint64_t>(next_check - ts + 1, cfg->max_steps - done);
-        if (cfg->use_graph && chunk == check && done > 0) {
+        uint64_t ran = 0;
+        while (tune_next < 4 && done > 0 && chunk - ran > TUNE_STEPS) {
+            const int q = tune_next++;
+            sw->ci = sw->tune_ci[q];
+            OE_TRY(build_tables(sw, active));
+            HIP_OK(sweep_step(sw, tab, dt));
+            HIP_OK(hipEventRecord(ev.a, sw->stream));
+            for (int w = 0; w < TUNE_STEPS; ++w) HIP_OK(sweep_step(sw, tab, dt));
+            HIP_OK(hipEventRecord(ev.b, sw->stream));
+            HIP_OK(hipEventSynchronize(ev.b));
+            float ms = 0.f;
+            HIP_OK(hipEventElapsedTime(&ms, ev.a, ev.b));
+            sw->tune_ms[q] = ms / TUNE_STEPS;
+            if (sw->tune_ms[q] < sw->tune_ms[tune_best]) tune_best = q;
+            ran += TUNE_STEPS + 1;
+            if (tune_next == 4 || chunk - ran <= TUNE_STEPS) {
+                sw->ci = sw->tune_ci[tune_best];
+                OE_TRY(build_tables(sw, active));
+                dirty = true;
+            }
+        }
+        if (cfg->use_graph && chunk == check && done > 0 && ran == 0) {
             // the graph holds a divisor of the check interval (at most 25
             // steps) and is launched check / gsteps times: the active set
             // changes at many checks, and instantiating a short graph costs
@@ -562,7 +704,7 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
             }
             for (uint64_t q = 0; q < chunk / gsteps; ++q) HIP_OK(hipGraphLaunch(sw->exec, sw->stream));
         } else {
-            for (uint64_t q = 0; q < chunk; ++q) HIP_OK(sweep_step(sw, tab, dt));
+            for (uint64_t q = ran; q < chunk; ++q) HIP_OK(sweep_step(sw, tab, dt));
         }
         done += chunk;
         const uint64_t cur = T0 + done - 1;  // timestep of the last step run
@@ -590,6 +732,10 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
             else keep.push_back(s);
         }
         if (keep.size() != active.size()) {
+            std::vector<int> stopping;
+            for (int s : active)
+                if (results[s].termination_reason == OE_TERM_ENERGY_DECAY) stopping.push_back(s);
+            OE_TRY(ride_last(sw, stopping));
             active.swap(keep);
             if (!active.empty()) {
                 OE_TRY(build_tables(sw, active));
@@ -598,6 +744,7 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
             }
         }
     }
+    OE_TRY(ride_last(sw, active));
     HIP_OK(hipStreamSynchronize(sw->stream));
     for (int s : active) results[s].timesteps_executed = done;
     // Engines and port DFTs advance by the steps each structure ran.

@@ -243,14 +243,13 @@ struct Rows {
     }
 };
 
-// Reads one word of each 64-byte line of the kernel's arguments at once.
+// Reads one word of each 64-byte line of a kernel's arguments at once.
 // Loaded where they are used, the lines (13 of a Yee launch) arrive one
 // after the other, each a miss of its work-group's scalar cache: a step of
 // 72x60x32 with CPML took 13.4 us, 12.5 with this.
+using ArgLine = const __attribute__((address_space(4))) unsigned*;
 template <int BYTES>
-__device__ __forceinline__ void touch_args() {
-    using Arg = const __attribute__((address_space(4))) unsigned*;
-    const Arg k = (Arg)__builtin_amdgcn_kernarg_segment_ptr();
+__device__ __forceinline__ void touch_lines(ArgLine k) {
     constexpr int L = (BYTES + 63) / 64;
     static_assert(L >= 1 && L <= 16, "arguments beyond 1 KB");
     unsigned t[16];
@@ -258,6 +257,9 @@ __device__ __forceinline__ void touch_args() {
     for (int q = 0; q < 16; ++q) t[q] = k[16 * (q < L ? q : L - 1)];
     __asm__ volatile("" ::"s"(t[0]), "s"(t[1]), "s"(t[2]), "s"(t[3]), "s"(t[4]), "s"(t[5]), "s"(t[6]), "s"(t[7]),
                      "s"(t[8]), "s"(t[9]), "s"(t[10]), "s"(t[11]), "s"(t[12]), "s"(t[13]), "s"(t[14]), "s"(t[15]));
+}
+__device__ __forceinline__ void touch_args() {
+    touch_lines<sizeof(YeeArgs) + sizeof(CpmlArgs)>((ArgLine)__builtin_amdgcn_kernarg_segment_ptr());
 }
 
 // kfirst / klast: the lane's left / right k neighbour along the row is not
@@ -276,8 +278,7 @@ struct Tile {
 // and each of the two kinds is spread over the XCDs by itself (their
 // work-groups do not cost the same); inner tells them apart.
 template <int V, bool MIX = false>
-__device__ __forceinline__ Tile decode(const YeeArgs& a, bool* inner = nullptr) {
-    int bid = blockIdx.x - a.n_ride;
+__device__ __forceinline__ Tile decode(const YeeArgs& a, int bid, bool* inner = nullptr) {
     int seg0 = 0, seg1 = a.first[a.nbox];
     if constexpr (MIX) {
         *inner = bid >= a.first[a.nbox - 1];
@@ -850,7 +851,7 @@ template <int V, int AX, bool PHYS, bool TAB, bool RAG = false>
 __global__ __launch_bounds__(256, V == 4 && AX == 7 ? 3 : 1) void k_update_h(YeeArgs a, CpmlArgs c) {
     extern __shared__ float2 lds_rows[];
     // the step's first launch advances the step counter (no H lane reads it)
-    touch_args<sizeof(YeeArgs) + sizeof(CpmlArgs)>();
+    touch_args();
     if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(a.step_inc);
     if constexpr (RIDES<AX>) {
         if ((int)blockIdx.x < a.n_ride) {
@@ -860,14 +861,14 @@ __global__ __launch_bounds__(256, V == 4 && AX == 7 ? 3 : 1) void k_update_h(Yee
     }
     Rows<TAB> rows{lds_rows, reinterpret_cast<const float2*>(a.tab_h), 3 * a.n_mat_h};
     h_body<V, AX, PHYS, TAB, RAG>(a.g, a.Fin, a.Fout, a.Cf, MatIndex{a.n_mat_h == 1 ? nullptr : a.mat_h, a.mat8_h}, rows, c,
-                             decode<V>(a));
+                             decode<V>(a, blockIdx.x - a.n_ride));
 }
 
 // The z-faces kernels are held to the 128 registers of 4 waves a SIMD.
 template <int V, int AX, bool PHYS, bool TAB, bool MUR = false, bool RAG = false>
 __global__ __launch_bounds__(256, V == 4 && AX == AX_Z ? 4 : V == 4 && AX == 7 ? 3 : 1) void k_update_e(YeeArgs a, CpmlArgs c) {
     extern __shared__ float2 lds_rows[];
-    touch_args<sizeof(YeeArgs) + sizeof(CpmlArgs)>();
+    touch_args();
     if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(a.step_inc);
     if constexpr (RIDES<AX>) {
         if ((int)blockIdx.x < a.n_ride) {
@@ -880,9 +881,9 @@ __global__ __launch_bounds__(256, V == 4 && AX == AX_Z ? 4 : V == 4 && AX == 7 ?
     const MatIndex mat_e{a.n_mat_e == 1 ? nullptr : a.mat_e, a.mat8_e};
     if (MUR || a.n_src) {
         const Sources src{a, TAB ? lds_val : a.src_val};
-        e_body<V, AX, PHYS, TAB, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat_e, rows, c, decode<V>(a), &src, a.mur_z);
+        e_body<V, AX, PHYS, TAB, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat_e, rows, c, decode<V>(a, blockIdx.x - a.n_ride), &src, a.mur_z);
     } else {
-        e_body<V, AX, PHYS, TAB, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat_e, rows, c, decode<V>(a));
+        e_body<V, AX, PHYS, TAB, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat_e, rows, c, decode<V>(a, blockIdx.x - a.n_ride));
     }
 }
 
@@ -894,48 +895,81 @@ __global__ __launch_bounds__(256, V == 4 && AX == AX_Z ? 4 : V == 4 && AX == 7 ?
 // each waited for once; large ones run at memory speed (256^3, 8 layers, 64
 // boxes' table: 109 us a launch, 121 when the slabs were a launch of their
 // own and a plane's loads came in three waits).
-template <int AXI, bool PHYS, bool RAG>
-__global__ __launch_bounds__(256, 3) void k_update_h_mix(YeeArgs a, CpmlArgs c) {
+template <int AXI, bool MIX, bool PHYS, bool RAG>
+__device__ __forceinline__ void h_group(const YeeArgs& a, const CpmlArgs& c, int bid, float2* lds_rows) {
     constexpr int V = 4;
-    extern __shared__ float2 lds_rows[];
-    touch_args<sizeof(YeeArgs) + sizeof(CpmlArgs)>();
-    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(a.step_inc);
-    if ((int)blockIdx.x < a.n_ride) {
-        ride(*a.ride, blockIdx.x, true);
+    if (bid < a.n_ride) {
+        ride(*a.ride, bid, true);
         return;
     }
     Rows<true> rows{lds_rows, reinterpret_cast<const float2*>(a.tab_h), 3 * a.n_mat_h};
     const MatIndex mat{a.n_mat_h == 1 ? nullptr : a.mat_h, a.mat8_h};
-    bool inner;
-    const Tile t = decode<V, true>(a, &inner);
-    if (inner) h_body<V, AXI, PHYS && AXI != 0, true, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t);
+    bool inner = true;
+    const Tile t = decode<V, MIX>(a, bid - a.n_ride, &inner);
+    if (!MIX || inner) h_body<V, AXI, PHYS && AXI != 0, true, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t);
     else h_body<V, AX_X | AX_Y | AX_Z, PHYS, true, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t);
 }
 
-template <int AXI, bool PHYS, bool MUR, bool RAG>
-__global__ __launch_bounds__(256, 3) void k_update_e_mix(YeeArgs a, CpmlArgs c) {
+template <int AXI, bool MIX, bool PHYS, bool MUR, bool RAG>
+__device__ __forceinline__ void e_group(const YeeArgs& a, const CpmlArgs& c, int bid, float2* lds_rows) {
     constexpr int V = 4;
-    extern __shared__ float2 lds_rows[];
-    touch_args<sizeof(YeeArgs) + sizeof(CpmlArgs)>();
-    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(a.step_inc);
-    if ((int)blockIdx.x < a.n_ride) {
-        ride(*a.ride, blockIdx.x, false);
+    if (bid < a.n_ride) {
+        ride(*a.ride, bid, false);
         return;
     }
     __shared__ SourceValue lds_val[MAX_FOLD_SOURCES];
     Rows<true> rows{lds_rows, reinterpret_cast<const float2*>(a.tab_e), 3 * a.n_mat_e, a.src_val, lds_val, a.n_src};
     const MatIndex mat{a.n_mat_e == 1 ? nullptr : a.mat_e, a.mat8_e};
     const Sources ex{a, lds_val};
-    bool inner;
-    const Tile t = decode<V, true>(a, &inner);
-    if (inner)
+    bool inner = true;
+    const Tile t = decode<V, MIX>(a, bid - a.n_ride, &inner);
+    if (!MIX || inner)
         e_body<V, AXI, PHYS && AXI != 0, true, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t, &ex, a.mur_z);
     else
         e_body<V, AX_X | AX_Y | AX_Z, PHYS, true, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t, &ex, a.mur_z);
 }
 
-// Many grids in one launch (a parameter sweep): work-group -> box of some
-// structure through the launch's table; each box has its own tile shape
+template <int AXI, bool PHYS, bool RAG>
+__global__ __launch_bounds__(256, 3) void k_update_h_mix(YeeArgs a, CpmlArgs c) {
+    extern __shared__ float2 lds_rows[];
+    touch_args();
+    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(a.step_inc);
+    h_group<AXI, true, PHYS, RAG>(a, c, blockIdx.x, lds_rows);
+}
+
+template <int AXI, bool PHYS, bool MUR, bool RAG>
+__global__ __launch_bounds__(256, 3) void k_update_e_mix(YeeArgs a, CpmlArgs c) {
+    extern __shared__ float2 lds_rows[];
+    touch_args();
+    if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(a.step_inc);
+    e_group<AXI, true, PHYS, MUR, RAG>(a, c, blockIdx.x, lds_rows);
+}
+
+// A parameter sweep: the launches of many grids as one.  A work-group finds
+// its grid in the launch's table and runs that grid's own launch from there
+// (its tiles, riders and sources), with the arguments in device memory
+// instead of the kernel's; consecutive work-groups, and so one grid's,
+// share an XCD.
+template <int AXI, bool MIX, bool RAG, bool H>
+__global__ __launch_bounds__(256, MIX ? 3 : AXI != 0 ? 4 : 1) void k_update_units(UnitArgs s) {
+    extern __shared__ float2 lds_rows[];
+    if (s.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(s.step_inc);
+    int bid = blockIdx.x;
+    if (s.xcd_remap) {
+        const int per = gridDim.x >> 3;
+        if (bid < (per << 3)) bid = (bid & 7) * per + (bid >> 3);
+    }
+    using Table = const __attribute__((address_space(4))) int*;
+    using Units = const __attribute__((address_space(4))) SweepUnit*;
+    const Units p = (Units)s.unit + ((Table)s.wg_unit)[bid];
+    touch_lines<sizeof(SweepUnit)>((ArgLine)p);
+    const SweepUnit& u = *(const SweepUnit*)p;
+    if constexpr (H) h_group<AXI, MIX, true, RAG>(u.a, u.c, bid - u.first, lds_rows);
+    else e_group<AXI, MIX, true, false, RAG>(u.a, u.c, bid - u.first, lds_rows);
+}
+
+// The sweep's grids that need scalar lanes or have no material table, many in
+// one launch: work-group -> box of some structure through the launch's table; each box has its own tile shape
 // (bx * by * ns <= 256 lanes: ns i-chunks of by rows of bx lanes; surplus
 // lanes exit).
 template <int V>
@@ -1642,6 +1676,26 @@ hipError_t launch_fused(const FusedArgs& a, const CpmlArgs* c, hipStream_t s) {
     if (c->physical)
         return tab ? launch_fused_t<AX_Z, true, true>(a, *c, s) : launch_fused_t<AX_Z, true, false>(a, *c, s);
     return tab ? launch_fused_t<AX_Z, false, true>(a, *c, s) : launch_fused_t<AX_Z, false, false>(a, *c, s);
+}
+
+template <bool H, int AXI, bool MIX>
+static hipError_t units_t(const UnitArgs& a, int n_wg, bool ragged, int rows, hipStream_t s) {
+    const size_t lds = 3 * rows * sizeof(float2);
+    if (ragged) hipLaunchKernelGGL((k_update_units<AXI, MIX, true, H>), dim3(n_wg), dim3(256), lds, s, a);
+    else hipLaunchKernelGGL((k_update_units<AXI, MIX, false, H>), dim3(n_wg), dim3(256), lds, s, a);
+    return hipGetLastError();
+}
+
+template <bool H>
+static hipError_t units_dispatch(const UnitArgs& a, int n_wg, int axes, bool ragged, int rows, hipStream_t s) {
+    if (axes & AX_MIX)
+        return axes & AX_Z ? units_t<H, AX_Z, true>(a, n_wg, ragged, rows, s) : units_t<H, 0, true>(a, n_wg, ragged, rows, s);
+    return axes & AX_Z ? units_t<H, AX_Z, false>(a, n_wg, ragged, rows, s) : units_t<H, 0, false>(a, n_wg, ragged, rows, s);
+}
+
+hipError_t launch_units(bool h, const UnitArgs& a, int n_wg, int axes, bool ragged, int rows, hipStream_t s) {
+    if (n_wg <= 0) return hipSuccess;
+    return h ? units_dispatch<true>(a, n_wg, axes, ragged, rows, s) : units_dispatch<false>(a, n_wg, axes, ragged, rows, s);
 }
 
 // Sweep launches: physical CPML only (every structure of a sweep carries the

@@ -187,3 +187,58 @@ def test_sweep_sources_on_repeated_cells_keep_list_order():
         eng2, port2 = keep[q]
         assert np.array_equal(np.concatenate(eng1.read_fields()), np.concatenate(eng2.read_fields()))
         assert np.array_equal(port1.series(), port2.series())
+
+
+@pytest.mark.parametrize("check,graph,tune", [(10, True, True), (7, False, True), (30, True, False), (3, True, True)])
+def test_kinds_of_structures_together(check, graph, tune):
+    """Structures of every kind in one sweep: with and without CPML, on z
+    only, on one x face, rows that are no whole float4 lanes, rows of scalar
+    lanes, no material table (1030 materials); sources that the E launch
+    adds (also hard ones whose samples end early, which hold their cell at
+    zero from then on), too many of them, ones on the j = 0 row; DFTs that
+    ride and ones too large to.  Each equals its own engine's run (samples
+    continued with zeros) bit for bit."""
+    from openems_amd import MODE_PHYSICAL, CpmlBoundaries, HipEngine, Operator, ScheduledExcitation
+
+    steps = 61
+    pulse = np.exp(-((np.arange(steps) - 15) / 6.0) ** 2).astype(np.float32)
+    f = np.linspace(2e9, 20e9, 5)
+    # shape, layers, sources (count, j), DFT signals, materials
+    kinds = [((20, 18, 24), (4,) * 6, (2, 9), 2, 3), ((20, 18, 24), None, (8, 9), 64, 1),
+             ((17, 23, 30), (0, 0, 0, 0, 5, 7), (3, 4), 5, 2), ((24, 30, 33), (0, 6, 0, 0, 0, 0), (9, 11), 3, 86),
+             ((19, 21, 6), (3, 3, 3, 3, 0, 0), (1, 8), 4, 2), ((22, 20, 16), (4, 4, 4, 4, 4, 4), (2, 0), 65, 2),
+             ((21, 20, 20), (3, 0, 0, 3, 4, 0), (2, 7), 3, 1030), ((16, 40, 64), (2, 2, 9, 3, 4, 4), (4, 20), 0, 300)]
+
+    def build(q):
+        shape, layers, (n_src, j), n_sig, rows = kinds[q]
+        rng = np.random.default_rng(q)
+        op = Operator.uniform(*shape, 0.5e-3)
+        for m in range(rows - 1):
+            at = [int(rng.integers(0, s)) for s in shape]
+            op.set_material(1.5 + 0.002 * m, 1.0, 0.0, 0.0, (at[0], at[0] + 1, at[1], at[1] + 1, at[2], at[2] + 1))
+        eng = HipEngine(op)
+        cp = eng.cpml(CpmlBoundaries(layers=layers, mode=MODE_PHYSICAL)) if layers else None
+        terms = [[(m % 6, *[int(rng.integers(0, s)) for s in shape], 0.5)] for m in range(n_sig)]
+        dft = eng.dft(terms, f, record_steps=steps) if n_sig else None
+        exc = [ScheduledExcitation((shape[0] // 2, j, m % shape[2]), m % 3, pulse[:steps - 4 * m], m % 2 == 0)
+               for m in range(n_src)]
+        return eng, cp, dft, exc
+
+    sw = Sweep()
+    got = [build(q) for q in range(len(kinds))]
+    for eng, cp, dft, exc in got:
+        sw.add(eng, cp, dft, exc)
+    res = sw.run(steps, check_interval=check, use_graph=graph, autotune=tune)
+    say(f"[sweep] kinds: tuning {sw.tuning()}")
+    for q in range(len(kinds)):
+        eng, cp, dft, exc = build(q)
+        exc = [ScheduledExcitation(x.position, x.direction, np.resize(np.append(x.samples, np.zeros(steps)), steps),
+                                   x.soft_source) for x in exc]
+        r = eng.run_batch(EngineBatch(num_steps=steps, excitations=exc, extensions=[x for x in (cp, dft) if x],
+                                      sample_interval=check))
+        assert res[q].timesteps_executed == r.timesteps_executed == steps
+        for a, b in zip(got[q][0].read_fields(), eng.read_fields()):
+            assert np.array_equal(a, b) and np.abs(b).max() > 0, kinds[q]
+        if dft:
+            assert np.array_equal(got[q][2].series(), dft.series()), kinds[q]
+            assert np.array_equal(got[q][2].dft_values(), dft.dft_values()), kinds[q]
