@@ -114,6 +114,14 @@ Box make_box(const Tiles& t, int i0, int i1, int j0, int j1) {
     return b;
 }
 
+// Fields and psi of a grid.
+size_t state_bytes(const Grid& g, const CpmlArgs* cp) {
+    size_t cells = 6 * g.N;
+    for (int f = 0; cp && f < 6; ++f)
+        if (cp->on_mask >> f & 1) cells += 4 * (g.N / (f < 2 ? g.nx : f < 4 ? g.ny : g.nz)) * cp->L[f];
+    return cells * sizeof(float);
+}
+
 YeeArgs launch_args(const oe_engine* e, const Tiles& t, const CpmlArgs* cp, const std::vector<Box>& boxes) {
     YeeArgs a{};
     a.g = e->g;
@@ -143,6 +151,7 @@ YeeArgs launch_args(const oe_engine* e, const Tiles& t, const CpmlArgs* cp, cons
         a.first[b + 1] = a.first[b] + a.n_kb * boxes[b].n_jb * boxes[b].n_ib;
     }
     a.xcd_remap = e->xcd_remap;
+    a.stream_own = stream_state(state_bytes(e->g, cp));
     return a;
 }
 
@@ -498,6 +507,18 @@ bool close_z_slabs(const CpmlArgs* cp) {
 }  // namespace
 
 namespace oe {
+
+// A half-step reads and writes its own field once; what it leaves behind is
+// read by the next half-step.  Where all of the state stays in the 256 MB
+// behind the L2s, plain loads of the old values are the faster ones (us per
+// step, past the caches / plain: 151x133x117 36.3 / 30.2, with CPML 50.5 /
+// 46.4; 200^3 93.6 / 84.9).  Beyond that size they would displace what the
+// next half-step wants (256^3 180 / 229, with CPML 215 / 263; 220^3 with CPML,
+// 292 MB, 153 / 170), and where the L2s (32 MB) hold the state, what is in
+// them (100^3 11.4 / 12.5).
+bool stream_state(size_t bytes) { return bytes <= ((size_t)30 << 20) || bytes > ((size_t)256 << 20); }
+
+size_t grid_state(const oe_engine* e, const CpmlArgs* cp) { return state_bytes(e->g, cp); }
 
 bool dft_rides(const oe_extension* x) {
     return x->dft_stride == 1 && x->dft.surf.n == 0 && x->dft.n_sig <= RIDE_SIGNALS &&

@@ -129,6 +129,7 @@ struct YeeArgs {
     Box box[MAX_BOXES];
     int first[MAX_BOXES + 1];
     int xcd_remap;         // 1: make consecutive tiles share an XCD (L2)
+    int stream_own;        // 1: the half's own old values are loaded past the caches (stream_state)
     // Point sources added by the E half-step after its update (when no
     // extension acts between the E update and the sources): the lane holding
     // a source's cell adds or sets its value, in list order.  The cell
@@ -239,6 +240,10 @@ struct SweepArgs {
 // table, rows being the largest table of the launch's half (LDS size).
 hipError_t launch_sweep(bool h, const SweepArgs& a, int n_wg, int axes, int vec, int rows, hipStream_t s);
 
+// Whether the half-steps of `bytes` of state (fields and CPML psi) load
+// their own old values past the caches.
+bool stream_state(size_t bytes);
+
 // The other grids of a sweep (float4 lanes, a material table for both halves):
 // one launch per kind of axes (0, AX_Z, with or without AX_MIX) and ragged.
 struct SweepUnit {
@@ -250,6 +255,7 @@ struct UnitArgs {
     const SweepUnit* unit;
     const int* wg_unit;  // work-group -> unit
     int xcd_remap;
+    int stream_own;      // as in YeeArgs, for all units
     uint64_t* step_inc;  // non-null on a half's first launch: lane 0 advances the counter
 };
 hipError_t launch_units(bool h, const UnitArgs& a, int n_wg, int axes, bool ragged, int rows, hipStream_t s);

@@ -181,6 +181,8 @@ struct oe_engine {
 };
 
 namespace oe {
+// Bytes of a grid's fields and psi.
+size_t grid_state(const oe_engine* e, const CpmlArgs* cp);
 // Whether a DFT is small enough to ride (oe_ride.h).
 bool dft_rides(const oe_extension* x);
 // The single launch of a half-step with ci planes per work-group; false for

@@ -78,6 +78,7 @@ struct oe_sweep {
     // take 317 / 305 / 306 / 320 us a step at 1 / 2 / 4 / 8
     int ci = 2;
     int xcd_remap = 1;
+    int stream_own = 1;
     // largest material table per half of the structures outside the units
     // (0: some structure reads its coefficient arrays, so every one does)
     int rows_h = 0, rows_e = 0;
@@ -199,6 +200,9 @@ void structure_boxes(const oe_sweep* sw, int sid, const Item& it, std::vector<Gr
 oe_status build_tables(oe_sweep* sw, const std::vector<int>& active) {
     sw->groups.clear();
     sw->unit_groups.clear();
+    size_t state = 0;
+    for (int sid : active) state += grid_state(sw->items[sid].eng, sw->items[sid].cpml ? &sw->items[sid].cpml->cpml : nullptr);
+    sw->stream_own = stream_state(state);
     for (int sid : active) {
         const Item& it = sw->items[sid];
         if (!it.unit) {
@@ -273,7 +277,7 @@ oe_status build_tables(oe_sweep* sw, const std::vector<int>& active) {
 hipError_t yee_half(oe_sweep* sw, bool h) {
     uint64_t* inc = sw->step.as<uint64_t>() + (h ? 0 : 1);
     for (const auto& G : sw->unit_groups) {
-        const UnitArgs a{G.d_unit, G.d_wg, sw->xcd_remap, inc};
+        const UnitArgs a{G.d_unit, G.d_wg, sw->xcd_remap, sw->stream_own, inc};
         inc = nullptr;
         HIP_RET(launch_units(h, a, (int)G.wg_unit.size(), G.axes, G.ragged, h ? G.rows_h : G.rows_e, sw->stream));
     }

@@ -439,7 +439,7 @@ __device__ __forceinline__ bool any_lane(bool on) {
 // AX: CPML axes compiled in (AX_X | AX_Y | AX_Z); PHYS: apply the field
 // correction (else psi only, as the reference); TAB: coefficients from the
 // material table (mat, tab in LDS) instead of the arrays in Cf.
-template <int V, int AX, bool PHYS, bool TAB, bool RAG = false, class R>
+template <int V, int AX, bool PHYS, bool TAB, bool RAG, bool STREAM, class R>
 __device__ __forceinline__ void h_body(const Grid& g, const float* Fin, float* Fout, const float* __restrict__ Cf,
                                        const MatIndex mat, R& rows,
                                        const CpmlArgs& c, const Tile& t) {
@@ -504,7 +504,7 @@ __device__ __forceinline__ void h_body(const Grid& g, const float* Fin, float* F
         ex_c = ldv<V, RAG>(at(Ex, u, o));
         ez_j = ldv<V, RAG>(at(Ez, u, oj));
         ex_j = ldv<V, RAG>(at(Ex, u, oj));
-        hx = ldn<V, OE_NT_OWN, RAG>(at(Hx, u, o)), hy = ldn<V, OE_NT_OWN, RAG>(at(Hy, u, o)), hz = ldn<V, OE_NT_OWN, RAG>(at(Hz, u, o));
+        hx = ldn<V, STREAM, RAG>(at(Hx, u, o)), hy = ldn<V, STREAM, RAG>(at(Hy, u, o)), hz = ldn<V, STREAM, RAG>(at(Hz, u, o));
         if constexpr (TAB) {
             mi = coef_index<V, RAG>(mat, u, o);
         } else {
@@ -635,7 +635,7 @@ __device__ __forceinline__ void apply_sources(const Sources& src, size_t plane, 
 // update skips (i = 0 or j = 0) get the same writes from their old values.
 // Valid when no other hook acts on those cells between the E update and the
 // Mur post step (the host checks it).
-template <int V, int AX, bool PHYS, bool TAB, bool MUR = false, bool RAG = false, class R>
+template <int V, int AX, bool PHYS, bool TAB, bool MUR, bool RAG, bool STREAM, class R>
 __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* Fout, const float* __restrict__ Cf,
                                        const MatIndex mat, R& rows,
                                        const CpmlArgs& c, const Tile& t, const Sources* src = nullptr,
@@ -707,7 +707,7 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
         hx_c = ldv<V, RAG>(at(Hx, u, o)), hy_c = ldv<V, RAG>(at(Hy, u, o)), hz_c = ldv<V, RAG>(at(Hz, u, o));
         hz_j = ldv<V, RAG>(at(Hz, u, oj));
         hx_j = ldv<V, RAG>(at(Hx, u, oj));
-        ex = ldn<V, OE_NT_OWN, RAG>(at(Ex, u, o)); ey = ldn<V, OE_NT_OWN, RAG>(at(Ey, u, o)); ez = ldn<V, OE_NT_OWN, RAG>(at(Ez, u, o));
+        ex = ldn<V, STREAM, RAG>(at(Ex, u, o)); ey = ldn<V, STREAM, RAG>(at(Ey, u, o)); ez = ldn<V, STREAM, RAG>(at(Ez, u, o));
         if constexpr (!TAB) {
             s0 = ldn<V, OE_NT_COEF, RAG>(at(ca0, u, o)); s1 = ldn<V, OE_NT_COEF, RAG>(at(ca1, u, o)); s2 = ldn<V, OE_NT_COEF, RAG>(at(ca2, u, o));
             c0 = ldn<V, OE_NT_COEF, RAG>(at(cb0, u, o)); c1 = ldn<V, OE_NT_COEF, RAG>(at(cb1, u, o)); c2 = ldn<V, OE_NT_COEF, RAG>(at(cb2, u, o));
@@ -847,7 +847,7 @@ constexpr bool RIDES = (AX & (AX_X | AX_Y)) == 0;
 // One grid: the tile comes from the launch's box list.  With TAB the
 // work-group copies its half's material rows into LDS (dynamic LDS of 24
 // bytes per row).
-template <int V, int AX, bool PHYS, bool TAB, bool RAG = false>
+template <int V, int AX, bool PHYS, bool TAB, bool RAG = false, bool STREAM = true>
 __global__ __launch_bounds__(256, V == 4 && AX == 7 ? 3 : 1) void k_update_h(YeeArgs a, CpmlArgs c) {
     extern __shared__ float2 lds_rows[];
     // the step's first launch advances the step counter (no H lane reads it)
@@ -860,12 +860,12 @@ __global__ __launch_bounds__(256, V == 4 && AX == 7 ? 3 : 1) void k_update_h(Yee
         }
     }
     Rows<TAB> rows{lds_rows, reinterpret_cast<const float2*>(a.tab_h), 3 * a.n_mat_h};
-    h_body<V, AX, PHYS, TAB, RAG>(a.g, a.Fin, a.Fout, a.Cf, MatIndex{a.n_mat_h == 1 ? nullptr : a.mat_h, a.mat8_h}, rows, c,
+    h_body<V, AX, PHYS, TAB, RAG, STREAM>(a.g, a.Fin, a.Fout, a.Cf, MatIndex{a.n_mat_h == 1 ? nullptr : a.mat_h, a.mat8_h}, rows, c,
                              decode<V>(a, blockIdx.x - a.n_ride));
 }
 
 // The z-faces kernels are held to the 128 registers of 4 waves a SIMD.
-template <int V, int AX, bool PHYS, bool TAB, bool MUR = false, bool RAG = false>
+template <int V, int AX, bool PHYS, bool TAB, bool MUR = false, bool RAG = false, bool STREAM = true>
 __global__ __launch_bounds__(256, V == 4 && AX == AX_Z ? 4 : V == 4 && AX == 7 ? 3 : 1) void k_update_e(YeeArgs a, CpmlArgs c) {
     extern __shared__ float2 lds_rows[];
     touch_args();
@@ -881,9 +881,9 @@ __global__ __launch_bounds__(256, V == 4 && AX == AX_Z ? 4 : V == 4 && AX == 7 ?
     const MatIndex mat_e{a.n_mat_e == 1 ? nullptr : a.mat_e, a.mat8_e};
     if (MUR || a.n_src) {
         const Sources src{a, TAB ? lds_val : a.src_val};
-        e_body<V, AX, PHYS, TAB, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat_e, rows, c, decode<V>(a, blockIdx.x - a.n_ride), &src, a.mur_z);
+        e_body<V, AX, PHYS, TAB, MUR, RAG, STREAM>(a.g, a.Fin, a.Fout, a.Cf, mat_e, rows, c, decode<V>(a, blockIdx.x - a.n_ride), &src, a.mur_z);
     } else {
-        e_body<V, AX, PHYS, TAB, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat_e, rows, c, decode<V>(a, blockIdx.x - a.n_ride));
+        e_body<V, AX, PHYS, TAB, MUR, RAG, STREAM>(a.g, a.Fin, a.Fout, a.Cf, mat_e, rows, c, decode<V>(a, blockIdx.x - a.n_ride));
     }
 }
 
@@ -895,7 +895,7 @@ __global__ __launch_bounds__(256, V == 4 && AX == AX_Z ? 4 : V == 4 && AX == 7 ?
 // each waited for once; large ones run at memory speed (256^3, 8 layers, 64
 // boxes' table: 109 us a launch, 121 when the slabs were a launch of their
 // own and a plane's loads came in three waits).
-template <int AXI, bool MIX, bool PHYS, bool RAG>
+template <int AXI, bool MIX, bool PHYS, bool RAG, bool STREAM>
 __device__ __forceinline__ void h_group(const YeeArgs& a, const CpmlArgs& c, int bid, float2* lds_rows) {
     constexpr int V = 4;
     if (bid < a.n_ride) {
@@ -906,11 +906,11 @@ __device__ __forceinline__ void h_group(const YeeArgs& a, const CpmlArgs& c, int
     const MatIndex mat{a.n_mat_h == 1 ? nullptr : a.mat_h, a.mat8_h};
     bool inner = true;
     const Tile t = decode<V, MIX>(a, bid - a.n_ride, &inner);
-    if (!MIX || inner) h_body<V, AXI, PHYS && AXI != 0, true, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t);
-    else h_body<V, AX_X | AX_Y | AX_Z, PHYS, true, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t);
+    if (!MIX || inner) h_body<V, AXI, PHYS && AXI != 0, true, RAG, STREAM>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t);
+    else h_body<V, AX_X | AX_Y | AX_Z, PHYS, true, RAG, STREAM>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t);
 }
 
-template <int AXI, bool MIX, bool PHYS, bool MUR, bool RAG>
+template <int AXI, bool MIX, bool PHYS, bool MUR, bool RAG, bool STREAM>
 __device__ __forceinline__ void e_group(const YeeArgs& a, const CpmlArgs& c, int bid, float2* lds_rows) {
     constexpr int V = 4;
     if (bid < a.n_ride) {
@@ -924,25 +924,25 @@ __device__ __forceinline__ void e_group(const YeeArgs& a, const CpmlArgs& c, int
     bool inner = true;
     const Tile t = decode<V, MIX>(a, bid - a.n_ride, &inner);
     if (!MIX || inner)
-        e_body<V, AXI, PHYS && AXI != 0, true, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t, &ex, a.mur_z);
+        e_body<V, AXI, PHYS && AXI != 0, true, MUR, RAG, STREAM>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t, &ex, a.mur_z);
     else
-        e_body<V, AX_X | AX_Y | AX_Z, PHYS, true, MUR, RAG>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t, &ex, a.mur_z);
+        e_body<V, AX_X | AX_Y | AX_Z, PHYS, true, MUR, RAG, STREAM>(a.g, a.Fin, a.Fout, a.Cf, mat, rows, c, t, &ex, a.mur_z);
 }
 
-template <int AXI, bool PHYS, bool RAG>
+template <int AXI, bool PHYS, bool RAG, bool STREAM>
 __global__ __launch_bounds__(256, 3) void k_update_h_mix(YeeArgs a, CpmlArgs c) {
     extern __shared__ float2 lds_rows[];
     touch_args();
     if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(a.step_inc);
-    h_group<AXI, true, PHYS, RAG>(a, c, blockIdx.x, lds_rows);
+    h_group<AXI, true, PHYS, RAG, STREAM>(a, c, blockIdx.x, lds_rows);
 }
 
-template <int AXI, bool PHYS, bool MUR, bool RAG>
+template <int AXI, bool PHYS, bool MUR, bool RAG, bool STREAM>
 __global__ __launch_bounds__(256, 3) void k_update_e_mix(YeeArgs a, CpmlArgs c) {
     extern __shared__ float2 lds_rows[];
     touch_args();
     if (a.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(a.step_inc);
-    e_group<AXI, true, PHYS, MUR, RAG>(a, c, blockIdx.x, lds_rows);
+    e_group<AXI, true, PHYS, MUR, RAG, STREAM>(a, c, blockIdx.x, lds_rows);
 }
 
 // A parameter sweep: the launches of many grids as one.  A work-group finds
@@ -950,7 +950,7 @@ __global__ __launch_bounds__(256, 3) void k_update_e_mix(YeeArgs a, CpmlArgs c) 
 // (its tiles, riders and sources), with the arguments in device memory
 // instead of the kernel's; consecutive work-groups, and so one grid's,
 // share an XCD.
-template <int AXI, bool MIX, bool RAG, bool H>
+template <int AXI, bool MIX, bool RAG, bool H, bool STREAM>
 __global__ __launch_bounds__(256, MIX ? 3 : AXI != 0 ? 4 : 1) void k_update_units(UnitArgs s) {
     extern __shared__ float2 lds_rows[];
     if (s.step_inc && blockIdx.x == 0 && threadIdx.x == 0) advance(s.step_inc);
@@ -964,8 +964,8 @@ __global__ __launch_bounds__(256, MIX ? 3 : AXI != 0 ? 4 : 1) void k_update_unit
     const Units p = (Units)s.unit + ((Table)s.wg_unit)[bid];
     touch_lines<sizeof(SweepUnit)>((ArgLine)p);
     const SweepUnit& u = *(const SweepUnit*)p;
-    if constexpr (H) h_group<AXI, MIX, true, RAG>(u.a, u.c, bid - u.first, lds_rows);
-    else e_group<AXI, MIX, true, false, RAG>(u.a, u.c, bid - u.first, lds_rows);
+    if constexpr (H) h_group<AXI, MIX, true, RAG, STREAM>(u.a, u.c, bid - u.first, lds_rows);
+    else e_group<AXI, MIX, true, false, RAG, STREAM>(u.a, u.c, bid - u.first, lds_rows);
 }
 
 // The sweep's grids that need scalar lanes or have no material table, many in
@@ -1017,7 +1017,7 @@ __global__ __launch_bounds__(256) void k_update_h_sweep(SweepArgs a) {
     if constexpr (TAB) {
             rows.fill();
     }
-    h_body<V, AX, PHYS, TAB>(S.g, S.F, S.F, S.Cf, MatIndex{S.n_mat_h == 1 ? nullptr : S.mat_h, S.mat8_h}, rows, S.c, t);
+    h_body<V, AX, PHYS, TAB, false, true>(S.g, S.F, S.F, S.Cf, MatIndex{S.n_mat_h == 1 ? nullptr : S.mat_h, S.mat8_h}, rows, S.c, t);
 }
 
 template <int V, int AX, bool PHYS, bool TAB>
@@ -1031,15 +1031,17 @@ __global__ __launch_bounds__(256) void k_update_e_sweep(SweepArgs a) {
     if constexpr (TAB) {
             rows.fill();
     }
-    e_body<V, AX, PHYS, TAB>(S.g, S.F, S.F, S.Cf, MatIndex{S.n_mat_e == 1 ? nullptr : S.mat_e, S.mat8_e}, rows, S.c, t);
+    e_body<V, AX, PHYS, TAB, false, false, true>(S.g, S.F, S.F, S.Cf, MatIndex{S.n_mat_e == 1 ? nullptr : S.mat_e, S.mat8_e}, rows, S.c, t);
 }
 
 template <int V, int AX, bool PHYS, bool RAG>
 hipError_t launch_h_t(const YeeArgs& a, const CpmlArgs& c, hipStream_t s) {
     const dim3 grid(a.n_ride + a.first[a.nbox]);
-    if (a.n_mat_h > 0)
-        hipLaunchKernelGGL((k_update_h<V, AX, PHYS, true, RAG>), grid, dim3(256), 3 * a.n_mat_h * sizeof(float2), s, a,
-                           c);
+    const size_t lds = 3 * (size_t)a.n_mat_h * sizeof(float2);
+    if (a.n_mat_h > 0 && !a.stream_own)
+        hipLaunchKernelGGL((k_update_h<V, AX, PHYS, true, RAG, false>), grid, dim3(256), lds, s, a, c);
+    else if (a.n_mat_h > 0)
+        hipLaunchKernelGGL((k_update_h<V, AX, PHYS, true, RAG>), grid, dim3(256), lds, s, a, c);
     else
         hipLaunchKernelGGL((k_update_h<V, AX, PHYS, false, RAG>), grid, dim3(256), 0, s, a, c);
     return hipGetLastError();
@@ -1051,7 +1053,9 @@ hipError_t launch_e_t(const YeeArgs& a, const CpmlArgs& c, hipStream_t s) {
     const size_t lds = 3 * (size_t)a.n_mat_e * sizeof(float2);
     if (a.mur_z.on[0] || a.mur_z.on[1]) {
         if constexpr (V == 4 && !RAG) {
-            if (a.n_mat_e > 0)
+            if (a.n_mat_e > 0 && !a.stream_own)
+                hipLaunchKernelGGL((k_update_e<V, AX, PHYS, true, true, false, false>), grid, dim3(256), lds, s, a, c);
+            else if (a.n_mat_e > 0)
                 hipLaunchKernelGGL((k_update_e<V, AX, PHYS, true, true>), grid, dim3(256), lds, s, a, c);
             else
                 hipLaunchKernelGGL((k_update_e<V, AX, PHYS, false, true>), grid, dim3(256), 0, s, a, c);
@@ -1060,7 +1064,9 @@ hipError_t launch_e_t(const YeeArgs& a, const CpmlArgs& c, hipStream_t s) {
             return hipErrorInvalidValue;  // needs whole float4 lanes
         }
     }
-    if (a.n_mat_e > 0)
+    if (a.n_mat_e > 0 && !a.stream_own)
+        hipLaunchKernelGGL((k_update_e<V, AX, PHYS, true, false, RAG, false>), grid, dim3(256), lds, s, a, c);
+    else if (a.n_mat_e > 0)
         hipLaunchKernelGGL((k_update_e<V, AX, PHYS, true, false, RAG>), grid, dim3(256), lds, s, a, c);
     else
         hipLaunchKernelGGL((k_update_e<V, AX, PHYS, false, false, RAG>), grid, dim3(256), 0, s, a, c);
@@ -1074,26 +1080,32 @@ template <bool H, int V, int AX, bool PHYS, bool RAG>
 hipError_t launch_t(const YeeArgs& a, const CpmlArgs& c, hipStream_t s) {
     return H ? launch_h_t<V, AX, PHYS, RAG>(a, c, s) : launch_e_t<V, AX, PHYS, RAG>(a, c, s);
 }
-template <bool H, int AXI, bool PHYS, bool RAG>
+template <bool H, int AXI, bool PHYS, bool RAG, bool STREAM>
 hipError_t launch_mix_t(const YeeArgs& a, const CpmlArgs& c, hipStream_t s) {
     const dim3 grid(a.n_ride + a.first[a.nbox]);
     const size_t lds = 3 * (size_t)(H ? a.n_mat_h : a.n_mat_e) * sizeof(float2);
     if constexpr (H) {
-        hipLaunchKernelGGL((k_update_h_mix<AXI, PHYS, RAG>), grid, dim3(256), lds, s, a, c);
+        hipLaunchKernelGGL((k_update_h_mix<AXI, PHYS, RAG, STREAM>), grid, dim3(256), lds, s, a, c);
     } else if (a.mur_z.on[0] || a.mur_z.on[1]) {
         if constexpr (RAG) return hipErrorInvalidValue;
-        else hipLaunchKernelGGL((k_update_e_mix<AXI, PHYS, true, false>), grid, dim3(256), lds, s, a, c);
+        else hipLaunchKernelGGL((k_update_e_mix<AXI, PHYS, true, false, STREAM>), grid, dim3(256), lds, s, a, c);
     } else {
-        hipLaunchKernelGGL((k_update_e_mix<AXI, PHYS, false, RAG>), grid, dim3(256), lds, s, a, c);
+        hipLaunchKernelGGL((k_update_e_mix<AXI, PHYS, false, RAG, STREAM>), grid, dim3(256), lds, s, a, c);
     }
     return hipGetLastError();
 }
 // One launch for slabs and interior: float4 lanes and a material table only.
+template <bool H, bool RAG, bool STREAM>
+hipError_t dispatch_mix_t(const YeeArgs& a, const CpmlArgs& c, int axes, hipStream_t s) {
+    if (axes & AX_Z)
+        return c.physical ? launch_mix_t<H, AX_Z, true, RAG, STREAM>(a, c, s) : launch_mix_t<H, AX_Z, false, RAG, STREAM>(a, c, s);
+    return c.physical ? launch_mix_t<H, 0, true, RAG, STREAM>(a, c, s) : launch_mix_t<H, 0, false, RAG, STREAM>(a, c, s);
+}
+
 template <bool H, bool RAG>
 hipError_t dispatch_mix(const YeeArgs& a, const CpmlArgs& c, int axes, hipStream_t s) {
     if (a.t.vec != 4 || (H ? a.n_mat_h : a.n_mat_e) <= 0 || a.nbox < 2) return hipErrorInvalidValue;
-    if (axes & AX_Z) return c.physical ? launch_mix_t<H, AX_Z, true, RAG>(a, c, s) : launch_mix_t<H, AX_Z, false, RAG>(a, c, s);
-    return c.physical ? launch_mix_t<H, 0, true, RAG>(a, c, s) : launch_mix_t<H, 0, false, RAG>(a, c, s);
+    return a.stream_own ? dispatch_mix_t<H, RAG, true>(a, c, axes, s) : dispatch_mix_t<H, RAG, false>(a, c, axes, s);
 }
 
 template <bool H, int V, bool RAG>
@@ -1678,24 +1690,25 @@ hipError_t launch_fused(const FusedArgs& a, const CpmlArgs* c, hipStream_t s) {
     return tab ? launch_fused_t<AX_Z, false, true>(a, *c, s) : launch_fused_t<AX_Z, false, false>(a, *c, s);
 }
 
-template <bool H, int AXI, bool MIX>
-static hipError_t units_t(const UnitArgs& a, int n_wg, bool ragged, int rows, hipStream_t s) {
+template <bool H, int AXI, bool MIX, bool RAG>
+static hipError_t units_t(const UnitArgs& a, int n_wg, int rows, hipStream_t s) {
     const size_t lds = 3 * rows * sizeof(float2);
-    if (ragged) hipLaunchKernelGGL((k_update_units<AXI, MIX, true, H>), dim3(n_wg), dim3(256), lds, s, a);
-    else hipLaunchKernelGGL((k_update_units<AXI, MIX, false, H>), dim3(n_wg), dim3(256), lds, s, a);
+    if (a.stream_own) hipLaunchKernelGGL((k_update_units<AXI, MIX, RAG, H, true>), dim3(n_wg), dim3(256), lds, s, a);
+    else hipLaunchKernelGGL((k_update_units<AXI, MIX, RAG, H, false>), dim3(n_wg), dim3(256), lds, s, a);
     return hipGetLastError();
 }
 
-template <bool H>
-static hipError_t units_dispatch(const UnitArgs& a, int n_wg, int axes, bool ragged, int rows, hipStream_t s) {
+template <bool H, bool RAG>
+static hipError_t units_dispatch(const UnitArgs& a, int n_wg, int axes, int rows, hipStream_t s) {
     if (axes & AX_MIX)
-        return axes & AX_Z ? units_t<H, AX_Z, true>(a, n_wg, ragged, rows, s) : units_t<H, 0, true>(a, n_wg, ragged, rows, s);
-    return axes & AX_Z ? units_t<H, AX_Z, false>(a, n_wg, ragged, rows, s) : units_t<H, 0, false>(a, n_wg, ragged, rows, s);
+        return axes & AX_Z ? units_t<H, AX_Z, true, RAG>(a, n_wg, rows, s) : units_t<H, 0, true, RAG>(a, n_wg, rows, s);
+    return axes & AX_Z ? units_t<H, AX_Z, false, RAG>(a, n_wg, rows, s) : units_t<H, 0, false, RAG>(a, n_wg, rows, s);
 }
 
 hipError_t launch_units(bool h, const UnitArgs& a, int n_wg, int axes, bool ragged, int rows, hipStream_t s) {
     if (n_wg <= 0) return hipSuccess;
-    return h ? units_dispatch<true>(a, n_wg, axes, ragged, rows, s) : units_dispatch<false>(a, n_wg, axes, ragged, rows, s);
+    if (ragged) return h ? units_dispatch<true, true>(a, n_wg, axes, rows, s) : units_dispatch<false, true>(a, n_wg, axes, rows, s);
+    return h ? units_dispatch<true, false>(a, n_wg, axes, rows, s) : units_dispatch<false, false>(a, n_wg, axes, rows, s);
 }
 
 // Sweep launches: physical CPML only (every structure of a sweep carries the

@@ -44,3 +44,16 @@ def test_row_lengths_that_are_no_power_of_two(shape):
         sc = Scenario(f"rows_{nx}x{ny}x{nz}", shape, 1e-3, 30, materials=[(4.0, 1.0, 0.02, 0.0, (0, nx, 1, ny, 3, nz // 2))],
                       excitations=[(src, 2, True, gauss_ref(20e9))], probes=[src], cpml=cpml)
         assert_parity(run_pair(sc), sc.name)
+
+
+
+@pytest.mark.parametrize("shape,layers", [((108, 108, 112), None), ((101, 99, 102), (5,) * 6)], ids=["plain", "cpml"])
+def test_state_held_by_the_caches(shape, layers):
+    """Grids whose state outgrows the L2s but not the cache behind them load
+    their own old values without the streaming hint."""
+    nx, ny, nz = shape
+    src = (nx // 2, ny // 2, nz // 2)
+    mats = [(2.5, 1.0, 0.01, 0.0, (nx // 4, nx // 2, ny // 4, ny // 2, nz // 4, nz // 2))]
+    sc = Scenario(f"state_{nx}x{ny}x{nz}", shape, 1e-3, 6, materials=mats,
+                  excitations=[(src, 2, True, gauss_ref(20e9))], probes=[src], cpml=layers and {"layers": layers})
+    assert_parity(run_pair(sc), sc.name)
