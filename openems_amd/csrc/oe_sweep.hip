@@ -10,7 +10,8 @@
 // need scalar lanes or have no material table go in launches per kernel
 // variant beside it, sources and DFTs too large to ride in a point launch
 // after it.  The step sequence between two termination checks is captured
-// once as a HIP graph and replayed.  Each structure stops on its own energy decay or at
+// once as a HIP graph and replayed; structures that together outgrow the
+// cache behind the L2s run it in sets that do not, one set after the other.  Each structure stops on its own energy decay or at
 // max_steps; stopped structures leave the tables.  Checks fall on the
 // engines' absolute timesteps and the peak is kept in the engine, so a run
 // can continue where an earlier one stopped with the same result as one run.
@@ -60,6 +61,18 @@ struct Group {      // one launch: all boxes of one (vec, axes) kind
     const int* d_wg = nullptr;
 };
 
+// Structures stepped together from check to check.
+struct Set {
+    std::vector<int> ids;
+    std::vector<Group> groups;
+    std::vector<UnitGroup> unit_groups;
+    int stream_own = 1;
+    uint64_t* step = nullptr;         // step under way, steps whose E half has begun
+    int first_point = 0, n_point = 0;  // its structures in the point launch's tables
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+};
+
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 #define HIP_RET(expr)                          \
@@ -75,10 +88,9 @@ struct oe_sweep {
     hipStream_t stream = nullptr;
     std::vector<Item> items;
     // planes per work-group along i: 32 microstrips of 0.2 to 1.3 M cells
-    // take 317 / 305 / 306 / 320 us a step at 1 / 2 / 4 / 8
+    // take 301 / 295 / 299 / 324 us a step at 1 / 2 / 4 / 8
     int ci = 2;
     int xcd_remap = 1;
-    int stream_own = 1;
     // largest material table per half of the structures outside the units
     // (0: some structure reads its coefficient arrays, so every one does)
     int rows_h = 0, rows_e = 0;
@@ -88,14 +100,11 @@ struct oe_sweep {
     DevBuf structs, tables, rides, excs, exc_first, exc_serial, exc_samples, dfts, dft_of, ids, partials, energy, step;
     double* energy_host = nullptr;
     size_t energy_host_n = 0;
-    std::vector<Group> groups;
-    std::vector<UnitGroup> unit_groups;
+    std::vector<Set> sets;
     std::vector<Ride> ride_host;  // per structure, of the run (n_wg 0: none)
     // per structure, the (timestep, E + H energy) of every check of the last run
     std::vector<std::vector<std::pair<uint64_t, double>>> history;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    int graph_steps = 0;
+    int graph_steps = 0;  // of every set's graph (0: not captured)
     // The CPML slab launches of a half-step run beside the interior launch,
     // each on a side stream of its own (forked and joined by events; graph
     // branches under capture).  OE_SWEEP_OVERLAP=1: all slab launches on one
@@ -105,10 +114,12 @@ struct oe_sweep {
     hipEvent_t ev_fork = nullptr, ev_join[3] = {nullptr, nullptr, nullptr};
 
     void drop_graph() {
-        if (exec) (void)hipGraphExecDestroy(exec);
-        if (graph) (void)hipGraphDestroy(graph);
-        exec = nullptr;
-        graph = nullptr;
+        for (Set& t : sets) {
+            if (t.exec) (void)hipGraphExecDestroy(t.exec);
+            if (t.graph) (void)hipGraphDestroy(t.graph);
+            t.exec = nullptr;
+            t.graph = nullptr;
+        }
         graph_steps = 0;
     }
     ~oe_sweep() {
@@ -196,47 +207,87 @@ void structure_boxes(const oe_sweep* sw, int sid, const Item& it, std::vector<Gr
     add((m & 48) ? AX_Z : 0, ix0, ix1, jy0, jy1);
 }
 
-// Launch tables of the active structures, uploaded into sw->tables.
-oe_status build_tables(oe_sweep* sw, const std::vector<int>& active) {
-    sw->groups.clear();
-    sw->unit_groups.clear();
-    size_t state = 0;
-    for (int sid : active) state += grid_state(sw->items[sid].eng, sw->items[sid].cpml ? &sw->items[sid].cpml->cpml : nullptr);
-    sw->stream_own = stream_state(state);
-    for (int sid : active) {
+// The active structures in sets.  State comes faster from the 256 MB behind
+// the L2s than from memory, so where all structures together outgrow it and
+// there are several steps from check to check, they are dealt to sets of up
+// to 200 MB (32 microstrips of 450 MB: 318 us a step in one set, 294 in three,
+// 357 in sets of 80 MB, whose launches are too small; 64 of 930 MB: 654 in
+// one, 627 in sets of 240 MB, 611 in sets of 200).
+void deal_sets(oe_sweep* sw, const std::vector<int>& active, uint64_t check) {
+    sw->drop_graph();
+    sw->sets.clear();
+    auto state = [&](int sid) {
         const Item& it = sw->items[sid];
-        if (!it.unit) {
-            structure_boxes(sw, sid, it, sw->groups);
-            continue;
+        return grid_state(it.eng, it.cpml ? &it.cpml->cpml : nullptr);
+    };
+    size_t total = 0;
+    for (int sid : active) total += state(sid);
+    const size_t most = (size_t)200 << 20;
+    const bool deal = stream_state(total) && total > most && check >= 8;
+    const size_t target = deal ? total / ((total + most - 1) / most) : total;
+    size_t held = 0;
+    for (int sid : active) {
+        const size_t b = state(sid);
+        if (sw->sets.empty() || (deal && held > 0 && (held + b > most || held + b / 2 > target))) {
+            sw->sets.emplace_back();
+            held = 0;
         }
-        SweepUnit u{};
-        int axes = 0;
-        if (!one_launch_plan(it.eng, it.cpml ? &it.cpml->cpml : nullptr, sw->ci, &u.a, &axes))
-            return fail(OE_ERR_CONFIG, "structure %d has no single launch", sid);
-        if (it.cpml) u.c = it.cpml->cpml;
-        u.a.xcd_remap = 0;
-        const Ride& r = sw->ride_host[sid];
-        if (r.n_wg > 0) {
-            u.a.ride = sw->rides.as<Ride>() + sid;
-            u.a.n_ride = r.n_wg;
-            u.a.src_val = r.src_val;
-            u.a.n_src = r.n_src;
-            for (int q = 0; q < r.n_src; ++q) u.a.src_idx[q] = (uint32_t)(it.exc_off[q] % it.eng->g.N);
+        sw->sets.back().ids.push_back(sid);
+        held += b;
+        sw->sets.back().stream_own = stream_state(held);
+    }
+}
+
+// Launch tables of the active structures, uploaded into sw->tables, and the
+// sets' step counters after `done` steps.
+oe_status build_tables(oe_sweep* sw, const std::vector<int>& active, uint64_t check, uint64_t done) {
+    deal_sets(sw, active, check);
+    const size_t n_sets = sw->sets.size();
+    if (sw->step.bytes < 2 * n_sets * sizeof(uint64_t)) HIP_OK(sw->step.alloc(2 * n_sets * sizeof(uint64_t)));
+    std::vector<uint64_t> counters;
+    for (size_t q = 0; q < n_sets; ++q) {
+        sw->sets[q].step = sw->step.as<uint64_t>() + 2 * q;
+        counters.push_back(done - 1);  // -1 at first: the first H launch makes it 0
+        counters.push_back(done);
+    }
+    for (Set& set : sw->sets) {
+        for (int sid : set.ids) {
+            const Item& it = sw->items[sid];
+            sw->ride_host[sid].step_a = set.step;
+            sw->ride_host[sid].step_b = set.step + 1;
+            if (!it.unit) {
+                structure_boxes(sw, sid, it, set.groups);
+                continue;
+            }
+            SweepUnit u{};
+            int axes = 0;
+            if (!one_launch_plan(it.eng, it.cpml ? &it.cpml->cpml : nullptr, sw->ci, &u.a, &axes))
+                return fail(OE_ERR_CONFIG, "structure %d has no single launch", sid);
+            if (it.cpml) u.c = it.cpml->cpml;
+            u.a.xcd_remap = 0;
+            const Ride& r = sw->ride_host[sid];
+            if (r.n_wg > 0) {
+                u.a.ride = sw->rides.as<Ride>() + sid;
+                u.a.n_ride = r.n_wg;
+                u.a.src_val = r.src_val;
+                u.a.n_src = r.n_src;
+                for (int q = 0; q < r.n_src; ++q) u.a.src_idx[q] = (uint32_t)(it.exc_off[q] % it.eng->g.N);
+            }
+            UnitGroup* G = nullptr;
+            for (auto& q : set.unit_groups)
+                if (q.axes == axes && q.ragged == (u.a.ragged != 0)) G = &q;
+            if (!G) {
+                set.unit_groups.emplace_back();
+                G = &set.unit_groups.back();
+                G->axes = axes;
+                G->ragged = u.a.ragged != 0;
+            }
+            u.first = (int)G->wg_unit.size();
+            G->wg_unit.insert(G->wg_unit.end(), u.a.n_ride + u.a.first[u.a.nbox], (int)G->units.size());
+            G->units.push_back(u);
+            G->rows_h = std::max(G->rows_h, u.a.n_mat_h);
+            G->rows_e = std::max(G->rows_e, u.a.n_mat_e);
         }
-        UnitGroup* G = nullptr;
-        for (auto& q : sw->unit_groups)
-            if (q.axes == axes && q.ragged == (u.a.ragged != 0)) G = &q;
-        if (!G) {
-            sw->unit_groups.emplace_back();
-            G = &sw->unit_groups.back();
-            G->axes = axes;
-            G->ragged = u.a.ragged != 0;
-        }
-        u.first = (int)G->wg_unit.size();
-        G->wg_unit.insert(G->wg_unit.end(), u.a.n_ride + u.a.first[u.a.nbox], (int)G->units.size());
-        G->units.push_back(u);
-        G->rows_h = std::max(G->rows_h, u.a.n_mat_h);
-        G->rows_e = std::max(G->rows_e, u.a.n_mat_e);
     }
     std::vector<char> host;
     auto put = [&](const void* p, size_t bytes) {
@@ -246,26 +297,34 @@ oe_status build_tables(oe_sweep* sw, const std::vector<int>& active) {
         return at;
     };
     std::vector<std::pair<size_t, size_t>> at;
-    for (const auto& G : sw->groups) {
-        const size_t b = put(G.boxes.data(), G.boxes.size() * sizeof(SweepBox));
-        at.push_back({b, put(G.wg_box.data(), G.wg_box.size() * sizeof(int))});
-    }
-    for (const auto& G : sw->unit_groups) {
-        const size_t b = put(G.units.data(), G.units.size() * sizeof(SweepUnit));
-        at.push_back({b, put(G.wg_unit.data(), G.wg_unit.size() * sizeof(int))});
+    for (const Set& set : sw->sets) {
+        for (const auto& G : set.groups) {
+            const size_t b = put(G.boxes.data(), G.boxes.size() * sizeof(SweepBox));
+            at.push_back({b, put(G.wg_box.data(), G.wg_box.size() * sizeof(int))});
+        }
+        for (const auto& G : set.unit_groups) {
+            const size_t b = put(G.units.data(), G.units.size() * sizeof(SweepUnit));
+            at.push_back({b, put(G.wg_unit.data(), G.wg_unit.size() * sizeof(int))});
+        }
     }
     if (sw->tables.bytes < host.size()) HIP_OK(sw->tables.alloc(host.size()));
     HIP_OK(hipMemcpyAsync(sw->tables.p, host.data(), host.size(), hipMemcpyHostToDevice, sw->stream));
+    HIP_OK(hipMemcpyAsync(sw->step.p, counters.data(), counters.size() * sizeof(uint64_t), hipMemcpyHostToDevice,
+                          sw->stream));
+    HIP_OK(hipMemcpyAsync(sw->rides.p, sw->ride_host.data(), sw->ride_host.size() * sizeof(Ride), hipMemcpyHostToDevice,
+                          sw->stream));
     HIP_OK(hipStreamSynchronize(sw->stream));
     const char* base = sw->tables.as<char>();
     size_t q = 0;
-    for (auto& G : sw->groups) {
-        G.d_box = reinterpret_cast<const SweepBox*>(base + at[q].first);
-        G.d_wg = reinterpret_cast<const int*>(base + at[q++].second);
-    }
-    for (auto& G : sw->unit_groups) {
-        G.d_unit = reinterpret_cast<const SweepUnit*>(base + at[q].first);
-        G.d_wg = reinterpret_cast<const int*>(base + at[q++].second);
+    for (Set& set : sw->sets) {
+        for (auto& G : set.groups) {
+            G.d_box = reinterpret_cast<const SweepBox*>(base + at[q].first);
+            G.d_wg = reinterpret_cast<const int*>(base + at[q++].second);
+        }
+        for (auto& G : set.unit_groups) {
+            G.d_unit = reinterpret_cast<const SweepUnit*>(base + at[q].first);
+            G.d_wg = reinterpret_cast<const int*>(base + at[q++].second);
+        }
     }
     return OE_OK;
 }
@@ -274,19 +333,19 @@ oe_status build_tables(oe_sweep* sw, const std::vector<int>& active) {
 // half write disjoint cells and read only the other field, so with
 // sw->overlap the slab groups (x/y CPML faces) go to side streams, forked
 // from and joined back into the sweep stream around its interior launch.
-hipError_t yee_half(oe_sweep* sw, bool h) {
-    uint64_t* inc = sw->step.as<uint64_t>() + (h ? 0 : 1);
-    for (const auto& G : sw->unit_groups) {
-        const UnitArgs a{G.d_unit, G.d_wg, sw->xcd_remap, sw->stream_own, inc};
+hipError_t yee_half(oe_sweep* sw, const Set& set, bool h) {
+    uint64_t* inc = set.step + (h ? 0 : 1);
+    for (const auto& G : set.unit_groups) {
+        const UnitArgs a{G.d_unit, G.d_wg, sw->xcd_remap, set.stream_own, inc};
         inc = nullptr;
         HIP_RET(launch_units(h, a, (int)G.wg_unit.size(), G.axes, G.ragged, h ? G.rows_h : G.rows_e, sw->stream));
     }
-    if (sw->groups.empty()) return hipSuccess;
-    const bool ov = sw->overlap && sw->groups.size() > 1;
+    if (set.groups.empty()) return hipSuccess;
+    const bool ov = sw->overlap && set.groups.size() > 1;
     const int n_side = sw->overlap == 2 ? 3 : 1;
     int used = 0;  // side streams forked so far
     if (ov) HIP_RET(hipEventRecord(sw->ev_fork, sw->stream));
-    for (const auto& G : sw->groups) {
+    for (const auto& G : set.groups) {
         SweepArgs a{};
         a.st = sw->structs.as<SweepStruct>();
         a.box = G.d_box;
@@ -314,41 +373,42 @@ hipError_t yee_half(oe_sweep* sw, bool h) {
     return hipSuccess;
 }
 
-// Point and DFT tables of the active structures.
-struct StepTables {
-    int n_struct = 0;  // structures with sources or a DFT of the point launch
-};
-
-oe_status build_step_tables(oe_sweep* sw, const std::vector<int>& active, StepTables& t) {
+// Point and DFT tables of the active structures, set by set.
+oe_status build_step_tables(oe_sweep* sw, const std::vector<int>& active) {
     std::vector<SweepExc> ex;
     std::vector<int> first{0};
     std::vector<int> serial, dft_of;
     std::vector<SweepDft> dft;
     int n = 0;
-    for (int sid : active) {
-        const Item& it = sw->items[sid];
-        const bool own_exc = !it.fold && !it.exc.empty(), own_dft = it.port && !it.ride_port;
-        if (!own_exc && !own_dft) continue;
-        ++n;
-        if (own_exc)
-            for (const auto& e : it.exc) ex.push_back(e);
-        first.push_back((int)ex.size());
-        // sources on one cell apply in list order: then one thread does them all
-        std::vector<const float*> cells;
-        if (own_exc)
-            for (const auto& e : it.exc) cells.push_back(e.target);
-        std::sort(cells.begin(), cells.end());
-        serial.push_back(std::adjacent_find(cells.begin(), cells.end()) != cells.end() ? 1 : 0);
-        dft_of.push_back(own_dft ? (int)dft.size() : -1);
-        if (own_dft) {
-            SweepDft d{};
-            d.F = it.eng->F;
-            d.N = it.eng->g.N;
-            d.d = it.port->dft;
-            d.sample0 = it.port->dft_count;
-            d.t0 = (double)it.eng->timestep;
-            dft.push_back(d);
-        }
+    for (Set& set : sw->sets) {
+        set.first_point = n;
+        set.n_point = 0;
+        for (int sid : set.ids) {
+            const Item& it = sw->items[sid];
+            const bool own_exc = !it.fold && !it.exc.empty(), own_dft = it.port && !it.ride_port;
+            if (!own_exc && !own_dft) continue;
+            ++n;
+            ++set.n_point;
+            if (own_exc)
+                for (const auto& e : it.exc) ex.push_back(e);
+            first.push_back((int)ex.size());
+            // sources on one cell apply in list order: then one thread does them all
+            std::vector<const float*> cells;
+            if (own_exc)
+                for (const auto& e : it.exc) cells.push_back(e.target);
+            std::sort(cells.begin(), cells.end());
+            serial.push_back(std::adjacent_find(cells.begin(), cells.end()) != cells.end() ? 1 : 0);
+            dft_of.push_back(own_dft ? (int)dft.size() : -1);
+            if (own_dft) {
+                SweepDft d{};
+                d.F = it.eng->F;
+                d.N = it.eng->g.N;
+                d.d = it.port->dft;
+                d.sample0 = it.port->dft_count;
+                d.t0 = (double)it.eng->timestep;
+                dft.push_back(d);
+            }
+    }
     }
     if (sw->excs.bytes < std::max<size_t>(ex.size(), 1) * sizeof(SweepExc))
         HIP_OK(sw->excs.alloc(std::max<size_t>(ex.size(), 1) * sizeof(SweepExc)));
@@ -372,41 +432,41 @@ oe_status build_step_tables(oe_sweep* sw, const std::vector<int>& active, StepTa
     if (!active.empty())
         HIP_OK(hipMemcpyAsync(sw->ids.p, active.data(), active.size() * sizeof(int), hipMemcpyHostToDevice, sw->stream));
     HIP_OK(hipStreamSynchronize(sw->stream));
-    t.n_struct = n;
     return OE_OK;
 }
 
-// One timestep of all active structures (no host synchronisation; capturable).
-hipError_t sweep_step(oe_sweep* sw, const StepTables& t, double dt) {
-    hipError_t e;
+// One timestep of a set's structures (no host synchronisation; capturable).
+hipError_t sweep_step(oe_sweep* sw, const Set& set, double dt) {
     // the first H launch advances the step counter (from -1: step st reads st)
-    if ((e = yee_half(sw, true)) != hipSuccess) return e;
-    if ((e = yee_half(sw, false)) != hipSuccess) return e;
-    if (t.n_struct == 0) return hipSuccess;
-    return launch_sweep_point(sw->excs.as<SweepExc>(), sw->exc_first.as<int>(), sw->exc_serial.as<int>(),
-                              sw->dfts.as<SweepDft>(), sw->dft_of.as<int>(), t.n_struct, sw->step.as<uint64_t>(), dt,
-                              sw->stream);
+    HIP_RET(yee_half(sw, set, true));
+    HIP_RET(yee_half(sw, set, false));
+    if (set.n_point == 0) return hipSuccess;
+    return launch_sweep_point(sw->excs.as<SweepExc>(), sw->exc_first.as<int>() + set.first_point,
+                              sw->exc_serial.as<int>() + set.first_point, sw->dfts.as<SweepDft>(),
+                              sw->dft_of.as<int>() + set.first_point, set.n_point, set.step, dt, sw->stream);
 }
 
-oe_status capture(oe_sweep* sw, const StepTables& t, double dt, int steps) {
+oe_status capture(oe_sweep* sw, double dt, int steps) {
     sw->drop_graph();
-    HIP_OK(hipStreamBeginCapture(sw->stream, hipStreamCaptureModeThreadLocal));
-    hipError_t err = hipSuccess;
-    for (int q = 0; q < steps && err == hipSuccess; ++q) err = sweep_step(sw, t, dt);
-    hipGraph_t g = nullptr;
-    const hipError_t ec = hipStreamEndCapture(sw->stream, &g);
-    if (err != hipSuccess || ec != hipSuccess) {
-        if (g) (void)hipGraphDestroy(g);
-        return fail(OE_ERR_DEVICE, "sweep graph capture failed: %s", hipGetErrorString(err != hipSuccess ? err : ec));
+    for (Set& set : sw->sets) {
+        HIP_OK(hipStreamBeginCapture(sw->stream, hipStreamCaptureModeThreadLocal));
+        hipError_t err = hipSuccess;
+        for (int q = 0; q < steps && err == hipSuccess; ++q) err = sweep_step(sw, set, dt);
+        hipGraph_t g = nullptr;
+        const hipError_t ec = hipStreamEndCapture(sw->stream, &g);
+        if (err != hipSuccess || ec != hipSuccess) {
+            if (g) (void)hipGraphDestroy(g);
+            return fail(OE_ERR_DEVICE, "sweep graph capture failed: %s", hipGetErrorString(err != hipSuccess ? err : ec));
+        }
+        set.graph = g;
+        HIP_OK(hipGraphInstantiate(&set.exec, set.graph, nullptr, nullptr, 0));
     }
-    sw->graph = g;
-    HIP_OK(hipGraphInstantiate(&sw->exec, sw->graph, nullptr, nullptr, 0));
     sw->graph_steps = steps;
     return OE_OK;
 }
 
 // The riders of the run: port DFTs and source values of the structures in
-// units.  Samples are on the device (it.exc[q].samples).
+// units (build_tables adds the set's counters and uploads them).  Samples are on the device (it.exc[q].samples).
 oe_status build_rides(oe_sweep* sw, uint64_t t0, double dt) {
     const size_t n = sw->items.size();
     sw->ride_host.assign(n, Ride{});
@@ -437,8 +497,6 @@ oe_status build_rides(oe_sweep* sw, uint64_t t0, double dt) {
         r.g = it.eng->g;
         r.t0 = (double)t0;
         r.dt = dt;
-        r.step_a = sw->step.as<uint64_t>();
-        r.step_b = sw->step.as<uint64_t>() + 1;
         if (it.fold) {
             r.n_src = (int)it.exc.size();
             r.src = reinterpret_cast<const PointExc*>(sw->rides.as<char>() + src_off) + at;
@@ -457,7 +515,6 @@ oe_status build_rides(oe_sweep* sw, uint64_t t0, double dt) {
         if (it.ride_port) r.dft[r.n_dft++] = RideDft{it.port->dft, it.port->dft_count};
         r.first_ade = r.first_mur = r.n_wg = r.first_dft + r.n_dft;
     }
-    HIP_OK(hipMemcpyAsync(sw->rides.p, sw->ride_host.data(), n * sizeof(Ride), hipMemcpyHostToDevice, sw->stream));
     if (!src.empty())
         HIP_OK(hipMemcpyAsync(sw->rides.as<char>() + src_off, src.data(), src.size() * sizeof(PointExc),
                               hipMemcpyHostToDevice, sw->stream));
@@ -517,7 +574,6 @@ oe_status oe_sweep_create(int device, oe_sweep** out) {
             HIP_OK(hipEventCreateWithFlags(&sw->ev_join[q], hipEventDisableTiming));
         }
     }
-    HIP_OK(sw->step.alloc(2 * sizeof(uint64_t)));  // step under way, steps whose E half has begun
     *out = sw.release();
     return OE_OK;
 }
@@ -616,8 +672,6 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
                                       it.samples[q].size() * sizeof(float), hipMemcpyHostToDevice, sw->stream));
             off += it.samples[q].size();
         }
-    HIP_OK(hipMemsetAsync(sw->step.p, 0xff, sizeof(uint64_t), sw->stream));  // -1: the first step's H launch makes it 0
-    HIP_OK(hipMemsetAsync(sw->step.as<uint64_t>() + 1, 0, sizeof(uint64_t), sw->stream));
     OE_TRY(build_rides(sw, T0, dt));
     sw->rows_e = sw->rows_h = 0;
     bool all_e = true, all_h = true;
@@ -642,8 +696,8 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
     }
 
     // The i-depth of the work-groups, timed over the run's own first steps
-    // after its first check (no result depends on it): TUNE_STEPS of each
-    // candidate, one more before them.
+    // after its first check (no result depends on it), TUNE_STEPS of each
+    // candidate.
     struct Events {
         hipEvent_t a = nullptr, b = nullptr;
         ~Events() {
@@ -651,7 +705,7 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
             if (b) (void)hipEventDestroy(b);
         }
     } ev;
-    constexpr int TUNE_STEPS = 4;
+    constexpr int TUNE_STEPS = 5;
     int tune_next = cfg->autotune ? 0 : 4, tune_best = 0;
     if (cfg->autotune) {
         HIP_OK(hipEventCreate(&ev.a));
@@ -659,11 +713,9 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
         for (double& ms : sw->tune_ms) ms = 0.0;
     }
 
-    OE_TRY(build_tables(sw, active));
-    StepTables tab;
-    OE_TRY(build_step_tables(sw, active, tab));
+    OE_TRY(build_tables(sw, active, check, 0));
+    OE_TRY(build_step_tables(sw, active));
     uint64_t done = 0;
-    bool dirty = false;  // tables changed since the last capture
     sw->drop_graph();
     while (!active.empty() && done < cfg->max_steps) {
         // Energy is sampled after the steps whose timestep is a multiple of
@@ -674,24 +726,25 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
         const uint64_t next_check = (ts + check - 1) / check * check;  // first check at or after it
         const uint64_t chunk = std::min<uint64_t>(next_check - ts + 1, cfg->max_steps - done);
         uint64_t ran = 0;
-        while (tune_next < 4 && done > 0 && chunk - ran > TUNE_STEPS) {
+        while (tune_next < 4 && done > 0 && chunk - ran >= TUNE_STEPS) {
             const int q = tune_next++;
             sw->ci = sw->tune_ci[q];
-            OE_TRY(build_tables(sw, active));
-            HIP_OK(sweep_step(sw, tab, dt));
+            OE_TRY(build_tables(sw, active, check, done + ran));
+            OE_TRY(build_step_tables(sw, active));
             HIP_OK(hipEventRecord(ev.a, sw->stream));
-            for (int w = 0; w < TUNE_STEPS; ++w) HIP_OK(sweep_step(sw, tab, dt));
+            for (const Set& set : sw->sets)
+                for (int w = 0; w < TUNE_STEPS; ++w) HIP_OK(sweep_step(sw, set, dt));
             HIP_OK(hipEventRecord(ev.b, sw->stream));
             HIP_OK(hipEventSynchronize(ev.b));
             float ms = 0.f;
             HIP_OK(hipEventElapsedTime(&ms, ev.a, ev.b));
             sw->tune_ms[q] = ms / TUNE_STEPS;
             if (sw->tune_ms[q] < sw->tune_ms[tune_best]) tune_best = q;
-            ran += TUNE_STEPS + 1;
-            if (tune_next == 4 || chunk - ran <= TUNE_STEPS) {
+            ran += TUNE_STEPS;
+            if (tune_next == 4 || chunk - ran < TUNE_STEPS) {
                 sw->ci = sw->tune_ci[tune_best];
-                OE_TRY(build_tables(sw, active));
-                dirty = true;
+                OE_TRY(build_tables(sw, active, check, done + ran));
+                OE_TRY(build_step_tables(sw, active));
             }
         }
         if (cfg->use_graph && chunk == check && done > 0 && ran == 0) {
@@ -702,13 +755,12 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
             int gsteps = 1;
             for (int q = 1; q <= 25; ++q)
                 if (check % q == 0) gsteps = q;
-            if (!sw->exec || dirty || sw->graph_steps != gsteps) {
-                OE_TRY(capture(sw, tab, dt, gsteps));
-                dirty = false;
-            }
-            for (uint64_t q = 0; q < chunk / gsteps; ++q) HIP_OK(hipGraphLaunch(sw->exec, sw->stream));
+            if (sw->graph_steps != gsteps) OE_TRY(capture(sw, dt, gsteps));
+            for (const Set& set : sw->sets)
+                for (uint64_t q = 0; q < chunk / gsteps; ++q) HIP_OK(hipGraphLaunch(set.exec, sw->stream));
         } else {
-            for (uint64_t q = ran; q < chunk; ++q) HIP_OK(sweep_step(sw, tab, dt));
+            for (const Set& set : sw->sets)
+                for (uint64_t q = ran; q < chunk; ++q) HIP_OK(sweep_step(sw, set, dt));
         }
         done += chunk;
         const uint64_t cur = T0 + done - 1;  // timestep of the last step run
@@ -742,9 +794,8 @@ oe_status oe_sweep_run(oe_sweep* sw, const oe_sweep_config* cfg, oe_sweep_entry*
             OE_TRY(ride_last(sw, stopping));
             active.swap(keep);
             if (!active.empty()) {
-                OE_TRY(build_tables(sw, active));
-                OE_TRY(build_step_tables(sw, active, tab));
-                dirty = true;
+                OE_TRY(build_tables(sw, active, check, done));
+                OE_TRY(build_step_tables(sw, active));
             }
         }
     }

@@ -242,3 +242,43 @@ def test_kinds_of_structures_together(check, graph, tune):
         if dft:
             assert np.array_equal(got[q][2].series(), dft.series()), kinds[q]
             assert np.array_equal(got[q][2].dft_values(), dft.dft_values()), kinds[q]
+
+
+@pytest.mark.parametrize("check", [25, 4])
+def test_structures_dealt_to_sets(check):
+    """Structures that together outgrow the cache behind the L2s (10 of 1.2 M
+    cells, 290 MB) run from check to check in sets, unless there are few
+    steps in between; some stop at different checks, after which the rest are
+    dealt anew.  Each equals its own engine's run bit for bit."""
+    from openems_amd import HipEngine, Operator, ScheduledExcitation
+
+    steps, n = 60, 10
+    pulse = np.zeros(steps, np.float32)
+    pulse[:4] = (1.0, 2.0, -1.0, 0.5)
+    f = np.linspace(2e9, 20e9, 3)
+
+    def build(q):
+        op = Operator.uniform(100, 110, 108, 0.5e-3)
+        # lossy to a different degree: decays at different checks
+        op.set_material(2.0, 1.0, 0.02 * q * q, 0.0, (0, 100, 0, 110, 0, 108))
+        eng = HipEngine(op)
+        dft = eng.dft([[(2, 50, 55, 50 + q, 1.0)], [(4, 52, 55, 54, 1.0)]], f, record_steps=steps)
+        return eng, dft, [ScheduledExcitation((50, 55, 54), 2, pulse, True)]
+
+    sw = Sweep()
+    got = [build(q) for q in range(n)]
+    for eng, dft, exc in got:
+        sw.add(eng, None, dft, exc)
+    res = sw.run(steps, energy_decay_db=3.0, check_interval=check)
+    for q in range(n):
+        eng, dft, exc = build(q)
+        r = eng.run_batch(EngineBatch(max_timesteps=steps, excitations=exc, extensions=[dft], energy_decay_db=3.0,
+                                      check_interval=check, sample_interval=check, track_peak=True,
+                                      persistent_peak=True))
+        assert res[q].timesteps_executed == r.timesteps_executed
+        assert res[q].termination_reason == r.termination_reason
+        for a, b in zip(got[q][0].read_fields(), eng.read_fields()):
+            assert np.array_equal(a, b)
+        assert np.array_equal(got[q][1].series(), dft.series())
+        assert np.array_equal(got[q][1].dft_values(), dft.dft_values())
+    say(f"[sweep] sets, check {check}: steps {[r.timesteps_executed for r in res]}")
