@@ -765,7 +765,7 @@ __device__ __forceinline__ void gather_nl(const FaceDev* __restrict__ fc, int nf
     }
 }
 
-// Surfaces of more than MAX_FACES faces: the sums of one set of them.
+// Surfaces of more than one set of faces: the sums of one set.
 __global__ __launch_bounds__(256) void k_nf2ff_gather(const FaceDev* __restrict__ fc, int nf, double* nl, int first,
                                                       size_t n_ang) {
     const size_t a = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -1097,61 +1097,66 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
     size_t rows[2];
     for (int l = 0; l < 2; ++l)
         rows[l] = std::min(std::max<size_t>(GBM, budget / Nmax[l] / GBM * GBM), round_up(2 * (size_t)Umax[l], GBM));
-    // sets of up to MAX_FACES faces share the launches and, from one set to
-    // the next, the buffers
-    const int n_sets = (nf + MAX_FACES - 1) / MAX_FACES;
-    std::vector<int> set_chunks(n_sets, 0);
-    size_t n_table = 0;
-    for (int q = 0; q < nf; ++q) {
-        Plan& pl = plans[q];
-        pl.chunk = (int)(rows[pl.lane] / 2);
-        pl.n_chunks = (C.ax[pl.p].U + pl.chunk - 1) / pl.chunk;
-        int& m = set_chunks[q / MAX_FACES];
-        m = std::max(m, pl.n_chunks);
-    }
-    for (int m : set_chunks) n_table += (size_t)m * MAX_FACES;
-
-    // device workspace: the tables (uploaded in one copy), then results,
-    // partials and per face slot the operands
-    const size_t pblocks = (n_ang + 255) / 256;
-    const size_t face_off = 0, chunk_off = round_up(nf * sizeof(FaceDev), 64);
-    const size_t coord_off = round_up(chunk_off + n_table * sizeof(ChunkDev), 64);
-    const size_t up_bytes = coord_off + coord_len * sizeof(double);
-    size_t off = round_up(up_bytes, 256);
-    const size_t out_off = off;  // E_theta, E_phi, block maxima of U, power partials
-    const size_t out_len = 4 * n_ang + pblocks + blocks;
-    off = round_up(off + out_len * sizeof(double), 256);
-    const size_t nl_off = off;
-    if (n_sets > 1) off = round_up(off + 12 * n_ang * sizeof(double), 256);
-    const size_t pmax_off = off;
-    off = round_up(off + blocks * sizeof(float), 256);
-    const size_t bsc_off = off;
-    off = round_up(off + 2 * (size_t)nf * sizeof(float), 256);
+    // Sets of up to `per` faces share the launches and, from one set to the
+    // next, the buffers: as many as MAX_FACES, fewer where the device has no
+    // room for their buffers at once.
     struct Slot {
         size_t B = 0, A = 0, G = 0, S = 0, b = 0, a = 0, g = 0;
     } slot[MAX_FACES];
-    for (int q = 0; q < nf; ++q) {
-        const Plan& pl = plans[q];
-        Slot& t = slot[q % MAX_FACES];
-        const size_t M = std::min(rows[pl.lane], round_up(2 * (size_t)C.ax[pl.p].U, GBM));
-        t.b = std::max(t.b, (size_t)pl.K * pl.N);
-        t.a = std::max(t.a, M * pl.K);
-        t.g = std::max(t.g, M * pl.N);
+    for (Plan& pl : plans) {
+        pl.chunk = (int)(rows[pl.lane] / 2);
+        pl.n_chunks = (C.ax[pl.p].U + pl.chunk - 1) / pl.chunk;
     }
-    for (int q = 0; q < std::min(nf, MAX_FACES); ++q) {
-        Slot& t = slot[q];
-        t.B = off;  // B, then its split halves [N][K] each
-        off = round_up(off + 2 * t.b * sizeof(float), 256);
-        t.A = off;
-        off = round_up(off + t.a * sizeof(float), 256);
-        t.G = off;
-        off = round_up(off + t.g * sizeof(float), 256);
-        t.S = off;
-        off = round_up(off + 8 * n_ang * sizeof(double), 256);
-    }
-    if (C.work.bytes < off) {
+    const size_t pblocks = (n_ang + 255) / 256;
+    const size_t out_len = 4 * n_ang + pblocks + blocks;  // E_theta, E_phi, block maxima of U, power partials
+    int per = MAX_FACES, n_sets = 0;
+    std::vector<int> set_chunks;
+    size_t face_off = 0, chunk_off = 0, coord_off = 0, up_bytes = 0, out_off = 0, nl_off = 0, pmax_off = 0, bsc_off = 0;
+    size_t off = 0;
+    // device workspace: the tables (uploaded in one copy), then results,
+    // partials and per face slot the operands
+    auto lay_out = [&] {
+        n_sets = (nf + per - 1) / per;
+        set_chunks.assign(n_sets, 0);
+        for (int q = 0; q < nf; ++q) set_chunks[q / per] = std::max(set_chunks[q / per], plans[q].n_chunks);
+        size_t n_table = 0;
+        for (int m : set_chunks) n_table += (size_t)m * MAX_FACES;
+        chunk_off = round_up(nf * sizeof(FaceDev), 64);
+        coord_off = round_up(chunk_off + n_table * sizeof(ChunkDev), 64);
+        up_bytes = coord_off + coord_len * sizeof(double);
+        out_off = round_up(up_bytes, 256);
+        nl_off = round_up(out_off + out_len * sizeof(double), 256);
+        pmax_off = nl_off + (n_sets > 1 ? round_up(12 * n_ang * sizeof(double), 256) : 0);
+        bsc_off = round_up(pmax_off + blocks * sizeof(float), 256);
+        off = round_up(bsc_off + 2 * (size_t)nf * sizeof(float), 256);
+        for (Slot& t : slot) t = Slot{};
+        for (int q = 0; q < nf; ++q) {
+            const Plan& pl = plans[q];
+            Slot& t = slot[q % per];
+            const size_t M = std::min(rows[pl.lane], round_up(2 * (size_t)C.ax[pl.p].U, GBM));
+            t.b = std::max(t.b, (size_t)pl.K * pl.N);
+            t.a = std::max(t.a, M * pl.K);
+            t.g = std::max(t.g, M * pl.N);
+        }
+        for (int q = 0; q < std::min(nf, per); ++q) {
+            Slot& t = slot[q];
+            t.B = off;  // B, then its split halves [N][K] each
+            t.A = round_up(t.B + 2 * t.b * sizeof(float), 256);
+            t.G = round_up(t.A + t.a * sizeof(float), 256);
+            t.S = round_up(t.G + t.g * sizeof(float), 256);
+            off = round_up(t.S + 8 * n_ang * sizeof(double), 256);
+        }
+    };
+    lay_out();
+    while (C.work.bytes < off) {
         NF_OK(hipStreamSynchronize(s));
-        NF_OK(C.work.alloc(off));
+        const hipError_t e = C.work.alloc(off);
+        if (e == hipSuccess) break;
+        C.work.bytes = 0;
+        if (e != hipErrorOutOfMemory || per == 1) return e;
+        (void)hipGetLastError();
+        per /= 2;
+        lay_out();
     }
     const size_t host_bytes = std::max(up_bytes, out_len * sizeof(double));
     if (C.host.bytes < host_bytes) NF_OK(C.host.alloc(host_bytes));
@@ -1176,12 +1181,12 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
         launches[set].resize(set_chunks[set]);
         for (size_t c = 0; c < launches[set].size(); ++c) launches[set][c].table = (int)(tb + c * MAX_FACES);
         std::memset(hc + tb, 0, launches[set].size() * MAX_FACES * sizeof(ChunkDev));
-        for (int q = set * MAX_FACES; q < std::min(nf, (set + 1) * MAX_FACES); ++q) {
+        for (int q = set * per; q < std::min(nf, (set + 1) * per); ++q) {
             const Nf2ffFace& f = faces[q];
             const Plan& pl = plans[q];
             const auto& A = C.ax[pl.p];
             const auto& M = C.mir[f.axis];
-            const Slot& t = slot[q % MAX_FACES];
+            const Slot& t = slot[q % per];
             FaceDev d{};
             d.src = f.src;
             d.scale = f.scale;
@@ -1230,7 +1235,7 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
             pack_blocks[set] = std::max(pack_blocks[set], d.nb);
             for (int c = 0; c < pl.n_chunks; ++c) {
                 Launch& L = launches[set][c];
-                ChunkDev& ck = hc[L.table + q % MAX_FACES];
+                ChunkDev& ck = hc[L.table + q % per];
                 ck.u0 = c * pl.chunk;
                 ck.u1 = std::min(A.U, ck.u0 + pl.chunk);
                 ck.M = (int)round_up(2 * (size_t)(ck.u1 - ck.u0), GBM);
@@ -1283,11 +1288,11 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
     const FaceDev* d_faces = reinterpret_cast<const FaceDev*>(wk + face_off);
     const ChunkDev* d_chunks = reinterpret_cast<const ChunkDev*>(wk + chunk_off);
     for (int set = 0; set < n_sets; ++set) {
-        const FaceDev* fd = d_faces + set * MAX_FACES;
-        const int n = std::min(MAX_FACES, nf - set * MAX_FACES);
+        const FaceDev* fd = d_faces + set * per;
+        const int n = std::min(per, nf - set * per);
         hipLaunchKernelGGL(k_nf2ff_pack, dim3(pack_blocks[set], n), dim3(256), 0, s, fd);
         bool any_split = false;
-        for (int q = 0; q < n; ++q) any_split = any_split || hf[set * MAX_FACES + q].split;
+        for (int q = 0; q < n; ++q) any_split = any_split || hf[set * per + q].split;
         for (size_t c = 0; c < launches[set].size(); ++c) {
             const Launch& L = launches[set][c];
             const ChunkDev* cd = d_chunks + L.table;
@@ -1316,8 +1321,8 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
     }
     typedef std::complex<double> cd;
     const cd fac = cd(0.0, k) * std::exp(cd(0.0, -k * r)) / (4.0 * M_PI * r);
-    hipLaunchKernelGGL(k_nf2ff_project, dim3((unsigned)pblocks), dim3(256), 0, s, d_faces + (n_sets - 1) * MAX_FACES,
-                       nf - (n_sets - 1) * MAX_FACES, d_nl, d_kap + 3 * n_ang, d_kap + 3 * n_ang + n_theta, n_phi, n_ang,
+    hipLaunchKernelGGL(k_nf2ff_project, dim3((unsigned)pblocks), dim3(256), 0, s, d_faces + (n_sets - 1) * per,
+                       nf - (n_sets - 1) * per, d_nl, d_kap + 3 * n_ang, d_kap + 3 * n_ang + n_theta, n_phi, n_ang,
                        fac.real(), fac.imag(), r, d_out, d_umax);
     NF_OK(hipGetLastError());
     NF_OK(hipEventRecord(all->b, s));
