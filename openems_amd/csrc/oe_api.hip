@@ -1851,9 +1851,11 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     // launches cost a second start and tail, and work-groups of a slab's few
     // rows leave most of their lanes idle.  us per step, two launches / one:
     // 72x60x32 22.0 / 11.2, 200x150x40 39 / 27.0, 144^3 61 / 52.5, 256x200x128
-    // 100.9 / 92.1, 256^3 227.8 / 218.5, 384x384x256 557 / 547, 800x500x40
-    // 287.6 / 262.7.  (Overlapped or separately tiled slab launches, scalar
-    // lanes and grids without a table keep the two.)
+    // 100.9 / 92.1, 256^3 227.8 / 218.5, 384x384x256 555 / 545, 800x500x40
+    // 287.6 / 262.7, 400^3 1074 / 1040.  On the largest grids, whose slabs are a
+    // few percent, the interior's fourth wave counts for more: 448^3 1279 /
+    // 1299, 512^3 1811 / 1850.  (Overlapped or separately tiled slab launches,
+    // scalar lanes and grids without a table keep the two.)
     const bool mix = cp && !fused && tl.vec == 4 && !e->overlap_slabs && e->slab_tiles.bx <= 0 && e->n_mat[0] > 0 &&
                      e->n_mat[1] > 0 && e->g.N <= e->mix_cells;
     if (mix && e->tiles_auto) {

@@ -148,7 +148,7 @@ struct oe_engine {
     DevBuf exc_samples;
     DevBuf step_dev;       // batch-relative step read by the kernels of a step, and steps begun
     DevBuf ride_table;     // the riders of the running batch (oe_ride.h)
-    size_t mix_cells = SIZE_MAX;  // most cells of a CPML grid whose slabs and interior share a launch
+    size_t mix_cells = 75000000;  // most cells of a CPML grid whose slabs and interior share a launch
     int ride = 1;          // probes, small DFTs and captures in the Yee launches: 1 on, 0 off
     int graph_steps = 16;  // steps per captured graph (0: no graphs)
     // CPML slab launches on a second stream beside the interior launch of

@@ -686,24 +686,18 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
     // lanes of the folded Mur faces held by this thread
     const bool mur_lo = MUR && live && mz.on[0] && k0 == 0;
     const bool mur_hi = MUR && live && mz.on[1] && k0 + V == nz;
-    // material-table row indices one plane ahead: the LDS row reads of a
-    // plane need not wait for that plane's field loads
-    MatIdx mi_c;
-    if constexpr (TAB) {
-        mi_c = coef_index<V, RAG>(mat, u, o);
-    }
-
     for (int i = t.i0; i < t.i1; ++i, u += plane) {
         keep_offset(o);
         keep_offset(oj);
         const bool gi = i > 0;
         const bool row = live && gi && gj;
-        MatIdx mi_n;
+        MatIdx mi;
         Vec<V> hx_c, hy_c, hz_c, hz_j, hx_j, ex, ey, ez, c0, c1, c2, s0, s1, s2;
         float hy_kf = 0.f, hx_kf = 0.f;
         Psi<V> px, py, pz;
         bool onx = false;
-        if constexpr (TAB) mi_n = coef_index<V, RAG>(mat, u + (i + 1 < t.i1 ? plane : 0), o);
+        // first: loads arrive in order, and the row reads wait for the index
+        if constexpr (TAB) mi = coef_index<V, RAG>(mat, u, o);
         hx_c = ldv<V, RAG>(at(Hx, u, o)), hy_c = ldv<V, RAG>(at(Hy, u, o)), hz_c = ldv<V, RAG>(at(Hz, u, o));
         hz_j = ldv<V, RAG>(at(Hz, u, oj));
         hx_j = ldv<V, RAG>(at(Hx, u, oj));
@@ -743,7 +737,7 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
             if (i == t.i0) rows.fill();
         }
         if constexpr (TAB) {
-            coef_from<V, RAG>(mat, mi_c, rows.lds, s0, s1, s2, c0, c1, c2, nv);
+            coef_from<V, RAG>(mat, mi, rows.lds, s0, s1, s2, c0, c1, c2, nv);
         }
         // Mur pre step on the old values: v = E(shift) - c E(line)
         float mvx[2] = {0.f, 0.f}, mvy[2] = {0.f, 0.f};
@@ -835,7 +829,6 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
         }
         hy_p = hy_c;
         hz_p = hz_c;
-        mi_c = mi_n;
     }
 }
 
