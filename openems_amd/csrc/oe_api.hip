@@ -73,11 +73,12 @@ bool narrow_plane(const Grid& g) { return ((size_t)g.ny + 2) * g.nz < ((size_t)1
 // 200x201x75 64 / 75 lanes 84.6 / 64.3.
 //
 // ci: one plane up to 12 M cells, where more work-groups and a shorter chain
-// of loads count (with CPML, ci 1 / 2 / 4: 72x60x32 20.2 / 26.8 / 39.8,
-// 100^3 29.5 / 35.7 / 51, 160x144x120 62.4 / 65.8 / 73.5, 200x180x232 136 /
-// 142 / 141); above, two planes, which reload half as many i +- 1 planes
-// (256^3 249 / 239 / 239; plain 192 / 191 / 197; 512^3 2040 / 1950 / 1961),
-// four where the row is cut into narrow blocks (256x320x384 511 / 511 / 497).
+// of loads count (plain, us per step at ci 1 / 2 / 4: 64^3 8.0 / 9.3 / 12.2,
+// 100^3 11.5 / 12.4 / 15.0, 160x144x120 37.0 / 39.2 / 38.2, 200^3 95.7 / 94.2 /
+// 97.3); above, two planes, which reload half as many i +- 1 planes (256^3 198 /
+// 186 / 184; 512^3 with CPML 2040 / 1950 / 1961), four where the row is cut
+// into narrow blocks (256x320x384 with CPML 511 / 511 / 497).  A CPML grid's
+// single launch takes one or two (oe_engine_run_batch).
 // Scalar lanes, whose planes are cheaper than their start, take two
 // (151x133x117 with CPML, ci 1 / 2 / 3: 82.5 / 75.0 / 81.0).
 Tiles auto_tiles(const Grid& g, int vec_req) {

@@ -379,9 +379,9 @@ class SweepResult:
 
 class Sweep:
     """Many structures stepped together (oe_sweep_*): each is a HipEngine with
-    its CPML, lumped-port DFT and excitations; all half-steps of all active
-    structures run as one launch per kernel variant, replayed from a captured
-    HIP graph between energy checks."""
+    its CPML, lumped-port DFT and excitations; a half-step of all active
+    structures (of a set that the caches hold, where they are many) is one
+    launch, replayed from a captured HIP graph between energy checks."""
 
     def __init__(self, device: int = 0):
         h = C.c_void_p()
