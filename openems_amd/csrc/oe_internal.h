@@ -3,6 +3,8 @@
 // public ABI.
 #pragma once
 
+#include "oe_tiles.h"
+
 #include <hip/hip_runtime.h>
 #include <cstddef>
 #include <cstdint>
@@ -30,23 +32,6 @@ struct DevBuf {
         return n ? hipMalloc(&p, n) : hipSuccess;
     }
     template <class T> T* as() const { return reinterpret_cast<T*>(p); }
-};
-
-// Field block: one allocation of 6 arrays of N floats, E(x,y,z) then H(x,y,z).
-// Coefficient block: 12 arrays of N floats, Ca(x,y,z) Cb(x,y,z) Da(x,y,z) Db(x,y,z).
-struct Grid {
-    int nx, ny, nz;
-    size_t N;
-};
-
-// Yee kernel launch shape.  A work-group covers bx*V consecutive k of `by`
-// rows (j) and marches along i over `ci` planes, keeping the i+1 (H update)
-// or i-1 (E update) plane of the marched components in registers.
-struct Tiles {
-    int vec;  // 4: float4 accesses, 1: scalar
-    int bx;   // lanes along k
-    int by;   // rows along j; bx * by <= 256
-    int ci;   // planes along i per work-group
 };
 
 // CPML state as the fused Yee kernels see it.  Face f = 2*dir + (max side).

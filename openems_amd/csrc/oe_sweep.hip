@@ -151,7 +151,7 @@ namespace {
 // (plain kernel).
 void structure_boxes(const oe_sweep* sw, int sid, const Item& it, std::vector<Group>& groups) {
     const Grid& g = it.eng->g;
-    const int vec = g.nz % 4 == 0 && (!it.cpml || it.cpml->cpml.zvec) ? 4 : 1;
+    const int vec = sweep_lanes(g, !it.cpml || it.cpml->cpml.zvec);
     const int nzv = ceil_div(g.nz, vec);
     SweepBox proto{};
     proto.sid = sid;
