@@ -1931,11 +1931,14 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     const uint64_t t_batch0 = e->timestep;
     // DFTs of a few signals sampled every step ride; the others are launches,
     // which read the step from the device when all of them sample every step.
+    // One that the batch lists twice adds twice a step, so it is launched
+    // twice: riders of one launch would add to its sums at the same time.
     std::vector<oe_extension*> ride_dfts;
     if (riding) {
         std::vector<oe_extension*> rest;
         for (auto* x : dfts) {
-            (dft_rides(x) && ride_dfts.size() < (size_t)MAX_RIDE_DFT ? ride_dfts : rest).push_back(x);
+            const bool one = std::count(dfts.begin(), dfts.end(), x) == 1;
+            (one && dft_rides(x) && ride_dfts.size() < (size_t)MAX_RIDE_DFT ? ride_dfts : rest).push_back(x);
         }
         dfts.swap(rest);
     }
@@ -2003,7 +2006,11 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     HIP_OK(hipMemsetAsync(step_dev, step_in_h ? 0xff : 0, sizeof(uint64_t), e->stream));
     HIP_OK(hipMemsetAsync(step_dev + 1, 0, sizeof(uint64_t), e->stream));
 
-    // The riders' table.  The captures ride where every one of them fits.
+    // The riders' table.  The captures ride where every one of them fits; of
+    // an extension listed twice one capture holds for both.
+    auto first_of = [](const std::vector<oe_extension*>& v, size_t q) {
+        return std::find(v.begin(), v.end(), v[q]) == v.begin() + q;
+    };
     bool ride_ade = riding && ades.size() <= (size_t)MAX_MERGE_ADE, ride_mur = riding && !fold_mur;
     size_t n_faces = 0;
     for (const auto* x : murs) n_faces += x->mur_faces.size();
@@ -2036,15 +2043,17 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         for (auto* x : ride_dfts) rt.dft[rt.n_dft++] = RideDft{x->dft, x->dft_count};
         rt.first_ade = rt.first_dft + rt.n_dft;
         int wg = rt.first_ade;
-        for (auto* x : ades) {
-            if (!ride_ade || x->ade.mode != OE_MODE_PHYSICAL || x->ade.n == 0) continue;
+        for (size_t q = 0; q < ades.size(); ++q) {
+            const oe_extension* x = ades[q];
+            if (!ride_ade || !first_of(ades, q) || x->ade.mode != OE_MODE_PHYSICAL || x->ade.n == 0) continue;
             rt.ade_first[rt.n_ade] = wg;
             rt.ade[rt.n_ade++] = x->ade;
             wg += (x->ade.n + 255) / 256;
         }
         rt.first_mur = wg;
-        for (auto* x : murs) {
-            if (!ride_mur) continue;
+        for (size_t q = 0; q < murs.size(); ++q) {
+            const oe_extension* x = murs[q];
+            if (!ride_mur || !first_of(murs, q)) continue;
             for (size_t f = 0; f < x->mur_faces.size(); ++f) {
                 rt.mur[rt.n_mur++] = RideMur{x->mur_dev.as<MurDev>() + f, wg};
                 wg += (x->mur_faces[f].s0 * x->mur_faces[f].s1 + 255) / 256;
@@ -2229,7 +2238,9 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         for (auto* x : murs) {
             if (fold_mur) break;
             Timed tm(e, "mur_post");
-            HIP_OK(launch_mur_post(e->F, e->g, x->mur_dev.as<MurDev>(), (int)x->mur_faces.size(), x->mur_thin, e->stream));
+            // listed twice: the second post step adds to the first one's values
+            const bool apart = x->mur_thin || std::count(murs.begin(), murs.end(), x) > 1;
+            HIP_OK(launch_mur_post(e->F, e->g, x->mur_dev.as<MurDev>(), (int)x->mur_faces.size(), apart, e->stream));
         }
         if (host) OE_TRY(run_hooks(3));
         if (point_ops) {

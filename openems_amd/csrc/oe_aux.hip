@@ -189,7 +189,8 @@ __global__ void k_mur_post_apply(float* __restrict__ F, Grid g, const MurDev* __
 }
 
 // The two steps apart, for a grid of 2 cells along a face's normal (its shift
-// plane is the opposite face's line plane).
+// plane is the opposite face's line plane) and for faces that a batch steps
+// twice.
 __global__ void k_mur_post(const float* __restrict__ F, Grid g, const MurDev* __restrict__ faces) {
     const MurDev m = faces[blockIdx.y];
     const int cnt = m.s0 * m.s1;
@@ -638,9 +639,9 @@ hipError_t launch_mur_pre(float* F, const Grid& g, const MurDev* faces, int n, h
     return hipGetLastError();
 }
 
-hipError_t launch_mur_post(float* F, const Grid& g, const MurDev* faces, int n, bool thin, hipStream_t s) {
+hipError_t launch_mur_post(float* F, const Grid& g, const MurDev* faces, int n, bool apart, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    if (!thin) {
+    if (!apart) {
         hipLaunchKernelGGL(k_mur_post_apply, dim3(mur_blocks(g), n), dim3(256), 0, s, F, g, faces);
         return hipGetLastError();
     }

@@ -316,8 +316,10 @@ struct MurDev {
     MurEdge e[2][2];  // [component nyp, nypp][face along the third axis: min, max]
 };
 hipError_t launch_mur_pre(float* F, const Grid& g, const MurDev* faces, int n, hipStream_t s);
-// thin: some face's axis holds only 2 cells.
-hipError_t launch_mur_post(float* F, const Grid& g, const MurDev* faces, int n, bool thin, hipStream_t s);
+// apart: the post step, stored to the faces' values, and each face's write in
+// launches of their own (some face's axis holds only 2 cells, or the step is
+// taken twice).
+hipError_t launch_mur_post(float* F, const Grid& g, const MurDev* faces, int n, bool apart, hipStream_t s);
 
 // ADE (src/extensions/dispersive.rs).  One thread per listed cell.
 struct AdeDev {
