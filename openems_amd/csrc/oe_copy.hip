@@ -40,6 +40,14 @@ struct Ring {
     std::vector<std::thread> threads;
     std::atomic<bool> stop{false};
     hipStream_t busy = nullptr;  // transfers into the ring may be under way on this stream
+    bool make(size_t piece) {
+        hipError_t err = hipHostMalloc((void**)&pinned, piece * STAGE_SLOTS, hipHostMallocDefault);
+        if (err != hipSuccess) pinned = nullptr;
+        for (int k = 0; k < STAGE_SLOTS && err == hipSuccess; ++k)
+            if ((err = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming)) != hipSuccess) ev[k] = nullptr;
+        if (err != hipSuccess) (void)hipGetLastError();
+        return err == hipSuccess;
+    }
     ~Ring() {
         stop.store(true);
         for (auto& t : threads) t.join();
@@ -50,17 +58,16 @@ struct Ring {
     }
 };
 
-hipError_t staged(const std::vector<Piece>& pieces, size_t piece, hipStream_t s) {
+// *began stays false where there is no ring (nothing was copied).
+hipError_t staged(const std::vector<Piece>& pieces, size_t piece, hipStream_t s, bool* began) {
     const size_t n = pieces.size();
     enum { EMPTY, FULL, DONE };
     std::unique_ptr<std::atomic<int>[]> state(new std::atomic<int>[n]);
     for (size_t q = 0; q < n; ++q) state[q].store(EMPTY);
     std::atomic<size_t> next{0};
     Ring r;
-    hipError_t err = hipHostMalloc((void**)&r.pinned, piece * STAGE_SLOTS, hipHostMallocDefault);
-    if (err != hipSuccess) return err;
-    for (hipEvent_t& e : r.ev)
-        if ((err = hipEventCreateWithFlags(&e, hipEventDisableTiming)) != hipSuccess) return err;
+    if (!r.make(piece)) return hipErrorOutOfMemory;
+    hipError_t err = hipSuccess;
     auto empty = [&] {
         for (;;) {
             const size_t c = next.fetch_add(1);
@@ -76,6 +83,7 @@ hipError_t staged(const std::vector<Piece>& pieces, size_t piece, hipStream_t s)
     r.threads.reserve(STAGE_THREADS);
     for (int t = 0; t < STAGE_THREADS; ++t) r.threads.emplace_back(empty);
     r.busy = s;
+    *began = true;
     size_t full = 0;  // pieces whose transfer has been seen to end
     auto poll = [&](size_t issued) -> hipError_t {
         while (full < issued) {
@@ -112,6 +120,7 @@ hipError_t copy_to_host(const HostCopy* c, int n, hipStream_t s) {
     size_t total = 0;
     for (int q = 0; q < n; ++q) total += c[q].bytes;
     if (total >= STAGE_MIN) {
+        bool began = false;  // without memory, events or threads for the ring: the runtime's copy below
         try {
             const size_t piece = 2u << 20;
             std::vector<Piece> pieces;
@@ -119,10 +128,9 @@ hipError_t copy_to_host(const HostCopy* c, int n, hipStream_t s) {
                 for (size_t o = 0; o < c[q].bytes; o += piece)
                     pieces.push_back({static_cast<char*>(c[q].dst) + o, static_cast<const char*>(c[q].src) + o,
                                       std::min(piece, c[q].bytes - o)});
-            return staged(pieces, piece, s);
+            const hipError_t err = staged(pieces, piece, s, &began);
+            if (began) return err;
         } catch (const std::exception&) {
-            // no memory or thread for the ring: the runtime's copy below
-            (void)hipStreamSynchronize(s);
         }
     }
     for (int q = 0; q < n; ++q) {
