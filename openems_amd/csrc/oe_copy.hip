@@ -8,8 +8,10 @@
 // pinned pieces while a few host threads empty it into the destination (and
 // take its page faults): 38 GB/s at 422 MB, 27 at 25 MB (MI355X host,
 // fresh pages; 1 MB pieces 30, 3 instead of 8 pieces 28, 6 threads instead of 4
-// no more).  The ring and the threads live for the call only, so
-// nothing is shared between calls, threads or streams.
+// no more).  A destination the runtime knows takes the transfers itself: pinned
+// memory at 56 GB/s (192 MB; 39 through the ring), managed or device memory.
+// The ring and the threads live for the call only, so nothing is shared
+// between calls, threads or streams.
 
 #include "oe_internal.h"
 
@@ -114,12 +116,24 @@ hipError_t staged(const std::vector<Piece>& pieces, size_t piece, hipStream_t s,
     return hipSuccess;
 }
 
+// Whether p is memory that the runtime does not know: ordinary host memory.
+bool pageable(const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return a.type == hipMemoryTypeUnregistered;
+}
+
 }  // namespace
 
 hipError_t copy_to_host(const HostCopy* c, int n, hipStream_t s) {
     size_t total = 0;
+    bool page = true;
     for (int q = 0; q < n; ++q) total += c[q].bytes;
-    if (total >= STAGE_MIN) {
+    for (int q = 0; q < n && page && total >= STAGE_MIN; ++q) page = pageable(c[q].dst);
+    if (page && total >= STAGE_MIN) {
         bool began = false;  // without memory, events or threads for the ring: the runtime's copy below
         try {
             const size_t piece = 2u << 20;

@@ -50,6 +50,11 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipSt
     memcpy(d, s, n);
     return hipSuccess;
 }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+    if (mode == "no_attributes") return last_error = 1, hipErrorInvalidValue;
+    a->type = mode == "pinned" && p == dst0 ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
+    return hipSuccess;
+}
 hipError_t hipMalloc(void**, size_t) { abort(); }
 hipError_t hipFree(void*) { abort(); }
 }
@@ -106,6 +111,12 @@ def test_ring_carries_all(copy, sizes):
 @pytest.mark.parametrize("sizes", SIZES)
 def test_without_a_ring_the_runtime_copies(copy, mode, sizes):
     assert copy(mode, *sizes) == (True, True, len(sizes))
+
+
+@pytest.mark.parametrize("sizes", SIZES)
+def test_a_pinned_destination_takes_the_transfers(copy, sizes):
+    assert copy("pinned", *sizes) == (True, True, len(sizes))
+    assert copy("no_attributes", *sizes) == (True, True, 0)
 
 
 @pytest.mark.parametrize("sizes", [(12 * MB - 4,), (1,), (5 * MB, 6 * MB)])
