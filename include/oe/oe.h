@@ -260,8 +260,10 @@ oe_status oe_engine_kernel_time(oe_engine* eng, const char* name, uint64_t* laun
 oe_status oe_engine_set_profiling(oe_engine* eng, int period);
 
 /* Tile shape of the Yee kernels: bx lanes along z (in vector units), by rows
- * along y, ci planes along x per work-group; 0 keeps the automatic choice.
- * vec = 4 uses 16-byte accesses (requires nz % 4 == 0), 1 scalar, 0 auto. */
+ * along y (bx * by at most 256; by 0 takes 256 / bx), ci planes along x per
+ * work-group; 0 keeps the automatic choice.  vec = 4 uses 16-byte accesses
+ * (nz a multiple of 4, or at least 8), 1 scalar, 0 auto.  What
+ * oe_engine_get_tiles reports is accepted. */
 oe_status oe_engine_set_tiles(oe_engine* eng, int bx, int by, int ci, int vec);
 oe_status oe_engine_get_tiles(const oe_engine* eng, int tiles[4]);
 

@@ -734,19 +734,24 @@ oe_status oe_engine_kernel_time(oe_engine* e, const char* name, uint64_t* launch
 oe_status oe_engine_set_tiles(oe_engine* e, int bx, int by, int ci, int vec) {
     if (!e) return fail(OE_ERR_CONFIG, "null argument");
     Tiles t = auto_tiles(e->g, vec);
-    if (vec == 4 && e->g.nz % 4 != 0) return fail(OE_ERR_CONFIG, "vec=4 needs nz %% 4 == 0 (nz=%d)", e->g.nz);
+    const Tiles own = t;
+    if (vec == 4 && t.vec != 4)
+        return fail(OE_ERR_CONFIG, "vec=4 needs rows of whole float4s or of 8 cells and more, in planes of fewer than 2^30 "
+                    "cells (ny=%d, nz=%d)", e->g.ny, e->g.nz);
+    if (bx > 256 || by > 256) return fail(OE_ERR_CONFIG, "bx and by must be at most 256");
     if (bx > 0) {
-        if ((bx & (bx - 1)) != 0 || bx > 256) return fail(OE_ERR_CONFIG, "bx must be a power of two <= 256");
         t.bx = bx;
         t.by = 256 / bx;
     }
     if (by > 0) {
         if (bx <= 0) t.bx = std::min(64, pow2ceil((e->g.nz + t.vec - 1) / t.vec));
-        if (by * t.bx != 256) return fail(OE_ERR_CONFIG, "bx * by must equal 256");
+        if (by * t.bx > 256) return fail(OE_ERR_CONFIG, "bx * by must be at most 256");
         t.by = by;
     }
     if (ci > 0) t.ci = std::min(ci, e->g.nx);
-    e->tiles_auto = bx <= 0 && by <= 0 && ci <= 0;
+    // the automatic shape given back (oe_engine_get_tiles) stays automatic
+    const bool same = bx == own.bx && by == own.by && ci == own.ci;
+    e->tiles_auto = same || (bx <= 0 && by <= 0 && ci <= 0);
     e->tiles = t;
     return OE_OK;
 }
