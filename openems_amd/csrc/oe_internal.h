@@ -28,8 +28,11 @@ struct DevBuf {
     ~DevBuf() { if (p) (void)hipFree(p); }
     hipError_t alloc(size_t n) {
         if (p) { (void)hipFree(p); p = nullptr; }
-        bytes = n;
-        return n ? hipMalloc(&p, n) : hipSuccess;
+        bytes = 0;  // of a failed allocation: callers ask for what is missing
+        const hipError_t e = n ? hipMalloc(&p, n) : hipSuccess;
+        if (e == hipSuccess) bytes = n;
+        else p = nullptr;
+        return e;
     }
     template <class T> T* as() const { return reinterpret_cast<T*>(p); }
 };

@@ -871,8 +871,11 @@ struct PinnedBuf {
     ~PinnedBuf() { if (p) (void)hipHostFree(p); }
     hipError_t alloc(size_t n) {
         if (p) { (void)hipHostFree(p); p = nullptr; }
-        bytes = n;
-        return n ? hipHostMalloc(&p, n, hipHostMallocDefault) : hipSuccess;
+        bytes = 0;  // as DevBuf
+        const hipError_t e = n ? hipHostMalloc(&p, n, hipHostMallocDefault) : hipSuccess;
+        if (e == hipSuccess) bytes = n;
+        else p = nullptr;
+        return e;
     }
 };
 
@@ -1152,7 +1155,6 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
         NF_OK(hipStreamSynchronize(s));
         const hipError_t e = C.work.alloc(off);
         if (e == hipSuccess) break;
-        C.work.bytes = 0;
         if (e != hipErrorOutOfMemory || per == 1) return e;
         (void)hipGetLastError();
         per /= 2;

@@ -543,6 +543,7 @@ oe_status energies(oe_sweep* sw, int n) {
     if (sw->energy_host_n < (size_t)n) {
         if (sw->energy_host) (void)hipHostFree(sw->energy_host);
         sw->energy_host = nullptr;
+        sw->energy_host_n = 0;
         HIP_OK(hipHostMalloc(&sw->energy_host, (size_t)n * 2 * sizeof(double), hipHostMallocDefault));
         sw->energy_host_n = n;
     }
