@@ -1034,8 +1034,15 @@ static hipError_t plan_angles(Nf2ffCache& c, const double* theta, int nt, const 
     return hipSuccess;
 }
 
-// G stays within 64 Mi floats per face; larger U is split into chunks of u,
-// each with the angles whose u falls in it.
+// Work buffers of at most about OE_NF2FF_MB MB (1024): fewer faces share the
+// launches and the buffers of more of them follow one another.
+size_t work_limit() {
+    const char* v = getenv("OE_NF2FF_MB");
+    return (size_t)std::max(0L, v ? atol(v) : 1024L) << 20;
+}
+
+// G stays within 64 Mi floats over the faces of a launch; larger U is split
+// into chunks of u, each with the angles whose u falls in it.
 hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const double* theta, int n_theta,
                          const double* phi, int n_phi, double r, const double center[3], hipStream_t s,
                          Nf2ffCache* cache, Nf2ffOut* out) {
@@ -1064,17 +1071,12 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
 
     // per face: first-contraction axis p (fewer distinct |kappa|), sizes
     struct Plan {
-        int p, q, np, nq, K, N, swap, lane, chunk, n_chunks;
+        int p, q, np, nq, K, N, swap, need, rows, chunk, n_chunks;  // need: rows of all of U, rows: of one chunk
         std::vector<double> xp, xq;
     };
     const int nf = (int)faces.size();
     std::vector<Plan> plans(nf);
-    // rows of one chunk: G within 64 Mi floats for the widest of the z faces,
-    // and of the others (of all, when there is only one kind)
-    bool kinds[2] = {false, false};
-    for (const auto& f : faces) kinds[f.axis != 2] = true;
-    size_t coord_len = 0, blocks = 0, Nmax[2] = {GBN, GBN};
-    int Umax[2] = {0, 0};
+    size_t coord_len = 0, blocks = 0;
     for (int q = 0; q < nf; ++q) {
         const Nf2ffFace& f = faces[q];
         Plan& pl = plans[q];
@@ -1092,24 +1094,20 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
         for (double v : cq) pl.xq.push_back(v - center[pl.q]);
         coord_len += 2 * ((size_t)pl.np + pl.nq);
         blocks += (cp.size() * cq.size() + 255) / 256;
-        pl.lane = kinds[0] && kinds[1] && f.axis != 2;
-        Nmax[pl.lane] = std::max(Nmax[pl.lane], (size_t)pl.N);
-        Umax[pl.lane] = std::max(Umax[pl.lane], C.ax[pl.p].U);
+        pl.need = (int)round_up(2 * (size_t)C.ax[pl.p].U, GBM);
     }
+    // Rows of one chunk: the most, the same for every face of a launch, for
+    // which G of all of them stays within 256 MB, the size of the cache that
+    // the reduction then reads it from.  349x349x221 nodes, us per transform
+    // with 256 MB a face / 256 MB together: 54300 irregular angles 3000 / 2884,
+    // 22500 1360 / 1313 (128 MB together 2950, 384 MB 2960).
     const size_t budget = (size_t)64 << 20;
-    size_t rows[2];
-    for (int l = 0; l < 2; ++l)
-        rows[l] = std::min(std::max<size_t>(GBM, budget / Nmax[l] / GBM * GBM), round_up(2 * (size_t)Umax[l], GBM));
     // Sets of up to `per` faces share the launches and, from one set to the
-    // next, the buffers: as many as MAX_FACES, fewer where the device has no
-    // room for their buffers at once.
+    // next, the buffers: as many as MAX_FACES, fewer where their buffers pass
+    // work_limit().
     struct Slot {
         size_t B = 0, A = 0, G = 0, S = 0, b = 0, a = 0, g = 0;
     } slot[MAX_FACES];
-    for (Plan& pl : plans) {
-        pl.chunk = (int)(rows[pl.lane] / 2);
-        pl.n_chunks = (C.ax[pl.p].U + pl.chunk - 1) / pl.chunk;
-    }
     const size_t pblocks = (n_ang + 255) / 256;
     const size_t out_len = 4 * n_ang + pblocks + blocks;  // E_theta, E_phi, block maxima of U, power partials
     int per = MAX_FACES, n_sets = 0;
@@ -1120,6 +1118,27 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
     // partials and per face slot the operands
     auto lay_out = [&] {
         n_sets = (nf + per - 1) / per;
+        for (int s0 = 0; s0 < nf; s0 += per) {
+            const int s1 = std::min(nf, s0 + per);
+            size_t rows = 0;
+            for (int q = s0; q < s1; ++q) rows = std::max(rows, (size_t)plans[q].need);
+            auto held = [&](size_t r) {
+                size_t g = 0;
+                for (int q = s0; q < s1; ++q) g += std::min(r, (size_t)plans[q].need) * plans[q].N;
+                return g;
+            };
+            size_t lo = GBM;  // the most rows within the budget, by halving
+            for (size_t hi = rows; lo < hi;) {
+                const size_t mid = round_up((lo + hi) / 2, GBM);
+                if (held(mid) <= budget) lo = mid;
+                else hi = mid - GBM;
+            }
+            for (int q = s0; q < s1; ++q) {
+                plans[q].rows = (int)std::min(lo, (size_t)plans[q].need);
+                plans[q].chunk = plans[q].rows / 2;
+                plans[q].n_chunks = (C.ax[plans[q].p].U + plans[q].chunk - 1) / plans[q].chunk;
+            }
+        }
         set_chunks.assign(n_sets, 0);
         for (int q = 0; q < nf; ++q) set_chunks[q / per] = std::max(set_chunks[q / per], plans[q].n_chunks);
         size_t n_table = 0;
@@ -1136,7 +1155,7 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
         for (int q = 0; q < nf; ++q) {
             const Plan& pl = plans[q];
             Slot& t = slot[q % per];
-            const size_t M = std::min(rows[pl.lane], round_up(2 * (size_t)C.ax[pl.p].U, GBM));
+            const size_t M = pl.rows;
             t.b = std::max(t.b, (size_t)pl.K * pl.N);
             t.a = std::max(t.a, M * pl.K);
             t.g = std::max(t.g, M * pl.N);
@@ -1151,14 +1170,13 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
         }
     };
     lay_out();
-    while (C.work.bytes < off) {
-        NF_OK(hipStreamSynchronize(s));
-        const hipError_t e = C.work.alloc(off);
-        if (e == hipSuccess) break;
-        if (e != hipErrorOutOfMemory || per == 1) return e;
-        (void)hipGetLastError();
-        per /= 2;
+    for (const size_t most = work_limit(); off > most && per > 1;) {
+        per = (per + 1) / 2;
         lay_out();
+    }
+    if (C.work.bytes < off) {
+        NF_OK(hipStreamSynchronize(s));
+        NF_OK(C.work.alloc(off));
     }
     const size_t host_bytes = std::max(up_bytes, out_len * sizeof(double));
     if (C.host.bytes < host_bytes) NF_OK(C.host.alloc(host_bytes));
