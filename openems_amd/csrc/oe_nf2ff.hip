@@ -98,6 +98,9 @@ struct ChunkDev {
 };
 constexpr int MAX_FACES = 6;
 
+// Whether a launch over the kinds of a bit mask takes this chunk.
+__device__ __forceinline__ bool takes(const ChunkDev& c, int kinds) { return c.kind >= 0 && (kinds >> c.kind & 1); }
+
 // The face whose work-groups hold blockIdx.x in a launch over kind.
 __device__ __forceinline__ int face_of_block(const ChunkDev* ch, int nf, int kind) {
     int f = -1;
@@ -413,20 +416,22 @@ __device__ __forceinline__ void phase_rows16(const FaceDev& f, const ChunkDev& c
     }
 }
 
-// The contraction's operands of one chunk, every face in one launch: grid
-// (work-groups, face, 2), z = 0 the phase rows, z = 1 (first chunk) the split
-// of B for the faces that need it.
+__device__ __forceinline__ void chunk_rows(const FaceDev& f, const ChunkDev& c, double k) {
+    if (c.M == 0) return;
+    if (c.kind == KIND_SPLIT16) phase_rows16(f, c, k);
+    else phase_rows(f, c, k);
+}
+
+// The contraction's operands of the first chunk, every face in one launch:
+// grid (work-groups, face, 2), z = 0 the phase rows, z = 1 the split of B for
+// the faces that need it.  The rows of the chunks that follow are formed in
+// the launch of the reduction before them (next): A is free by then, and the
+// arithmetic of the rows (31 us a chunk) runs beside the reduction's loads.
 __global__ __launch_bounds__(256) void k_nf2ff_operands(const FaceDev* __restrict__ fc, const ChunkDev* __restrict__ ch,
                                                         double k) {
     const FaceDev& f = fc[blockIdx.y];
-    const ChunkDev& c = ch[blockIdx.y];
-    if (blockIdx.z == 0) {
-        if (c.M == 0) return;
-        if (c.kind == KIND_SPLIT16) phase_rows16(f, c, k);
-        else phase_rows(f, c, k);
-    } else if (f.split) {
-        bsplit(f);
-    }
+    if (blockIdx.z == 0) chunk_rows(f, ch[blockIdx.y], k);
+    else if (f.split) bsplit(f);
 }
 
 // The large contractions on the FP16 matrix cores when split16 (operands
@@ -523,11 +528,17 @@ constexpr int REDUCE_THREADS = 256;
 constexpr int REDUCE_GROUPS = REDUCE_THREADS / QL;
 
 __global__ __launch_bounds__(REDUCE_THREADS) void k_nf2ff_reduce(const FaceDev* __restrict__ fc,
-                                                                 const ChunkDev* __restrict__ ch, double k) {
+                                                                 const ChunkDev* __restrict__ ch,
+                                                                 const ChunkDev* __restrict__ next, int kinds,
+                                                                 double k) {
     constexpr int M = REDUCE_M;
     const FaceDev& r = fc[blockIdx.y];
+    if (blockIdx.z == 1) {
+        chunk_rows(r, next[blockIdx.y], k);
+        return;
+    }
     const ChunkDev& ck = ch[blockIdx.y];
-    if (ck.mirror) return;
+    if (ck.mirror || !takes(ck, kinds)) return;
     const int ql = threadIdx.x & (QL - 1);
     const int gi = ck.g0 + blockIdx.x * REDUCE_GROUPS + (int)(threadIdx.x / QL);
     if (gi >= ck.g1) return;  // whole groups of QL lanes
@@ -735,10 +746,16 @@ __device__ __forceinline__ void mirror_reduce(const FaceDev& r, const ChunkDev& 
 }
 
 __global__ __launch_bounds__(MIRROR_THREADS) void k_nf2ff_reduce_mirror(const FaceDev* __restrict__ fc,
-                                                                        const ChunkDev* __restrict__ ch, double k) {
+                                                                        const ChunkDev* __restrict__ ch,
+                                                                        const ChunkDev* __restrict__ next, int kinds,
+                                                                        double k) {
     const FaceDev& r = fc[blockIdx.y];
+    if (blockIdx.z == 1) {
+        chunk_rows(r, next[blockIdx.y], k);
+        return;
+    }
     const ChunkDev& ck = ch[blockIdx.y];
-    if (!ck.mirror || ck.g0 + (int)blockIdx.x * MIRROR_GROUPS >= ck.g1) return;
+    if (!ck.mirror || !takes(ck, kinds) || ck.g0 + (int)blockIdx.x * MIRROR_GROUPS >= ck.g1) return;
     if (r.uni_q) mirror_reduce<true>(r, ck, k);
     else mirror_reduce<false>(r, ck, k);
 }
@@ -908,6 +925,15 @@ struct Nf2ffCache {
     // timing events, created on first use and kept: [0] brackets the whole
     // transform, the others one GEMM launch each
     std::vector<std::unique_ptr<EventPair>> events;
+    // beside the large contractions: the faces of the small ones
+    hipStream_t side = nullptr;
+    hipEvent_t fork = nullptr, join = nullptr;
+    ~Nf2ffCache() {
+        if (side) (void)hipStreamSynchronize(side);
+        if (fork) (void)hipEventDestroy(fork);
+        if (join) (void)hipEventDestroy(join);
+        if (side) (void)hipStreamDestroy(side);
+    }
     Nf2ffCache() = default;
     Nf2ffCache(const Nf2ffCache&) = delete;
     Nf2ffCache& operator=(const Nf2ffCache&) = delete;
@@ -1192,7 +1218,8 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
     double flop = 0.0, flop_split = 0.0;
     struct Launch {  // one chunk of one set
         int wg[3] = {0, 0, 0};  // work-groups per KIND_*
-        int operands = 0, mirror = 0, plain = 0, table = 0;
+        int operands = 0, table = 0;
+        int mirror[2] = {0, 0}, plain[2] = {0, 0};  // work-groups of the reductions, [1] of KIND_SPLIT16
     };
     std::vector<std::vector<Launch>> launches(n_sets);
     std::vector<int> pack_blocks(n_sets, 0);
@@ -1271,8 +1298,9 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
                 ck.g0 = gs[ck.u0];
                 ck.g1 = gs[ck.u1];
                 const int ng = ck.g1 - ck.g0;
-                if (ck.mirror) L.mirror = std::max(L.mirror, (ng + MIRROR_GROUPS - 1) / MIRROR_GROUPS);
-                else L.plain = std::max(L.plain, (ng + REDUCE_GROUPS - 1) / REDUCE_GROUPS);
+                int& wgs = (ck.mirror ? L.mirror : L.plain)[ck.kind == KIND_SPLIT16];
+                wgs = std::max(wgs, ck.mirror ? (ng + MIRROR_GROUPS - 1) / MIRROR_GROUPS
+                                              : (ng + REDUCE_GROUPS - 1) / REDUCE_GROUPS);
                 const size_t work = (size_t)ck.M * pl.K / (ck.kind == KIND_SPLIT16 ? 8 : 1);
                 L.operands = std::max(L.operands, (int)std::min<size_t>((work + 255) / 256, 2048));
                 const double fl = 2.0 * (2.0 * (ck.u1 - ck.u0)) * (8.0 * pl.nq) * pl.np;  // useful (unpadded) work
@@ -1316,24 +1344,60 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
         for (size_t c = 0; c < launches[set].size(); ++c) {
             const Launch& L = launches[set][c];
             const ChunkDev* cd = d_chunks + L.table;
-            hipLaunchKernelGGL(k_nf2ff_operands, dim3(L.operands, n, c == 0 && any_split ? 2 : 1), dim3(256), 0, s, fd, cd,
-                               k);
-            for (int kind : {KIND_SPLIT16, KIND_FP32_LARGE, KIND_FP32}) {
-                if (!L.wg[kind]) continue;
+            if (c == 0)
+                hipLaunchKernelGGL(k_nf2ff_operands, dim3(L.operands, n, any_split ? 2 : 1), dim3(256), 0, s, fd, cd, k);
+            auto gemm = [&](int kind, hipStream_t on) -> hipError_t {
+                if (!L.wg[kind]) return hipSuccess;
                 EventPair* ev = nullptr;
                 NF_OK(next_events(&ev));
                 gemm_ev.push_back(ev);
                 gemm_split.push_back(kind == KIND_SPLIT16);
-                NF_OK(hipEventRecord(ev->a, s));
+                NF_OK(hipEventRecord(ev->a, on));
                 const dim3 grid(L.wg[kind]);
-                if (kind == KIND_SPLIT16) hipLaunchKernelGGL(k_hgemm3, grid, dim3(256), 0, s, fd, cd, n);
-                else if (kind == KIND_FP32) hipLaunchKernelGGL(k_sgemm_mfma<64>, grid, dim3(256), 0, s, fd, cd, n);
-                else hipLaunchKernelGGL(k_sgemm_mfma<128>, grid, dim3(256), 0, s, fd, cd, n);
-                NF_OK(hipEventRecord(ev->b, s));
+                if (kind == KIND_SPLIT16) hipLaunchKernelGGL(k_hgemm3, grid, dim3(256), 0, on, fd, cd, n);
+                else if (kind == KIND_FP32) hipLaunchKernelGGL(k_sgemm_mfma<64>, grid, dim3(256), 0, on, fd, cd, n);
+                else hipLaunchKernelGGL(k_sgemm_mfma<128>, grid, dim3(256), 0, on, fd, cd, n);
+                return hipEventRecord(ev->b, on);
+            };
+            // the reductions of some kinds; the next chunk's rows go with the
+            // first of them when asked for
+            auto reduce = [&](int kinds, int mirror, int plain, int rows, hipStream_t on) {
+                const ChunkDev* nx = cd + MAX_FACES;
+                if (mirror) {
+                    hipLaunchKernelGGL(k_nf2ff_reduce_mirror, dim3(std::max(mirror, rows), n, rows ? 2 : 1),
+                                       dim3(MIRROR_THREADS), 0, on, fd, cd, nx, kinds, k);
+                    rows = 0;
+                }
+                if (plain)
+                    hipLaunchKernelGGL(k_nf2ff_reduce, dim3(std::max(plain, rows), n, rows ? 2 : 1), dim3(REDUCE_THREADS), 0,
+                                       on, fd, cd, nx, kinds, k);
+            };
+            const int rows = c + 1 < launches[set].size() ? launches[set][c + 1].operands : 0;
+            const int split = 1 << KIND_SPLIT16, fp32 = 1 << KIND_FP32 | 1 << KIND_FP32_LARGE;
+            // The faces of the small contractions go beside the large ones of
+            // the others (349x349x221 nodes, us per transform with their rows in
+            // launches of their own and one stream / rows with the reductions /
+            // and beside: 181x360 regular angles 490 / 490 / 476, 22500
+            // irregular ones 1313 / 1314 / 1291, 54300 2884 / 2858 / 2820).
+            const bool both = L.wg[KIND_SPLIT16] && (L.wg[KIND_FP32] || L.wg[KIND_FP32_LARGE]);
+            if (both) {
+                if (!C.side) {
+                    NF_OK(hipStreamCreateWithFlags(&C.side, hipStreamNonBlocking));
+                    NF_OK(hipEventCreateWithFlags(&C.fork, hipEventDisableTiming));
+                    NF_OK(hipEventCreateWithFlags(&C.join, hipEventDisableTiming));
+                }
+                NF_OK(hipEventRecord(C.fork, s));
+                NF_OK(hipStreamWaitEvent(C.side, C.fork, 0));
+                NF_OK(gemm(KIND_SPLIT16, s));
+                for (int kind : {KIND_FP32_LARGE, KIND_FP32}) NF_OK(gemm(kind, C.side));
+                reduce(fp32, L.mirror[0], L.plain[0], 0, C.side);
+                NF_OK(hipEventRecord(C.join, C.side));
+                NF_OK(hipStreamWaitEvent(s, C.join, 0));
+                reduce(split, L.mirror[1], L.plain[1], rows, s);
+            } else {
+                for (int kind : {KIND_SPLIT16, KIND_FP32_LARGE, KIND_FP32}) NF_OK(gemm(kind, s));
+                reduce(split | fp32, std::max(L.mirror[0], L.mirror[1]), std::max(L.plain[0], L.plain[1]), rows, s);
             }
-            if (L.mirror)
-                hipLaunchKernelGGL(k_nf2ff_reduce_mirror, dim3(L.mirror, n), dim3(MIRROR_THREADS), 0, s, fd, cd, k);
-            if (L.plain) hipLaunchKernelGGL(k_nf2ff_reduce, dim3(L.plain, n), dim3(REDUCE_THREADS), 0, s, fd, cd, k);
         }
         if (set + 1 < n_sets)
             hipLaunchKernelGGL(k_nf2ff_gather, dim3((unsigned)pblocks), dim3(256), 0, s, fd, n, d_nl, set == 0, n_ang);
