@@ -1773,9 +1773,6 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
             HIP_OK(hipMemcpyAsync(e->exc_samples.as<float>() + off, x.samples, x.n_samples * sizeof(float), hipMemcpyHostToDevice, e->stream));
         off += x.n_samples;
     }
-    if (px.size() * sizeof(PointExc) > e->exc_table.bytes) HIP_OK(e->exc_table.alloc(px.size() * sizeof(PointExc) + 64));
-    if (!px.empty())
-        HIP_OK(hipMemcpyAsync(e->exc_table.p, px.data(), px.size() * sizeof(PointExc), hipMemcpyHostToDevice, e->stream));
 
     // Probe tables.
     // (count0: the probe's samples so far)
@@ -1793,9 +1790,22 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         pp[q].count = x->probe_cnt.as<uint64_t>();
         pp[q].count0 = cnt;
     }
-    if (pp.size() * sizeof(PointProbe) > e->probe_table.bytes) HIP_OK(e->probe_table.alloc(pp.size() * sizeof(PointProbe) + 64));
-    if (!pp.empty())
-        HIP_OK(hipMemcpyAsync(e->probe_table.p, pp.data(), pp.size() * sizeof(PointProbe), hipMemcpyHostToDevice, e->stream));
+    // The batch's tables in one block of device memory, uploaded in one copy
+    // once all is known: step counters, sources, probes, riders and (written by
+    // these) the folded sources' values.
+    auto al64 = [](size_t n) { return (n + 63) & ~(size_t)63; };
+    const size_t exc_at = al64(2 * sizeof(uint64_t)), probe_at = exc_at + al64(px.size() * sizeof(PointExc));
+    const size_t ride_at = probe_at + al64(pp.size() * sizeof(PointProbe)), val_at = ride_at + al64(sizeof(Ride));
+    const size_t tables_len = val_at + MAX_FOLD_SOURCES * sizeof(SourceValue);
+    if (e->batch_tables.bytes < tables_len) HIP_OK(e->batch_tables.alloc(tables_len));
+    char* tables_dev = e->batch_tables.as<char>();
+    const PointExc* exc_dev = reinterpret_cast<const PointExc*>(tables_dev + exc_at);
+    const PointProbe* probe_dev = reinterpret_cast<const PointProbe*>(tables_dev + probe_at);
+    const Ride* ride_dev = reinterpret_cast<const Ride*>(tables_dev + ride_at);
+    uint64_t* step_dev = reinterpret_cast<uint64_t*>(tables_dev);
+    std::vector<char> tables(val_at, 0);
+    if (!px.empty()) std::memcpy(tables.data() + exc_at, px.data(), px.size() * sizeof(PointExc));
+    if (!pp.empty()) std::memcpy(tables.data() + probe_at, pp.data(), pp.size() * sizeof(PointProbe));
     Tiles tl = e->tiles;
     // a float4 lane meets at most one z slab, or lanes are scalar
     if (tl.vec == 4 && !narrow_plane(e->g)) tl = auto_tiles(e->g, 1);
@@ -1931,8 +1941,6 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     // so a run of steps without host work in between (no energy sample, decay
     // check or timed step) is replayed from one captured graph.  The DFTs
     // then form their sample times from the batch's first step.
-    if (e->step_dev.bytes < 2 * sizeof(uint64_t)) HIP_OK(e->step_dev.alloc(2 * sizeof(uint64_t)));
-    uint64_t* step_dev = e->step_dev.as<uint64_t>();  // reset below, once the step scheme is known
     const uint64_t t_batch0 = e->timestep;
     // DFTs of a few signals sampled every step ride; the others are launches,
     // which read the step from the device when all of them sample every step.
@@ -2008,8 +2016,7 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     std::vector<Launch> plan_h = plan;
     const bool step_in_h = !fused && !plan_h.empty();
     if (step_in_h) plan_h[0].a.step_inc = step_dev;
-    HIP_OK(hipMemsetAsync(step_dev, step_in_h ? 0xff : 0, sizeof(uint64_t), e->stream));
-    HIP_OK(hipMemsetAsync(step_dev + 1, 0, sizeof(uint64_t), e->stream));
+    if (step_in_h) std::memset(tables.data(), 0xff, sizeof(uint64_t));
 
     // The riders' table.  The captures ride where every one of them fits; of
     // an extension listed twice one capture holds for both.
@@ -2021,6 +2028,7 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
     for (const auto* x : murs) n_faces += x->mur_faces.size();
     ride_mur = ride_mur && n_faces > 0 && n_faces <= (size_t)MAX_RIDE_MUR;
     int n_ride_h = 0, n_ride_e = 0;
+    bool records = false;  // some rider records E values, a step late
     if (riding) {
         Ride rt{};
         rt.F = e->F;
@@ -2030,14 +2038,11 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         rt.step_a = step_dev;
         rt.step_b = step_dev + 1;
         rt.n_probe = (int)pp.size();
-        rt.probe = e->probe_table.as<PointProbe>();
-        const size_t val_off = (sizeof(Ride) + 63) / 64 * 64;
-        const size_t ride_bytes = val_off + MAX_FOLD_SOURCES * sizeof(SourceValue);
-        if (e->ride_table.bytes < ride_bytes) HIP_OK(e->ride_table.alloc(ride_bytes));
+        rt.probe = probe_dev;
         if (fold_sources) {
             rt.n_src = (int)px.size();
-            rt.src = e->exc_table.as<PointExc>();
-            rt.src_val = reinterpret_cast<SourceValue*>(e->ride_table.as<char>() + val_off);
+            rt.src = exc_dev;
+            rt.src_val = reinterpret_cast<SourceValue*>(tables_dev + val_at);
             for (Launch& L : plan_e) {
                 L.a.src_val = rt.src_val;
                 L.a.n_src = rt.n_src;
@@ -2067,12 +2072,14 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         rt.n_wg = wg;
         n_ride_h = wg;
         n_ride_e = rt.first_ade;
-        HIP_OK(hipMemcpy(e->ride_table.p, &rt, sizeof(Ride), hipMemcpyHostToDevice));
-        plan_h.back().a.ride = plan_e.back().a.ride = e->ride_table.as<Ride>();
+        std::memcpy(tables.data() + ride_at, &rt, sizeof(Ride));
+        records = rt.n_probe + rt.n_dft > 0;
+        plan_h.back().a.ride = plan_e.back().a.ride = ride_dev;
         plan_h.back().a.n_ride = n_ride_h;
         plan_e.back().a.n_ride = n_ride_e;
         plan_e[0].a.step_inc = step_dev + 1;
     }
+    HIP_OK(hipMemcpyAsync(tables_dev, tables.data(), tables.size(), hipMemcpyHostToDevice, e->stream));
 
     // The slab launches of a half-step write other cells than the interior
     // launch and read only the other field (and their own psi), so they run
@@ -2250,8 +2257,8 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         if (host) OE_TRY(run_hooks(3));
         if (point_ops) {
             Timed tm(e, "point_ops");
-            HIP_OK(launch_point_ops(e->F, e->g.N, e->exc_table.as<PointExc>(), fold_sources ? 0 : (int)px.size(), st,
-                                    e->probe_table.as<PointProbe>(), riding ? 0 : (int)pp.size(), e->stream, step_dev));
+            HIP_OK(launch_point_ops(e->F, e->g.N, exc_dev, fold_sources ? 0 : (int)px.size(), st, probe_dev,
+                                    riding ? 0 : (int)pp.size(), e->stream, step_dev));
         }
         for (size_t q = 0; q < dfts.size(); ++q) {
             oe_extension* x = dfts[q];
@@ -2381,7 +2388,7 @@ oe_status oe_engine_run_batch(oe_engine* e, const oe_batch_desc* b, oe_batch_res
         }
     }
     // the last step's E values (nothing follows that would carry them)
-    if (executed && n_ride_e) HIP_OK(launch_ride_last(e->ride_table.as<Ride>(), n_ride_e, e->stream));
+    if (executed && records) HIP_OK(launch_ride_last(ride_dev, n_ride_e, e->stream));
     OE_TRY(drain());
     HIP_OK(hipStreamSynchronize(e->stream));
     if (e->profiling) collect_timing(e);

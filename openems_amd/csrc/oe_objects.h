@@ -146,8 +146,7 @@ struct oe_engine {
     double* energy_host = nullptr;  // pinned
     // point ops
     DevBuf exc_samples;
-    DevBuf step_dev;       // batch-relative step read by the kernels of a step, and steps begun
-    DevBuf ride_table;     // the riders of the running batch (oe_ride.h)
+    DevBuf batch_tables;   // the running batch's step counters, sources, probes and riders (oe_ride.h)
     size_t mix_cells = 75000000;  // most cells of a CPML grid whose slabs and interior share a launch
     int ride = 1;          // probes, small DFTs and captures in the Yee launches: 1 on, 0 off
     int graph_steps = 16;  // steps per captured graph (0: no graphs)
@@ -167,8 +166,6 @@ struct oe_engine {
     int byte_index = 1;
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-    DevBuf exc_table;
-    DevBuf probe_table;
     // profiling: 0 off, n > 0 times every launch of every n-th step
     int profiling = 0;
     bool prof_step = false;
