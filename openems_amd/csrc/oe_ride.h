@@ -78,9 +78,44 @@ __device__ __forceinline__ void mur_pre_cell(const float* __restrict__ F, const 
     m.v_nypp[q] = B[ps] - m.coeff * B[pb];
 }
 
+// Signal m of a DFT: its terms in order, four loaded at a time (one after
+// the other, a term costs the 0.35 us of its two dependent loads).
+__device__ __forceinline__ double dft_signal(const float* __restrict__ F, size_t N, const DftDev& d, int m) {
+    double s = 0.0;
+    uint64_t k = d.off[m];
+    const uint64_t end = d.off[m + 1];
+    for (; k + 4 <= end; k += 4) {
+        double w[4];
+        float f[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            w[q] = d.w[k + q];
+            f[q] = F[(size_t)d.comp[k + q] * N + d.cell[k + q]];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s += w[q] * (double)f[q];
+    }
+    for (; k < end; ++k) s += d.w[k] * (double)F[(size_t)d.comp[k] * N + d.cell[k]];
+    return s;
+}
+
 // Work-group wg (256 lanes) of the riders of an H (h) or E launch.
+//
+// A DFT's two halves ride in different launches, so what each of them does is
+// what its half needs: the half's signals are listed, a phasor is formed once
+// for each frequency, and the (frequency, signal) pairs are those of the list.
+// What bounds it is latency, and a DFT rides on any grid, so this may not take
+// longer than the grid's half-step and a launch of the DFT's own.  us per step
+// at 72x60x32, plain, as a launch / riding with a phasor a pair and a term at a
+// time / in this form: 64 signals of 4 terms at 64 frequencies 18.9 / 30.1 /
+// 13.7, 64 of 32 terms at 10 frequencies 35.2 / 42.9 / 18.6, voltage and
+// current of 4 terms at 64 frequencies 14.4 / 10.4 / 8.5.
 __device__ __forceinline__ void ride(const Ride& r, int wg, bool h) {
-    __shared__ double sv[RIDE_SIGNALS];
+    constexpr int FC = 256;  // frequencies at a time
+    __shared__ double sv[RIDE_SIGNALS];     // the half's signals
+    __shared__ int sig[RIDE_SIGNALS];       // and their numbers
+    __shared__ double ph[FC][2];
+    __shared__ int n_half;
     const int tid = threadIdx.x;
     if (wg >= r.first_ade) {  // H launches only
         if (wg >= r.first_mur) {
@@ -130,21 +165,30 @@ __device__ __forceinline__ void ride(const Ride& r, int wg, bool h) {
     const RideDft& x = r.dft[wg - r.first_dft];
     const DftDev& d = x.d;
     const uint64_t sample = x.sample0 + st;
-    if (tid < d.n_sig && (d.is_h[tid] != 0) != h) {
-        double s = 0.0;
-        for (uint64_t k = d.off[tid]; k < d.off[tid + 1]; ++k)
-            s += d.w[k] * (double)r.F[(size_t)d.comp[k] * r.g.N + d.cell[k]];
-        if (d.series && sample < d.series_cap) d.series[sample * d.n_sig + tid] = s;
-        sv[tid] = s;
+    if (tid < 64) {  // RIDE_SIGNALS lanes, one wave
+        const bool mine = tid < d.n_sig && (d.is_h[tid] != 0) != h;
+        const unsigned long long all = __ballot(mine);
+        if (tid == 0) n_half = __popcll(all);
+        if (mine) {
+            const int at = __popcll(all & ((1ull << tid) - 1));
+            const double s = dft_signal(r.F, r.g.N, d, tid);
+            if (d.series && sample < d.series_cap) d.series[sample * d.n_sig + tid] = s;
+            sv[at] = s;
+            sig[at] = tid;
+        }
     }
-    __syncthreads();
     const double t = (r.t0 + (double)st + (h ? 1.0 : 0.5)) * r.dt;
-    for (int q = tid; q < d.n_f * d.n_sig; q += 256) {
-        const int f = q / d.n_sig, m = q - f * d.n_sig;
-        if ((d.is_h[m] != 0) == h) continue;
-        double c, s;
-        dft_phasor(d.freqs[f], t, c, s);
-        dft_add(d, (size_t)q, sv[m], c, s);
+    for (int f0 = 0; f0 < d.n_f; f0 += FC) {
+        const int nf = min(FC, d.n_f - f0);
+        if (f0) __syncthreads();  // the phasors before are read
+        const int p = nf <= 128 ? tid - 128 : tid;  // waves that have no signals, where they hold all
+        if (p >= 0 && p < nf) dft_phasor(d.freqs[f0 + p], t, ph[p][0], ph[p][1]);
+        __syncthreads();
+        const int n = n_half;
+        for (int q = tid; q < nf * n; q += 256) {
+            const int f = q / n, g = q - f * n;
+            dft_add(d, (size_t)(f0 + f) * d.n_sig + sig[g], sv[g], ph[f][0], ph[f][1]);
+        }
     }
 }
 #endif  // __HIPCC__
