@@ -3,6 +3,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <cstddef>
 
 namespace oe {
@@ -48,6 +49,13 @@ inline bool narrow_plane(const Grid& g) { return ((size_t)g.ny + 2) * g.nz < ((s
 // single launch takes one or two (oe_engine_run_batch).
 // Scalar lanes, whose planes are cheaper than their start, take two
 // (151x133x117 with CPML, ci 1 / 2 / 3: 82.5 / 75.0 / 81.0).
+//
+// Where a plane fills less than half of its work-groups' lanes, the start of a
+// work-group costs more than the plane it works on, and the depth that pays
+// grows as the square root of the work-groups (ci 1 or 2 / this: 100000x4x4
+// 312 / 98, 100000x8x8 329 / 119, 20000x16x16 82 / 63, 1000x2x1000 30.5 / 28.7).
+// No grid is cut into more than 2^23 work-groups of its tiles: a launch holds
+// 2^32 lanes.
 inline Tiles auto_tiles(const Grid& g, int vec_req) {
     Tiles t{};
     t.vec = vec_req == 1 || (g.nz % 4 != 0 && g.nz < 8) || !narrow_plane(g) ? 1 : 4;
@@ -64,8 +72,13 @@ inline Tiles auto_tiles(const Grid& g, int vec_req) {
         }
     }
     t.by = 256 / t.bx;
+    const int n_kb = (nzv + t.bx - 1) / t.bx;
     const int ci4 = g.N <= 12000000 ? 1 : (t.bx <= 32 && nzv > 64) ? 4 : 2;
-    t.ci = std::min(g.nx, t.vec == 4 ? ci4 : 2);
+    int ci = t.vec == 4 ? ci4 : 2;
+    const double blocks = (double)n_kb * ((g.ny + t.by - 1) / t.by);  // work-groups of a plane
+    if ((double)nzv * g.ny < 128.0 * blocks) ci = std::max(ci, (int)(std::sqrt(blocks * g.nx) / 16));
+    ci = std::max(ci, (int)std::ceil(blocks * g.nx / (1 << 23)));
+    t.ci = std::min(g.nx, ci);
     return t;
 }
 

@@ -679,6 +679,12 @@ __device__ __forceinline__ void e_body(const Grid& g, const float* Fin, float* F
     int ly = 0, lz = 0;
     int fy = -1, fz = -1;
     if constexpr ((AX & AX_Y) != 0) fy = live ? face_of(c, 1, j, ly) : -1;
+    if constexpr (AX == 0 && !MUR) {  // rows of j = 0 keep their value: nothing to do where there are no others
+        if (ny == 1 && !copy_all) {
+            if constexpr (R::late) rows.fill();
+            return;
+        }
+    }
     const bool ony = (AX & AX_Y) != 0 && any_lane<AX>(fy >= 0);
     if constexpr ((AX & AX_Z) != 0) fz = live ? zface_of<V, RAG>(c, k0, lz) : -1;
     const int nv = RAG ? min(V, nz - k0) : V;  // the lane's cells

@@ -6,6 +6,7 @@ import pytest
 
 from openems_amd import MODE_PHYSICAL, CpmlBoundaries, EngineBatch, HipEngine, Operator, ScheduledExcitation
 from openems_amd._ffi import OEError
+from tests.parity_util import Scenario, assert_parity, gauss_ref, run_pair
 
 pytestmark = pytest.mark.gpu
 
@@ -53,3 +54,18 @@ def test_shapes_no_work_group_holds_are_refused():
         assert eng.tiles() == before
     with pytest.raises(OEError):  # rows too short for float4 lanes
         _engine((24, 20, 7)).set_tiles(vec=4)
+
+
+@pytest.mark.parametrize("shape", [(4, 1, 300), (4, 2, 256), (3, 5, 512), (5, 3, 262), (2500, 4, 4), (3000, 3, 2), (700, 2, 40)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("absorber", ["none", "cpml"])
+def test_waves_of_first_rows_and_deep_marches(shape, absorber):
+    """Waves that hold only rows of j = 0, which the E update leaves alone, and
+    thin planes marched many at a time, against the oracle bit for bit."""
+    src = tuple(m // 2 for m in shape)
+    layers = [min(3, (shape[f // 2] - 1) // 2) for f in range(6)]
+    sc = Scenario(f"rows_{absorber}_{'x'.join(map(str, shape))}", shape, 1e-3, 30,
+                  materials=[(4.0, 1.0, 0.02, 0.0, (0, max(1, shape[0] // 2), 0, shape[1], 0, max(1, shape[2] // 2)))],
+                  excitations=[(src, 2, True, gauss_ref(20e9)), ((0, 0, 0), 1, True, gauss_ref(25e9))], probes=[src],
+                  cpml=dict(layers=layers, mode=MODE_PHYSICAL) if absorber == "cpml" else None)
+    assert_parity(run_pair(sc), sc.name)

@@ -52,3 +52,31 @@ def test_wide_planes_take_scalar_lanes(rules):
         fits = (ny + 2) * nz * 4 < 2 ** 32
         assert (r["vec"], r["sweep"]) == ((4, 4) if fits else (1, 1)), (ny, nz)
         assert r["sweep_ragged"] == 1
+
+
+def _work_groups(shape, r):
+    nx, ny, nz = shape
+    lanes = -(-nz // r["vec"])
+    return -(-lanes // r["bx"]) * -(-ny // r["by"]) * -(-nx // r["ci"])
+
+
+def test_every_cell_has_a_lane_and_every_launch_fits(rules):
+    """bx by at most 256 lanes, and no more lanes in a launch than 2^32 hold,
+    on grids of any proportion up to 2^32 cells."""
+    shapes = [(1 << 30, 1, 1), (1 << 25, 1, 1), (1 << 28, 2, 4), (1 << 29, 1, 5), (300_000_000, 3, 3), (40_000_000, 1, 64), (1, 1, 1),
+              (1 << 20, 64, 64), (512, 512, 512), (1 << 26, 8, 4), (1 << 16, 1 << 8, 1 << 8), (3, 1 << 29, 2), (2, 2, 1 << 30)]
+    for s, r in zip(shapes, rules(*shapes)):
+        assert 1 <= r["bx"] and 1 <= r["by"] and r["bx"] * r["by"] <= 256 and 1 <= r["ci"] <= s[0], (s, r)
+        assert _work_groups(s, r) * 256 < 2 ** 32, (s, r)
+
+
+def test_nearly_empty_planes_are_marched_deep(rules):
+    """Planes that fill less than half of their lanes: no more than a few
+    thousand work-groups for each sixteenfold depth; full ones as before."""
+    thin = [(100_000, 4, 4), (1_000_000, 1, 1), (20_000, 16, 16), (2000, 1, 2000), (100_000, 8, 8), (200_000, 2, 2)]
+    for s, r in zip(thin, rules(*thin)):
+        assert r["ci"] > 2 and _work_groups(s, r) <= 20_000, (s, r)
+    full = [((100, 100, 100), 1), ((144, 144, 144), 1), ((256, 256, 256), 2), ((512, 512, 512), 2), ((64, 64, 64), 1), ((256, 320, 384), 4),
+            ((2000, 4, 1000), 1), ((5000, 32, 32), 1)]
+    for (s, ci), r in zip(full, rules(*(s for s, _ in full))):
+        assert r["ci"] == ci, (s, r)
