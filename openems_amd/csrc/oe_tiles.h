@@ -38,7 +38,10 @@ inline bool narrow_plane(const Grid& g) { return ((size_t)g.ny + 2) * g.nz < ((s
 // of two left lanes idle on most grids: us per step at 100^3 (25 lanes)
 // 32 / 25 lanes 13.9 / 11.9; 128x192x320 (80 lanes) 64 / 40 lanes 120 / 94;
 // 256x320x384 (96 lanes) 64 / 32 lanes 466 / 426, with CPML 568 / 497; scalar
-// 200x201x75 64 / 75 lanes 84.6 / 64.3.
+// 200x201x75 64 / 75 lanes 84.6 / 64.3.  Parts of a row are widened to a
+// multiple of 8 lanes where as many rows still fit: a wave of 63 lanes' parts
+// straddles two rows (200x200x1000, 63 / 64 lanes 632 / 596; 2000x18x2000 with
+// CPML 1551 / 1428).
 //
 // ci: one plane up to 12 M cells, where more work-groups and a shorter chain
 // of loads count (plain, us per step at ci 1 / 2 / 4: 64^3 8.0 / 9.3 / 12.2,
@@ -73,6 +76,7 @@ inline Tiles auto_tiles(const Grid& g, int vec_req) {
     }
     t.by = 256 / t.bx;
     const int n_kb = (nzv + t.bx - 1) / t.bx;
+    if (n_kb > 1) t.bx = std::max(t.bx, 256 / t.by / 8 * 8);
     const int ci4 = g.N <= 12000000 ? 1 : (t.bx <= 32 && nzv > 64) ? 4 : 2;
     int ci = t.vec == 4 ? ci4 : 2;
     const double blocks = (double)n_kb * ((g.ny + t.by - 1) / t.by);  // work-groups of a plane

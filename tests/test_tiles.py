@@ -80,3 +80,12 @@ def test_nearly_empty_planes_are_marched_deep(rules):
             ((2000, 4, 1000), 1), ((5000, 32, 32), 1)]
     for (s, ci), r in zip(full, rules(*(s for s, _ in full))):
         assert r["ci"] == ci, (s, r)
+
+
+def test_row_parts_hold_whole_eighths_where_rows_still_fit(rules):
+    shapes = [(200, 200, 1000), (256, 320, 384), (128, 192, 320), (150, 150, 400), (64, 64, 520), (100, 100, 100), (40, 40, 3000)]
+    want = [(64, 4), (32, 8), (40, 6), (50, 5), (None, None), (25, 10), (64, 4)]
+    for s, w, r in zip(shapes, want, rules(*shapes)):
+        parts = -(-(-(-s[2] // r["vec"])) // r["bx"])
+        assert w[0] is None or (r["bx"], r["by"]) == w, (s, r)
+        assert r["by"] == 256 // r["bx"] and (parts == 1 or r["bx"] % 8 == 0 or (r["bx"] // 8 + 1) * 8 * r["by"] > 256), (s, r)
