@@ -1095,6 +1095,11 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
     bool mirror = true;
     if (const char* v = getenv("OE_NF2FF_MIRROR")) mirror = atoi(v) != 0;
 
+    // faces of small contractions on a side stream beside the large ones unless
+    // OE_NF2FF_STREAMS=1
+    bool beside = true;
+    if (const char* v = getenv("OE_NF2FF_STREAMS")) beside = atoi(v) != 1;
+
     // per face: first-contraction axis p (fewer distinct |kappa|), sizes
     struct Plan {
         int p, q, np, nq, K, N, swap, need, rows, chunk, n_chunks;  // need: rows of all of U, rows: of one chunk
@@ -1379,7 +1384,7 @@ hipError_t nf2ff_compute(const std::vector<Nf2ffFace>& faces, double freq, const
             // launches of their own and one stream / rows with the reductions /
             // and beside: 181x360 regular angles 490 / 490 / 476, 22500
             // irregular ones 1313 / 1314 / 1291, 54300 2884 / 2858 / 2820).
-            const bool both = L.wg[KIND_SPLIT16] && (L.wg[KIND_FP32] || L.wg[KIND_FP32_LARGE]);
+            const bool both = beside && L.wg[KIND_SPLIT16] && (L.wg[KIND_FP32] || L.wg[KIND_FP32_LARGE]);
             if (both) {
                 if (!C.side) {
                     NF_OK(hipStreamCreateWithFlags(&C.side, hipStreamNonBlocking));

@@ -73,5 +73,7 @@ def test_chunks_of_rows(monkeypatch, split, kind):
                     / (np.linalg.norm(Et) ** 2 + np.linalg.norm(Ep) ** 2))
     say(f"[nf2ff] {kind} {g.e_theta.shape}, split {split}: rel L2 {err:.2e}; {g.total_ms:.3f} ms")
     assert err <= PATTERN_TOL and abs(g.prad - prad) <= 1e-12 * abs(prad)
-    again = nf.calculate(th, ph)
-    assert np.array_equal(again.e_theta, g.e_theta) and np.array_equal(again.e_phi, g.e_phi)
+    for streams in ("2", "1"):  # with the small contractions beside the large ones, and after them
+        monkeypatch.setenv("OE_NF2FF_STREAMS", streams)
+        again = nf.calculate(th, ph)
+        assert np.array_equal(again.e_theta, g.e_theta) and np.array_equal(again.e_phi, g.e_phi)
