@@ -252,7 +252,9 @@ oe_status oe_engine_run_batch(oe_engine* eng, const oe_batch_desc* batch, oe_bat
  * "update_e:grid" (one launch over the grid), or "update_h:interior" /
  * "update_h:slabs" and the "update_e:" pair (CPML in two launches: interior
  * box with z-face CPML, x/y face slabs with all faces), "mur_pre", "mur_post", "ade_pre", "ade_post",
- * "point_ops", "energy".  Returns the launch count and total milliseconds. */
+ * "point_ops", "energy".  Work that rides in the Yee launches (small DFTs and
+ * probes, the Mur and ADE captures, source values) has no name of its own: its
+ * time is theirs.  Returns the launch count and total milliseconds. */
 oe_status oe_engine_kernel_time(oe_engine* eng, const char* name, uint64_t* launches, double* total_ms);
 
 /* Per-launch event timing: 0 off (default); n > 0 records HIP events around
